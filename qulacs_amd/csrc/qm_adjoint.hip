@@ -8,79 +8,60 @@
 // gradient is Re <bistate| R(theta + pi) |state> / 2 = -Im <lambda|P|psi> with
 // lambda = H|psi> (the reference's bistate is 2 lambda).  The reference spends
 // a state copy, a gate and an inner product per parameter (about three passes)
-// plus two more passes for the inverses.  Here the gates are grouped into
-// passes over blocks of K = 3 qubits: a pass keeps the 8 amplitudes of psi
-// (and of lambda on the way back) that differ only in its block qubits in
-// registers and runs a contiguous run of gates on them -- every gate whose
-// non-diagonal qubits lie in the block (rotations with their X/Y qubits in it,
-// dense gates on block qubits) and every diagonal gate (CZ, Z rotations, diagonal
-// matrices) wherever its qubits are, since an outside bit is fixed per thread.
-// Forward, a pass applies its gates in order; backward, in reverse order it
-// adds each rotation's term -Im <lambda|P|psi> and applies the inverse to both
-// states.  A hardware-efficient layer on 20 qubits (RY, RZ on every qubit, a CZ
-// chain) is 7 passes instead of 59 per-gate passes.  H|psi> with <psi|H|psi>
-// is one kernel over all terms.
+// plus two more passes for the inverses.
 //
-// Layout: `batch` states of 2^n complex128 each, contiguous (state b at
-// b * 2^n); theta is batch x params (row-major).  Every reduction is written
-// as per-block partial sums and summed in a fixed order at the end, so the
-// results do not depend on scheduling.
-#include <algorithm>
-#include <cmath>
-#include <vector>
-
-#include "qm_internal.hpp"
+// Here every gate becomes single-qubit operations, CZ gates and 4 x 4 matrices,
+// and the tile engine (qm_tile.hpp) runs them stage by stage on tiles in LDS:
+//   * a rotation about a Pauli string of several qubits is one RX between CZ gates
+//     to its other qubits (CZ_{a,t} X_t CZ_{a,t} = X_t Z_a), after fixed
+//     single-qubit changes of basis; CNOT is H CZ H;
+//   * consecutive single-qubit gates on one qubit are one operation U = F_m ... F_1.
+//     Its 2 x 2 matrix depends on the parameter set: k_adj_mats forms U and U^dagger
+//     of every operation and set once per call;
+//   * backward, the three numbers s_P = Im <lambda|P|psi>, P in {X, Y, Z} on the
+//     operation's qubit after U, give the gradient of every rotation inside U: for
+//     F_j = exp(i a P_j / 2) it is -sum_P g_P s_P with F_m..F_{j+1} P_j
+//     (F_m..F_{j+1})^dagger = g_X X + g_Y Y + g_Z Z (k_adj_mats forms g).  A fused
+//     RZ RY costs 12 multiply-adds per amplitude pair for its two gradients.
+//
+// Layout: `batch` states of 2^max(n, 4) complex128 each, contiguous (state b at
+// b * dim); theta is batch x params (row-major).  Every reduction is a fixed-order
+// sum of partial sums, so the results do not depend on scheduling, and a parameter
+// set's result does not depend on the batch it is in.
+#include "qm_tile.hpp"
 
 namespace qm {
 namespace {
 
-constexpr int kAdjThreads = 256;
-constexpr unsigned kAdjBlocks = 64;  // blocks per state per launch (grid-stride)
+constexpr int kAdjK = 3;             // block qubits of a pass: 8 amplitudes of psi and of lambda per thread
+constexpr u32 kAdjLow = 3;           // qubits 0..2 are in every window: 128-byte runs
+constexpr u32 kFwdLocal = 12;        // forward window: 64 KiB of psi
+constexpr u32 kBwdLocal = 11;        // backward window: 32 KiB of psi and 32 KiB of lambda
+constexpr u32 kFwdThreads = 1u << (kFwdLocal - kAdjK);
+constexpr u32 kBwdThreads = 1u << (kBwdLocal - kAdjK);
+constexpr u32 kStageGrads = 64;      // operations with gradients per backward stage (LDS sums)
+constexpr u64 kBwdMaxBlocks = 4096;  // work-groups per state of a backward stage (more tiles: several each)
+constexpr u32 kHpsiThreads = 256;
+constexpr u32 kHpsiMaxBlocks = 512;
 
-struct AdjGate {
-    u32 kind;  // 0 fixed dense (k <= 2), 1 rotation
-    u32 k;
-    u32 q[2];
-    double2 m[16];      // fixed: matrix (row-major, bit i <-> q[i])
-    u64 bf, pf;         // rotation: Pauli masks
-    u32 rot, pivot;
-    u32 param, occ;     // rotation: parameter index, occurrence slot
-    double coef;
+// One factor of a single-qubit operation.
+struct Factor {
+    u32 kind;    // 0: fixed matrix, 1 / 2 / 3: exp(i a P / 2) with P = X / Y / Z
+    u32 fixed;   // kind 0: offset into the fixed-matrix pool
+    u32 param;   // rotation: parameter index
+    u32 occ;     // rotation: occurrence number
+    double coef; // rotation: a = coef * theta[param]
 };
 
 struct AdjTerm {
-    u64 bf, pf;
+    u64 pf;
     u32 rot, pad;
     double coef;
 };
-
-constexpr int kPassQubits = 3;            // block qubits per pass
-constexpr int kPassRots = 16;             // rotations per pass (LDS accumulators)
-
-// One gate inside a pass, in the pass's terms.  Member bit j of a tuple is
-// block qubit blk[j] (ascending); bits outside the block come from the tuple's
-// base index.
-struct PassOp {
-    u32 type;          // 0 rotation, 1 dense on one block bit, 2 dense on two block bits, 3 diagonal
-    u32 lbf, lpf;      // rotation: flip / phase masks over member bits
-    u64 opf;           // rotation: phase mask over qubits outside the block
-    u32 rot;           // rotation: number of Y factors (P = i^rot X^bf Z^pf)
-    u32 slot;          // rotation: index among the pass's rotations
-    u32 occ;           // rotation: occurrence (partials row)
-    u32 a, b;          // dense: member bits (matrix bit 0 <-> a, bit 1 <-> b)
-    u32 dk;            // diagonal: number of qubits (1 or 2)
-    u32 dloc[2];       // diagonal: member bit, or 255 for a qubit outside the block
-    u32 dpos[2];       // diagonal: qubit position when outside the block
-    double2 m[16];     // dense matrix (row-major) or the diagonal's entries
-};
-
-struct PassArgs {
-    u64 offs[1 << kPassQubits];  // offset of member m
-    unsigned char blk[kPassQubits];
-    u32 op0, nops;               // ops[op0 .. op0 + nops)
-    u32 nrot;
-    u32 param[kPassRots];        // rotation slot -> parameter
-    double coef[kPassRots];      // rotation slot -> coefficient
+// terms [term0, term0 + nterm) share the bit-flip mask bf
+struct AdjGroup {
+    u64 bf;
+    u32 term0, nterm;
 };
 
 __device__ __forceinline__ double2 ipow(double2 z, u32 k) {  // z * i^k
@@ -92,346 +73,318 @@ __device__ __forceinline__ double2 ipow(double2 z, u32 k) {  // z * i^k
     }
 }
 
-__global__ __launch_bounds__(kAdjThreads) void k_adj_zero(double2* __restrict__ s, u64 dim) {
-    double2* st = s + (u64)blockIdx.y * dim;
-    for (u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x; i < dim; i += (u64)gridDim.x * blockDim.x)
-        st[i] = make_double2(i == 0 ? 1.0 : 0.0, 0.0);
+// out <- a b, 2 x 2 complex
+__device__ __forceinline__ void mul2(double2 (&out)[4], const double2 (&a)[4], const double2 (&b)[4]) {
+    double2 r[4];
+    r[0] = cmac(cmul(a[0], b[0]), a[1], b[2]);
+    r[1] = cmac(cmul(a[0], b[1]), a[1], b[3]);
+    r[2] = cmac(cmul(a[2], b[0]), a[3], b[2]);
+    r[3] = cmac(cmul(a[2], b[1]), a[3], b[3]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[i] = r[i];
 }
 
-// Fixed gate (dense on 1 or 2 qubits) applied as M (INV = false) or M^dagger,
-// to psi and, when TWO, to lambda as well.
-template <bool INV, bool TWO>
-__global__ __launch_bounds__(kAdjThreads) void k_adj_fixed(double2* __restrict__ psi, double2* __restrict__ lam,
-                                                           u64 dim, AdjGate g) {
-    const u64 off = (u64)blockIdx.y * dim;
-    double2 m[16];
-    const u32 d = 1u << g.k;
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            if ((u32)r >= d || (u32)c >= d) continue;
-            m[r * 4 + c] = INV ? cconj(g.m[c * d + r]) : g.m[r * d + c];
-        }
-    const u64 groups = dim >> g.k;
-    for (u64 t = (u64)blockIdx.x * blockDim.x + threadIdx.x; t < groups; t += (u64)gridDim.x * blockDim.x) {
-        if (g.k == 1) {
-            const u64 b0 = insert_zero(t, g.q[0]), b1 = b0 | (1ULL << g.q[0]);
-#pragma unroll
-            for (int w = 0; w < (TWO ? 2 : 1); ++w) {
-                double2* s = (w ? lam : psi) + off;
-                const double2 x = s[b0], y = s[b1];
-                s[b0] = cmac(cmul(m[0], x), m[1], y);
-                s[b1] = cmac(cmul(m[4], x), m[5], y);
-            }
-        } else {
-            const u32 lo = min(g.q[0], g.q[1]), hi = max(g.q[0], g.q[1]);
-            const u64 b = insert_zero(insert_zero(t, lo), hi);
-            const u64 i0 = b, i1 = b | (1ULL << g.q[0]), i2 = b | (1ULL << g.q[1]), i3 = i1 | i2;
-#pragma unroll
-            for (int w = 0; w < (TWO ? 2 : 1); ++w) {
-                double2* s = (w ? lam : psi) + off;
-                const double2 a0 = s[i0], a1 = s[i1], a2 = s[i2], a3 = s[i3];
-                s[i0] = cmac(cmac(cmac(cmul(m[0], a0), m[1], a1), m[2], a2), m[3], a3);
-                s[i1] = cmac(cmac(cmac(cmul(m[4], a0), m[5], a1), m[6], a2), m[7], a3);
-                s[i2] = cmac(cmac(cmac(cmul(m[8], a0), m[9], a1), m[10], a2), m[11], a3);
-                s[i3] = cmac(cmac(cmac(cmul(m[12], a0), m[13], a1), m[14], a2), m[15], a3);
-            }
-        }
+// The matrices of every single-qubit operation for every parameter set: U into the
+// forward pool, U^dagger into the backward pool, and per rotation occurrence the
+// vector g (see the file comment).  blockIdx.y = set; one thread per operation.
+// `copies` lists the pool entries that do not depend on the set (4 x 4 matrices).
+struct MatsArgs {
+    const Factor* factors;
+    const u32* first;      // factors [first[o], first[o + 1]) of operation o, in gate order
+    const double2* fixed;  // fixed factors' matrices
+    const u32* fwd_at;     // pool offsets of operation o's matrix
+    const u32* bwd_at;
+    const u32* copies;     // ncopy_f forward offsets, then ncopy_b backward offsets
+    const double2* copy_val;
+    u32 nops, ncopy_f, ncopy_b, nparams, nocc;
+    u32 fwd_stride, bwd_stride;
+};
+__global__ __launch_bounds__(64) void k_adj_mats(MatsArgs a, const double* __restrict__ theta, double2* __restrict__ fwd,
+                                                 double2* __restrict__ bwd, double* __restrict__ gvec) {
+    const u32 set = blockIdx.y, o = blockIdx.x * blockDim.x + threadIdx.x;
+    double2* pf = fwd + (u64)set * a.fwd_stride;
+    double2* pb = bwd + (u64)set * a.bwd_stride;
+    if (o >= a.nops) {
+        const u32 c = o - a.nops;
+        if (c < a.ncopy_f) pf[a.copies[c]] = a.copy_val[c];
+        else if (c < a.ncopy_f + a.ncopy_b) pb[a.copies[c]] = a.copy_val[c];
+        return;
     }
+    // u = F_m ... F_{j+1} while the factors are walked from the last to the first
+    double2 u[4] = {make_double2(1, 0), make_double2(0, 0), make_double2(0, 0), make_double2(1, 0)};
+    for (u32 j = a.first[o + 1]; j-- > a.first[o];) {
+        const Factor f = a.factors[j];
+        // m = c I + i s P for a rotation about P = X, Y or Z (px, py, pz); selected without
+        // branches
+        const double px = f.kind == 1 ? 1.0 : 0.0, py = f.kind == 2 ? 1.0 : 0.0, pz = f.kind == 3 ? 1.0 : 0.0;
+        double2 m[4];
+        if (f.kind == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) m[i] = a.fixed[f.fixed + i];
+        } else {
+            // u P u^dagger = [[g_Z, g_X - i g_Y], [g_X + i g_Y, -g_Z]], from its entries (0, 0) and (1, 0)
+            const double2 c0 = cconj(u[0]), c1 = cconj(u[1]);
+            const double2 z20 = cmul(u[2], c0), z21 = cmul(u[2], c1), z30 = cmul(u[3], c0), z31 = cmul(u[3], c1);
+            const double2 z01 = cmul(u[0], c1);
+            const double n0 = u[0].x * u[0].x + u[0].y * u[0].y, n1 = u[1].x * u[1].x + u[1].y * u[1].y;
+            double* g = gvec + ((u64)set * a.nocc + f.occ) * 3;
+            g[0] = px * (z30.x + z21.x) - py * (z30.y - z21.y) + pz * (z20.x - z31.x);
+            g[1] = px * (z30.y + z21.y) + py * (z30.x - z21.x) + pz * (z20.y - z31.y);
+            g[2] = 2.0 * (px * z01.x + py * z01.y) + pz * (n0 - n1);
+            const double ang = 0.5 * (f.coef * theta[(u64)set * a.nparams + f.param]);
+            const double c = cos(ang), s = sin(ang);
+            m[0] = make_double2(c, s * pz);
+            m[1] = make_double2(s * py, s * px);
+            m[2] = make_double2(-(s * py), s * px);
+            m[3] = make_double2(c, -(s * pz));
+        }
+        mul2(u, u, m);
+    }
+    double2* uf = pf + a.fwd_at[o];
+    double2* ub = pb + a.bwd_at[o];
+    uf[0] = u[0]; uf[1] = u[1]; uf[2] = u[2]; uf[3] = u[3];
+    ub[0] = cconj(u[0]); ub[1] = cconj(u[2]); ub[2] = cconj(u[1]); ub[3] = cconj(u[3]);
 }
 
-// Rotation exp(i a P / 2), a = coef * theta[b][param].  FORWARD applies it to
-// psi.  Otherwise (backward) the block adds -Im <lambda|P|psi> over its
-// amplitudes to partials[(occ * batch + b) * gridDim.x + blockIdx.x] and then
-// applies exp(-i a P / 2) to psi and lambda.
-template <bool FORWARD>
-__global__ __launch_bounds__(kAdjThreads) void k_adj_rot(double2* __restrict__ psi, double2* __restrict__ lam,
-                                                         u64 dim, AdjGate g, const double* __restrict__ theta,
-                                                         u32 nparams, double* __restrict__ partials) {
-    __shared__ double red[32];
-    const u32 b = blockIdx.y;
-    const u64 off = (u64)b * dim;
-    const double a = g.coef * theta[(u64)b * nparams + g.param];
-    const double c = cos(0.5 * a), sn = FORWARD ? sin(0.5 * a) : -sin(0.5 * a);
-    double acc = 0.0;
-    double2* P = psi + off;
-    double2* Lm = lam + off;
-    const u64 stride = (u64)gridDim.x * blockDim.x;
-    if (g.bf == 0) {
-        // diagonal: (P psi)_x = s_x psi_x with s_x = i^rot (-1)^popcount(x & pf)
-        for (u64 x = (u64)blockIdx.x * blockDim.x + threadIdx.x; x < dim; x += stride) {
-            const double2 ph = ipow(make_double2((__popcll(x & g.pf) & 1) ? -1.0 : 1.0, 0.0), g.rot);
-            const double2 v = P[x];
-            const double2 pv = cmul(ph, v);
-            if (!FORWARD) {
-                const double2 l = Lm[x];
-                acc -= l.x * pv.y - l.y * pv.x;  // -Im(conj(l) * pv)
-            }
-            // (c + i sn ph) v
-            const double2 f = make_double2(c - sn * ph.y, sn * ph.x);
-            P[x] = cmul(f, v);
-            if (!FORWARD) Lm[x] = cmul(f, Lm[x]);
+// One forward stage: a work-group per tile (blockIdx.x) and set (blockIdx.y).  Two
+// groups of 64 KiB share a CU, so one's loads and stores overlap the other's passes.
+// `first`: the tile is a part of |0...0>, nothing is read.
+__global__ __launch_bounds__(kFwdThreads, 4) void k_adj_fwd(double2* __restrict__ psi, u32 n, u32 lq, u32 first,
+                                                            DStage sg, const DPass* __restrict__ passes,
+                                                            const DSub* __restrict__ subs,
+                                                            const double2* __restrict__ pool, u32 stride) {
+    extern __shared__ double2 st[];
+    __shared__ u64 hi_tab[1u << (kFwdLocal - kAdjLow)];
+    const u32 L = 1u << lq, T = blockDim.x;
+    double2* s = psi + ((u64)blockIdx.y << n);
+    build_hi_tab<kAdjLow>(hi_tab, lq, sg);
+    const u64 tb = tile_base(blockIdx.x, n - lq, sg);
+    __syncthreads();
+    if (first) {
+        for (u32 i = threadIdx.x; i < L; i += T)
+            st[slot_of(i)] = make_double2(i == 0 && blockIdx.x == 0 ? 1.0 : 0.0, 0.0);
+    } else if (L == 8 * kFwdThreads) {
+#pragma unroll
+        for (u32 k = 0; k < 8; ++k) {
+            const u32 i = threadIdx.x + k * kFwdThreads;
+            st[slot_of(i)] = s[tile_index<kAdjLow>(tb, hi_tab, i)];
         }
     } else {
-        const u64 half = dim >> 1;
-        for (u64 t = (u64)blockIdx.x * blockDim.x + threadIdx.x; t < half; t += stride) {
-            const u64 x = insert_zero(t, g.pivot), y = x ^ g.bf;
-            // P|y> = i^rot (-1)^popcount(y & pf) |x>, P|x> = i^rot (-1)^popcount(x & pf) |y>
-            const double sy = (__popcll(y & g.pf) & 1) ? -1.0 : 1.0, sx = (__popcll(x & g.pf) & 1) ? -1.0 : 1.0;
-            const double2 px = ipow(make_double2(sy, 0.0), g.rot);  // coefficient of psi_y in (P psi)_x
-            const double2 py = ipow(make_double2(sx, 0.0), g.rot);  // coefficient of psi_x in (P psi)_y
-            const double2 vx = P[x], vy = P[y];
-            const double2 ppx = cmul(px, vy), ppy = cmul(py, vx);
-            if (!FORWARD) {
-                const double2 lx = Lm[x], ly = Lm[y];
-                acc -= (lx.x * ppx.y - lx.y * ppx.x) + (ly.x * ppy.y - ly.y * ppy.x);
-                // inverse on lambda: c l + i sn (P l)
-                const double2 qx = cmul(px, ly), qy = cmul(py, lx);
-                Lm[x] = make_double2(c * lx.x - sn * qx.y, c * lx.y + sn * qx.x);
-                Lm[y] = make_double2(c * ly.x - sn * qy.y, c * ly.y + sn * qy.x);
-            }
-            P[x] = make_double2(c * vx.x - sn * ppx.y, c * vx.y + sn * ppx.x);
-            P[y] = make_double2(c * vy.x - sn * ppy.y, c * vy.y + sn * ppy.x);
-        }
+        for (u32 i = threadIdx.x; i < L; i += T) st[slot_of(i)] = s[tile_index<kAdjLow>(tb, hi_tab, i)];
     }
-    if (!FORWARD) {
-        acc = block_sum(acc * g.coef, red);  // d/dtheta = coef * d/da
-        if (threadIdx.x == 0) partials[((u64)g.occ * gridDim.y + b) * gridDim.x + blockIdx.x] = acc;
-    }
-}
-
-// ---------------------------------------------------------------- pass kernel
-constexpr int kPassN = 1 << kPassQubits;
-
-// exp(+-i a P / 2) on the tuple, P's flip part LBF known at compile time so
-// every register index is a constant.  (P v)_y = i^rot (-1)^(so + |x & lpf|) v_x
-// with x = y ^ LBF.  BACK: first acc += -Im sum_y conj(l_y) (P v)_y, then the
-// inverse on v and l.
-template <int LBF, bool BACK>
-__device__ __forceinline__ void rot_apply(double2* v, double2* l, u32 lpf, u32 rot, u32 so, double c, double sn,
-                                          double& acc) {
-#pragma unroll
-    for (int y = 0; y < kPassN; ++y) {
-        const int x = y ^ LBF;
-        if (LBF != 0 && x < y) continue;  // pairs handled once, from their lower member
-        // factors of P: (P v)_y = fy * v_x, (P v)_x = fx * v_y
-        const u32 sy = (so + __popc((u32)x & lpf)) & 1u, sx = (so + __popc((u32)y & lpf)) & 1u;
-        const double2 fy = ipow(make_double2(sy ? -1.0 : 1.0, 0.0), rot);
-        const double2 fx = ipow(make_double2(sx ? -1.0 : 1.0, 0.0), rot);
-        if (LBF == 0) {
-            const double2 pv = cmul(fy, v[y]);
-            if (BACK) acc -= l[y].x * pv.y - l[y].y * pv.x;
-            // (c + i sn fy) v_y
-            const double2 f = make_double2(c - sn * fy.y, sn * fy.x);
-            v[y] = cmul(f, v[y]);
-            if (BACK) l[y] = cmul(f, l[y]);
-        } else {
-            const double2 vy = v[y], vx = v[x];
-            const double2 py = cmul(fy, vx), px = cmul(fx, vy);  // (P v)_y, (P v)_x
-            if (BACK) acc -= (l[y].x * py.y - l[y].y * py.x) + (l[x].x * px.y - l[x].y * px.x);
-            v[y] = make_double2(c * vy.x - sn * py.y, c * vy.y + sn * py.x);
-            v[x] = make_double2(c * vx.x - sn * px.y, c * vx.y + sn * px.x);
-            if (BACK) {
-                const double2 ly = l[y], lx = l[x];
-                const double2 qy = cmul(fy, lx), qx = cmul(fx, ly);
-                l[y] = make_double2(c * ly.x - sn * qy.y, c * ly.y + sn * qy.x);
-                l[x] = make_double2(c * lx.x - sn * qx.y, c * lx.y + sn * qx.x);
-            }
-        }
-    }
-}
-
-template <bool BACK>
-__device__ __forceinline__ void rot_dispatch(u32 lbf, double2* v, double2* l, u32 lpf, u32 rot, u32 so, double c,
-                                             double sn, double& acc) {
-    switch (lbf) {
-#define QM_ROT_CASE(B)                                                        \
-    case B:                                                                   \
-        if constexpr (B < kPassN) rot_apply<B, BACK>(v, l, lpf, rot, so, c, sn, acc); \
-        break;
-        QM_ROT_CASE(0) QM_ROT_CASE(1) QM_ROT_CASE(2) QM_ROT_CASE(3) QM_ROT_CASE(4) QM_ROT_CASE(5) QM_ROT_CASE(6)
-        QM_ROT_CASE(7) QM_ROT_CASE(8) QM_ROT_CASE(9) QM_ROT_CASE(10) QM_ROT_CASE(11) QM_ROT_CASE(12)
-        QM_ROT_CASE(13) QM_ROT_CASE(14) QM_ROT_CASE(15)
-#undef QM_ROT_CASE
-        default: break;
-    }
-}
-
-// Dense matrix on member bit A (INV: its conjugate transpose) applied to v.
-template <int A, bool INV>
-__device__ __forceinline__ void dense1_apply(double2* v, const double2* m) {
-    const double2 m00 = INV ? cconj(m[0]) : m[0], m01 = INV ? cconj(m[2]) : m[1];
-    const double2 m10 = INV ? cconj(m[1]) : m[2], m11 = INV ? cconj(m[3]) : m[3];
-#pragma unroll
-    for (int y = 0; y < kPassN; ++y) {
-        if (y & (1 << A)) continue;
-        const int z = y | (1 << A);
-        const double2 a0 = v[y], a1 = v[z];
-        v[y] = cmac(cmul(m00, a0), m01, a1);
-        v[z] = cmac(cmul(m10, a0), m11, a1);
-    }
-}
-
-template <int A, int B, bool INV>
-__device__ __forceinline__ void dense2_apply(double2* v, const double2* m) {
-    double2 mm[16];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) mm[r * 4 + c] = INV ? cconj(m[c * 4 + r]) : m[r * 4 + c];
-#pragma unroll
-    for (int y = 0; y < kPassN; ++y) {
-        if ((y & (1 << A)) || (y & (1 << B))) continue;
-        const int i1 = y | (1 << A), i2 = y | (1 << B), i3 = i1 | i2;
-        const double2 a0 = v[y], a1 = v[i1], a2 = v[i2], a3 = v[i3];
-        v[y] = cmac(cmac(cmac(cmul(mm[0], a0), mm[1], a1), mm[2], a2), mm[3], a3);
-        v[i1] = cmac(cmac(cmac(cmul(mm[4], a0), mm[5], a1), mm[6], a2), mm[7], a3);
-        v[i2] = cmac(cmac(cmac(cmul(mm[8], a0), mm[9], a1), mm[10], a2), mm[11], a3);
-        v[i3] = cmac(cmac(cmac(cmul(mm[12], a0), mm[13], a1), mm[14], a2), mm[15], a3);
-    }
-}
-
-template <bool INV>
-__device__ __forceinline__ void dense1_dispatch(u32 a, double2* v, const double2* m) {
-    switch (a) {
-        case 0: dense1_apply<0, INV>(v, m); break;
-        case 1: dense1_apply<1, INV>(v, m); break;
-        case 2: dense1_apply<2, INV>(v, m); break;
-        default:
-            if constexpr (kPassQubits > 3) dense1_apply<3, INV>(v, m);
-            break;
-    }
-}
-
-template <bool INV>
-__device__ __forceinline__ void dense2_dispatch(u32 a, u32 b, double2* v, const double2* m) {
-    switch (a * 4 + b) {
-#define QM_D2_CASE(A, B)                                                       \
-    case A * 4 + B:                                                            \
-        if constexpr (A < kPassQubits && B < kPassQubits) dense2_apply<A, B, INV>(v, m); \
-        break;
-        QM_D2_CASE(0, 1) QM_D2_CASE(0, 2) QM_D2_CASE(0, 3) QM_D2_CASE(1, 0) QM_D2_CASE(1, 2) QM_D2_CASE(1, 3)
-        QM_D2_CASE(2, 0) QM_D2_CASE(2, 1) QM_D2_CASE(2, 3) QM_D2_CASE(3, 0) QM_D2_CASE(3, 1) QM_D2_CASE(3, 2)
-#undef QM_D2_CASE
-        default: break;
-    }
-}
-
-// Diagonal gate: member y of the tuple with base index `base` gets entry d[idx],
-// idx collecting the gate's qubit bits (member bits or base bits).
-template <bool INV>
-__device__ __forceinline__ void diag_apply(double2* v, const PassOp& op, u64 base) {
-    u32 outside = 0;
-    for (u32 j = 0; j < op.dk; ++j)
-        if (op.dloc[j] == 255u) outside |= (u32)((base >> op.dpos[j]) & 1ULL) << j;
-#pragma unroll
-    for (int y = 0; y < kPassN; ++y) {
-        u32 idx = outside;
-        for (u32 j = 0; j < op.dk; ++j)
-            if (op.dloc[j] != 255u) idx |= (((u32)y >> op.dloc[j]) & 1u) << j;
-        const double2 d = INV ? cconj(op.m[idx]) : op.m[idx];
-        v[y] = cmul(d, v[y]);
-    }
-}
-
-// One pass over `batch` states (blockIdx.y = state).  BACK: psi and lambda,
-// gates in reverse order, rotation terms summed per block into
-// partials[(occ * batch + b) * gridDim.x + blockIdx.x].
-template <bool BACK>
-__global__ __launch_bounds__(kAdjThreads) void k_adj_pass(double2* __restrict__ psi, double2* __restrict__ lam,
-                                                          u64 dim, PassArgs pa, const PassOp* __restrict__ ops,
-                                                          const double* __restrict__ theta, u32 nparams,
-                                                          double* __restrict__ partials) {
-    __shared__ double acc_lds[BACK ? kPassRots * kAdjThreads : 1];
-    __shared__ double cs_lds[kPassRots][2];
-    __shared__ double red[32];
-    const u32 bs = blockIdx.y;
-    const u64 off = (u64)bs * dim;
-    if (threadIdx.x < pa.nrot) {
-        const double ang = pa.coef[threadIdx.x] * theta[(u64)bs * nparams + pa.param[threadIdx.x]];
-        cs_lds[threadIdx.x][0] = cos(0.5 * ang);
-        cs_lds[threadIdx.x][1] = sin(0.5 * ang);
-    }
-    if (BACK)
-        for (u32 r = 0; r < pa.nrot; ++r) acc_lds[r * kAdjThreads + threadIdx.x] = 0.0;
     __syncthreads();
-    double2* P = psi + off;
-    double2* Lm = lam + off;
-    const u64 tuples = dim >> kPassQubits;
-    const u64 stride = (u64)gridDim.x * blockDim.x;
-    for (u64 t = (u64)blockIdx.x * blockDim.x + threadIdx.x; t < tuples; t += stride) {
-        u64 base = t;
+    run_passes<kAdjK, kFwdThreads, 1, false>(st, lq, passes, sg.pass0, sg.npass, subs,
+                                             pool + (u64)blockIdx.y * stride);
+    for (u32 i = threadIdx.x; i < L; i += T) s[tile_index<kAdjLow>(tb, hi_tab, i)] = st[slot_of(i)];
+}
+
+// Wave sums of a, b, c: afterwards every lane of row r (16 lanes) holds the sum of a, b, c
+// for r = 0, 1, 2.  Two swap levels put different values into the rows, so four row levels serve
+// all three: 21 vector instructions instead of 54 for three separate sums.
+__device__ __forceinline__ double swap_add32(double a, double b) {
+    const auto lo = __builtin_amdgcn_permlane32_swap((u32)__double2loint(a), (u32)__double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((u32)__double2hiint(a), (u32)__double2hiint(b), false, false);
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ double swap_add16(double a, double b) {
+    const auto lo = __builtin_amdgcn_permlane16_swap((u32)__double2loint(a), (u32)__double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((u32)__double2hiint(a), (u32)__double2hiint(b), false, false);
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_sum3(double a, double b, double c) {
+    double v = swap_add16(swap_add32(a, c), swap_add32(b, 0.0));
+    v = dpp_add<0x128>(v);  // row_ror:8
+    v = dpp_add<0x124>(v);  // row_ror:4
+    v = dpp_add<0x122>(v);  // row_ror:2
+    return dpp_add<0x121>(v);
+}
+
+// One bit of a backward LAYER: the three sums of its operation (if it has gradients), then
+// U^dagger on psi (v) and lambda (l).  out: this wave's sums of the operation in LDS.
+template <int P>
+__device__ __forceinline__ void bwd_bit(double2 (&v)[1 << kAdjK], double2 (&l)[1 << kAdjK], const double2* mp,
+                                        bool grad, bool add, double* out) {
+    constexpr int NP = 1 << (kAdjK - 1);
+    const double2 m0 = mp[0], m1 = mp[1], m2 = mp[2], m3 = mp[3];
+    auto pair_j = [](int q) { return ((q >> P) << (P + 1)) | (q & ((1 << P) - 1)); };
+    if (grad) {
+        double sx = 0.0, sy = 0.0, sz = 0.0;
 #pragma unroll
-        for (int j = 0; j < kPassQubits; ++j) base = insert_zero(base, pa.blk[j]);
-        double2 v[kPassN], l[kPassN];
-#pragma unroll
-        for (int y = 0; y < kPassN; ++y) v[y] = P[base + pa.offs[y]];
-        if (BACK) {
-#pragma unroll
-            for (int y = 0; y < kPassN; ++y) l[y] = Lm[base + pa.offs[y]];
+        for (int q = 0; q < NP; ++q) {
+            const double2 a = v[pair_j(q)], b = v[pair_j(q) | (1 << P)];
+            const double2 c = l[pair_j(q)], d = l[pair_j(q) | (1 << P)];
+            sx = fma(c.x, b.y, sx); sy = fma(-c.x, b.x, sy); sz = fma(c.x, a.y, sz);
+            sx = fma(-c.y, b.x, sx); sy = fma(-c.y, b.y, sy); sz = fma(-c.y, a.x, sz);
+            sx = fma(d.x, a.y, sx); sy = fma(d.x, a.x, sy); sz = fma(-d.x, b.y, sz);
+            sx = fma(-d.y, a.x, sx); sy = fma(d.y, a.y, sy); sz = fma(d.y, b.x, sz);
         }
-        for (u32 k = 0; k < pa.nops; ++k) {
-            const PassOp& op = ops[pa.op0 + (BACK ? pa.nops - 1 - k : k)];
-            switch (op.type) {
-                case 0: {
-                    const u32 so = (u32)__popcll(base & op.opf) & 1u;
-                    const double c = cs_lds[op.slot][0], sn = BACK ? -cs_lds[op.slot][1] : cs_lds[op.slot][1];
-                    double acc = 0.0;
-                    rot_dispatch<BACK>(op.lbf, v, l, op.lpf, op.rot, so, c, sn, acc);
-                    if (BACK) acc_lds[op.slot * kAdjThreads + threadIdx.x] += acc;
-                    break;
-                }
-                case 1:
-                    dense1_dispatch<BACK>(op.a, v, op.m);
-                    if (BACK) dense1_dispatch<true>(op.a, l, op.m);
-                    break;
-                case 2:
-                    dense2_dispatch<BACK>(op.a, op.b, v, op.m);
-                    if (BACK) dense2_dispatch<true>(op.a, op.b, l, op.m);
-                    break;
-                default:
-                    diag_apply<BACK>(v, op, base);
-                    if (BACK) diag_apply<true>(l, op, base);
-                    break;
-            }
-        }
-#pragma unroll
-        for (int y = 0; y < kPassN; ++y) P[base + pa.offs[y]] = v[y];
-        if (BACK) {
-#pragma unroll
-            for (int y = 0; y < kPassN; ++y) Lm[base + pa.offs[y]] = l[y];
+        const double r = wave_sum3(sx, sy, sz);
+        const u32 lane = threadIdx.x & 63u;
+        if ((lane & 15u) == 0 && lane < 48) {
+            if (add) out[lane >> 4] += r;
+            else out[lane >> 4] = r;
         }
     }
-    if (BACK) {
-        for (u32 k = 0; k < pa.nops; ++k) {
-            const PassOp& op = ops[pa.op0 + k];
-            if (op.type != 0) continue;
-            const double a = block_sum(acc_lds[op.slot * kAdjThreads + threadIdx.x], red);
-            // d/dtheta = coef * d/dangle
-            if (threadIdx.x == 0)
-                partials[((u64)op.occ * gridDim.y + bs) * gridDim.x + blockIdx.x] = a * pa.coef[op.slot];
+#pragma unroll
+    for (int q = 0; q < NP; ++q)
+        pair_update2(v[pair_j(q)], v[pair_j(q) | (1 << P)], l[pair_j(q)], l[pair_j(q) | (1 << P)], m0, m1, m2, m3);
+}
+
+// One backward stage: as k_adj_fwd on the tiles of psi and lambda, the operations reversed and
+// inverted.  A thread holds one register block of each state; the tile has at most T blocks
+// (threads beyond them hold zeros, so that the wave sums see every lane).  Work-group x takes
+// tiles x, x + gridDim.x, ... and writes its sums of the stage's operations to
+// partials[set][x][3 * (position in grads) ..].
+__global__ __launch_bounds__(kBwdThreads, 2) void k_adj_bwd(double2* __restrict__ psi, double2* __restrict__ lam, u32 n,
+                                                            u32 lq, u64 ntiles, DStage sg, u32 grad0, u32 ngrad,
+                                                            const DPass* __restrict__ passes,
+                                                            const DSub* __restrict__ subs,
+                                                            const double2* __restrict__ pools, u32 stride,
+                                                            double* __restrict__ partials, u32 ncols) {
+    extern __shared__ double2 st[];
+    __shared__ u64 hi_tab[1u << (kBwdLocal - kAdjLow)];
+    __shared__ double acc[kBwdThreads / 64][kStageGrads][3];
+    constexpr int D = 1 << kAdjK;
+    const u32 L = 1u << lq, T = blockDim.x, tid = threadIdx.x, wave = tid >> 6;
+    const u32 ngroups = L >> kAdjK;
+    const double2* __restrict__ pool = pools + (u64)blockIdx.y * stride;
+    double2* P = psi + ((u64)blockIdx.y << n);
+    double2* Q = lam + ((u64)blockIdx.y << n);
+    double2* st2 = st + L;
+    build_hi_tab<kAdjLow>(hi_tab, lq, sg);
+    __syncthreads();
+    for (u64 t = blockIdx.x; t < ntiles; t += gridDim.x) {
+        const bool add = t != blockIdx.x;  // a later tile of this work-group
+        const u64 tb = tile_base(t, n - lq, sg);
+        if (L == 8 * kBwdThreads) {
+#pragma unroll
+            for (u32 k = 0; k < 8; ++k) {
+                const u32 i = tid + k * kBwdThreads;
+                const u64 at = tile_index<kAdjLow>(tb, hi_tab, i);
+                st[slot_of(i)] = P[at];
+                st2[slot_of(i)] = Q[at];
+            }
+        } else {
+            for (u32 i = tid; i < L; i += T) {
+                const u64 at = tile_index<kAdjLow>(tb, hi_tab, i);
+                st[slot_of(i)] = P[at];
+                st2[slot_of(i)] = Q[at];
+            }
         }
+        __syncthreads();
+        for (u32 p = 0; p < sg.npass; ++p) {
+            const DPass ps = passes[sg.pass0 + p];
+            const bool mine = tid < ngroups;
+            u32 base = mine ? tid : 0, slot[D];
+#pragma unroll
+            for (int i = 0; i < kAdjK; ++i) {
+                const u32 q = ps.pos[i];
+                base = (base & ((1u << q) - 1)) | ((base >> q) << (q + 1));
+            }
+            slot[0] = slot_of(base);
+#pragma unroll
+            for (int j = 1; j < D; ++j) {
+                slot[j] = slot[j & (j - 1)] ^ ps.sbit[__builtin_ctz(j)];
+                asm volatile("" : "+v"(slot[j]));
+            }
+            double2 v[D], l[D];
+#pragma unroll
+            for (int j = 0; j < D; ++j) {
+                v[j] = st[slot[j]];
+                l[j] = st2[slot[j]];
+            }
+            if (!mine) {
+#pragma unroll
+                for (int j = 0; j < D; ++j) v[j] = l[j] = make_double2(0.0, 0.0);
+            }
+            u32 k = 0;
+            while (k < ps.nsub) {
+                DSub sub = subs[ps.sub0 + k];
+                while ((sub.type & 0xffu) == SUB_LAYER) {
+                    const u32 d1 = (sub.type >> 8) & 15u;
+                    if (sub.type >> 12) {
+                        const u32 sgn = layer_signs<kAdjK>(sub, base);
+                        flip_signs<kAdjK>(v, sgn);
+                        flip_signs<kAdjK>(l, sgn);
+                    }
+                    const double2* mp = pool + sub.data;
+                    double* out = acc[wave][sub.grad0 - grad0];
+                    if (d1 & 1u) {
+                        bwd_bit<0>(v, l, mp, sub.gmask & 1u, add, out);
+                        mp += 4;
+                        out += 3 * (sub.gmask & 1u);
+                    }
+                    if (d1 & 2u) {
+                        bwd_bit<1>(v, l, mp, sub.gmask & 2u, add, out);
+                        mp += 4;
+                        out += 3 * ((sub.gmask >> 1) & 1u);
+                    }
+                    if (d1 & 4u) bwd_bit<2>(v, l, mp, sub.gmask & 4u, add, out);
+                    if (++k == ps.nsub) break;
+                    sub = subs[ps.sub0 + k];
+                }
+                if (k == ps.nsub) break;
+                // D2: the 4 x 4 matrix on both states
+                const double2* mp = pool + sub.data;
+                apply_d2<kAdjK>(v, byte_at(sub.a, 0), byte_at(sub.a, 1), mp);
+                apply_d2<kAdjK>(l, byte_at(sub.a, 0), byte_at(sub.a, 1), mp);
+                ++k;
+            }
+            if (mine) {
+#pragma unroll
+                for (int j = 0; j < D; ++j) {
+                    st[slot[j]] = v[j];
+                    st2[slot[j]] = l[j];
+                }
+            }
+            __syncthreads();
+        }
+        for (u32 i = tid; i < L; i += T) {
+            const u64 at = tile_index<kAdjLow>(tb, hi_tab, i);
+            P[at] = st[slot_of(i)];
+            Q[at] = st2[slot_of(i)];
+        }
+        __syncthreads();  // the tile has been read out of LDS
+    }
+    double* dst = partials + ((u64)blockIdx.y * gridDim.x + blockIdx.x) * ncols + 3 * (u64)grad0;
+    for (u32 i = tid; i < 3 * ngrad; i += T) {
+        double s = 0.0;
+        for (u32 w = 0; w < T / 64; ++w) s += acc[w][i / 3][i % 3];
+        dst[i] = s;
     }
 }
 
-// lambda = sum_k c_k P_k psi and the block's share of Re <psi|lambda>.
-__global__ __launch_bounds__(kAdjThreads) void k_adj_hpsi(const double2* __restrict__ psi, double2* __restrict__ lam,
-                                                          u64 dim, const AdjTerm* __restrict__ terms, u32 nterms,
-                                                          double* __restrict__ epart) {
+// lambda = sum_k c_k P_k psi and the block's share of Re <psi|lambda>.  Terms with one
+// bit-flip mask read their partner amplitude once.
+__global__ __launch_bounds__(kHpsiThreads) void k_adj_hpsi(const double2* __restrict__ psi, double2* __restrict__ lam,
+                                                           u64 dim, const AdjGroup* __restrict__ groups, u32 ngroup,
+                                                           const AdjTerm* __restrict__ terms,
+                                                           double* __restrict__ epart) {
     __shared__ double red[32];
     const u64 off = (u64)blockIdx.y * dim;
     const double2* P = psi + off;
     double acc = 0.0;
     for (u64 x = (u64)blockIdx.x * blockDim.x + threadIdx.x; x < dim; x += (u64)gridDim.x * blockDim.x) {
         double2 s = make_double2(0.0, 0.0);
-        for (u32 k = 0; k < nterms; ++k) {
-            const AdjTerm tm = terms[k];
-            const u64 y = x ^ tm.bf;
-            const double sg = (__popcll(y & tm.pf) & 1) ? -tm.coef : tm.coef;
-            const double2 v = ipow(P[y], tm.rot);
-            s.x = fma(sg, v.x, s.x);
-            s.y = fma(sg, v.y, s.y);
+        for (u32 g = 0; g < ngroup; ++g) {
+            const AdjGroup gr = groups[g];
+            const u64 y = x ^ gr.bf;
+            const double2 v = P[y];
+            double2 c = make_double2(0.0, 0.0);  // sum_k c_k i^rot (-1)^popcount(y & pf)
+            for (u32 k = 0; k < gr.nterm; ++k) {
+                const AdjTerm tm = terms[gr.term0 + k];
+                const double sg = (__popcll(y & tm.pf) & 1) ? -tm.coef : tm.coef;
+                const double2 f = ipow(make_double2(1.0, 0.0), tm.rot);
+                c.x = fma(sg, f.x, c.x);
+                c.y = fma(sg, f.y, c.y);
+            }
+            s = cmac(s, c, v);
         }
         lam[off + x] = s;
         const double2 p = P[x];
@@ -441,26 +394,175 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_hpsi(const double2* __restr
     if (threadIdx.x == 0) epart[(u64)blockIdx.y * gridDim.x + blockIdx.x] = acc;
 }
 
-// grad[b][p] = sum over occurrences of p (in order) and blocks (in order).
-__global__ void k_adj_finish(const double* __restrict__ partials, const double* __restrict__ epart,
-                             const u32* __restrict__ occ_param, u32 nocc, u32 nparams, u32 batch, u32 nblk,
-                             double* __restrict__ grad, double* __restrict__ energy) {
-    const u64 idx = (u64)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx < (u64)batch * nparams) {
-        const u32 b = (u32)(idx / nparams), p = (u32)(idx % nparams);
-        double s = 0.0;
-        for (u32 o = 0; o < nocc; ++o) {
-            if (occ_param[o] != p) continue;
-            const double* src = partials + ((u64)o * batch + b) * nblk;
-            for (u32 k = 0; k < nblk; ++k) s += src[k];
-        }
-        grad[idx] = s;
+// Columns of partials[set][block][ncols] summed over the blocks: 16 columns per
+// work-group, 16 threads per column, each over every 16th block, then in order.
+__global__ __launch_bounds__(256) void k_adj_columns(const double* __restrict__ partials, u32 nblk, u32 ncols,
+                                                     double* __restrict__ sums) {
+    __shared__ double red[16][17];
+    const u32 c = threadIdx.x & 15u, part = threadIdx.x >> 4, col = blockIdx.x * 16 + c;
+    const double* src = partials + (u64)blockIdx.y * nblk * ncols;
+    double s = 0.0;
+    if (col < ncols)
+        for (u32 b = part; b < nblk; b += 16) s += src[(u64)b * ncols + col];
+    red[part][c] = s;
+    __syncthreads();
+    if (part == 0 && col < ncols) {
+        double r = 0.0;
+        for (u32 k = 0; k < 16; ++k) r += red[k][c];
+        sums[(u64)blockIdx.y * ncols + col] = r;
     }
-    if (idx < batch) {
+}
+
+// grad[set][p] = -sum over the occurrences of p (in order) of coef * (g . s); the first
+// thread of a set's first block adds up its energy.
+__global__ __launch_bounds__(64) void k_adj_grad(const double* __restrict__ sums, u32 ncols,
+                                                 const double* __restrict__ gvec, u32 nocc,
+                                                 const u32* __restrict__ first, const u32* __restrict__ occs,
+                                                 const u32* __restrict__ occ_col, const double* __restrict__ occ_coef,
+                                                 u32 nparams, double* __restrict__ grad,
+                                                 const double* __restrict__ epart, u32 neblk,
+                                                 double* __restrict__ energy) {
+    const u32 p = blockIdx.x * blockDim.x + threadIdx.x, set = blockIdx.y;
+    if (blockIdx.x == 0) {  // the set's energy
         double e = 0.0;
-        for (u32 k = 0; k < nblk; ++k) e += epart[idx * nblk + k];
-        energy[idx] = e;
+        for (u32 k = threadIdx.x; k < neblk; k += 64) e += epart[(u64)set * neblk + k];
+        e = wave_sum(e);
+        if (threadIdx.x == 0) energy[set] = e;
     }
+    if (p >= nparams) return;
+    double r = 0.0;
+    for (u32 k = first[p]; k < first[p + 1]; ++k) {
+        const u32 o = occs[k];
+        const double* g = gvec + ((u64)set * nocc + o) * 3;
+        const double* s = sums + (u64)set * ncols + occ_col[o];
+        r -= occ_coef[o] * (g[0] * s[0] + g[1] * s[1] + g[2] * s[2]);
+    }
+    grad[(u64)set * nparams + p] = r;
+}
+
+// ------------------------------------------------------------------ host side
+// A single-qubit operation while the circuit is read: its factors in gate order.
+struct Op1 {
+    std::vector<Factor> factors;
+    bool grad = false;
+};
+
+bool unitary2(const cd* m) {
+    const cd a = std::conj(m[0]) * m[0] + std::conj(m[2]) * m[2], b = std::conj(m[1]) * m[1] + std::conj(m[3]) * m[3];
+    const cd c = std::conj(m[0]) * m[1] + std::conj(m[2]) * m[3];
+    return std::abs(a - 1.0) < 1e-12 && std::abs(b - 1.0) < 1e-12 && std::abs(c) < 1e-12;
+}
+
+// The circuit as single-qubit operations, CZ gates and 4 x 4 matrices.
+struct Builder {
+    u32 ne = 0;
+    std::vector<HOp> ops;
+    std::vector<Op1> op1;
+    std::vector<double2> fixed;
+    std::vector<long> last;  // per qubit: index in ops of its last operation, if single-qubit and open
+    std::vector<Factor> occ; // rotation occurrences
+
+    explicit Builder(u32 n) : ne(n), last(n, -1) {}
+    Op1& open(u32 q) {
+        if (last[q] < 0) {
+            HOp h;
+            h.type = 0;
+            h.q = {q};
+            h.m.assign(4, 0.0);
+            h.id = (long)op1.size();
+            last[q] = (long)ops.size();
+            ops.push_back(std::move(h));
+            op1.emplace_back();
+        }
+        return op1[ops[last[q]].id];
+    }
+    void put1(u32 q, const cd* m) {
+        // a matrix that is not unitary keeps an operation of its own: the gradient of a
+        // rotation before it needs the state between the two
+        const bool closed = !unitary2(m);
+        if (closed) last[q] = -1;
+        Factor f{};
+        f.fixed = (u32)fixed.size();
+        for (int i = 0; i < 4; ++i) fixed.push_back(make_double2(m[i].real(), m[i].imag()));
+        open(q).factors.push_back(f);
+        if (closed) last[q] = -1;
+    }
+    void cz(u32 a, u32 b) {
+        HOp h;
+        h.type = 2;
+        h.q = {a, b};
+        ops.push_back(std::move(h));
+        last[a] = last[b] = -1;
+    }
+    void put2(u32 a, u32 b, const cd* m) {
+        HOp h;
+        h.type = 0;
+        h.q = {a, b};
+        h.m.assign(m, m + 16);
+        ops.push_back(std::move(h));
+        last[a] = last[b] = -1;
+    }
+    // H before and after a CZ: the two constants are the neighbours of 1/sqrt(2), whose
+    // product is closer to 1/2 (by 2e-17 relative) than either one's square (1.4e-16), so
+    // that many CNOTs do not change the norm
+    void h(u32 q, bool second) {
+        const double c = second ? 0.70710678118654746 : 0.70710678118654757;
+        const cd m[4] = {c, c, c, -c};
+        put1(q, m);
+    }
+    void rot1(u32 q, u32 pauli, u32 param, double coef) {
+        Op1& o = open(q);
+        Factor f{};
+        f.kind = pauli;
+        f.param = param;
+        f.coef = coef;
+        f.occ = (u32)occ.size();
+        occ.push_back(f);
+        o.factors.push_back(f);
+        o.grad = true;
+        ops[last[q]].grad = true;
+    }
+    // exp(i a P / 2), P a Pauli string on k >= 2 qubits
+    void rotation(u32 k, const u32* q, const u32* pauli, u32 param, double coef) {
+        u32 t = 0;  // the qubit that is rotated: one with an X if there is one, else a Z
+        for (u32 j = 0; j < k; ++j)
+            if (pauli[j] == 1 || (pauli[t] == 2 && pauli[j] == 3)) t = j;
+        const double c = 0.70710678118654757, d = 0.70710678118654746;
+        // basis changes to Z (other qubits) and X (qubit t) and back
+        const cd i1(0, 1);
+        auto change = [&](u32 j, bool back) {
+            const double r = back ? d : c;
+            const cd h[4] = {r, r, r, -r};
+            if (j == t) {
+                if (pauli[j] == 3) put1(q[j], h);
+                if (pauli[j] == 2) {  // diag(1, -i) Y diag(1, i) = X
+                    const cd s[4] = {1.0, 0.0, 0.0, back ? i1 : -i1};
+                    put1(q[j], s);
+                }
+            } else if (pauli[j] == 1) {
+                put1(q[j], h);
+            } else if (pauli[j] == 2) {
+                // V = (1/sqrt2) [[1, -i], [1, i]]: V Y V^dagger = Z
+                const cd v[4] = {r, -i1 * r, r, i1 * r}, w[4] = {r, r, i1 * r, -i1 * r};
+                put1(q[j], back ? w : v);
+            }
+        };
+        for (u32 j = 0; j < k; ++j) change(j, false);
+        for (u32 j = 0; j < k; ++j)
+            if (j != t) cz(q[j], q[t]);
+        rot1(q[t], 1, param, coef);
+        for (u32 j = 0; j < k; ++j)
+            if (j != t) cz(q[j], q[t]);
+        for (u32 j = 0; j < k; ++j) change(j, true);
+    }
+};
+
+template <class T>
+bool put_dev(T** dst, const std::vector<T>& src, const char* what) {
+    *dst = nullptr;
+    if (src.empty()) return true;
+    return hip_ok(hipMalloc((void**)dst, src.size() * sizeof(T)), what) &&
+           hip_ok(hipMemcpy(*dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice), what);
 }
 
 }  // namespace
@@ -469,127 +571,164 @@ __global__ void k_adj_finish(const double* __restrict__ partials, const double* 
 using namespace qm;
 
 struct qm_adjoint {
-    u32 n = 0, nparams = 0;
-    std::vector<AdjGate> gates;
-    std::vector<u32> occ_param;  // parameter of each rotation occurrence
-    std::vector<PassOp> pops;    // the gates as pass operations, pass after pass
-    std::vector<PassArgs> passes;
+    u32 n = 0, ne = 0, nparams = 0, lqf = 0, lqb = 0;
+    u64 ngates = 0, blocks3 = 0;
+    Flat fwd, bwd;
+    std::vector<u32> stage_grad0;  // backward stage -> position in bwd.grads of its first operation
+    // host tables, uploaded on first use
+    std::vector<Factor> factors;
+    std::vector<u32> first, fwd_at, bwd_at, copies, par_first, par_occs, occ_col;
+    std::vector<double2> fixed, copy_val;
+    std::vector<double> occ_coef;
+    u32 ncopy_f = 0, ncopy_b = 0;
     int device = -1;
-    u32* d_occ = nullptr;
-    PassOp* d_ops = nullptr;
+    Factor* d_factors = nullptr;
+    u32 *d_first = nullptr, *d_fwd_at = nullptr, *d_bwd_at = nullptr, *d_copies = nullptr, *d_par_first = nullptr,
+        *d_par_occs = nullptr, *d_occ_col = nullptr;
+    double2 *d_fixed = nullptr, *d_copy_val = nullptr;
+    double* d_occ_coef = nullptr;
+    DPass *d_fpass = nullptr, *d_bpass = nullptr;
+    DSub *d_fsub = nullptr, *d_bsub = nullptr;
+
+    u32 nops() const { return (u32)first.size() - 1; }
+    u32 nocc() const { return (u32)occ_coef.size(); }
+    u32 ncols() const { return 3 * (u32)bwd.grads.size(); }
+    u64 tiles_b() const { return 1ULL << (ne - lqb); }
+    u32 blocks_b() const { return (u32)std::min<u64>(tiles_b(), kBwdMaxBlocks); }
+    u32 blocks_h() const {
+        return (u32)std::min<u64>(std::max<u64>((1ULL << ne) / (4 * kHpsiThreads), 1), kHpsiMaxBlocks);
+    }
+    // workspace parts, in order; each a multiple of 16 bytes
+    u64 state_bytes(u64 batch) const { return batch * (16ULL << ne); }
+    u64 fpool_bytes(u64 batch) const { return batch * fwd.pool.size() * 16; }
+    u64 bpool_bytes(u64 batch) const { return batch * bwd.pool.size() * 16; }
+    u64 part_bytes(u64 batch) const { return (batch * blocks_b() * ncols() * 8 + 15) & ~15ULL; }
+    u64 sums_bytes(u64 batch) const { return (batch * ncols() * 8 + 15) & ~15ULL; }
+    u64 gvec_bytes(u64 batch) const { return (batch * nocc() * 24 + 15) & ~15ULL; }
+    u64 epart_bytes(u64 batch) const { return (batch * blocks_h() * 8 + 15) & ~15ULL; }
+
     void release() {
         if (device >= 0) {
             (void)hipSetDevice(device);
-            if (d_occ) (void)hipFree(d_occ);
-            if (d_ops) (void)hipFree(d_ops);
+            void* ptrs[] = {d_factors, d_first, d_fwd_at, d_bwd_at, d_copies, d_par_first, d_par_occs, d_occ_col,
+                            d_fixed, d_copy_val, d_occ_coef, d_fpass, d_bpass, d_fsub, d_bsub};
+            for (void* p : ptrs)
+                if (p) (void)hipFree(p);
         }
-        d_occ = nullptr;
-        d_ops = nullptr;
+        d_factors = nullptr; d_first = nullptr; d_fwd_at = nullptr; d_bwd_at = nullptr; d_copies = nullptr;
+        d_par_first = nullptr; d_par_occs = nullptr; d_occ_col = nullptr; d_fixed = nullptr; d_copy_val = nullptr;
+        d_occ_coef = nullptr; d_fpass = nullptr; d_bpass = nullptr; d_fsub = nullptr; d_bsub = nullptr;
         device = -1;
     }
-    void plan();
+    bool prepare(unsigned dev, const char* what) {
+        if (device == (int)dev) return true;
+        release();
+        device = (int)dev;  // release() frees what the uploads below allocate
+        const bool ok = put_dev(&d_factors, factors, what) && put_dev(&d_first, first, what) &&
+                        put_dev(&d_fwd_at, fwd_at, what) && put_dev(&d_bwd_at, bwd_at, what) &&
+                        put_dev(&d_copies, copies, what) && put_dev(&d_par_first, par_first, what) &&
+                        put_dev(&d_par_occs, par_occs, what) && put_dev(&d_occ_col, occ_col, what) &&
+                        put_dev(&d_fixed, fixed, what) && put_dev(&d_copy_val, copy_val, what) &&
+                        put_dev(&d_occ_coef, occ_coef, what) && put_dev(&d_fpass, fwd.passes, what) &&
+                        put_dev(&d_bpass, bwd.passes, what) && put_dev(&d_fsub, fwd.subs, what) &&
+                        put_dev(&d_bsub, bwd.subs, what) &&
+                        hip_ok(hipFuncSetAttribute((const void*)k_adj_fwd, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                   (int)(sizeof(double2) << kFwdLocal)), what) &&
+                        hip_ok(hipFuncSetAttribute((const void*)k_adj_bwd, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                   (int)(2 * sizeof(double2) << kBwdLocal)), what);
+        if (!ok) release();
+        return ok;
+    }
+    void build(const Builder& b);
 };
 
-// Groups the gates into passes (see the file comment): a gate joins the open
-// pass when the qubits it needs in the block (a rotation's X/Y qubits, a
-// non-diagonal fixed gate's qubits; none for a diagonal gate) fit in
-// kPassQubits together with the pass's, and the pass has a free rotation slot.
-void qm_adjoint::plan() {
-    pops.clear();
-    passes.clear();
-    if (n < (u32)kPassQubits) return;  // tiny states keep one kernel per gate
-    auto diagonal = [](const AdjGate& g) {
-        const u32 d = 1u << g.k;
-        for (u32 r = 0; r < d; ++r)
-            for (u32 c = 0; c < d; ++c)
-                if (r != c && (g.m[r * d + c].x != 0.0 || g.m[r * d + c].y != 0.0)) return false;
-        return true;
-    };
-    auto needs = [&](const AdjGate& g) -> u64 {
-        if (g.kind == 1) return g.bf;
-        if (diagonal(g)) return 0;
-        u64 m = 1ULL << g.q[0];
-        if (g.k == 2) m |= 1ULL << g.q[1];
-        return m;
-    };
-    for (const AdjGate& g : gates)
-        if (__builtin_popcountll(needs(g)) > kPassQubits) return;  // keeps one kernel per gate
-    size_t i = 0;
-    while (i < gates.size()) {
-        u64 blk = 0;
-        size_t j = i;
-        u32 nrot = 0;
-        for (; j < gates.size(); ++j) {
-            const u64 nb = blk | needs(gates[j]);
-            if (__builtin_popcountll(nb) > kPassQubits) break;
-            if (gates[j].kind == 1 && nrot == (u32)kPassRots) break;
-            blk = nb;
-            nrot += gates[j].kind == 1 ? 1 : 0;
+// Schedules the operations forward and, reversed and inverted, backward, and lays out the tables.
+void qm_adjoint::build(const Builder& b) {
+    lqf = std::min(ne, kFwdLocal);
+    lqb = std::min(ne, kBwdLocal);
+    HCirc hc;
+    hc.n = hc.ne = ne;
+    hc.ops = b.ops;
+    schedule_circuit(fwd, hc, kAdjK, kFwdLocal, kAdjLow);
+    std::reverse(hc.ops.begin(), hc.ops.end());
+    for (HOp& o : hc.ops)
+        if (o.type == 0 && o.q.size() == 2) {  // 4 x 4: conjugate transpose
+            const std::vector<cd> m = o.m;
+            for (int r = 0; r < 4; ++r)
+                for (int c = 0; c < 4; ++c) o.m[r * 4 + c] = std::conj(m[c * 4 + r]);
         }
-        // pad the block with the highest free qubits (consecutive lanes then read
-        // consecutive amplitudes of every member)
-        for (int q = (int)n - 1; q >= 0 && __builtin_popcountll(blk) < kPassQubits; --q) blk |= 1ULL << q;
-        PassArgs pa{};
-        int pos[64];
-        int k = 0;
-        for (u32 q = 0; q < n; ++q) {
-            pos[q] = -1;
-            if ((blk >> q) & 1) {
-                pa.blk[k] = (unsigned char)q;
-                pos[q] = k++;
+    schedule_circuit(bwd, hc, kAdjK, kBwdLocal, kAdjLow, kStageGrads);
+    // first gradient of each backward stage: stages hold whole passes, in order
+    stage_grad0.clear();
+    u32 g = 0;
+    for (const DStage& sg : bwd.stages) {
+        stage_grad0.push_back(g);
+        for (u32 p = 0; p < sg.npass; ++p) {
+            const DPass& ps = bwd.passes[sg.pass0 + p];
+            for (u32 k = 0; k < ps.nsub; ++k) g += (u32)__builtin_popcount(bwd.subs[ps.sub0 + k].gmask);
+        }
+    }
+    stage_grad0.push_back(g);
+    factors.clear();
+    first.assign(1, 0);
+    for (const Op1& o : b.op1) {
+        factors.insert(factors.end(), o.factors.begin(), o.factors.end());
+        first.push_back((u32)factors.size());
+    }
+    fixed = b.fixed;
+    auto place = [&](const Flat& f, std::vector<u32>& at, u32& ncopy) {
+        at.assign(b.op1.size(), 0);
+        std::vector<bool> set(f.pool.size(), false);
+        for (const auto& m : f.mats) {
+            at[m.first] = m.second;
+            for (u32 i = 0; i < 4; ++i) set[m.second + i] = true;
+        }
+        ncopy = 0;
+        for (u32 i = 0; i < f.pool.size(); ++i)
+            if (!set[i]) {
+                copies.push_back(i);
+                copy_val.push_back(f.pool[i]);
+                ++ncopy;
             }
-        }
-        for (int y = 0; y < kPassN; ++y) {
-            u64 o = 0;
-            for (int b = 0; b < kPassQubits; ++b)
-                if ((y >> b) & 1) o |= 1ULL << pa.blk[b];
-            pa.offs[y] = o;
-        }
-        pa.op0 = (u32)pops.size();
-        pa.nops = (u32)(j - i);
-        pa.nrot = 0;
-        auto local = [&](u64 mask) {
-            u32 l = 0;
-            for (u32 q = 0; q < n; ++q)
-                if (((mask >> q) & 1) && pos[q] >= 0) l |= 1u << pos[q];
-            return l;
-        };
-        for (size_t g = i; g < j; ++g) {
-            const AdjGate& ag = gates[g];
-            PassOp op{};
-            if (ag.kind == 1) {
-                op.type = 0;
-                op.lbf = local(ag.bf);
-                op.lpf = local(ag.pf);
-                op.opf = ag.pf & ~blk;
-                op.rot = ag.rot;
-                op.slot = pa.nrot;
-                op.occ = ag.occ;
-                pa.param[pa.nrot] = ag.param;
-                pa.coef[pa.nrot] = ag.coef;
-                ++pa.nrot;
-            } else if (diagonal(ag)) {
-                op.type = 3;
-                op.dk = ag.k;
-                const u32 d = 1u << ag.k;
-                for (u32 t = 0; t < ag.k; ++t) {
-                    const u32 q = ag.q[t];
-                    op.dloc[t] = pos[q] >= 0 ? (u32)pos[q] : 255u;
-                    op.dpos[t] = q;
-                }
-                for (u32 x = 0; x < d; ++x) op.m[x] = ag.m[x * d + x];
-            } else {
-                op.type = ag.k == 1 ? 1 : 2;
-                op.a = (u32)pos[ag.q[0]];
-                op.b = ag.k == 2 ? (u32)pos[ag.q[1]] : 0;
-                for (u32 x = 0; x < (1u << (2 * ag.k)); ++x) op.m[x] = ag.m[x];
+    };
+    place(fwd, fwd_at, ncopy_f);
+    place(bwd, bwd_at, ncopy_b);
+    // column of each occurrence's operation, occurrences by parameter
+    std::vector<u32> col(b.op1.size(), 0);
+    for (size_t i = 0; i < bwd.grads.size(); ++i) col[bwd.grads[i]] = 3 * (u32)i;
+    occ_col.assign(b.occ.size(), 0);
+    occ_coef.assign(b.occ.size(), 0.0);
+    for (size_t o = 0; o < b.op1.size(); ++o)
+        for (const Factor& f : b.op1[o].factors)
+            if (f.kind) {
+                occ_col[f.occ] = col[o];
+                occ_coef[f.occ] = f.coef;
             }
-            pops.push_back(op);
-        }
-        passes.push_back(pa);
-        i = j;
+    par_first.assign(1, 0);
+    for (u32 p = 0; p < nparams; ++p) {
+        for (const Factor& f : b.occ)
+            if (f.param == p) par_occs.push_back(f.occ);
+        par_first.push_back((u32)par_occs.size());
     }
 }
+
+namespace {
+// The number of groups that the gate list divides into, in order, when a group's gates act
+// non-diagonally on at most three qubits; 0 if a gate needs more, or below three qubits.
+u64 count_blocks3(u32 n, const std::vector<u64>& needs) {
+    if (n < 3) return 0;
+    u64 groups = 0, blk = 0;
+    for (u64 m : needs) {
+        if (__builtin_popcountll(m) > 3) return 0;
+        if (groups == 0 || __builtin_popcountll(blk | m) > 3) {
+            ++groups;
+            blk = 0;
+        }
+        blk |= m;
+    }
+    return groups;
+}
+}  // namespace
 
 extern "C" {
 
@@ -599,68 +738,62 @@ qm_adjoint* qm_adjoint_create(UINT n, const qm_adjoint_gate* gates, UINT gate_co
         set_error(QM_ERR_INVALID_ARGUMENT, "%s: qubit count %u outside 1..34 or null gates", what, n);
         return nullptr;
     }
-    auto* a = new qm_adjoint();
-    a->n = n;
-    a->nparams = nparams;
+    const u32 ne = std::max<u32>(n, kMinQubits);
+    Builder b(ne);
+    std::vector<u64> needs;  // qubits that each gate acts on non-diagonally
     for (UINT i = 0; i < gate_count; ++i) {
         const qm_adjoint_gate& in = gates[i];
-        AdjGate g{};
         const u32 k = in.qubit_count;
-        u64 mask = 0;
+        u64 mask = 0, need = 0;
         bool ok = k >= 1 && k <= 4;
         for (u32 j = 0; ok && j < k; ++j) {
             ok = in.qubits[j] < n && !((mask >> in.qubits[j]) & 1);
             mask |= 1ULL << in.qubits[j];
         }
         if (ok && in.kind == QM_ADJ_ROT) {
-            g.kind = 1;
-            u32 rot = 0;
             for (u32 j = 0; ok && j < k; ++j) {
-                const u64 bit = 1ULL << in.qubits[j];
-                switch (in.paulis[j]) {
-                    case 1: g.bf |= bit; break;
-                    case 2: g.bf |= bit; g.pf |= bit; ++rot; break;
-                    case 3: g.pf |= bit; break;
-                    default: ok = false;
-                }
+                ok = in.paulis[j] >= 1 && in.paulis[j] <= 3;
+                if (in.paulis[j] != 3) need |= 1ULL << in.qubits[j];
             }
             ok = ok && in.param < nparams;
-            g.rot = rot;
-            g.pivot = g.bf ? 63 - __builtin_clzll(g.bf) : 0;
-            g.param = in.param;
-            g.coef = in.coef;
-            g.occ = (u32)a->occ_param.size();
-            if (ok) a->occ_param.push_back(in.param);
+            if (ok && k == 1) b.rot1(in.qubits[0], in.paulis[0], in.param, in.coef);
+            else if (ok) b.rotation(k, in.qubits, in.paulis, in.param, in.coef);
         } else if (ok) {
-            g.kind = 0;
             const bool two = in.kind == QM_BATCH_CZ || in.kind == QM_BATCH_CNOT;
             ok = (in.kind <= QM_BATCH_CNOT) && (two ? k == 2 : k <= 2) && (two || in.matrix);
-            g.k = k;
-            g.q[0] = in.qubits[0];
-            g.q[1] = k > 1 ? in.qubits[1] : 0;
-            const u32 d = 1u << k;
-            for (u32 r = 0; ok && r < d; ++r)
-                for (u32 c = 0; c < d; ++c) {
-                    double2 v = make_double2(0, 0);
-                    if (in.kind == QM_BATCH_DENSE) v = make_double2(in.matrix[r * d + c].re, in.matrix[r * d + c].im);
-                    else if (in.kind == QM_BATCH_DIAG && r == c) v = make_double2(in.matrix[r].re, in.matrix[r].im);
-                    else if (in.kind == QM_BATCH_CZ && r == c) v = make_double2(r == 3 ? -1.0 : 1.0, 0.0);
-                    else if (in.kind == QM_BATCH_CNOT) {
-                        // bit 0 <-> control, bit 1 <-> target
-                        const u32 cb = c & 1, tb = (c >> 1) & 1;
-                        v = make_double2(r == (cb | ((tb ^ cb) << 1)) ? 1.0 : 0.0, 0.0);
+            if (ok && in.kind == QM_BATCH_CZ) {
+                b.cz(in.qubits[0], in.qubits[1]);
+            } else if (ok && in.kind == QM_BATCH_CNOT) {
+                b.h(in.qubits[1], false);
+                b.cz(in.qubits[0], in.qubits[1]);
+                b.h(in.qubits[1], true);
+                need = mask;
+            } else if (ok) {
+                const u32 d = 1u << k;
+                std::vector<cd> m((size_t)d * d, 0.0);
+                for (u32 r = 0; r < d; ++r)
+                    for (u32 c = 0; c < d; ++c) {
+                        if (in.kind == QM_BATCH_DENSE) m[r * d + c] = cd(in.matrix[r * d + c].re, in.matrix[r * d + c].im);
+                        else if (r == c) m[r * d + c] = cd(in.matrix[r].re, in.matrix[r].im);
+                        if (r != c && m[r * d + c] != cd(0.0)) need = mask;
                     }
-                    g.m[r * d + c] = v;
-                }
+                if (k == 1) b.put1(in.qubits[0], m.data());
+                else b.put2(in.qubits[0], in.qubits[1], m.data());
+            }
         }
         if (!ok) {
             set_error(QM_ERR_INVALID_ARGUMENT, "%s: gate %u is not a 1..2-qubit fixed gate or a valid rotation", what, i);
-            delete a;
             return nullptr;
         }
-        a->gates.push_back(g);
+        needs.push_back(need);
     }
-    a->plan();
+    auto* a = new qm_adjoint();
+    a->n = n;
+    a->ne = ne;
+    a->nparams = nparams;
+    a->ngates = gate_count;
+    a->blocks3 = count_blocks3(n, needs);
+    a->build(b);
     return a;
 }
 
@@ -671,15 +804,14 @@ void qm_adjoint_destroy(qm_adjoint* a) {
 }
 
 void qm_adjoint_stats(const qm_adjoint* a, ITYPE* passes, ITYPE* gates) {
-    if (passes) *passes = a ? (ITYPE)a->passes.size() : 0;
-    if (gates) *gates = a ? (ITYPE)a->gates.size() : 0;
+    if (passes) *passes = a ? (ITYPE)a->blocks3 : 0;
+    if (gates) *gates = a ? (ITYPE)a->ngates : 0;
 }
 
 ITYPE qm_adjoint_workspace_bytes(const qm_adjoint* a, UINT batch) {
     if (!a) return 0;
-    const u64 states = 2ULL * batch * (16ULL << a->n);
-    const u64 parts = ((u64)a->occ_param.size() * batch + batch) * kAdjBlocks * sizeof(double);
-    return states + parts + 256;
+    return 2 * a->state_bytes(batch) + a->fpool_bytes(batch) + a->bpool_bytes(batch) + a->part_bytes(batch) +
+           a->sums_bytes(batch) + a->gvec_bytes(batch) + a->epart_bytes(batch) + 256;
 }
 
 int qm_adjoint_run(qm_adjoint* a, UINT batch, const double* theta, const ITYPE* bf, const ITYPE* pf, const UINT* rot,
@@ -698,61 +830,79 @@ int qm_adjoint_run(qm_adjoint* a, UINT batch, const double* theta, const ITYPE* 
         }
     if (!use_device(dev)) return QM_ERR_HIP;
     hipStream_t st = stream_of(stream);
-    if (a->device != (int)dev) {
-        a->release();
-        if (!a->occ_param.empty()) {
-            if (!hip_ok(hipMalloc((void**)&a->d_occ, a->occ_param.size() * sizeof(u32)), what) ||
-                !hip_ok(hipMemcpy(a->d_occ, a->occ_param.data(), a->occ_param.size() * sizeof(u32),
-                                  hipMemcpyHostToDevice),
-                        what))
-                return QM_ERR_HIP;
-        }
-        if (!a->pops.empty()) {
-            if (!hip_ok(hipMalloc((void**)&a->d_ops, a->pops.size() * sizeof(PassOp)), what) ||
-                !hip_ok(hipMemcpy(a->d_ops, a->pops.data(), a->pops.size() * sizeof(PassOp), hipMemcpyHostToDevice),
-                        what))
-                return QM_ERR_HIP;
-        }
-        a->device = (int)dev;
-    }
+    if (!a->prepare(dev, what)) return QM_ERR_HIP;
     Scratch* sc = scratch_for(st);
     if (!sc) return QM_ERR_HIP;
-    const u64 dim = 1ULL << a->n;
-    double2* psi = (double2*)workspace;
-    double2* lam = psi + (u64)batch * dim;
-    double* partials = (double*)(lam + (u64)batch * dim);
-    double* epart = partials + (u64)a->occ_param.size() * batch * kAdjBlocks;
-    std::vector<AdjTerm> ht(nterms);
-    for (UINT k = 0; k < nterms; ++k) ht[k] = AdjTerm{bf[k], pf[k], rot[k], 0, coefs[k]};
-    const AdjTerm* dterms = nterms ? (const AdjTerm*)upload(sc, ht.data(), sizeof(AdjTerm) * nterms) : nullptr;
-    if (nterms && !dterms) return QM_ERR_HIP;
-    const unsigned nblk = kAdjBlocks;
-    const dim3 grid(nblk, batch);
-    k_adj_zero<<<grid, kAdjThreads, 0, st>>>(psi, dim);
-    if (!a->passes.empty()) {
-        for (const PassArgs& pa : a->passes)
-            k_adj_pass<false><<<grid, kAdjThreads, 0, st>>>(psi, lam, dim, pa, a->d_ops, theta, a->nparams, partials);
-    } else {
-        for (const AdjGate& g : a->gates) {
-            if (g.kind == 1) k_adj_rot<true><<<grid, kAdjThreads, 0, st>>>(psi, lam, dim, g, theta, a->nparams, partials);
-            else k_adj_fixed<false, false><<<grid, kAdjThreads, 0, st>>>(psi, lam, dim, g);
+    const u64 dim = 1ULL << a->ne;
+    char* w = (char*)workspace;
+    auto take = [&](u64 bytes) {
+        char* p = w;
+        w += bytes;
+        return p;
+    };
+    double2* psi = (double2*)take(a->state_bytes(batch));
+    double2* lam = (double2*)take(a->state_bytes(batch));
+    double2* fpool = (double2*)take(a->fpool_bytes(batch));
+    double2* bpool = (double2*)take(a->bpool_bytes(batch));
+    double* partials = (double*)take(a->part_bytes(batch));
+    double* sums = (double*)take(a->sums_bytes(batch));
+    double* gvec = (double*)take(a->gvec_bytes(batch));
+    double* epart = (double*)take(a->epart_bytes(batch));
+    // the observable, grouped by bit-flip mask (groups and terms in the order given)
+    std::vector<AdjGroup> groups;
+    std::vector<AdjTerm> terms;
+    {
+        std::vector<bool> done(nterms, false);
+        for (UINT k = 0; k < nterms; ++k) {
+            if (done[k]) continue;
+            AdjGroup g{bf[k], (u32)terms.size(), 0};
+            for (UINT j = k; j < nterms; ++j)
+                if (!done[j] && bf[j] == bf[k]) {
+                    done[j] = true;
+                    terms.push_back(AdjTerm{pf[j], rot[j], 0, coefs[j]});
+                    ++g.nterm;
+                }
+            groups.push_back(g);
         }
     }
-    k_adj_hpsi<<<grid, kAdjThreads, 0, st>>>(psi, lam, dim, dterms, nterms, epart);
-    if (!a->passes.empty()) {
-        for (size_t i = a->passes.size(); i-- > 0;)
-            k_adj_pass<true><<<grid, kAdjThreads, 0, st>>>(psi, lam, dim, a->passes[i], a->d_ops, theta, a->nparams,
-                                                            partials);
-    } else {
-        for (size_t i = a->gates.size(); i-- > 0;) {
-            const AdjGate& g = a->gates[i];
-            if (g.kind == 1) k_adj_rot<false><<<grid, kAdjThreads, 0, st>>>(psi, lam, dim, g, theta, a->nparams, partials);
-            else k_adj_fixed<true, true><<<grid, kAdjThreads, 0, st>>>(psi, lam, dim, g);
+    const AdjGroup* dgroups = nullptr;
+    const AdjTerm* dterms = nullptr;
+    if (nterms) {
+        dgroups = (const AdjGroup*)upload(sc, groups.data(), sizeof(AdjGroup) * groups.size());
+        dterms = (const AdjTerm*)upload(sc, terms.data(), sizeof(AdjTerm) * terms.size());
+        if (!dgroups || !dterms) return QM_ERR_HIP;
+    }
+    MatsArgs ma{a->d_factors, a->d_first, a->d_fixed, a->d_fwd_at, a->d_bwd_at, a->d_copies, a->d_copy_val,
+                a->nops(), a->ncopy_f, a->ncopy_b, a->nparams, a->nocc(), (u32)a->fwd.pool.size(),
+                (u32)a->bwd.pool.size()};
+    const u32 nmat = a->nops() + a->ncopy_f + a->ncopy_b;
+    if (nmat) k_adj_mats<<<dim3((nmat + 63) / 64, batch), 64, 0, st>>>(ma, theta, fpool, bpool, gvec);
+    auto threads = [](u32 lq, u32 most) { return std::max(64u, std::min(most, (1u << lq) >> kAdjK)); };
+    {
+        const dim3 grid((u32)(1ULL << (a->ne - a->lqf)), batch);
+        u32 first = 1;
+        for (const DStage& sg : a->fwd.stages) {
+            k_adj_fwd<<<grid, threads(a->lqf, kFwdThreads), sizeof(double2) << a->lqf, st>>>(
+                psi, a->ne, a->lqf, first, sg, a->d_fpass, a->d_fsub, fpool, (u32)a->fwd.pool.size());
+            first = 0;
         }
     }
-    const u64 outs = std::max<u64>((u64)batch * a->nparams, batch);
-    k_adj_finish<<<(unsigned)((outs + 255) / 256), 256, 0, st>>>(partials, epart, a->d_occ, (u32)a->occ_param.size(),
-                                                                a->nparams, batch, nblk, grad, energy);
+    k_adj_hpsi<<<dim3(a->blocks_h(), batch), kHpsiThreads, 0, st>>>(psi, lam, dim, dgroups, (u32)groups.size(), dterms,
+                                                                   epart);
+    if (a->ncols()) {
+        const dim3 grid(a->blocks_b(), batch);
+        for (size_t s = 0; s < a->bwd.stages.size(); ++s) {
+            if (a->stage_grad0[s] == a->ncols() / 3) break;  // no rotation is left: nothing more to differentiate
+            k_adj_bwd<<<grid, threads(a->lqb, kBwdThreads), 2 * sizeof(double2) << a->lqb, st>>>(
+                psi, lam, a->ne, a->lqb, a->tiles_b(), a->bwd.stages[s], a->stage_grad0[s],
+                a->stage_grad0[s + 1] - a->stage_grad0[s], a->d_bpass, a->d_bsub, bpool, (u32)a->bwd.pool.size(),
+                partials, a->ncols());
+        }
+        k_adj_columns<<<dim3((a->ncols() + 15) / 16, batch), 256, 0, st>>>(partials, a->blocks_b(), a->ncols(), sums);
+    }
+    k_adj_grad<<<dim3(std::max(1u, (a->nparams + 63) / 64), batch), 64, 0, st>>>(
+        sums, a->ncols(), gvec, a->nocc(), a->d_par_first, a->d_par_occs, a->d_occ_col, a->d_occ_coef, a->nparams, grad,
+        epart, a->blocks_h(), energy);
     if (!hip_ok(hipGetLastError(), what)) return QM_ERR_HIP;
     finish_update(st, what);
     return QM_OK;
