@@ -393,8 +393,9 @@ typedef struct qm_adjoint_gate {
 typedef struct qm_adjoint qm_adjoint;
 QM_EXPORT qm_adjoint* qm_adjoint_create(UINT qubit_count, const qm_adjoint_gate* gates, UINT gate_count, UINT param_count);
 QM_EXPORT void qm_adjoint_destroy(qm_adjoint* circuit);
-/* Register-block passes one sweep issues (0: one kernel per gate, for states
- * below 3 qubits or rotations with more than 3 X/Y qubits) and gates. */
+/* Two measures of the gate list: the number of groups it divides into, in order,
+ * when the gates of a group act non-diagonally on at most 3 qubits together (0 for
+ * states below 3 qubits and when a gate alone needs more), and its gates. */
 QM_EXPORT void qm_adjoint_stats(const qm_adjoint* circuit, ITYPE* passes, ITYPE* gates);
 /* Device memory qm_adjoint_run needs for `batch` parameter sets. */
 QM_EXPORT ITYPE qm_adjoint_workspace_bytes(const qm_adjoint* circuit, UINT batch);

@@ -57,7 +57,8 @@ class AdjointCircuit:
             raise _lib.QulacsMI355Error("qm_adjoint_create failed")
 
     def stats(self) -> dict:
-        """Register-block passes per sweep (0: one kernel per gate) and gates."""
+        """Groups of gates over at most three non-diagonal qubits, in order (0: none, see
+        qm_adjoint_stats), and gates."""
         p, g = C.c_ulonglong(), C.c_ulonglong()
         _lib.call("qm_adjoint_stats", self.h, C.byref(p), C.byref(g))
         return {"passes": int(p.value), "gates": int(g.value)}
