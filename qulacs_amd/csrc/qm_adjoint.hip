@@ -24,10 +24,10 @@
 //     (F_m..F_{j+1})^dagger = g_X X + g_Y Y + g_Z Z (k_adj_mats forms g).  A fused
 //     RZ RY costs 12 multiply-adds per amplitude pair for its two gradients.
 //
-// Bound: HBM traffic per stage, then FP64 issue.  20 qubits, 12 layers of RY RZ and a CZ
-// chain, 16 parameter sets (256 MiB per state array): 42.3 ms with one kernel per
-// 3-qubit register block straight from memory (160 passes at 3.0-3.6 TB/s), 11.3 ms
-// with tiles (21 forward stages of 153 us, 24 backward of 327 us: 3.3-3.5 TB/s).
+// Bound: FP64 issue and LDS round trips.  20 qubits, 12 layers of RY RZ and a CZ chain, 16
+// parameter sets (256 MiB per state array): 42.3 ms with one kernel per 3-qubit register block
+// straight from memory (160 passes at 3.0-3.6 TB/s), 11.3 ms with tiles in the order of the gate
+// list (21 forward and 24 backward stages), 7.5 ms with Picker's 6 and 8 stages.
 //
 // Layout: `batch` states of 2^max(n, 4) complex128 each, contiguous (state b at
 // b * dim); theta is batch x params (row-major).  Every reduction is a fixed-order
@@ -39,7 +39,6 @@ namespace qm {
 namespace {
 
 constexpr int kAdjK = 3;             // block qubits of a pass: 8 amplitudes of psi and of lambda per thread
-constexpr u32 kAdjLow = 3;           // qubits 0..2 are in every window: 128-byte runs
 constexpr u32 kFwdLocal = 12;        // forward window: 64 KiB of psi
 constexpr u32 kBwdLocal = 11;        // backward window: 32 KiB of psi and 32 KiB of lambda
 constexpr u32 kFwdThreads = 1u << (kFwdLocal - kAdjK);
@@ -159,12 +158,13 @@ __global__ __launch_bounds__(kFwdThreads, 4) void k_adj_fwd(double2* __restrict_
                                                             const DSub* __restrict__ subs,
                                                             const double2* __restrict__ pool, u32 stride) {
     extern __shared__ double2 st[];
-    __shared__ u64 hi_tab[1u << (kFwdLocal - kAdjLow)];
+    __shared__ u64 hi_tab[1u << (kFwdLocal - kLowFixed)];
     const u32 L = 1u << lq, T = blockDim.x;
     double2* s = psi + ((u64)blockIdx.y << n);
-    build_hi_tab<kAdjLow>(hi_tab, lq, sg);
+    build_hi_tab(hi_tab, lq, sg);
     const u64 tb = tile_base(blockIdx.x, n - lq, sg);
     __syncthreads();
+    if (sg.npass) warm_program(passes[sg.pass0], subs, pool + (u64)blockIdx.y * stride);
     if (first) {
         for (u32 i = threadIdx.x; i < L; i += T)
             st[slot_of(i)] = make_double2(i == 0 && blockIdx.x == 0 ? 1.0 : 0.0, 0.0);
@@ -172,15 +172,15 @@ __global__ __launch_bounds__(kFwdThreads, 4) void k_adj_fwd(double2* __restrict_
 #pragma unroll
         for (u32 k = 0; k < 8; ++k) {
             const u32 i = threadIdx.x + k * kFwdThreads;
-            st[slot_of(i)] = s[tile_index<kAdjLow>(tb, hi_tab, i)];
+            st[slot_of(i)] = s[tile_index(tb, hi_tab, i)];
         }
     } else {
-        for (u32 i = threadIdx.x; i < L; i += T) st[slot_of(i)] = s[tile_index<kAdjLow>(tb, hi_tab, i)];
+        for (u32 i = threadIdx.x; i < L; i += T) st[slot_of(i)] = s[tile_index(tb, hi_tab, i)];
     }
     __syncthreads();
     run_passes<kAdjK, kFwdThreads, 1, false>(st, lq, passes, sg.pass0, sg.npass, subs,
-                                             pool + (u64)blockIdx.y * stride);
-    for (u32 i = threadIdx.x; i < L; i += T) s[tile_index<kAdjLow>(tb, hi_tab, i)] = st[slot_of(i)];
+                                             pool + (u64)blockIdx.y * stride, blockIdx.x);
+    for (u32 i = threadIdx.x; i < L; i += T) s[tile_index(tb, hi_tab, i)] = st[slot_of(i)];
 }
 
 // Wave sums of a, b, c: afterwards every lane of row r (16 lanes) holds the sum of a, b, c
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void k_adj_bwd(double2* __restrict_
                                                             const double2* __restrict__ pools, u32 stride,
                                                             double* __restrict__ partials, u32 ncols) {
     extern __shared__ double2 st[];
-    __shared__ u64 hi_tab[1u << (kBwdLocal - kAdjLow)];
+    __shared__ u64 hi_tab[1u << (kBwdLocal - kLowFixed)];
     __shared__ double acc[kBwdThreads / 64][kStageGrads][3];
     constexpr int D = 1 << kAdjK;
     const u32 L = 1u << lq, T = blockDim.x, tid = threadIdx.x, wave = tid >> 6;
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void k_adj_bwd(double2* __restrict_
     double2* P = psi + ((u64)blockIdx.y << n);
     double2* Q = lam + ((u64)blockIdx.y << n);
     double2* st2 = st + L;
-    build_hi_tab<kAdjLow>(hi_tab, lq, sg);
+    build_hi_tab(hi_tab, lq, sg);
     __syncthreads();
     for (u64 t = blockIdx.x; t < ntiles; t += gridDim.x) {
         const bool add = t != blockIdx.x;  // a later tile of this work-group
@@ -271,13 +271,13 @@ __global__ __launch_bounds__(kBwdThreads, 2) void k_adj_bwd(double2* __restrict_
 #pragma unroll
             for (u32 k = 0; k < 8; ++k) {
                 const u32 i = tid + k * kBwdThreads;
-                const u64 at = tile_index<kAdjLow>(tb, hi_tab, i);
+                const u64 at = tile_index(tb, hi_tab, i);
                 st[slot_of(i)] = P[at];
                 st2[slot_of(i)] = Q[at];
             }
         } else {
             for (u32 i = tid; i < L; i += T) {
-                const u64 at = tile_index<kAdjLow>(tb, hi_tab, i);
+                const u64 at = tile_index(tb, hi_tab, i);
                 st[slot_of(i)] = P[at];
                 st2[slot_of(i)] = Q[at];
             }
@@ -285,6 +285,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void k_adj_bwd(double2* __restrict_
         __syncthreads();
         for (u32 p = 0; p < sg.npass; ++p) {
             const DPass ps = passes[sg.pass0 + p];
+            if (ps.warm) warm_program(ps, subs, pool);
             const bool mine = tid < ngroups;
             u32 base = mine ? tid : 0, slot[D];
 #pragma unroll
@@ -311,10 +312,10 @@ __global__ __launch_bounds__(kBwdThreads, 2) void k_adj_bwd(double2* __restrict_
             u32 k = 0;
             while (k < ps.nsub) {
                 DSub sub = subs[ps.sub0 + k];
-                while ((sub.type & 0xffu) == SUB_LAYER) {
+                while ((sub.type & 15u) == SUB_LAYER) {
                     const u32 d1 = (sub.type >> 8) & 15u;
-                    if (sub.type >> 12) {
-                        const u32 sgn = layer_signs<kAdjK>(sub, base);
+                    if ((sub.type >> 12) | sub.nx) {
+                        const u32 sgn = layer_signs<kAdjK>(sub, base, t);
                         flip_signs<kAdjK>(v, sgn);
                         flip_signs<kAdjK>(l, sgn);
                     }
@@ -351,7 +352,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void k_adj_bwd(double2* __restrict_
             __syncthreads();
         }
         for (u32 i = tid; i < L; i += T) {
-            const u64 at = tile_index<kAdjLow>(tb, hi_tab, i);
+            const u64 at = tile_index(tb, hi_tab, i);
             P[at] = st[slot_of(i)];
             Q[at] = st2[slot_of(i)];
         }
@@ -654,7 +655,7 @@ void qm_adjoint::build(const Builder& b) {
     HCirc hc;
     hc.n = hc.ne = ne;
     hc.ops = b.ops;
-    schedule_circuit(fwd, hc, kAdjK, kFwdLocal, kAdjLow);
+    schedule_circuit(fwd, hc, kAdjK, kFwdLocal);
     std::reverse(hc.ops.begin(), hc.ops.end());
     for (HOp& o : hc.ops)
         if (o.type == 0 && o.q.size() == 2) {  // 4 x 4: conjugate transpose
@@ -662,7 +663,7 @@ void qm_adjoint::build(const Builder& b) {
             for (int r = 0; r < 4; ++r)
                 for (int c = 0; c < 4; ++c) o.m[r * 4 + c] = std::conj(m[c * 4 + r]);
         }
-    schedule_circuit(bwd, hc, kAdjK, kBwdLocal, kAdjLow, kStageGrads);
+    schedule_circuit(bwd, hc, kAdjK, kBwdLocal, kStageGrads);
     // first gradient of each backward stage: stages hold whole passes, in order
     stage_grad0.clear();
     u32 g = 0;

@@ -8,14 +8,15 @@
 // reduction per term).
 //
 // Design:
-//   * one work-group (1024 threads, 512 at K = 4) per circuit, circuits taken from a queue
-//     (an atomic counter) in descending-cost order, so one launch covers a batch
-//     of uneven sizes; every work-group leaves the loop once the queue is empty;
-//   * the state lives in LDS: 2^lq complex128 with lq = min(n, 13) (128 KiB at
-//     13 qubits); circuits of 14..20 qubits keep the state in device memory and
-//     are processed in 2^13-amplitude tiles, one "stage" at a time: a stage is a
-//     set of gates whose qubits all lie in one 13-qubit window (qubits 0..3 are
-//     always in the window, so a tile is made of 256-byte contiguous runs);
+//   * the state lives in LDS, 2^lq complex128 with lq = min(n, 12) (64 KiB at 12 qubits): two
+//     work-groups share a CU, and since they drift apart, one's memory phases and sub-operation
+//     handling overlap the other's FP64 arithmetic;
+//   * a circuit of at most 12 qubits is one work-group, from |0> to its energy; circuits of 13..20
+//     qubits keep the state in device memory and are processed in 2^12-amplitude tiles, one
+//     "stage" at a time: a stage is a set of gates whose dense part lies in one 12-qubit window
+//     (qubits 0..2 are always in the window, so a tile is made of 128-byte contiguous runs;
+//     diagonal gates may touch qubits outside, which are constants of a tile);
+//   * one launch per stage number covers that stage's tiles of every circuit, in descending cost;
 //   * inside a stage the gates are grouped into passes: each pass names K
 //     "block" qubits; a thread loads the 2^K amplitudes that differ in those
 //     bits into registers, applies every gate of the pass (dense gates on block
@@ -28,12 +29,16 @@
 //     (deterministic), with P_k in the mask form of the reference
 //     (src/csim/utility.cpp:12-43): P|x> = i^rot (-1)^popcount(x & pf) |x ^ bf>.
 //
-// Scheduling (host): gates are scanned in order; a gate joins the current
-// stage / pass unless it touches a qubit of a gate skipped earlier in the same
-// scan (then it is skipped too and its qubits are blocked) or it does not fit
-// the window / block.  A gate is therefore only moved ahead of gates it
-// commutes with trivially (disjoint qubits), and every scan schedules at least
-// its first gate.
+// Scheduling (host): see Picker in qm_tile.hpp.
+//
+// Bound: FP64 issue and the latency of the steps around it (sub-operation decoding, LDS round trips,
+// barriers), not HBM: a stage of a 26-qubit brickwork circuit takes 1.13 ms of which its 2.1 GB
+// need 0.4 ms.  26 qubits, 10 layers: 9.87 ms with 13 stages of 13-qubit windows picked in
+// gate order and one work-group per CU; 6.55 ms with Picker's 5 stages and two work-groups per
+// CU; 5.64 ms with shears for three quarters of the matrices.  QAOA (4 layers, ring and
+// chords, 26 qubits): 13.7 -> 10.2 -> 6.0 ms, the last from Z rotations in place of
+// diagonals read per amplitude.  512 circuits of 8 to 16 qubits: 1.75 -> 0.69 ms, from one
+// work-group per tile instead of per circuit.
 #include <cstring>
 
 #include "qm_tile.hpp"
@@ -41,24 +46,25 @@
 namespace qm {
 namespace {
 
-// Work-group size per register-block width: 8 waves at K = 4 (the register
-// block limits a SIMD to 2 waves), 16 waves below, so a CU holding one
-// 128 KiB tile still has 4 waves per SIMD to hide LDS latency.
-template <int K>
-constexpr u32 block_threads() { return K >= 4 ? 512u : 1024u; }
-constexpr u32 kMaxBlockThreads = 1024;
 struct DCirc {
     u32 n, lq, nstage, stage0, term0, nterm;
     u64 state_off;  // complex128 offset of the circuit's state in the scratch buffer
+    u32 chunk0;     // first entry of the circuit's partial energies (circuits of several tiles)
+    u32 pad;
 };
-// This thread's share of sum_k c_k Re <psi|P_k|psi>, reading the state from LDS
-// (swizzled slots) or from device memory.
+struct DItem {
+    u32 circ, tile;
+};
+// Circuits above this size run in tiles; a tile is 64 KiB, so two work-groups share a CU.
+constexpr u32 kTileLocal = 12;
+// This thread's share of sum_k c_k Re <psi|P_k|psi> over amplitudes [x0, x1), reading the
+// state from LDS (swizzled slots) or from device memory; threads [0, stride) take part.
 template <bool FROM_LDS>
 __device__ __forceinline__ double energy_sum(const double2* __restrict__ gs, const double2* st, const DCirc& c,
-                                             const DTerm* __restrict__ terms) {
+                                             const DTerm* __restrict__ terms, u64 x0, u64 x1, u32 stride) {
     double acc = 0.0;
-    const u64 dim = 1ULL << c.n;
-    for (u64 x = threadIdx.x; x < dim; x += blockDim.x) {
+    if (threadIdx.x >= stride) return acc;
+    for (u64 x = x0 + threadIdx.x; x < x1; x += stride) {
         const double2 px = FROM_LDS ? st[slot_of((u32)x)] : gs[x];
         for (u32 k = 0; k < c.nterm; ++k) {
             const DTerm tm = terms[c.term0 + k];
@@ -80,114 +86,78 @@ __device__ __forceinline__ double energy_sum(const double2* __restrict__ gs, con
     return acc;
 }
 
-__global__ void k_batch_reset(int* counter) {
-    if (threadIdx.x == 0) *counter = 0;
-}
-
-// Tiles of one stage of a batched circuit held in device memory (every stage
-// after the first), the next tile loaded into registers while the passes run
-// on the current one.  P amplitudes per thread, T threads.  The loop is laid
-// out as in stage_tiles: unconditional loads of the next tile at the top, the
-// LDS fill from them after the stores of the current tile.
-constexpr u32 kBatchTile = 1u << kMaxLocal;
-template <int K, u32 P, u32 T, int G>
-__device__ __forceinline__ void batch_tiles(double2* st, double2* __restrict__ gs, const u32* hi_tab, u32 lq, u32 tl,
-                                            const DStage& sg, const DPass* __restrict__ passes,
-                                            const DSub* __restrict__ subs, const double2* __restrict__ pool) {
-    const u32 tid = threadIdx.x, ntiles = 1u << tl;
-    {
-        const u64 tb = tile_base(0, tl, sg);
-#pragma unroll
-        for (u32 k = 0; k < P; ++k) st[slot_of(tid + k * T)] = gs[tile_index(tb, hi_tab, tid + k * T)];
-        __syncthreads();
-    }
-    for (u32 t = 0;; ++t) {
-        double rx[P], ry[P];
-        const bool more = t + 1 < ntiles;
-        {
-            const u64 tb = tile_base(t + 1, tl, sg);
-#pragma unroll
-            for (u32 k = 0; k < P; ++k) {
-                const double2 a = gs[more ? tile_index(tb, hi_tab, tid + k * T) : 0];
-                rx[k] = a.x;
-                ry[k] = a.y;
-            }
-        }
-        run_passes<K, T, G>(st, lq, passes, sg.pass0, sg.npass, subs, pool);
-        const u64 tb = tile_base(t, tl, sg);
-#pragma unroll
-        for (u32 k = 0; k < P; ++k) gs[tile_index(tb, hi_tab, tid + k * T)] = st[slot_of(tid + k * T)];
-        __syncthreads();
-        if (!more) break;
-#pragma unroll
-        for (u32 k = 0; k < P; ++k) st[slot_of(tid + k * T)] = make_double2(rx[k], ry[k]);
-        __syncthreads();
-    }
-}
-
-// The program arrays arrive as separate read-only, non-aliasing arguments so the
-// compiler reads them through the scalar cache (inside a by-value struct they
-// became per-lane vector loads).
 template <int K>
-__global__ __launch_bounds__(block_threads<K>()) void k_batch(
+constexpr u32 tile_threads() { return K == 4 ? 256u : 512u; }
+
+// Stage `level` of every circuit that has one, a work-group per (circuit, tile): a circuit of at
+// most 12 qubits is one tile and one stage, from |0> to its energy in LDS; a larger one keeps its
+// state in device memory.  The tiles of a stage are independent, so a 16-qubit circuit is 16
+// work-groups of a launch instead of one work-group's loop over them: 512 circuits of 8 to 16
+// qubits, 4 to 8 layers, were bound by that chain on the largest ones.
+template <int K>
+__global__ __launch_bounds__(tile_threads<K>(), K == 4 ? 2 : 4) void k_batch_level(
     const DCirc* __restrict__ circs, const DStage* __restrict__ stages, const DPass* __restrict__ passes,
     const DSub* __restrict__ subs, const double2* __restrict__ pool, const DTerm* __restrict__ terms,
-    const u32* __restrict__ order, double2* __restrict__ scratch, double* __restrict__ energies, int* counter,
-    u32 ncirc, int keep) {
+    const DItem* __restrict__ items, u32 level, double2* __restrict__ scratch, double* __restrict__ energies, int keep) {
     extern __shared__ double2 st[];
-    __shared__ u32 hi_tab[1u << (kMaxLocal - kLowFixed)];
+    __shared__ u32 hi_tab[1u << (kTileLocal - kLowFixed)];
     __shared__ double red[16];
-    __shared__ int s_slot;
     const u32 tid = threadIdx.x, bd = blockDim.x;
-
-    for (;;) {
-        if (tid == 0) s_slot = atomicAdd(counter, 1);
-        __syncthreads();
-        const int slot = s_slot;
-        __syncthreads();
-        if (slot >= (int)ncirc) break;  // uniform: every thread read the same slot
-        const u32 ci = order[slot];
-        const DCirc c = circs[ci];
-        const u32 lq = c.lq, L = 1u << lq, tl = c.n - lq;
-        double2* gs = scratch + c.state_off;
-
-        for (u32 s = 0; s < c.nstage; ++s) {
-            const DStage sg = stages[c.stage0 + s];
-            if (tl > 0) {
-                build_hi_tab(hi_tab, lq, sg);
-                __syncthreads();
-            }
-            if (tl > 0 && s > 0 && L == kBatchTile) {
-                // one register block per thread (two measured slower here)
-                batch_tiles<K, kBatchTile / block_threads<K>(), block_threads<K>(), 1>(st, gs, hi_tab, lq, tl,
-                                                                                        sg, passes, subs, pool);
-                continue;
-            }
-            for (u32 t = 0; t < (1u << tl); ++t) {
-                const u64 tb = tile_base(t, tl, sg);
-                if (s == 0) {
-                    // |0...0>: slot_of(0) == 0 and amplitude 0 lies in tile 0
-                    for (u32 i = tid; i < L; i += bd) st[i] = make_double2((i == 0 && t == 0) ? 1.0 : 0.0, 0.0);
-                } else {
-                    for (u32 i = tid; i < L; i += bd) st[slot_of(i)] = gs[tile_index(tb, hi_tab, i)];
-                }
-                __syncthreads();
-                run_passes<K, block_threads<K>(), 1>(st, lq, passes, sg.pass0, sg.npass, subs, pool);
-                if (tl > 0) {
-                    for (u32 i = tid; i < L; i += bd) gs[tile_index(tb, hi_tab, i)] = st[slot_of(i)];
-                } else if (keep) {
-                    for (u32 i = tid; i < L; i += bd) gs[i] = st[slot_of(i)];
-                }
-                __syncthreads();
-            }
-        }
-
-        // sum_k c_k Re <psi| P_k |psi>
-        const double acc = tl ? energy_sum<false>(gs, st, c, terms) : energy_sum<true>(gs, st, c, terms);
-        const double total = block_sum(acc, red);
-        if (tid == 0) energies[ci] = total;
+    const DItem it = items[blockIdx.x];
+    const DCirc c = circs[it.circ];
+    const DStage sg = stages[c.stage0 + level];
+    const u32 lq = c.lq, L = 1u << lq, tl = c.n - lq;
+    double2* gs = scratch + c.state_off;
+    const u64 tb = tile_base(it.tile, tl, sg);
+    if (tl > 0) {
+        build_hi_tab(hi_tab, lq, sg);
         __syncthreads();
     }
+    warm_program(passes[sg.pass0], subs, pool);
+    if (level == 0) {
+        // |0...0>: slot_of(0) == 0 and amplitude 0 lies in tile 0
+        for (u32 i = tid; i < L; i += bd) st[i] = make_double2((i == 0 && it.tile == 0) ? 1.0 : 0.0, 0.0);
+    } else {
+        for (u32 i = tid; i < L; i += bd) st[slot_of(i)] = gs[tile_index(tb, hi_tab, i)];
+    }
+    __syncthreads();
+    run_passes<K, tile_threads<K>(), 1>(st, lq, passes, sg.pass0, sg.npass, subs, pool, it.tile);
+    if (tl > 0) {
+        for (u32 i = tid; i < L; i += bd) gs[tile_index(tb, hi_tab, i)] = st[slot_of(i)];
+        return;
+    }
+    if (keep)
+        for (u32 i = tid; i < L; i += bd) gs[i] = st[slot_of(i)];
+    // a thread count that depends on the circuit alone: its energy does not depend on the batch
+    const u32 part = min(tile_threads<K>(), max(64u, L >> K));
+    const double total = block_sum(energy_sum<true>(gs, st, c, terms, 0, L, part), red);
+    if (tid == 0) energies[it.circ] = total;
+}
+
+// Energies of the circuits of several tiles: partial sums over 2^12 amplitudes, then one thread per
+// circuit adds them in order.
+__global__ __launch_bounds__(256) void k_batch_energy(const DCirc* __restrict__ circs, const DTerm* __restrict__ terms,
+                                                      const DItem* __restrict__ items, const double2* __restrict__ scratch,
+                                                      double* __restrict__ partials) {
+    __shared__ double red[16];
+    const DItem it = items[blockIdx.x];
+    const DCirc c = circs[it.circ];
+    const u64 x0 = (u64)it.tile << kTileLocal;
+    const u64 x1 = x0 + (1ULL << kTileLocal), dim = 1ULL << c.n;
+    const double total =
+        block_sum(energy_sum<false>(scratch + c.state_off, nullptr, c, terms, x0, x1 < dim ? x1 : dim, 256), red);
+    if (threadIdx.x == 0) partials[c.chunk0 + it.tile] = total;
+}
+__global__ __launch_bounds__(64) void k_batch_finish(const DCirc* __restrict__ circs, const u32* __restrict__ large,
+                                                     u32 nlarge, const double* __restrict__ partials,
+                                                     double* __restrict__ energies) {
+    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nlarge) return;
+    const DCirc c = circs[large[i]];
+    const u32 chunks = c.n > kTileLocal ? 1u << (c.n - kTileLocal) : 1u;
+    double e = 0.0;
+    for (u32 k = 0; k < chunks; ++k) e += partials[c.chunk0 + k];
+    energies[large[i]] = e;
 }
 
 // One stage of a single-state circuit: every work-group takes tiles of 2^lq
@@ -244,7 +214,7 @@ __device__ __forceinline__ void stage_tiles(double2* __restrict__ state, double2
                 ry[k] = x.y;
             }
         }
-        run_passes<K, T, stage_blocks<K>()>(st, lq, passes, sg.pass0, sg.npass, subs, pool);
+        run_passes<K, T, stage_blocks<K>()>(st, lq, passes, sg.pass0, sg.npass, subs, pool, t);
         const u64 tb = tile_base(t, tl, sg);
 #pragma unroll
         for (u32 k = 0; k < P; ++k) state[tile_index(tb, hi_tab, tid + k * T)] = st[slot_of(tid + k * T)];
@@ -291,9 +261,48 @@ __global__ __launch_bounds__(stage_threads<K>()) void k_stage(double2* __restric
         const u64 tb = tile_base(t, tl, sg);
         for (u32 i = threadIdx.x; i < L; i += T) st[slot_of(i)] = state[tile_index(tb, hi_tab, i)];
         __syncthreads();
-        run_passes<K, T, stage_blocks<K>()>(st, lq, passes, sg.pass0, sg.npass, subs, pool);
+        run_passes<K, T, stage_blocks<K>()>(st, lq, passes, sg.pass0, sg.npass, subs, pool, t);
         for (u32 i = threadIdx.x; i < L; i += T) state[tile_index(tb, hi_tab, i)] = st[slot_of(i)];
         __syncthreads();
+    }
+}
+
+// One stage of a single-state circuit with a work-group per tile of at most 2^12 amplitudes: two or more groups share a
+// CU and drift apart, so one's memory phase overlaps another's passes without a prefetch.
+template <int K>
+__global__ __launch_bounds__(tile_threads<K>(), K == 4 ? 2 : 4) void k_tile(double2* __restrict__ state, u32 lq, u32 tl,
+                                                                            DStage sg, const DPass* __restrict__ passes,
+                                                                            const DSub* __restrict__ subs,
+                                                                            const double2* __restrict__ pool) {
+    extern __shared__ double2 st[];
+    __shared__ u64 hi_tab[1u << (kTileLocal - kLowFixed)];
+    constexpr u32 T = tile_threads<K>();
+    const u32 L = 1u << lq;
+    build_hi_tab(hi_tab, lq, sg);
+    const u64 tb = tile_base(blockIdx.x, tl, sg);
+    __syncthreads();
+    constexpr u32 P = (1u << kTileLocal) / T;
+    if (L == P * T) {
+        double2 r[P];
+#pragma unroll
+        for (u32 k = 0; k < P; ++k) r[k] = state[tile_index(tb, hi_tab, threadIdx.x + k * T)];
+        warm_program(passes[sg.pass0], subs, pool);  // while the tile is on its way
+#pragma unroll
+        for (u32 k = 0; k < P; ++k) st[slot_of(threadIdx.x + k * T)] = r[k];
+    } else {
+        warm_program(passes[sg.pass0], subs, pool);
+        for (u32 i = threadIdx.x; i < L; i += blockDim.x) st[slot_of(i)] = state[tile_index(tb, hi_tab, i)];
+    }
+    __syncthreads();
+    run_passes<K, T, 1>(st, lq, passes, sg.pass0, sg.npass, subs, pool, blockIdx.x);
+    if (L == P * T) {
+#pragma unroll
+        for (u32 k = 0; k < P; ++k) {
+            const u32 i = threadIdx.x + k * T;
+            state[tile_index(tb, hi_tab, i)] = st[slot_of(i)];
+        }
+    } else {
+        for (u32 i = threadIdx.x; i < L; i += blockDim.x) state[tile_index(tb, hi_tab, i)] = st[slot_of(i)];
     }
 }
 
@@ -334,7 +343,6 @@ struct qm_batch {
     int device = -1;
     unsigned K = 0;
     int keep = 0;
-    unsigned lq_max = 0;
     std::vector<qm::DCirc> h_circs;
     qm::u64 n_stages = 0, n_passes = 0, n_subs = 0;
     qm::DCirc* d_circs = nullptr;
@@ -343,12 +351,19 @@ struct qm_batch {
     qm::DSub* d_subs = nullptr;
     double2* d_pool = nullptr;
     qm::DTerm* d_terms = nullptr;
-    qm::u32* d_order = nullptr;
+    qm::DItem* d_items = nullptr;     // the launches' items one after another, then the energy items
+    qm::u32* d_large = nullptr;       // circuits of several tiles
     double2* d_scratch = nullptr;
     double* d_energies = nullptr;
-    int* d_counter = nullptr;
-    size_t cap[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};  // bytes held by each device buffer above
-    int grid = 0;                       // work-groups of the launch (computed once per compile)
+    double* d_partials = nullptr;
+    struct Level {
+        qm::u32 first, count, lq;  // items; the largest tile among them
+    };
+    std::vector<Level> levels;
+    Level energy_items{0, 0, 0};
+    qm::u32 n_large = 0;
+    size_t cap[11] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};  // bytes held by each device buffer above
+    bool lds_set = false;               // the kernel's LDS limit has been raised on this device
     unsigned lq_cap = 13;               // qubits held in LDS per tile (qm_batch_set_local_qubits)
     hipGraph_t graph = nullptr;         // captured launch (qm_batch_capture)
     hipGraphExec_t graph_exec = nullptr;
@@ -361,15 +376,16 @@ struct qm_batch {
 
     void release() {
         drop_graph();
-        grid = 0;
+        lds_set = false;
         if (device >= 0) {
             (void)hipSetDevice(device);
-            void* ptrs[] = {d_circs, d_stages, d_passes, d_subs, d_pool, d_terms, d_order, d_scratch, d_energies, d_counter};
+            void* ptrs[] = {d_circs, d_stages, d_passes, d_subs, d_pool, d_terms, d_items, d_large, d_scratch, d_energies, d_partials};
             for (void* p : ptrs)
                 if (p) (void)hipFree(p);
         }
         d_circs = nullptr; d_stages = nullptr; d_passes = nullptr; d_subs = nullptr; d_pool = nullptr;
-        d_terms = nullptr; d_order = nullptr; d_scratch = nullptr; d_energies = nullptr; d_counter = nullptr;
+        d_terms = nullptr; d_items = nullptr; d_large = nullptr; d_scratch = nullptr; d_energies = nullptr;
+        d_partials = nullptr;
         for (size_t& c : cap) c = 0;
         device = -1;
         h_circs.clear();
@@ -403,22 +419,16 @@ struct qm_circuit {
 namespace qm {
 namespace {
 
-// Sets the kernel's LDS limit and sizes the grid (resident work-groups, at most
-// one per circuit).  Kept out of the launch path so a graph capture only sees
+// Raises the kernel's LDS limit.  Kept out of the launch path so a graph capture only sees
 // stream operations.
-bool batch_prepare_launch(qm_batch* b, unsigned dev, const char* what) {
-    const size_t lds = sizeof(double2) << b->lq_max;
-    const void* fn = b->K == 2 ? (const void*)k_batch<2> : b->K == 3 ? (const void*)k_batch<3> : (const void*)k_batch<4>;
-    if (!hip_ok(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), what)) return false;
-    int per_cu = 0, cus = 0;
-    const int threads = (int)(b->K == 2 ? block_threads<2>() : b->K == 3 ? block_threads<3>() : block_threads<4>());
-    if (!hip_ok(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, lds), what)) return false;
-    if (!hip_ok(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, (int)dev), what)) return false;
-    if (per_cu < 1) {
-        set_error(QM_ERR_HIP, "%s: the kernel does not fit a compute unit with %zu bytes of LDS", what, lds);
+bool batch_prepare_launch(qm_batch* b, const char* what) {
+    const void* fn = b->K == 2   ? (const void*)k_batch_level<2>
+                     : b->K == 3 ? (const void*)k_batch_level<3>
+                                 : (const void*)k_batch_level<4>;
+    if (!hip_ok(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(sizeof(double2) << kTileLocal)),
+                what))
         return false;
-    }
-    b->grid = (int)std::min<u64>(b->h_circs.size(), (u64)per_cu * cus);
+    b->lds_set = true;
     return true;
 }
 
@@ -491,60 +501,86 @@ int qm_batch_compile(qm_batch* b, UINT block_qubits, int keep_states, unsigned d
                 return QM_ERR_INVALID_ARGUMENT;
             }
     if (b->device >= 0 && b->device != (int)dev) b->release();
-    b->drop_graph();  // device buffers and the queue length may change
-    b->grid = 0;
+    b->drop_graph();  // device buffers and the launches may change
+    b->lds_set = false;
     b->h_circs.clear();
     if (!use_device(dev)) return QM_ERR_HIP;
-    Flat f;    std::vector<DTerm> terms;
+    Flat f;
+    std::vector<DTerm> terms;
     std::vector<DCirc> dc;
     u64 state_off = 0;
-    u32 lq_max = kMinQubits;
+    const u32 lq_cap = std::min((u32)b->lq_cap, kTileLocal);
+    u32 nlevel = 0, nchunk = 0;
+    std::vector<u32> large;
+    std::vector<DItem> energy;
     for (const HCirc& c : b->circs) {
         DCirc d{};
         d.n = c.ne;
-        d.lq = std::min(c.ne, (u32)b->lq_cap);
+        d.lq = std::min(c.ne, lq_cap);
         d.stage0 = (u32)f.stages.size();
-        d.nstage = schedule_circuit(f, c, K, b->lq_cap);
+        d.nstage = schedule_circuit(f, c, K, lq_cap);
         d.term0 = (u32)terms.size();
         d.nterm = (u32)c.terms.size();
         terms.insert(terms.end(), c.terms.begin(), c.terms.end());
         d.state_off = state_off;
-        if (c.ne > b->lq_cap || keep_states) state_off += 1ULL << c.ne;
-        lq_max = std::max(lq_max, d.lq);
+        if (c.ne > lq_cap || keep_states) state_off += 1ULL << c.ne;
+        nlevel = std::max(nlevel, d.nstage);
+        if (c.ne > lq_cap) {
+            const u32 chunks = c.ne > kTileLocal ? 1u << (c.ne - kTileLocal) : 1u;
+            d.chunk0 = nchunk;
+            for (u32 k = 0; k < chunks; ++k) energy.push_back({(u32)dc.size(), k});
+            nchunk += chunks;
+            large.push_back((u32)dc.size());
+        }
         dc.push_back(d);
     }
-    // descending cost: amplitudes x (passes + terms)
-    std::vector<u32> order(dc.size());
-    std::vector<double> cost(dc.size());
-    for (size_t i = 0; i < dc.size(); ++i) {
-        u64 np = 0;
-        for (u32 s = 0; s < dc[i].nstage; ++s) np += f.stages[dc[i].stage0 + s].npass;
-        cost[i] = std::ldexp(1.0, (int)dc[i].n) * (double)(np + dc[i].nterm + 1);
-        order[i] = (u32)i;
+    // each level's items in descending cost (amplitudes x (passes + terms of a single tile), so that
+    // the last work-groups of a launch are short ones
+    std::vector<DItem> items;
+    std::vector<qm_batch::Level> levels;
+    for (u32 lv = 0; lv < nlevel; ++lv) {
+        std::vector<std::pair<double, u32>> order;
+        for (u32 i = 0; i < dc.size(); ++i) {
+            if (dc[i].nstage <= lv) continue;
+            const double work = f.stages[dc[i].stage0 + lv].npass + (dc[i].n == dc[i].lq ? dc[i].nterm + 1 : 1);
+            order.emplace_back(std::ldexp(work, (int)dc[i].lq), i);
+        }
+        std::stable_sort(order.begin(), order.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
+        qm_batch::Level L{(u32)items.size(), 0, kMinQubits};
+        for (const auto& o : order) {
+            L.lq = std::max(L.lq, dc[o.second].lq);
+            for (u32 t = 0; t < 1u << (dc[o.second].n - dc[o.second].lq); ++t) items.push_back({o.second, t});
+        }
+        L.count = (u32)items.size() - L.first;
+        levels.push_back(L);
     }
-    std::stable_sort(order.begin(), order.end(), [&](u32 x, u32 y) { return cost[x] > cost[y]; });
+    const qm_batch::Level energy_items{(u32)items.size(), (u32)energy.size(), 0};
+    items.insert(items.end(), energy.begin(), energy.end());
     if (f.pool.empty()) f.pool.push_back(make_double2(0, 0));
     if (f.subs.empty()) f.subs.push_back(DSub{});
     if (f.passes.empty()) f.passes.push_back(DPass{});
     if (terms.empty()) terms.push_back(DTerm{});
+    if (items.empty()) items.push_back(DItem{});
     b->device = (int)dev;
     bool ok = dev_put(&b->d_circs, &b->cap[0], dc, what) && dev_put(&b->d_stages, &b->cap[1], f.stages, what) &&
               dev_put(&b->d_passes, &b->cap[2], f.passes, what) && dev_put(&b->d_subs, &b->cap[3], f.subs, what) &&
               dev_put(&b->d_pool, &b->cap[4], f.pool, what) && dev_put(&b->d_terms, &b->cap[5], terms, what) &&
-              dev_put(&b->d_order, &b->cap[6], order, what);
+              dev_put(&b->d_items, &b->cap[6], items, what) && dev_put(&b->d_large, &b->cap[10], large, what);
     if (ok && state_off) {
         ok = dev_reserve((void**)&b->d_scratch, &b->cap[7], state_off * sizeof(double2), what);
         if (!ok) set_error(QM_ERR_OUT_OF_MEMORY, "%s: %llu bytes of state memory", what, state_off * 16ULL);
     }
     if (ok) ok = dev_reserve((void**)&b->d_energies, &b->cap[8], std::max<size_t>(1, dc.size()) * sizeof(double), what);
-    if (ok) ok = dev_reserve((void**)&b->d_counter, &b->cap[9], sizeof(int), what);
+    if (ok) ok = dev_reserve((void**)&b->d_partials, &b->cap[9], std::max<size_t>(1, nchunk) * sizeof(double), what);
     if (!ok) {
         b->release();
         return QM_ERR_HIP;
     }
     b->K = K;
     b->keep = keep_states ? 1 : 0;
-    b->lq_max = lq_max;
+    b->levels = levels;
+    b->energy_items = energy_items;
+    b->n_large = (u32)large.size();
     b->h_circs = dc;
     b->n_stages = f.stages.size();
     b->n_passes = 0;
@@ -565,19 +601,28 @@ const double* qm_batch_run_async(qm_batch* b, void* stream, unsigned dev) {
     hipStream_t st = stream_of(stream);
     const u32 ncirc = (u32)b->h_circs.size();
     if (ncirc == 0) return b->d_energies;
-    const size_t lds = sizeof(double2) << b->lq_max;
-    if (b->grid == 0 && !batch_prepare_launch(b, dev, what)) return nullptr;
-    const u32 grid = (u32)b->grid;
-#define QM_BATCH_ARGS                                                                                       \
-    b->d_circs, b->d_stages, b->d_passes, b->d_subs, b->d_pool, b->d_terms, b->d_order, b->d_scratch, b->d_energies, \
-        b->d_counter, ncirc, b->keep
-    k_batch_reset<<<1, 64, 0, st>>>(b->d_counter);
-    switch (b->K) {
-        case 2: k_batch<2><<<grid, block_threads<2>(), lds, st>>>(QM_BATCH_ARGS); break;
-        case 3: k_batch<3><<<grid, block_threads<3>(), lds, st>>>(QM_BATCH_ARGS); break;
-        default: k_batch<4><<<grid, block_threads<4>(), lds, st>>>(QM_BATCH_ARGS); break;
+    if (!b->lds_set && !batch_prepare_launch(b, what)) return nullptr;
+    for (size_t lv = 0; lv < b->levels.size(); ++lv) {
+        const qm_batch::Level& L = b->levels[lv];
+        const size_t lds = sizeof(double2) << L.lq;
+        const u32 groups = (1u << L.lq) >> b->K;
+#define QM_BATCH_LEVEL(KK)                                                                                         \
+    k_batch_level<KK><<<L.count, std::max(64u, std::min(tile_threads<KK>(), groups)), lds, st>>>(                  \
+        b->d_circs, b->d_stages, b->d_passes, b->d_subs, b->d_pool, b->d_terms, b->d_items + L.first, (u32)lv,     \
+        b->d_scratch, b->d_energies, b->keep)
+        switch (b->K) {
+            case 2: QM_BATCH_LEVEL(2); break;
+            case 3: QM_BATCH_LEVEL(3); break;
+            default: QM_BATCH_LEVEL(4); break;
+        }
+#undef QM_BATCH_LEVEL
     }
-#undef QM_BATCH_ARGS
+    if (b->n_large) {
+        k_batch_energy<<<b->energy_items.count, 256, 0, st>>>(b->d_circs, b->d_terms, b->d_items + b->energy_items.first,
+                                                             b->d_scratch, b->d_partials);
+        k_batch_finish<<<(b->n_large + 63) / 64, 64, 0, st>>>(b->d_circs, b->d_large, b->n_large, b->d_partials,
+                                                              b->d_energies);
+    }
     if (!hip_ok(hipGetLastError(), what)) return nullptr;
     return b->d_energies;
 }
@@ -620,7 +665,7 @@ int qm_batch_capture(qm_batch* b, void* stream, unsigned dev) {
         return QM_ERR_INVALID_ARGUMENT;
     }
     if (!use_device(dev)) return QM_ERR_HIP;
-    if (b->grid == 0 && !batch_prepare_launch(b, dev, what)) return QM_ERR_HIP;
+    if (!b->lds_set && !batch_prepare_launch(b, what)) return QM_ERR_HIP;
     b->drop_graph();
     hipStream_t st = stream_of(stream);
     if (!hip_ok(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal), what)) return QM_ERR_HIP;
@@ -684,14 +729,19 @@ void* qm_batch_state_device_ptr(qm_batch* b, UINT index) {
 qm_circuit* qm_circuit_create(UINT n, const qm_batch_gate* gates, UINT gate_count, UINT block_qubits,
                               UINT local_qubits) {
     const char* what = "qm_circuit_create";
-    // Defaults (0): up to 19 qubits a 13-qubit window leaves at most 64 tiles
-    // per stage for 256 CUs; 12-qubit windows with 3-qubit blocks were 11-28 %
-    // faster there on brickwork circuits (13 q: 0.198 -> 0.149 ms, 14 q: 0.130
-    // -> 0.093 ms, 18 q: 0.179 -> 0.133 ms; 10-12 q, one stage: 15-20 % from the
-    // block width alone), equal at 20 and slower from 21 qubits up.
-    const bool small_state = n <= 19;
-    u32 K = block_qubits ? block_qubits : (small_state ? 3 : 4);
-    const u32 lq = local_qubits ? local_qubits : (small_state ? 12 : kMaxLocal);
+    // Defaults (0): 3-qubit blocks and 12-qubit windows (two work-groups per CU).  Against 4-qubit
+    // blocks and 13-qubit windows (one per CU, prefetched), brickwork of 10 layers: 52 / 67 us
+    // at 12 qubits, 83 / 116 at 16, 166 / 191 at 20, 405 / 398 at 22, 1377 / 1654 at 24,
+    // 5.64 / 6.59 ms at 26; QAOA and random circuits alike.  A 13-qubit window only pays where
+    // it saves a stage of a circuit with next to no arithmetic: one layer at 22 qubits 114 / 108 us
+    // (at 20 qubits 37 / 48, at 24 371 / 509), so 20 to 22 qubits with at most one
+    // matrix per qubit keep it.
+    UINT dense = 0;
+    if (gates)
+        for (UINT i = 0; i < gate_count; ++i) dense += gates[i].kind == QM_BATCH_DENSE;
+    const bool wide = n >= 20 && n <= 22 && dense <= n;
+    u32 K = block_qubits ? block_qubits : (wide ? 4 : 3);
+    const u32 lq = local_qubits ? local_qubits : (wide ? kMaxLocal : kTileLocal);
     if (n < kMinQubits || n > QM_CIRCUIT_MAX_QUBITS || K < 2 || K > 4 || lq < 8 || lq > kMaxLocal ||
         (gate_count && !gates)) {
         set_error(QM_ERR_INVALID_ARGUMENT,
@@ -774,6 +824,23 @@ bool circuit_enqueue(qm_circuit* c, void* state, u64 dim, hipStream_t st, unsign
     }
     if (!circuit_prepare(c, dev)) return false;
     const size_t lds = sizeof(double2) << c->lq;
+    const u32 tl = c->n - c->lq;
+    const u64 ntiles = 1ULL << tl;
+    if (c->lq <= 12 && c->K >= 3) {
+        const void* kt = c->K == 3 ? (const void*)k_tile<3> : (const void*)k_tile<4>;
+        if (c->per_cu == 0) {
+            if (!hip_ok(hipFuncSetAttribute(kt, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(sizeof(double2) << 12)), what))
+                return false;
+            c->per_cu = 1;
+        }
+        const u32 T = std::max(64u, std::min(c->K == 3 ? tile_threads<3>() : tile_threads<4>(), (1u << c->lq) >> c->K));
+        for (const DStage& sg : c->stages) {
+            if (sg.npass == 0) continue;
+            if (c->K == 3) k_tile<3><<<(u32)ntiles, T, lds, st>>>((double2*)state, c->lq, tl, sg, c->d_passes, c->d_subs, c->d_pool);
+            else k_tile<4><<<(u32)ntiles, T, lds, st>>>((double2*)state, c->lq, tl, sg, c->d_passes, c->d_subs, c->d_pool);
+        }
+        return hip_ok(hipGetLastError(), what);
+    }
     const void* fn = c->K == 2 ? (const void*)k_stage<2> : c->K == 3 ? (const void*)k_stage<3> : (const void*)k_stage<4>;
     if (c->per_cu == 0) {
         int per_cu = 0, cus = 0;
@@ -788,8 +855,6 @@ bool circuit_enqueue(qm_circuit* c, void* state, u64 dim, hipStream_t st, unsign
         c->per_cu = per_cu;
         c->cus = cus;
     }
-    const u32 tl = c->n - c->lq;
-    const u64 ntiles = 1ULL << tl;
     const u32 grid = (u32)std::min<u64>(ntiles, (u64)c->per_cu * c->cus);
     for (const DStage& sg : c->stages) {
         if (sg.npass == 0) continue;

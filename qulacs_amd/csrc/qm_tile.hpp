@@ -19,31 +19,40 @@ namespace {
 using cd = std::complex<double>;
 
 constexpr u32 kMaxLocal = 13;   // qubits resident in LDS
-constexpr u32 kLowFixed = 4;    // qubits 0..3 are local in every stage (the executors; LOW below)
+constexpr u32 kLowFixed = 3;    // qubits 0..2 are local in every stage: a tile is made of 128-byte runs
 constexpr u32 kMinQubits = 4;   // smaller circuits run on 4 qubits (extra qubits stay |0>)
 
-// Sub-operation kinds (low byte of DSub::type).
+// Sub-operation kinds (low 4 bits of DSub::type).
 // LAYER: CZ gates, then one 2x2 matrix on each block bit of a mask.  type bits
-//   8..11: the block-bit mask; bits 16..31: the sign pattern over the register
+//   8..11: the block-bit mask; bits 4..7: those whose matrix is two shears; bits 16..31: the sign pattern over the register
 //   block of the CZs between two block bits; bit 15: a and m hold, for block
 //   bit i, the mask of local positions outside the block that share a CZ with
 //   it (16 bits each: a = M0 | M1 << 16, m = M2 | M3 << 16), so the sign of
 //   register slot j changes with the parity of base & M_i where bit i of j is
 //   set; bits 12..14: the number (<= 4) of CZs between two positions outside
-//   the block, byte c of pairs = p | q << 4.
-//   data: the matrices (4 complex each) of the mask's bits in ascending order.
+//   the block, byte c of pairs = p | q << 4; nx: the number (<= 8) of CZs between a
+//   local position and a qubit outside the window, item c of x (16 bits each) =
+//   tile bit | p << 8, p the local position or 0x80 | block bit.
+//   data: the matrices (4 complex each; a, b and two unused for shears) of the mask's bits
+//   in ascending order.
 // D2: 4x4 on block bits byte 0 / byte 1 of a; DK: 2^K x 2^K on the block;
-// DIAG: diagonal on the m local positions in the bytes of a.
-enum : u32 { SUB_LAYER = 0, SUB_D2 = 1, SUB_DK = 2, SUB_DIAG = 3 };
+// DIAG: diagonal on the m qubits in the bytes of a (a local position, or kTileQubit
+// | tile bit for a qubit outside the window).
+// ZROT: amplitudes with even parity of the index bits of a mask times c + i s, the others
+// times c - i s; a = mask of local positions outside the block | block-bit mask << 16, x[0]:
+// mask of tile bits, data: c + i s.
+enum : u32 { SUB_LAYER = 0, SUB_D2 = 1, SUB_DK = 2, SUB_DIAG = 3, SUB_ZROT = 4 };
 // bits 16 i .. 16 i + 15: the register-block indices j (< 16) with bit i set
 constexpr u64 kBlockPatterns = 0xFF00F0F0CCCCAAAAull;
 constexpr u32 kCzPairsMax = 4;
+constexpr u32 kCzTileMax = 8;
+constexpr u32 kTileQubit = 0x40;  // in a stage's operations: qubit kTileQubit | i is tile bit i
 
 // Qubit lists are packed one byte per entry into 64-bit words so that the
 // kernel indexes them with shifts (a runtime index into an array would put it
 // in private memory).
 struct DStage {
-    u64 win[2];   // local bit LOW + i <-> qubit byte i of win (i < lq - LOW <= 10)
+    u64 win[2];   // local bit kLowFixed + i <-> qubit byte i of win (i < lq - kLowFixed <= 10)
     u64 comp[4];  // tile bit i <-> qubit byte i of comp (i < n - lq <= 32)
     u32 npass, pass0;
 };
@@ -54,7 +63,12 @@ struct DPass {
     u32 nsub, sub0;
     u32 flags;             // kPassHasDiag: a DIAG sub-operation (one register block per thread)
     unsigned short sbit[4];   // slot_of(1 << pos[i]), computed on the host
+    u32 pool0;                // first pool entry of the pass
+    // set in the first pass of a chunk of passes: bytes of the chunk's sub-operations, and of its
+    // pool entries << 16, for warm_program
+    u32 warm;
 };
+constexpr u32 kWarmBytes = 6144;  // per chunk: the scalar cache holds 16 KiB for two CUs
 constexpr u32 kPassHasDiag = 1;
 struct DSub {
     u32 type;
@@ -64,7 +78,8 @@ struct DSub {
     u32 pairs;  // LAYER: CZs between two positions outside the block
     u32 grad0;  // LAYER: position in Flat::grads of the first matrix in gmask
     u32 gmask;  // LAYER: block bits whose matrix belongs to an operation with grad set
-    u32 pad;
+    u32 nx;     // LAYER: CZs with a qubit outside the window
+    u64 x[2];
 };
 struct DTerm {
     u64 bf, pf;
@@ -73,14 +88,17 @@ struct DTerm {
 };
 
 struct HOp {
-    u32 type;  // 0 dense, 1 diag, 2 cz
+    // 0 dense, 1 diag, 2 cz, 3 exp(i phi Z...Z) on q with m[0] = exp(i phi)
+    u32 type;
     std::vector<u32> q;
     std::vector<cd> m;
+    bool reduced = false;  // single-qubit dense: m = {a, b, 0, 0} for [[1, 0], [b, 1]] [[1, a], [0, 1]]
     long id = -1;       // the caller's number of a single-qubit dense operation (see Flat::mats)
     bool grad = false;  // listed in Flat::grads
-    u64 mask() const {
+    u64 mask() const {  // tile bits aside
         u64 r = 0;
-        for (u32 x : q) r |= 1ULL << x;
+        for (u32 x : q)
+            if (x < kTileQubit) r |= 1ULL << x;
         return r;
     }
 };
@@ -95,38 +113,6 @@ struct HCirc {
 __host__ __device__ __forceinline__ u32 fold3(u32 x) { return ((x >> 3) ^ (x >> 6) ^ (x >> 9) ^ (x >> 12)) & 7u; }
 __host__ __device__ __forceinline__ u32 slot_of(u32 x) { return x ^ fold3(x); }
 
-// (x, y) <- (m0 x + m1 y, m2 x + m3 y), complex, updated in place; the matrix
-// entries are wave-uniform (scalar registers).  Written as one asm block so the
-// four results land in the registers of the four inputs: the sub-operation loop
-// of run_passes then keeps the register block at fixed registers across all
-// sub-operation kinds instead of copying it at every merge point.  The last
-// reader of each input writes a result into it (x.re holds the x.re chain from
-// its 4th op on), so three temporaries suffice.
-__device__ __forceinline__ void pair_update(double2& x, double2& y, const double2 m0, const double2 m1,
-                                            const double2 m2, const double2 m3) {
-    double tb, tc, td;
-    asm("v_mul_f64 %[tb], %[m0i], %[xr]\n\t"          // B = x'.im
-        "v_mul_f64 %[tc], %[m2r], %[xr]\n\t"          // C = y'.re
-        "v_mul_f64 %[td], %[m2i], %[xr]\n\t"          // D = y'.im
-        "v_mul_f64 %[xr], %[m0r], %[xr]\n\t"          // A = x'.re
-        "v_fma_f64 %[xr], -%[m0i], %[xi], %[xr]\n\t"
-        "v_fma_f64 %[tb], %[m0r], %[xi], %[tb]\n\t"
-        "v_fma_f64 %[tc], -%[m2i], %[xi], %[tc]\n\t"
-        "v_fma_f64 %[td], %[m2r], %[xi], %[td]\n\t"
-        "v_fma_f64 %[xr], %[m1r], %[yr], %[xr]\n\t"
-        "v_fma_f64 %[tb], %[m1i], %[yr], %[tb]\n\t"
-        "v_fma_f64 %[tc], %[m3r], %[yr], %[tc]\n\t"
-        "v_fma_f64 %[td], %[m3i], %[yr], %[td]\n\t"
-        "v_fma_f64 %[xi], %[m1r], %[yi], %[tb]\n\t"
-        "v_fma_f64 %[yr], -%[m3i], %[yi], %[tc]\n\t"
-        "v_fma_f64 %[xr], -%[m1i], %[yi], %[xr]\n\t"
-        "v_fma_f64 %[yi], %[m3r], %[yi], %[td]"
-        : [xr] "+v"(x.x), [xi] "+v"(x.y), [yr] "+v"(y.x), [yi] "+v"(y.y), [tb] "=&v"(tb), [tc] "=&v"(tc),
-          [td] "=&v"(td)
-        : [m0r] "s"(m0.x), [m0i] "s"(m0.y), [m1r] "s"(m1.x), [m1i] "s"(m1.y), [m2r] "s"(m2.x), [m2i] "s"(m2.y),
-          [m3r] "s"(m3.x), [m3i] "s"(m3.y));
-}
-
 // v <- v * z, complex, in place.
 __device__ __forceinline__ void cmul_inplace(double2& v, const double2 z) {
     double t;
@@ -138,9 +124,14 @@ __device__ __forceinline__ void cmul_inplace(double2& v, const double2 z) {
         : [zr] "v"(z.x), [zi] "v"(z.y));
 }
 
-// Two independent pair updates interleaved instruction by instruction, so a
-// dependent FMA follows its producer 8 instructions later (pair_update alone:
-// 4), which keeps the FP64 pipeline busy with only two waves per SIMD.
+// (x, y) <- (m0 x + m1 y, m2 x + m3 y), complex, on two pairs, updated in place; the matrix
+// entries are wave-uniform (scalar registers).  Written as one asm block so the results land in
+// the registers of the inputs: the sub-operation loop then keeps the register block at
+// fixed registers instead of copying it at every merge point.  The last reader of each input
+// writes a result into it (x.re holds the x.re chain from its 4th op on), so three temporaries
+// per pair suffice.  The two pairs are interleaved instruction by instruction: a dependent FMA
+// follows its producer 8 instructions later, which keeps the FP64 pipeline busy with only
+// two waves per SIMD.
 __device__ __forceinline__ void pair_update2(double2& x0, double2& y0, double2& x1, double2& y1, const double2 m0,
                                              const double2 m1, const double2 m2, const double2 m3) {
     double tb0, tc0, td0, tb1, tc1, td1;
@@ -183,25 +174,126 @@ __device__ __forceinline__ void pair_update2(double2& x0, double2& y0, double2& 
           [m3r] "s"(m3.x), [m3i] "s"(m3.y));
 }
 
+// pair_update2, or with `shear` set x += m0 y, then y += m1 x on both pairs: 8 multiply-adds
+// per pair instead of 16.  The (uniform) choice is a branch inside the asm block: as two
+// blocks under an if, the compiler copies the whole register block at the merge (16 64-bit moves
+// per bit at K = 3, which cost what the shears save).
+__device__ __forceinline__ void pair_either2(double2& x0, double2& y0, double2& x1, double2& y1, const double2 m0,
+                                             const double2 m1, const double2 m2, const double2 m3, const u32 shear) {
+    double tb0, tc0, td0, tb1, tc1, td1;
+    asm("s_cmp_lg_u32 %[shear], 0\n\t"
+        "s_cbranch_scc1 .Lshear%=\n\t"
+        "v_mul_f64 %[tb0], %[m0i], %[xr0]\n\t"
+        "v_mul_f64 %[tb1], %[m0i], %[xr1]\n\t"
+        "v_mul_f64 %[tc0], %[m2r], %[xr0]\n\t"
+        "v_mul_f64 %[tc1], %[m2r], %[xr1]\n\t"
+        "v_mul_f64 %[td0], %[m2i], %[xr0]\n\t"
+        "v_mul_f64 %[td1], %[m2i], %[xr1]\n\t"
+        "v_mul_f64 %[xr0], %[m0r], %[xr0]\n\t"
+        "v_mul_f64 %[xr1], %[m0r], %[xr1]\n\t"
+        "v_fma_f64 %[xr0], -%[m0i], %[xi0], %[xr0]\n\t"
+        "v_fma_f64 %[xr1], -%[m0i], %[xi1], %[xr1]\n\t"
+        "v_fma_f64 %[tb0], %[m0r], %[xi0], %[tb0]\n\t"
+        "v_fma_f64 %[tb1], %[m0r], %[xi1], %[tb1]\n\t"
+        "v_fma_f64 %[tc0], -%[m2i], %[xi0], %[tc0]\n\t"
+        "v_fma_f64 %[tc1], -%[m2i], %[xi1], %[tc1]\n\t"
+        "v_fma_f64 %[td0], %[m2r], %[xi0], %[td0]\n\t"
+        "v_fma_f64 %[td1], %[m2r], %[xi1], %[td1]\n\t"
+        "v_fma_f64 %[xr0], %[m1r], %[yr0], %[xr0]\n\t"
+        "v_fma_f64 %[xr1], %[m1r], %[yr1], %[xr1]\n\t"
+        "v_fma_f64 %[tb0], %[m1i], %[yr0], %[tb0]\n\t"
+        "v_fma_f64 %[tb1], %[m1i], %[yr1], %[tb1]\n\t"
+        "v_fma_f64 %[tc0], %[m3r], %[yr0], %[tc0]\n\t"
+        "v_fma_f64 %[tc1], %[m3r], %[yr1], %[tc1]\n\t"
+        "v_fma_f64 %[td0], %[m3i], %[yr0], %[td0]\n\t"
+        "v_fma_f64 %[td1], %[m3i], %[yr1], %[td1]\n\t"
+        "v_fma_f64 %[xi0], %[m1r], %[yi0], %[tb0]\n\t"
+        "v_fma_f64 %[xi1], %[m1r], %[yi1], %[tb1]\n\t"
+        "v_fma_f64 %[yr0], -%[m3i], %[yi0], %[tc0]\n\t"
+        "v_fma_f64 %[yr1], -%[m3i], %[yi1], %[tc1]\n\t"
+        "v_fma_f64 %[xr0], -%[m1i], %[yi0], %[xr0]\n\t"
+        "v_fma_f64 %[xr1], -%[m1i], %[yi1], %[xr1]\n\t"
+        "v_fma_f64 %[yi0], %[m3r], %[yi0], %[td0]\n\t"
+        "v_fma_f64 %[yi1], %[m3r], %[yi1], %[td1]\n\t"
+        "s_branch .Ldone%=\n\t"
+        ".Lshear%=:\n\t"
+        "v_fma_f64 %[xr0], %[m0r], %[yr0], %[xr0]\n\t"
+        "v_fma_f64 %[xr1], %[m0r], %[yr1], %[xr1]\n\t"
+        "v_fma_f64 %[xi0], %[m0r], %[yi0], %[xi0]\n\t"
+        "v_fma_f64 %[xi1], %[m0r], %[yi1], %[xi1]\n\t"
+        "v_fma_f64 %[xr0], -%[m0i], %[yi0], %[xr0]\n\t"
+        "v_fma_f64 %[xr1], -%[m0i], %[yi1], %[xr1]\n\t"
+        "v_fma_f64 %[xi0], %[m0i], %[yr0], %[xi0]\n\t"
+        "v_fma_f64 %[xi1], %[m0i], %[yr1], %[xi1]\n\t"
+        "v_fma_f64 %[yr0], %[m1r], %[xr0], %[yr0]\n\t"
+        "v_fma_f64 %[yr1], %[m1r], %[xr1], %[yr1]\n\t"
+        "v_fma_f64 %[yi0], %[m1r], %[xi0], %[yi0]\n\t"
+        "v_fma_f64 %[yi1], %[m1r], %[xi1], %[yi1]\n\t"
+        "v_fma_f64 %[yr0], -%[m1i], %[xi0], %[yr0]\n\t"
+        "v_fma_f64 %[yr1], -%[m1i], %[xi1], %[yr1]\n\t"
+        "v_fma_f64 %[yi0], %[m1i], %[xr0], %[yi0]\n\t"
+        "v_fma_f64 %[yi1], %[m1i], %[xr1], %[yi1]\n\t"
+        ".Ldone%=:"
+        : [xr0] "+v"(x0.x), [xi0] "+v"(x0.y), [yr0] "+v"(y0.x), [yi0] "+v"(y0.y), [xr1] "+v"(x1.x),
+          [xi1] "+v"(x1.y), [yr1] "+v"(y1.x), [yi1] "+v"(y1.y), [tb0] "=&v"(tb0), [tc0] "=&v"(tc0),
+          [td0] "=&v"(td0), [tb1] "=&v"(tb1), [tc1] "=&v"(tc1), [td1] "=&v"(td1)
+        : [m0r] "s"(m0.x), [m0i] "s"(m0.y), [m1r] "s"(m1.x), [m1i] "s"(m1.y), [m2r] "s"(m2.x), [m2i] "s"(m2.y),
+          [m3r] "s"(m3.x), [m3i] "s"(m3.y), [shear] "s"(shear)
+        : "scc");
+}
+
+// v <- v (c + i s) on two amplitudes, complex, in place; c uniform, s per lane.
+__device__ __forceinline__ void phase2(double2& v, double2& w, const double c, const double sv, const double sw) {
+    double t0, u0, t1, u1;
+    asm("v_mul_f64 %[t0], %[sv], %[vi]\n\t"
+        "v_mul_f64 %[t1], %[sw], %[wi]\n\t"
+        "v_mul_f64 %[u0], %[sv], %[vr]\n\t"
+        "v_mul_f64 %[u1], %[sw], %[wr]\n\t"
+        "v_fma_f64 %[vr], %[c], %[vr], -%[t0]\n\t"
+        "v_fma_f64 %[wr], %[c], %[wr], -%[t1]\n\t"
+        "v_fma_f64 %[vi], %[c], %[vi], %[u0]\n\t"
+        "v_fma_f64 %[wi], %[c], %[wi], %[u1]"
+        : [vr] "+v"(v.x), [vi] "+v"(v.y), [wr] "+v"(w.x), [wi] "+v"(w.y), [t0] "=&v"(t0), [t1] "=&v"(t1),
+          [u0] "=&v"(u0), [u1] "=&v"(u1)
+        : [c] "s"(c), [sv] "v"(sv), [sw] "v"(sw));
+}
+// exp(i phi Z...Z) on a register block: slot j gets c + i s or c - i s by the parity of its
+// block bits in bm (uniform) and the sign that s already carries.
+template <int K>
+__device__ __forceinline__ void zrot_block(double2 (&v)[1 << K], u32 bm, const double c, const double s) {
+    u32 pat = 0;  // bit j: odd parity of j & bm
+#pragma unroll
+    for (int b = 0; b < K; ++b) pat ^= (0u - ((bm >> b) & 1u)) & (u32)((kBlockPatterns >> (16 * b)) & 0xffffu);
+    const int hi = __double2hiint(s), lo = __double2loint(s);
+#pragma unroll
+    for (int j = 0; j < (1 << K); j += 2)
+        phase2(v[j], v[j + 1], c, __hiloint2double(hi ^ (int)((pat << (31 - j)) & 0x80000000u), lo),
+               __hiloint2double(hi ^ (int)((pat << (30 - j)) & 0x80000000u), lo));
+}
+
+
 // One 2x2 matrix on block bit P of each of the G register blocks of a thread.
 // With two blocks, the pair updates interleave pair q of block 0 with pair q of
 // block 1; with one block, pairs q and q + 1.
-template <int K, int P, int G>
-__device__ __forceinline__ void sub_d1(double2 (&v)[G][1 << K], const double2* mp) {
+// REDUCE: bit P of `reduced` marks a matrix given as two shears.
+template <int K, int P, int G, bool REDUCE>
+__device__ __forceinline__ void sub_d1(double2 (&v)[G][1 << K], const double2* mp, u32 reduced) {
     const double2 m0 = mp[0], m1 = mp[1], m2 = mp[2], m3 = mp[3];
     // the 2^(K-1) pairs (j, j | 2^P)
     constexpr int NP = 1 << (K - 1);
     auto pair_j = [](int q) { return ((q >> P) << (P + 1)) | (q & ((1 << P) - 1)); };
+    auto update = [&](double2& x0, double2& y0, double2& x1, double2& y1) {
+        if constexpr (REDUCE) pair_either2(x0, y0, x1, y1, m0, m1, m2, m3, reduced & (1u << P));
+        else pair_update2(x0, y0, x1, y1, m0, m1, m2, m3);
+    };
     if constexpr (G == 2) {
 #pragma unroll
         for (int q = 0; q < NP; ++q)
-            pair_update2(v[0][pair_j(q)], v[0][pair_j(q) | (1 << P)], v[1][pair_j(q)], v[1][pair_j(q) | (1 << P)], m0,
-                         m1, m2, m3);
+            update(v[0][pair_j(q)], v[0][pair_j(q) | (1 << P)], v[1][pair_j(q)], v[1][pair_j(q) | (1 << P)]);
     } else {
 #pragma unroll
         for (int q = 0; q < NP; q += 2)
-            pair_update2(v[0][pair_j(q)], v[0][pair_j(q) | (1 << P)], v[0][pair_j(q + 1)],
-                         v[0][pair_j(q + 1) | (1 << P)], m0, m1, m2, m3);
+            update(v[0][pair_j(q)], v[0][pair_j(q) | (1 << P)], v[0][pair_j(q + 1)], v[0][pair_j(q + 1) | (1 << P)]);
     }
 }
 
@@ -252,15 +344,15 @@ __device__ __forceinline__ void apply_d2(double2* v, u32 p0, u32 p1, const doubl
 }
 #undef QM_D2_CASE
 
-// hi_tab[j] = global offset of local index j << LOW (the window qubits LOW.. of the
+// hi_tab[j] = global offset of local index j << kLowFixed (the window qubits kLowFixed.. of the
 // stage).  TI = u32 holds offsets below 2^32 (states of at most 32 qubits);
 // larger states use u64.
-template <u32 LOW = kLowFixed, typename TI>
+template <typename TI>
 __device__ __forceinline__ void build_hi_tab(TI* hi_tab, u32 lq, const DStage& sg) {
     const u64 win0 = sg.win[0], win1 = sg.win[1];
-    for (u32 j = threadIdx.x; j < (1u << (lq - LOW)); j += blockDim.x) {
+    for (u32 j = threadIdx.x; j < (1u << (lq - kLowFixed)); j += blockDim.x) {
         TI o = 0;
-        for (u32 i = 0; i + LOW < lq; ++i) o |= (TI)((j >> i) & 1u) << byte_at(i < 8 ? win0 : win1, i & 7);
+        for (u32 i = 0; i + kLowFixed < lq; ++i) o |= (TI)((j >> i) & 1u) << byte_at(i < 8 ? win0 : win1, i & 7);
         hi_tab[j] = o;
     }
 }
@@ -276,18 +368,30 @@ __device__ __forceinline__ u64 tile_base(u64 t, u32 tl, const DStage& sg) {
     return tb;
 }
 
-template <u32 LOW = kLowFixed, typename TI>
+template <typename TI>
 __device__ __forceinline__ u64 tile_index(u64 tb, const TI* hi_tab, u32 i) {
-    return tb + hi_tab[i >> LOW] + (i & ((1u << LOW) - 1));
+    return tb + hi_tab[i >> kLowFixed] + (i & ((1u << kLowFixed) - 1));
 }
 
 // The signs that the CZ gates of a LAYER give a register block with block base
 // `base` (local index with zeros at the block positions): bit j of the result set
 // means that amplitude j changes sign.  base is zero at the block positions, so a
 // local position p outside the block is (base >> p) & 1 for the whole block.
+// A qubit outside the window is a bit of the tile index: those CZs turn into uniform bits
+// (block positions) or into one more mask of local positions (scalar work).
 template <int K>
-__device__ __forceinline__ u32 layer_signs(const DSub& sub, u32 base) {
+__device__ __forceinline__ u32 layer_signs(const DSub& sub, u32 base, u64 tile) {
     u32 sgn = sub.type >> 16;
+    if (sub.nx) {
+        u32 mask = 0;
+        for (u32 c = 0; c < sub.nx; ++c) {
+            const u32 w = (u32)((c < 4 ? sub.x[0] : sub.x[1]) >> (16 * (c & 3u))) & 0xffffu, p = w >> 8;
+            const u32 on = (u32)(tile >> (w & 63u)) & 1u;
+            if (p & 0x80u) sgn ^= (0u - on) & (u32)(kBlockPatterns >> (16 * (p & 3u))) & 0xffffu;
+            else mask ^= on << p;
+        }
+        sgn ^= 0u - ((u32)__popc(base & mask) & 1u);
+    }
     if (sub.type & 0x8000u) {
 #pragma unroll
         for (int i = 0; i < K; ++i) {
@@ -316,34 +420,36 @@ __device__ __forceinline__ void flip_signs(double2 (&v)[1 << K], u32 sgn) {
 }
 
 // One LAYER sub-operation on the G register blocks of a thread, block g with
-// block base base[g].  The sub-operation is decoded once for all blocks.
-template <int K, int G>
+// block base base[g].  The sub-operation is decoded once for all blocks.  REDUCE = false: no
+// reduced matrices occur.
+template <int K, int G, bool REDUCE = true>
 __device__ __forceinline__ void apply_layer(double2 (&v)[G][1 << K], const DSub& sub, const u32 (&base)[G],
-                                            const double2* __restrict__ pool) {
+                                            const double2* __restrict__ pool, u64 tile) {
     const u32 d1 = (sub.type >> 8) & 15u;
-    if (sub.type >> 12) {
+    if ((sub.type >> 12) | sub.nx) {
         u32 sgn[G];
 #pragma unroll
-        for (int g = 0; g < G; ++g) sgn[g] = layer_signs<K>(sub, base[g]);
+        for (int g = 0; g < G; ++g) sgn[g] = layer_signs<K>(sub, base[g], tile);
 #pragma unroll
         for (int g = 0; g < G; ++g) flip_signs<K>(v[g], sgn[g]);
     }
     const double2* mp = pool + sub.data;
+    const u32 red = (sub.type >> 4) & 15u;
     if (d1 & 1u) {
-        sub_d1<K, 0, G>(v, mp);
+        sub_d1<K, 0, G, REDUCE>(v, mp, red);
         mp += 4;
     }
     if (d1 & 2u) {
-        sub_d1<K, 1, G>(v, mp);
+        sub_d1<K, 1, G, REDUCE>(v, mp, red);
         mp += 4;
     }
     if constexpr (K > 2)
         if (d1 & 4u) {
-            sub_d1<K, 2, G>(v, mp);
+            sub_d1<K, 2, G, REDUCE>(v, mp, red);
             mp += 4;
         }
     if constexpr (K > 3)
-        if (d1 & 8u) sub_d1<K, 3, G>(v, mp);
+        if (d1 & 8u) sub_d1<K, 3, G, REDUCE>(v, mp, red);
 }
 
 // The sub-operations of one pass on the G register blocks of groups gi0,
@@ -352,10 +458,11 @@ __device__ __forceinline__ void apply_layer(double2 (&v)[G][1 << K], const DSub&
 // the bits i of j): each lane forms its 2^K slots from the K per-bit offsets
 // (the empty asm keeps every partial XOR in a vector register, so the compiler
 // does not form the 2^K uniform combinations in scalar registers, which spill).
-// WIDE = false: only LAYER and D2 sub-operations occur.
+// WIDE = false: only LAYER (with full matrices) and D2 sub-operations occur.
 template <int K, u32 T, int G, bool WIDE = true>
 __device__ __forceinline__ void pass_groups(double2* st, const DPass& ps, const u32 (&sbit)[K], u32 gi0,
-                                            const DSub* __restrict__ subs, const double2* __restrict__ pool) {
+                                            const DSub* __restrict__ subs, const double2* __restrict__ pool,
+                                            u64 tile) {
     constexpr int D = 1 << K;
     u32 base[G], slot[G][D];
     double2 v[G][D];
@@ -389,13 +496,24 @@ __device__ __forceinline__ void pass_groups(double2* st, const DPass& ps, const 
     u32 k = 0;
     while (k < ps.nsub) {
         DSub sub = subs[ps.sub0 + k];
-        while ((sub.type & 0xffu) == SUB_LAYER) {
-            apply_layer<K, G>(v, sub, base, pool);
+        static_assert(SUB_LAYER == 0 && SUB_ZROT == 4, "the test below");
+        while ((sub.type & 11u) == 0) {
+            // a chain of conditional in-place updates (a ZROT has none of LAYER's parts)
+            if (WIDE && (sub.type & 4u)) {
+                const double2 z = pool[sub.data];
+                const u32 odd = (u32)__popcll(tile & sub.x[0]);
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const int f = (int)((odd + (u32)__popc(base[g] & sub.a & 0xffffu)) << 31);
+                    zrot_block<K>(v[g], sub.a >> 16, z.x, __hiloint2double(__double2hiint(z.y) ^ f, __double2loint(z.y)));
+                }
+            }
+            apply_layer<K, G, WIDE>(v, sub, base, pool, tile);
             if (++k == ps.nsub) break;
             sub = subs[ps.sub0 + k];
         }
         if (k == ps.nsub) break;
-        const u32 kind = sub.type & 0xffu;
+        const u32 kind = sub.type & 15u;
         const double2* mp = pool + sub.data;
         if (kind == SUB_D2) {
 #pragma unroll
@@ -407,7 +525,7 @@ __device__ __forceinline__ void pass_groups(double2* st, const DPass& ps, const 
             // (passes with a DIAG run with one block per thread: the per-lane
             // reads of the diagonal for two blocks exhaust the registers)
             // bit i of the diagonal index: local position p_i, i.e. bit p_i of
-            // base or, for a block position, bit j of the block pattern
+            // base or, for a block position, bit j of the block pattern; or a tile bit
             u32 pat[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -421,7 +539,11 @@ __device__ __forceinline__ void pass_groups(double2* st, const DPass& ps, const 
             for (int g = 0; g < G; ++g) {
                 u32 tbit[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) tbit[i] = i < (int)sub.m ? (base[g] >> byte_at(sub.a, i)) & 1u : 0u;
+                for (int i = 0; i < 4; ++i) {
+                    const u32 p = byte_at(sub.a, i);
+                    const u32 bit = p & kTileQubit ? (u32)(tile >> (p & 63u)) & 1u : (base[g] >> (p & 31u)) & 1u;
+                    tbit[i] = i < (int)sub.m ? bit : 0u;
+                }
 #pragma unroll
                 for (int j = 0; j < D; ++j) {
                     u32 idx = 0;
@@ -439,28 +561,52 @@ __device__ __forceinline__ void pass_groups(double2* st, const DPass& ps, const 
         for (int j = 0; j < D; ++j) st[slot[g][j]] = v[g][j];
 }
 
+// Brings a chunk of the program into the scalar cache: every wave reads its share of the cache
+// lines, all at once.  Read on demand, each line is a miss of several hundred cycles in a chain
+// (descriptor, then matrix) that nothing hides when a CU runs a single tile: a 20-qubit
+// circuit of 10 brickwork layers (256 tiles for 256 CUs) takes 127 us instead of 166.
+// (Plain indexed reads: turning the pointer into an integer would let the compiler assume that
+// stores change the program, and read it with vector loads.)
+__device__ __forceinline__ void warm_lines(const u32* __restrict__ p, u32 bytes) {
+    const u32 n = (bytes + 63) / 64;  // steps of a line, and the last word
+    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    for (u32 i = wave; i <= n && bytes; i += 4 * nw) {
+        u32 x[4];
+#pragma unroll
+        for (u32 k = 0; k < 4; ++k) x[k] = p[min((i + k * nw) * 16, bytes / 4 - 1)];
+        asm volatile("" ::"s"(x[0]), "s"(x[1]), "s"(x[2]), "s"(x[3]));
+    }
+}
+__device__ __forceinline__ void warm_program(const DPass& ps, const DSub* __restrict__ subs,
+                                             const double2* __restrict__ pool) {
+    warm_lines(reinterpret_cast<const u32*>(subs + ps.sub0), ps.warm & 0xffffu);
+    warm_lines(reinterpret_cast<const u32*>(pool + ps.pool0), ps.warm >> 16);
+}
+
 // Applies passes [pass0, pass0 + npass) to the 2^lq amplitudes in LDS with a
-// work-group of T threads (of at most T if it has fewer groups than T); ends with a barrier after every pass.  With G = 2
+// work-group of T threads (of at most T if it has fewer groups than T), `tile`: the
+// tile's index; ends with a barrier after every pass.  With G = 2
 // and exactly 2 T groups of 2^K amplitudes, every thread holds two register
 // blocks and decodes each sub-operation once for both.
 template <int K, u32 T, int G, bool WIDE = true>
 __device__ __forceinline__ void run_passes(double2* st, u32 lq, const DPass* __restrict__ passes, u32 pass0,
                                            u32 npass, const DSub* __restrict__ subs,
-                                           const double2* __restrict__ pool) {
+                                           const double2* __restrict__ pool, u64 tile) {
     constexpr int D = 1 << K;
     const u32 ngroups = (1u << lq) >> K;
     for (u32 p = 0; p < npass; ++p) {
         const DPass ps = passes[pass0 + p];
+        if (p > 0 && ps.warm) warm_program(ps, subs, pool);  // the first chunk: see the callers
         u32 sbit[K];
 #pragma unroll
         for (int i = 0; i < K; ++i) sbit[i] = ps.sbit[i];
         if (G == 2 && ngroups == 2 * T && !(ps.flags & kPassHasDiag)) {
-            pass_groups<K, T, G, WIDE>(st, ps, sbit, threadIdx.x, subs, pool);
+            pass_groups<K, T, G, WIDE>(st, ps, sbit, threadIdx.x, subs, pool, tile);
         } else if (ngroups == T) {
-            pass_groups<K, T, 1, WIDE>(st, ps, sbit, threadIdx.x, subs, pool);
+            pass_groups<K, T, 1, WIDE>(st, ps, sbit, threadIdx.x, subs, pool, tile);
         } else {
             for (u32 g = threadIdx.x; g < ngroups; g += blockDim.x)
-                pass_groups<K, T, 1, WIDE>(st, ps, sbit, g, subs, pool);
+                pass_groups<K, T, 1, WIDE>(st, ps, sbit, g, subs, pool, tile);
         }
         __syncthreads();
     }
@@ -492,36 +638,113 @@ u32 pool_put(Flat& f, const std::vector<cd>& m) {
     return off;
 }
 
-// Passes of one stage: ops (already in local positions) -> DPass/DSub.
-void schedule_passes(Flat& f, std::vector<HOp> ops, u32 lq, u32 K, DStage& sg) {
-    sg.pass0 = (u32)f.passes.size();
-    sg.npass = 0;
-    std::vector<bool> done(ops.size(), false);
-    size_t left = ops.size();
-    while (left > 0) {
-        u64 blocked = 0, block = 0;
-        std::vector<size_t> sel;
-        for (size_t i = 0; i < ops.size(); ++i) {
-            if (done[i]) continue;
-            const HOp& o = ops[i];
-            const u64 m = o.mask();
-            if (m & blocked) {
-                blocked |= m;
+// The window (or block) of the next stage (or pass).  Operations are scanned in order; a
+// dense operation is taken if its qubits lie in the window, a diagonal one if it touches
+// the window at all (a qubit outside is a constant there); a dense operation that is not
+// taken blocks its qubits for everything after it.  Diagonal operations that do not touch the
+// window block nothing: they commute with what is taken.  Candidates: the window that grows
+// in scan order (any circuit), and every run of adjacent qubits (chains and grids, where the
+// order of the gate list would spread the window over the register and leave each stage a few
+// layers: 26-qubit brickwork, 20 layers: 26 -> 8 stages; 20-qubit ansatz: 25 -> 8).
+// The one with the most dense work wins.
+struct Picker {
+    struct Item {
+        u64 mask;
+        u32 weight;  // 0: diagonal
+        bool grad;
+    };
+    std::vector<Item> items;
+    std::vector<u32> rest;  // what is left, in order
+
+    static u32 weight_of(const HOp& o) { return o.type == 0 ? 1u << (o.q.size() - 1) : 0u; }
+    void add(const HOp& o) {
+        rest.push_back((u32)items.size());
+        items.push_back({o.mask(), weight_of(o), o.grad});
+    }
+    // Scans with window w (grown up to `most` qubits if `grow`); returns the dense work taken.
+    u64 scan(u64& w, bool grow, u32 most, size_t max_grads, std::vector<u32>* sel) const {
+        u64 blocked = 0, work = 0;
+        size_t grads = 0;
+        for (u32 i : rest) {
+            const Item& it = items[i];
+            if (it.mask & blocked) {
+                // (a diagonal one that a fixed window does not touch orders nothing in it)
+                if (it.weight || grow || (it.mask & w)) blocked |= it.mask;
+                if ((blocked & w) == w && (!grow || (u32)__builtin_popcountll(w) >= most)) break;
                 continue;
             }
-            if (o.type != 0) {
-                sel.push_back(i);
+            if (it.weight == 0) {
+                if (sel) sel->push_back(i);
                 continue;
             }
-            if ((u32)__builtin_popcountll(block | m) <= K) {
-                block |= m;
-                sel.push_back(i);
+            const u64 m = it.mask | w;
+            const bool fits = m == w || (grow && (u32)__builtin_popcountll(m) <= most);
+            if (fits && (!it.grad || grads < max_grads)) {
+                w = m;
+                work += it.weight;
+                grads += it.grad ? 1 : 0;
+                if (sel) sel->push_back(i);
             } else {
-                blocked |= m;
+                blocked |= it.mask;
+                if ((blocked & w) == w && (!grow || (u32)__builtin_popcountll(w) >= most)) break;
             }
         }
-        // pad the block to K local positions
-        for (u32 p = 0; p < lq && (u32)__builtin_popcountll(block) < K; ++p) block |= 1ULL << p;
+        return work;
+    }
+    // Picks a window of at most `most` positions out of [0, n) that contains `fixed`, and
+    // what it takes; the window is filled up to min(n, most) positions.
+    u64 pick(u32 n, u64 fixed, u32 low, u32 most, size_t max_grads, std::vector<u32>& sel) {
+        u64 best = fixed;
+        u64 work = scan(best, true, most, max_grads, nullptr);
+        const u32 f = most - low;
+        bool grow = true;
+        for (u32 s = low; s + f <= n; ++s) {
+            u64 w = fixed | (((1ULL << f) - 1) << s);
+            const u64 c = scan(w, false, most, max_grads, nullptr);
+            if (c > work) {
+                work = c;
+                best = w;
+                grow = false;
+            }
+        }
+        u64 w = grow ? fixed : best;
+        sel.clear();
+        scan(w, grow, most, max_grads, &sel);
+        // fill the window: with the qubits of diagonal operations that wait, then the lowest
+        auto room = [&] { return (u32)__builtin_popcountll(w) < std::min(n, most); };
+        for (u32 i : sel)
+            for (u64 m = items[i].mask & ~w; m && room(); m &= m - 1) w |= m & (~m + 1);
+        for (u32 q = 0; q < n && room(); ++q) w |= 1ULL << q;
+        // a diagonal operation outside the window stays for a later one
+        sel.erase(std::remove_if(sel.begin(), sel.end(), [&](u32 i) { return !(items[i].mask & w); }), sel.end());
+        return w;
+    }
+    void take(const std::vector<u32>& sel) {  // sel is ascending in `rest` order
+        size_t k = 0, out = 0;
+        for (size_t i = 0; i < rest.size(); ++i) {
+            if (k < sel.size() && rest[i] == sel[k]) ++k;
+            else rest[out++] = rest[i];
+        }
+        rest.resize(out);
+    }
+};
+
+// Passes of one stage: ops (already in local positions) -> DPass/DSub.
+void schedule_passes(Flat& f, const std::vector<HOp>& ops, u32 lq, u32 K, DStage& sg) {
+    sg.pass0 = (u32)f.passes.size();
+    sg.npass = 0;
+    Picker pk;
+    size_t dense_left = 0;
+    for (const HOp& o : ops) {
+        pk.add(o);
+        dense_left += o.type == 0;
+    }
+    std::vector<u32> sel;
+    while (!pk.rest.empty()) {
+        const u64 block = pk.pick(lq, 0, 0, K, ~size_t(0), sel);
+        for (u32 i : sel) dense_left -= ops[i].type == 0;
+        if (dense_left == 0) sel = pk.rest;  // the last pass takes every diagonal operation that is left
+        pk.take(sel);
         DPass ps{};
         u32 bpos[4] = {0, 0, 0, 0};
         {
@@ -532,25 +755,52 @@ void schedule_passes(Flat& f, std::vector<HOp> ops, u32 lq, u32 K, DStage& sg) {
         for (u32 i = 0; i < 4; ++i) ps.pos[i] = (unsigned char)bpos[i];
         for (u32 i = 0; i < K; ++i) ps.sbit[i] = (unsigned short)slot_of(1u << bpos[i]);
         ps.sub0 = (u32)f.subs.size();
+        ps.pool0 = (u32)f.pool.size();
         auto bit_of = [&](u32 p) -> u32 {
             for (u32 i = 0; i < K; ++i)
                 if (bpos[i] == p) return i;
             return 0;
         };
-        // Consecutive CZ gates, then consecutive single-qubit matrices on distinct
-        // block bits (these commute with each other), become one LAYER.
+        // Levels: an operation goes to the first level after what it does not commute
+        // with (only block bits carry dense operations); a level is its diagonal
+        // operations, then its matrices on distinct block bits.
+        std::vector<std::vector<u32>> levels;
+        {
+            u32 dense_at[4] = {0, 0, 0, 0}, diag_at[4] = {0, 0, 0, 0};
+            for (u32 i : sel) {
+                const HOp& o = ops[i];
+                u32 lv = 1;
+                for (u32 q : o.q) {
+                    if (q >= kTileQubit || !((block >> q) & 1)) continue;
+                    const u32 b = bit_of(q);
+                    lv = std::max(lv, dense_at[b] + 1);
+                    if (o.type == 0) lv = std::max(lv, diag_at[b]);
+                }
+                for (u32 q : o.q) {
+                    if (q >= kTileQubit || !((block >> q) & 1)) continue;
+                    u32& at = (o.type == 0 ? dense_at : diag_at)[bit_of(q)];
+                    at = std::max(at, lv);
+                }
+                if (levels.size() < lv) levels.resize(lv);
+                levels[lv - 1].push_back(i);
+            }
+        }
         std::vector<const HOp*> pend_d1(K, nullptr);
-        u32 d1mask = 0, cz_const = 0, npair = 0, pairs = 0;
+        u32 d1mask = 0, redmask = 0, cz_const = 0, npair = 0, pairs = 0, nx = 0;
+        u64 xs[2] = {0, 0};
         u32 czmask[4] = {0, 0, 0, 0};
         bool cz_any = false;
         auto flush = [&]() {
             if (d1mask == 0 && !cz_any) return;
             DSub sb{};
             const bool masks = (czmask[0] | czmask[1] | czmask[2] | czmask[3]) != 0;
-            sb.type = SUB_LAYER | (d1mask << 8) | (npair << 12) | (masks ? 0x8000u : 0u) | (cz_const << 16);
+            sb.type = SUB_LAYER | (redmask << 4) | (d1mask << 8) | (npair << 12) | (masks ? 0x8000u : 0u) | (cz_const << 16);
             sb.a = czmask[0] | (czmask[1] << 16);
             sb.m = czmask[2] | (czmask[3] << 16);
             sb.pairs = pairs;
+            sb.nx = nx;
+            sb.x[0] = xs[0];
+            sb.x[1] = xs[1];
             sb.data = (u32)f.pool.size();
             sb.grad0 = (u32)f.grads.size();
             for (u32 b = 0; b < K; ++b) {
@@ -564,15 +814,26 @@ void schedule_passes(Flat& f, std::vector<HOp> ops, u32 lq, u32 K, DStage& sg) {
             }
             f.subs.push_back(sb);
             std::fill(pend_d1.begin(), pend_d1.end(), nullptr);
-            d1mask = 0;
+            d1mask = redmask = 0;
             cz_const = 0;
             npair = 0;
             pairs = 0;
+            nx = 0;
+            xs[0] = xs[1] = 0;
             std::fill(czmask, czmask + 4, 0u);
             cz_any = false;
         };
         const u32 jmask = (1u << (1u << K)) - 1;
         auto add_cz = [&](u32 p0, u32 p1) {
+            if (p0 >= kTileQubit) std::swap(p0, p1);
+            if (p1 >= kTileQubit) {
+                if (nx == kCzTileMax) flush();
+                const u32 in = ((block >> p0) & 1) ? 0x80u | bit_of(p0) : p0;
+                xs[nx >> 2] |= (u64)((p1 & 63u) | (in << 8)) << (16 * (nx & 3));
+                ++nx;
+                cz_any = true;
+                return;
+            }
             const bool in0 = (block >> p0) & 1, in1 = (block >> p1) & 1;
             if (in0 && in1) {
                 cz_const ^= (u32)(kBlockPatterns >> (16 * bit_of(p0))) & (u32)(kBlockPatterns >> (16 * bit_of(p1))) &
@@ -586,184 +847,349 @@ void schedule_passes(Flat& f, std::vector<HOp> ops, u32 lq, u32 K, DStage& sg) {
             }
             cz_any = true;
         };
-        for (size_t i : sel) {
-            const HOp& o = ops[i];
-            done[i] = true;
-            --left;
-            if (o.type == 2) {
-                if (d1mask) flush();
-                add_cz(o.q[0], o.q[1]);
-                continue;
-            }
-            if (o.type == 0 && o.q.size() == 1) {
-                const u32 b = bit_of(o.q[0]);
-                if ((d1mask >> b) & 1) flush();
-                pend_d1[b] = &o;
-                d1mask |= 1u << b;
-                continue;
-            }
-            flush();
-            DSub sb{};
-            if (o.type == 1) {
+        for (const auto& level : levels) {
+            for (u32 i : level) {
+                const HOp& o = ops[i];
+                if (o.type != 1) continue;
+                DSub sb{};
                 ps.flags |= kPassHasDiag;
                 sb.type = SUB_DIAG;
                 sb.m = (u32)o.q.size();
                 for (size_t k = 0; k < o.q.size(); ++k) sb.a |= o.q[k] << (8 * k);
                 sb.data = pool_put(f, o.m);
-            } else if (o.q.size() == 2) {
-                sb.type = SUB_D2;
-                sb.a = bit_of(o.q[0]) | (bit_of(o.q[1]) << 8);
-                sb.data = pool_put(f, o.m);
-            } else {
-                // embed into the K block bits (ascending) with the identity elsewhere
-                const u32 k = (u32)o.q.size(), D = 1u << K;
-                std::vector<u32> bits(k);
-                u32 omask = 0;
-                for (u32 t = 0; t < k; ++t) {
-                    bits[t] = bit_of(o.q[t]);
-                    omask |= 1u << bits[t];
-                }
-                std::vector<cd> M((size_t)D * D, 0.0);
-                for (u32 col = 0; col < D; ++col) {
-                    u32 x = 0;
-                    for (u32 t = 0; t < k; ++t) x |= ((col >> bits[t]) & 1u) << t;
-                    for (u32 y = 0; y < (1u << k); ++y) {
-                        u32 row = col & ~omask;
-                        for (u32 t = 0; t < k; ++t) row |= ((y >> t) & 1u) << bits[t];
-                        M[(size_t)row * D + col] += o.m[(size_t)y * (1u << k) + x];
-                    }
-                }
-                sb.type = SUB_DK;
-                sb.data = pool_put(f, M);
+                f.subs.push_back(sb);
             }
-            f.subs.push_back(sb);
+            for (u32 i : level) {
+                const HOp& o = ops[i];
+                if (o.type != 3) continue;
+                DSub sb{};
+                sb.type = SUB_ZROT;
+                for (u32 q : o.q) {
+                    if (q >= kTileQubit) sb.x[0] |= 1ULL << (q & 63u);
+                    else if ((block >> q) & 1) sb.a |= 0x10000u << bit_of(q);
+                    else sb.a |= 1u << q;
+                }
+                sb.data = pool_put(f, o.m);
+                f.subs.push_back(sb);
+            }
+            for (u32 i : level)
+                if (ops[i].type == 2) add_cz(ops[i].q[0], ops[i].q[1]);
+            for (u32 i : level) {
+                const HOp& o = ops[i];
+                if (o.type != 0 || o.q.size() != 1) continue;
+                pend_d1[bit_of(o.q[0])] = &o;
+                d1mask |= 1u << bit_of(o.q[0]);
+                if (o.reduced) redmask |= 1u << bit_of(o.q[0]);
+            }
+            flush();
+            for (u32 i : level) {
+                const HOp& o = ops[i];
+                if (o.type != 0 || o.q.size() == 1) continue;
+                DSub sb{};
+                if (o.q.size() == 2) {
+                    sb.type = SUB_D2;
+                    sb.a = bit_of(o.q[0]) | (bit_of(o.q[1]) << 8);
+                    sb.data = pool_put(f, o.m);
+                } else {
+                    // embed into the K block bits (ascending) with the identity elsewhere
+                    const u32 k = (u32)o.q.size(), D = 1u << K;
+                    std::vector<u32> bits(k);
+                    u32 omask = 0;
+                    for (u32 t = 0; t < k; ++t) {
+                        bits[t] = bit_of(o.q[t]);
+                        omask |= 1u << bits[t];
+                    }
+                    std::vector<cd> M((size_t)D * D, 0.0);
+                    for (u32 col = 0; col < D; ++col) {
+                        u32 x = 0;
+                        for (u32 t = 0; t < k; ++t) x |= ((col >> bits[t]) & 1u) << t;
+                        for (u32 y = 0; y < (1u << k); ++y) {
+                            u32 row = col & ~omask;
+                            for (u32 t = 0; t < k; ++t) row |= ((y >> t) & 1u) << bits[t];
+                            M[(size_t)row * D + col] += o.m[(size_t)y * (1u << k) + x];
+                        }
+                    }
+                    sb.type = SUB_DK;
+                    sb.data = pool_put(f, M);
+                }
+                f.subs.push_back(sb);
+            }
         }
-        flush();
         ps.nsub = (u32)f.subs.size() - ps.sub0;
         f.passes.push_back(ps);
         ++sg.npass;
     }
+    // chunks of passes for warm_program
+    for (u32 p = sg.pass0; p < sg.pass0 + sg.npass;) {
+        auto end_of = [&](u32 q, bool pool) {
+            const bool last = q + 1 == f.passes.size();
+            return pool ? (last ? (u32)f.pool.size() : f.passes[q + 1].pool0)
+                        : (last ? (u32)f.subs.size() : f.passes[q + 1].sub0);
+        };
+        DPass& head = f.passes[p];
+        u32 q = p;
+        for (;; ++q) {
+            const u32 bs = (end_of(q, false) - head.sub0) * (u32)sizeof(DSub);
+            const u32 bp = (end_of(q, true) - head.pool0) * (u32)sizeof(double2);
+            if (q > p && bs + bp > kWarmBytes) break;
+            head.warm = std::min(bs, 2 * kWarmBytes) | std::min(bp, 2 * kWarmBytes) << 16;
+            if (q + 1 == sg.pass0 + sg.npass) {
+                ++q;
+                break;
+            }
+        }
+        p = q;
+    }
 }
 
-// Stages (windows of lq_cap qubits including 0..3) for circuits above lq_cap
-// qubits; a single identity stage otherwise.  Returns the number of stages appended.
-// `low`: the qubits below it are in every window.  `max_grads`: a stage takes at
-// most that many operations with grad set.
-u32 schedule_circuit(Flat& f, const HCirc& c, u32 K, u32 lq_cap = kMaxLocal, u32 low_fixed = kLowFixed,
-                     size_t max_grads = ~size_t(0)) {
+// Stages (windows of lq_cap qubits including those below `low_fixed`) for circuits above
+// lq_cap qubits; a single identity stage otherwise.  A stage takes at most `max_grads`
+// operations with grad set.  Returns the number of stages appended.
+u32 schedule_circuit(Flat& f, const HCirc& c, u32 K, u32 lq_cap = kMaxLocal, size_t max_grads = ~size_t(0)) {
     const u32 n = c.ne, lq = std::min(n, lq_cap);
     if (n <= lq_cap && max_grads == ~size_t(0)) {
         DStage sg{};
-        for (u32 i = 0; i + low_fixed < lq; ++i) set_byte(sg.win[i >> 3], i & 7, low_fixed + i);
+        for (u32 i = 0; i + kLowFixed < lq; ++i) set_byte(sg.win[i >> 3], i & 7, kLowFixed + i);
         schedule_passes(f, c.ops, lq, K, sg);
         f.stages.push_back(sg);
         return 1;
     }
-    std::vector<bool> done(c.ops.size(), false);
-    size_t left = c.ops.size();
+    Picker pk;
+    for (const HOp& o : c.ops) pk.add(o);
+    const u64 low = (1ULL << kLowFixed) - 1;
     u32 count = 0;
-    const u64 low = (1ULL << low_fixed) - 1;
-    while (left > 0) {
-        u64 win = low, blocked = 0;
-        size_t grads = 0;
-        std::vector<size_t> sel;
-        for (size_t i = 0; i < c.ops.size(); ++i) {
-            if (done[i]) continue;
-            const u64 m = c.ops[i].mask();
-            if (m & blocked) {
-                blocked |= m;
-                continue;
-            }
-            if ((u32)__builtin_popcountll(win | m) <= lq && (!c.ops[i].grad || grads < max_grads)) {
-                win |= m;
-                grads += c.ops[i].grad ? 1 : 0;
-                sel.push_back(i);
-            } else {
-                blocked |= m;
-            }
-        }
-        for (u32 q = 0; q < n && (u32)__builtin_popcountll(win) < lq; ++q) win |= 1ULL << q;
+    std::vector<u32> sel;
+    do {  // a circuit without gates still needs one stage to initialise |0>
+        const u64 win = pk.pick(n, low, kLowFixed, lq, max_grads, sel);
+        pk.take(sel);
         DStage sg{};
         u32 local_of[64];
         u32 wi = 0, ci = 0;
         for (u32 q = 0; q < n; ++q) {
-            if (q < low_fixed) {
+            if (q < kLowFixed) {
                 local_of[q] = q;
             } else if ((win >> q) & 1) {
-                local_of[q] = low_fixed + wi;
+                local_of[q] = kLowFixed + wi;
                 set_byte(sg.win[wi >> 3], wi & 7, q);
                 ++wi;
             } else {
+                local_of[q] = kTileQubit | ci;
                 set_byte(sg.comp[ci >> 3], ci & 7, q);
                 ++ci;
             }
         }
         std::vector<HOp> ops;
         ops.reserve(sel.size());
-        for (size_t i : sel) {
-            HOp o = c.ops[i];
-            for (u32& q : o.q) q = local_of[q];
-            ops.push_back(std::move(o));
-            done[i] = true;
-            --left;
+        for (u32 i : sel) {
+            ops.push_back(c.ops[i]);
+            for (u32& q : ops.back().q) q = local_of[q];
         }
         schedule_passes(f, ops, lq, K, sg);
         f.stages.push_back(sg);
         ++count;
-    }
-    if (count == 0) {  // a circuit without gates still needs one stage to initialise |0>
-        DStage sg{};
-        u32 wi = 0, ci = 0;
-        for (u32 q = low_fixed; q < n; ++q) {
-            if (wi + low_fixed < lq) {
-                set_byte(sg.win[wi >> 3], wi & 7, q);
-                ++wi;
-            } else {
-                set_byte(sg.comp[ci >> 3], ci & 7, q);
-                ++ci;
-            }
-        }
-        sg.npass = 0;
-        sg.pass0 = (u32)f.passes.size();
-        f.stages.push_back(sg);
-        count = 1;
-    }
+    } while (!pk.rest.empty());
     return count;
 }
 
-// Gates in the C ABI form -> internal ops, with consecutive single-qubit dense /
-// diagonal gates on the same qubit multiplied together.
-// Appends o; a single-qubit dense / diagonal gate is fused into the previous
-// op on its qubit when that is one too (last[q]: index of the last op on q).
-void push_op(HCirc& c, std::vector<long>& last, HOp o) {
-    if (o.q.size() == 1 && o.type != 2) {
-        const long p = last[o.q[0]];
-        if (p >= 0 && c.ops[p].q.size() == 1 && c.ops[p].type != 2) {
-            HOp& prev = c.ops[p];
-            auto full = [](const HOp& h) {
-                if (h.type == 0) return h.m;
-                return std::vector<cd>{h.m[0], 0.0, 0.0, h.m[1]};
-            };
-            if (prev.type == 1 && o.type == 1) {
-                prev.m[0] *= o.m[0];
-                prev.m[1] *= o.m[1];
-            } else {
-                std::vector<cd> prod;
-                mat_mul(full(o), full(prev), prod, 2);  // new after old
-                prev.m = prod;
-                prev.type = 0;
-            }
-            return;
+// Gates in the C ABI form -> internal operations.
+//   * Consecutive single-qubit gates on a qubit are multiplied together.
+//   * Diagonal operations (CZ, ZROT, DIAG) commute, so a single-qubit diagonal waits in `pend`
+//     and is multiplied into the next dense operation on its qubit, or, at the end, into
+//     the last one.
+//   * CNOT(c, t) = H_t CZ(c, t) H_t with H = [[1, 1], [1, -1]] before and half of it after
+//     the CZ: both exact, where 1/sqrt(2) twice would change the norm by 1.4e-16 per CNOT.
+//   * A diagonal gate with entries of modulus 1 is a product of exp(i phi Z...Z) over subsets of
+//     its qubits: phases on single qubits wait as above, the others become ZROT when they
+//     are few (a two-qubit gate has one), else the gate stays a DIAG.
+struct Converter {
+    HCirc& c;
+    std::vector<long> last;        // last operation that touches each qubit
+    std::vector<long> last_dense;  // last dense one
+    struct Phase {
+        cd d[2] = {1.0, 1.0};
+        bool any = false;
+    };
+    std::vector<Phase> pend;
+
+    explicit Converter(HCirc& circ) : c(circ), last(circ.ne, -1), last_dense(circ.ne, -1), pend(circ.ne) {}
+
+    void push(HOp o) {
+        c.ops.push_back(std::move(o));
+        const long i = (long)c.ops.size() - 1;
+        for (u32 q : c.ops.back().q) {
+            last[q] = i;
+            if (c.ops.back().type == 0) last_dense[q] = i;
         }
     }
-    c.ops.push_back(std::move(o));
-    for (u32 q : c.ops.back().q) last[q] = (long)c.ops.size() - 1;
+    void phase(u32 q, cd d0, cd d1) {
+        pend[q].d[0] *= d0;
+        pend[q].d[1] *= d1;
+        pend[q].any = true;
+    }
+    void dense(const std::vector<u32>& q, std::vector<cd> m) {
+        const u32 d = 1u << q.size();
+        for (u32 t = 0; t < q.size(); ++t) {
+            Phase& ph = pend[q[t]];
+            if (!ph.any) continue;
+            for (u32 r = 0; r < d; ++r)
+                for (u32 col = 0; col < d; ++col) m[r * d + col] *= ph.d[(col >> t) & 1u];
+            ph = Phase{};
+        }
+        const long p = last[q[0]];
+        if (q.size() == 1 && p >= 0 && c.ops[p].type == 0 && c.ops[p].q.size() == 1) {
+            std::vector<cd> prod;
+            mat_mul(m, c.ops[p].m, prod, 2);  // new after old
+            c.ops[p].m = prod;
+            return;
+        }
+        HOp o;
+        o.type = 0;
+        o.q = q;
+        o.m = std::move(m);
+        push(std::move(o));
+    }
+    void zrot(const std::vector<u32>& q, cd z) {
+        if (q.size() == 1) {
+            phase(q[0], z, std::conj(z));
+            return;
+        }
+        HOp o;
+        o.type = 3;
+        o.q = q;
+        o.m = {z};
+        push(std::move(o));
+    }
+    void diagonal(const std::vector<u32>& q, const std::vector<cd>& m) {
+        const u32 k = (u32)q.size(), d = 1u << k;
+        if (k == 1) {
+            phase(q[0], m[0], m[1]);
+            return;
+        }
+        auto subset = [&](u32 s) {
+            std::vector<u32> r;
+            for (u32 t = 0; t < k; ++t)
+                if ((s >> t) & 1) r.push_back(q[t]);
+            return r;
+        };
+        for (u32 s = 1; s < d; ++s) {  // one exp(i phi Z...Z), entries as they are
+            bool is = std::abs(std::abs(m[0]) - 1.0) < 1e-14;
+            for (u32 i = 1; i < d && is; ++i) is = m[i] == ((__builtin_popcount(i & s) & 1) ? std::conj(m[0]) : m[0]);
+            if (is) {
+                zrot(subset(s), m[0]);
+                return;
+            }
+        }
+        bool unit = true;
+        for (u32 i = 0; i < d && unit; ++i) unit = std::abs(std::abs(m[i]) - 1.0) < 1e-14;
+        if (unit) {
+            double phi[16];
+            for (u32 i = 0; i < d; ++i) phi[i] = std::arg(m[i]);
+            for (u32 h = 1; h < d; h <<= 1)  // phi[s] <- sum_i (-1)^popcount(i & s) arg m_i
+                for (u32 i = 0; i < d; ++i)
+                    if (!(i & h)) {
+                        const double a = phi[i], b = phi[i | h];
+                        phi[i] = a + b;
+                        phi[i | h] = a - b;
+                    }
+            u32 many = 0;
+            for (u32 s = 1; s < d; ++s) many += (s & (s - 1)) && std::abs(phi[s]) > 1e-15;
+            if (many <= 2) {
+                const cd g = std::polar(1.0, phi[0] / d);
+                phase(q[0], g, g);
+                for (u32 s = 1; s < d; ++s)
+                    if (std::abs(phi[s]) > 1e-15) zrot(subset(s), std::polar(1.0, phi[s] / d));
+                return;
+            }
+        }
+        HOp o;
+        o.type = 1;
+        o.q = q;
+        o.m = m;
+        push(std::move(o));
+    }
+    // What is left in pend: into the last dense operation on the qubit (only diagonal ones
+    // follow it), else a diagonal operation of its own.
+    void finish() {
+        for (u32 q = 0; q < c.ne; ++q) {
+            Phase& ph = pend[q];
+            if (!ph.any) continue;
+            if (last_dense[q] >= 0) {
+                HOp& o = c.ops[last_dense[q]];
+                const u32 d = 1u << o.q.size(), t = (u32)(std::find(o.q.begin(), o.q.end(), q) - o.q.begin());
+                for (u32 r = 0; r < d; ++r)
+                    for (u32 col = 0; col < d; ++col) o.m[r * d + col] *= ph.d[(r >> t) & 1u];
+            } else if (ph.d[0] != 1.0 || ph.d[1] != 1.0) {
+                HOp o;
+                o.type = 1;
+                o.q = {q};
+                o.m = {ph.d[0], ph.d[1]};
+                push(std::move(o));
+            }
+            ph = Phase{};
+        }
+    }
+};
+
+// A single-qubit unitary U = diag(p, q) [[1, 0], [b, 1]] [[1, a], [0, 1]] with p = u00,
+// a = u01 / u00, q = det / u00, b = u10 / q.  The diagonal factor commutes with everything
+// diagonal that follows and is multiplied into the next dense operation on the qubit, so most
+// single-qubit matrices but the last on a qubit cost 8 multiply-adds per pair instead of 16 (the
+// fused executors are bound by FP64 issue: see qm_batch.hip).
+// Scaling rows or columns by a diagonal changes no relative rounding error, and with
+// |u00| >= 1/2 the two shears add terms of at most twice the result's size, so the error
+// is that of the full matrix.  Amplitudes are off by 1/p or 1/q until the diagonal is
+// applied.  A matrix is left whole when |u00| < 1/2, when that factor would exceed 2^200 in
+// all, and when it is not unitary (or a multiple of a unitary).
+void reduce_matrices(std::vector<HOp>& ops, u32 n) {
+    std::vector<long> last_dense(n, -1);
+    for (size_t i = 0; i < ops.size(); ++i)
+        if (ops[i].type == 0)
+            for (u32 q : ops[i].q) last_dense[q] = (long)i;
+    struct Left {
+        cd d[2] = {1.0, 1.0};
+        bool any = false;
+        double bits = 0.0;  // |log2| of the larger factor that waits in d
+    };
+    std::vector<Left> left(n);
+    double total = 0.0;
+    for (size_t i = 0; i < ops.size(); ++i) {
+        HOp& o = ops[i];
+        if (o.type != 0) continue;
+        bool shear = false;
+        if (o.q.size() == 1 && (long)i != last_dense[o.q[0]]) {
+            const double c0 = std::norm(o.m[0]) + std::norm(o.m[2]), c1 = std::norm(o.m[1]) + std::norm(o.m[3]);
+            const cd dot = std::conj(o.m[0]) * o.m[1] + std::conj(o.m[2]) * o.m[3];
+            shear = c0 > 1e-6 && c0 < 1e6 && std::abs(c1 - c0) < 1e-12 * c0 && std::abs(dot) < 1e-12 * c0 &&
+                    std::norm(o.m[0]) >= 0.25 * c0;
+        }
+        const u32 d = 1u << o.q.size();
+        for (u32 t = 0; t < o.q.size(); ++t) {
+            Left& l = left[o.q[t]];
+            if (!l.any) continue;
+            for (u32 r = 0; r < d; ++r)
+                for (u32 col = 0; col < d; ++col) o.m[r * d + col] *= l.d[(col >> t) & 1u];
+            total -= l.bits;
+            l = Left{};
+        }
+        if (!shear) continue;
+        const cd p = o.m[0], a = o.m[1] / o.m[0], q = o.m[3] - o.m[2] * a;
+        const double bits = std::max(std::abs(std::log2(std::abs(p))), std::abs(std::log2(std::abs(q))));
+        if (!(total + bits < 200.0)) continue;
+        Left& l = left[o.q[0]];
+        l.d[0] = p;
+        l.d[1] = q;
+        l.any = true;
+        l.bits = bits;
+        total += bits;
+        o.m = {a, o.m[2] / q, 0.0, 0.0};
+        o.reduced = true;
+    }
 }
 
 bool convert_gates(u32 n, const qm_batch_gate* gates, UINT gate_count, HCirc& c, const char* what) {
     c.n = n;
     c.ne = std::max<u32>(n, kMinQubits);
-    std::vector<long> last(c.ne, -1);  // last op touching each qubit
+    Converter cv(c);
     for (UINT gi = 0; gi < gate_count; ++gi) {
         const qm_batch_gate& g = gates[gi];
         const u32 k = g.qubit_count;
@@ -784,36 +1210,26 @@ bool convert_gates(u32 n, const qm_batch_gate* gates, UINT gate_count, HCirc& c,
             set_error(QM_ERR_INVALID_ARGUMENT, "%s: gate %u: null matrix", what, gi);
             return false;
         }
-        if (g.kind == QM_BATCH_CNOT) {
-            // CNOT(c, t) = H_t CZ(c, t) H_t; the Hadamards fuse into the
-            // single-qubit gates next to them on t
-            const double h = 0.70710678118654752440;
-            HOp hd;
-            hd.type = 0;
-            hd.q = {g.qubits[1]};
-            hd.m = {h, h, h, -h};
+        const std::vector<u32> q(g.qubits, g.qubits + k);
+        const u32 d = 1u << k;
+        std::vector<cd> m;
+        if (two) {
             HOp cz;
             cz.type = 2;
-            cz.q = {g.qubits[0], g.qubits[1]};
-            push_op(c, last, hd);
-            push_op(c, last, std::move(cz));
-            push_op(c, last, std::move(hd));
-            continue;
-        }
-        HOp o;
-        o.q.assign(g.qubits, g.qubits + k);
-        const u32 d = 1u << k;
-        if (g.kind == QM_BATCH_CZ) {
-            o.type = 2;
+            cz.q = q;
+            if (g.kind == QM_BATCH_CNOT) cv.dense({q[1]}, {1.0, 1.0, 1.0, -1.0});
+            cv.push(std::move(cz));
+            if (g.kind == QM_BATCH_CNOT) cv.dense({q[1]}, {0.5, 0.5, 0.5, -0.5});
         } else if (g.kind == QM_BATCH_DIAG) {
-            o.type = 1;
-            for (u32 i = 0; i < d; ++i) o.m.push_back(cd(g.matrix[i].re, g.matrix[i].im));
+            for (u32 i = 0; i < d; ++i) m.push_back(cd(g.matrix[i].re, g.matrix[i].im));
+            cv.diagonal(q, m);
         } else {
-            o.type = 0;
-            for (u32 i = 0; i < d * d; ++i) o.m.push_back(cd(g.matrix[i].re, g.matrix[i].im));
+            for (u32 i = 0; i < d * d; ++i) m.push_back(cd(g.matrix[i].re, g.matrix[i].im));
+            cv.dense(q, std::move(m));
         }
-        push_op(c, last, std::move(o));
     }
+    cv.finish();
+    reduce_matrices(c.ops, c.ne);
     return true;
 }
 
