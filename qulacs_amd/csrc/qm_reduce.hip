@@ -7,6 +7,7 @@
 // Reference loops restated: src/csim/stat_ops.cpp:13-86,
 // stat_ops_probability.cpp:11-100, stat_ops_expectation_value.cpp:352-482,
 // stat_ops_transition_amplitude.cpp:19-128, update_ops_named_state.cpp:21-98.
+#include <algorithm>
 #include <cmath>
 
 #include "qm_internal.hpp"
@@ -57,8 +58,9 @@ struct RArgs {
     const double2* __restrict__ b;  // bra (R_TRANS, R_INNER)
     u64 dim;
     u64 mask, value;                // R_MASKED
-    const Term* __restrict__ terms; // R_PAULI / R_TRANS: one per blockIdx.y
+    Term term;                      // R_PAULI / R_TRANS
     double* __restrict__ partials;  // [gridDim.y][gridDim.x][2]
+    double* __restrict__ out;       // a grid of one block: its result goes here, and nothing follows
 };
 
 template <int KIND>
@@ -79,7 +81,7 @@ __global__ __launch_bounds__(kRBlock) void k_reduce(RArgs r) {
         for (u64 i = t0; i < r.dim; i += stride)
             if ((i & r.mask) == r.value) acc_re += norm2(r.a[i]);
     } else if (KIND == R_PAULI) {
-        const Term tm = r.terms[blockIdx.y];
+        const Term tm = r.term;
         if (tm.bf == 0) {
             for (u64 i = t0; i < r.dim; i += stride) {
                 const double p = norm2(r.a[i]);
@@ -96,7 +98,7 @@ __global__ __launch_bounds__(kRBlock) void k_reduce(RArgs r) {
             }
         }
     } else if (KIND == R_TRANS) {
-        const Term tm = r.terms[blockIdx.y];
+        const Term tm = r.term;
         const double2* ket = r.a;
         const double2* bra = r.b;
         if (tm.bf == 0) {
@@ -133,142 +135,331 @@ __global__ __launch_bounds__(kRBlock) void k_reduce(RArgs r) {
     double s_im = 0.0;
     if (KIND == R_TRANS || KIND == R_INNER) s_im = block_sum(acc_im, lds);
     if (threadIdx.x == 0) {
-        double* out = r.partials + ((u64)blockIdx.y * gridDim.x + blockIdx.x) * 2;
+        double* out = r.out ? r.out : r.partials + ((u64)blockIdx.y * gridDim.x + blockIdx.x) * 2;
         out[0] = s_re;
         out[1] = s_im;
     }
 }
 
-// Sums partials[term][0..nb) per term, multiplies by the term's coefficient
-// and writes per-term values plus their total.  One wave per term (16 terms at
-// a time): lane-strided sums in index order, then a fixed shuffle tree; the
-// per-term values are added in term order.  Deterministic, and with no block
-// barriers inside the term loop.
-constexpr int kFinishThreads = 1024;
-__global__ __launch_bounds__(kFinishThreads) void k_finish(const double* __restrict__ partials, unsigned nb,
-                                                           unsigned nterms, const double2* __restrict__ coefs,
+// Sums `count` (re, im) pairs of partials in a fixed order (thread-strided, then a fixed tree)
+// into out, which may be pinned host memory: a copy command for 16 bytes costs more than the
+// kernel.
+constexpr int kFinishThreads = 256;
+__global__ __launch_bounds__(kFinishThreads) void k_finish(const double* __restrict__ partials, unsigned count,
                                                            double* __restrict__ out) {
-    const unsigned lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    for (unsigned t = wid; t < nterms; t += nw) {
-        const double* p = partials + (u64)t * nb * 2;
-        double re = 0.0, im = 0.0;
-        for (unsigned k = lane; k < nb; k += 64) {
-            re += p[2 * k];
-            im += p[2 * k + 1];
-        }
-        re = wave_sum(re);
-        im = wave_sum(im);
-        if (coefs) {
-            const double2 c = coefs[t];
-            const double pr = c.x * re - c.y * im, pi = c.x * im + c.y * re;
-            re = pr;
-            im = pi;
-        }
-        if (lane == 0) {
-            out[2 + 2 * t] = re;
-            out[3 + 2 * t] = im;
-        }
+    __shared__ double lds[32];
+    double re = 0.0, im = 0.0;
+    for (unsigned k = threadIdx.x; k < count; k += kFinishThreads) {
+        re += partials[2 * k];
+        im += partials[2 * k + 1];
     }
-    __syncthreads();  // the per-term values written above are visible to the whole block
+    re = block_sum(re, lds);
+    im = block_sum(im, lds);
     if (threadIdx.x == 0) {
-        double total_re = 0.0, total_im = 0.0;
-        for (unsigned t = 0; t < nterms; ++t) {
-            total_re += out[2 + 2 * t];
-            total_im += out[3 + 2 * t];
-        }
-        out[0] = total_re;
-        out[1] = total_im;
+        out[0] = re;
+        out[1] = im;
     }
 }
 
 unsigned reduce_blocks(u64 work) { return grid_for(work, (u64)kRBlock * 16, kMaxRBlocks); }
 
-// Enqueues one reduction family; on success *dout points at the device result
-// (2 + 2 * max(nterms, 1) doubles: the ordered total, then per-term values),
-// valid until the next reduction on the same stream.
+// Runs one reduction and waits for it; `term` for R_PAULI and R_TRANS.  Returns false on error;
+// the result (re, im) in res.
 template <int KIND>
-bool enqueue_reduce(RArgs r, u64 work, const Term* host_terms, unsigned nterms, const qm_complex* coefs, hipStream_t st,
-                    double** dout, unsigned* ny_out) {
+bool run_reduce(RArgs r, u64 work, const Term* term, hipStream_t st, double res[2]) {
     Scratch* sc = scratch_for(st);
     if (!sc) return false;
     const unsigned nb = reduce_blocks(work);
-    const unsigned ny = nterms ? nterms : 1;
-    if ((u64)nb * ny * 2 + 2 + 2 * (u64)ny > kPartialsCap || 2 + 2 * (u64)ny > kHostResultCap) {
-        set_error(QM_ERR_UNSUPPORTED, "too many terms in one reduction (%u)", ny);
-        return false;
-    }
-    if (nterms) {
-        r.terms = (const Term*)upload(sc, host_terms, sizeof(Term) * nterms);
-        if (!r.terms) return false;
-    }
-    const double2* dcoefs = nullptr;
-    if (coefs) {
-        dcoefs = (const double2*)upload(sc, coefs, sizeof(double2) * ny);
-        if (!dcoefs) return false;
-    }
+    if (term) r.term = *term;
     r.partials = sc->partials;
-    double* out = sc->partials + (u64)nb * ny * 2;
-    k_reduce<KIND><<<dim3(nb, ny), kRBlock, 0, st>>>(r);
-    k_finish<<<1, kFinishThreads, 0, st>>>(sc->partials, nb, ny, dcoefs, out);
-    *dout = out;
-    *ny_out = ny;
+    r.out = nb == 1 ? sc->host_result : nullptr;
+    k_reduce<KIND><<<nb, kRBlock, 0, st>>>(r);
+    if (nb > 1) k_finish<<<1, kFinishThreads, 0, st>>>(sc->partials, nb, sc->host_result);
+    if (!hip_ok(hipGetLastError(), "reduce") || !hip_ok(hipStreamSynchronize(st), "reduce sync")) return false;
+    res[0] = sc->host_result[0];
+    res[1] = sc->host_result[1];
     return true;
 }
 
-// Runs one reduction family and waits for it.  `nterms` > 0 for term-indexed
-// kinds.  Returns false on error; result (re, im) of the ordered total in res.
-template <int KIND>
-bool run_reduce(RArgs r, u64 work, const Term* host_terms, unsigned nterms, const qm_complex* coefs, hipStream_t st,
-                double res[2], std::vector<double>* per_term = nullptr) {
-    double* dout = nullptr;
-    unsigned ny = 0;
-    if (!enqueue_reduce<KIND>(r, work, host_terms, nterms, coefs, st, &dout, &ny)) return false;
-    Scratch* sc = scratch_for(st);
-    const size_t nout = 2 + 2 * (size_t)ny;
-    if (!hip_ok(hipMemcpyAsync(sc->host_result, dout, nout * sizeof(double), hipMemcpyDeviceToHost, st), "reduce"))
-        return false;
-    if (!hip_ok(hipStreamSynchronize(st), "reduce sync")) return false;
-    res[0] = sc->host_result[0];
-    res[1] = sc->host_result[1];
-    if (per_term) per_term->assign(sc->host_result + 2, sc->host_result + nout);
-    return true;
+// ------------------------------------------------------------------ observables
+// sum_k c_k <psi|P_k|psi>.  A term with bit-flip mask bf pairs index x with x ^ bf, so one pass
+// per term reads the whole state for one number.  Terms are put into groups whose masks span at
+// most 4 dimensions over GF(2): the 16 amplitudes of a coset of the span meet only each other
+// in all of a group's terms, so a thread loads one coset and evaluates them all, and the state
+// is read once per group.  With the span in reduced echelon form (pivot bits p_0..p_3), cosets
+// are numbered by the index bits that are no pivots, and member m is base ^ (sum of the
+// basis vectors in m); a term is the pairs (m, m ^ e), e = its mask's pivot bits, with the
+// sign (-1)^popcount(index & pf) = (lane: base & pf) x (uniform: bit m of a 16-bit pattern).
+// Bound: HBM.  25 qubits, 24 random terms: 24 passes, 1.91 ms; with 6 groups 0.51 ms (6.3 TB/s).  One block for all up
+// to 2^13 amplitudes, which needs no second launch.
+constexpr int kObsRank = 4;
+constexpr int kObsMembers = 1 << kObsRank;
+constexpr unsigned kObsInlineTerms = 48, kObsInlineGroups = 16;  // passed as kernel arguments
+constexpr unsigned kObsMaxBlocks = 2048, kObsMaxGroups = 256;   // per launch
+constexpr u64 kObsOneBlock = 1ULL << 13;                         // states up to here: one block does all
+
+struct ObsTerm {
+    u64 bf, pf;
+    u32 e, pattern;   // e: pairs (m, m ^ e), odd: 16 set if the imaginary part counts
+    double cre, cim;  // coefficient with the factor 2 of a pair and the sign of i^rot
+};
+struct ObsGroup {
+    u64 basis[kObsRank];
+    u32 term0, nterm;
+    unsigned char piv[kObsRank];  // ascending
+    u32 pad;
+};
+struct ObsArgs {
+    const double2* state;
+    u64 dim;
+    double* partials;  // [group][gridDim.x][2]
+    double* out;       // a single block writes the total here
+    u32 ngroup;
+    const ObsTerm* terms;    // more than the arrays below hold
+    const ObsGroup* groups;
+    ObsTerm term[kObsInlineTerms];
+    ObsGroup group[kObsInlineGroups];
+};
+
+template <int E, bool ODD>
+__device__ __forceinline__ double pair_sum(const double2 (&v)[kObsMembers], u32 pattern) {
+    double s = 0.0;
+#pragma unroll
+    for (int m = 0; m < kObsMembers; ++m) {
+        if (m > (m ^ E)) continue;
+        const double2 a = v[m], b = v[m ^ E];
+        const double t = ODD ? fma(a.y, b.x, -a.x * b.y) : fma(a.x, b.x, a.y * b.y);
+        s = fma(t, ((pattern >> m) & 1u) ? -1.0 : 1.0, s);
+    }
+    return s;
+}
+__device__ __forceinline__ double term_sum(const double2 (&v)[kObsMembers], u32 e, u32 pattern) {
+    switch (e) {
+#define QM_OBS_CASE(E)                                     \
+    case E: return pair_sum<E, false>(v, pattern);         \
+    case E + 16: return pair_sum<E, true>(v, pattern);
+        QM_OBS_CASE(1) QM_OBS_CASE(2) QM_OBS_CASE(3) QM_OBS_CASE(4) QM_OBS_CASE(5) QM_OBS_CASE(6) QM_OBS_CASE(7)
+        QM_OBS_CASE(8) QM_OBS_CASE(9) QM_OBS_CASE(10) QM_OBS_CASE(11) QM_OBS_CASE(12) QM_OBS_CASE(13) QM_OBS_CASE(14)
+        QM_OBS_CASE(15)
+#undef QM_OBS_CASE
+        default: return pair_sum<0, false>(v, pattern);
+    }
+}
+
+template <bool INLINE>
+__global__ __launch_bounds__(kRBlock) void k_observable(ObsArgs a) {
+    __shared__ double lds[32];
+    double re = 0.0, im = 0.0;
+    // up to 64 cosets: a group per wave instead of the groups one after another
+    const bool by_wave = a.dim <= 64 * kObsMembers;
+    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const u64 stride = by_wave ? 64 : (u64)gridDim.x * blockDim.x;
+    const u64 t0 = by_wave ? threadIdx.x & 63 : (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    const double2* __restrict__ psi = a.state;
+    for (u32 g = by_wave ? wave : blockIdx.y; g < a.ngroup; g += by_wave ? kRBlock / 64 : gridDim.y) {
+        const ObsGroup gr = INLINE ? a.group[g] : a.groups[g];
+        if (a.dim < (u64)kObsMembers) {  // fewer amplitudes than a coset has
+            if (t0 < a.dim) {
+                for (u32 k = 0; k < gr.nterm; ++k) {
+                    const ObsTerm tm = INLINE ? a.term[gr.term0 + k] : a.terms[gr.term0 + k];
+                    const double2 x = psi[t0], y = psi[t0 ^ tm.bf];
+                    double t = (tm.e & 16u) ? fma(x.y, y.x, -x.x * y.y) : fma(x.x, y.x, x.y * y.y);
+                    if (tm.bf) t *= 0.5;  // every pair is met from both sides
+                    if (par(t0 & tm.pf)) t = -t;
+                    re = fma(tm.cre, t, re);
+                    im = fma(tm.cim, t, im);
+                }
+            }
+            continue;
+        }
+        for (u64 i = t0; i < a.dim / kObsMembers; i += stride) {
+            u64 base = i;
+#pragma unroll
+            for (int k = 0; k < kObsRank; ++k) base = insert_zero(base, gr.piv[k]);
+            double2 v[kObsMembers];
+#pragma unroll
+            for (int m = 0; m < kObsMembers; ++m) {
+                const u64 off = ((m & 1) ? gr.basis[0] : 0) ^ ((m & 2) ? gr.basis[1] : 0) ^ ((m & 4) ? gr.basis[2] : 0) ^
+                                ((m & 8) ? gr.basis[3] : 0);
+                v[m] = psi[base ^ off];
+            }
+            for (u32 k = 0; k < gr.nterm; ++k) {
+                const ObsTerm tm = INLINE ? a.term[gr.term0 + k] : a.terms[gr.term0 + k];
+                // keeps the products of all 31 cases from being formed in front of the loop
+#pragma unroll
+                for (int m = 0; m < kObsMembers; ++m) asm volatile("" : "+v"(v[m].x), "+v"(v[m].y));
+                double t = term_sum(v, tm.e, tm.pattern);
+                if (par(base & tm.pf)) t = -t;
+                re = fma(tm.cre, t, re);
+                im = fma(tm.cim, t, im);
+            }
+        }
+    }
+    re = block_sum(re, lds);
+    im = block_sum(im, lds);
+    if (threadIdx.x == 0) {
+        double* out = a.out ? a.out : a.partials + ((u64)blockIdx.y * gridDim.x + blockIdx.x) * 2;
+        out[0] = re;
+        out[1] = im;
+    }
+}
+
+// Groups the terms of an observable on n qubits.
+struct ObsPlan {
+    std::vector<ObsTerm> terms;  // group after group
+    std::vector<ObsGroup> groups;
+};
+ObsPlan plan_observable(const u64* bf, const u64* pf, const u32* rot, const qm_complex* coef, u32 nterms, int n) {
+    ObsPlan pl;
+    // the distinct flip masks, by their highest bit, dealt out so that the pivots of a group are
+    // spread over the register: low pivots alone would make a wave's loads touch 16-byte pieces
+    // of distant lines
+    std::vector<u64> masks;
+    for (u32 k = 0; k < nterms; ++k)
+        if (bf[k]) masks.push_back(bf[k]);
+    std::sort(masks.begin(), masks.end());
+    masks.erase(std::unique(masks.begin(), masks.end()), masks.end());
+    const size_t D = masks.size(), deal = std::max<size_t>(1, (D + kObsRank - 1) / kObsRank);
+    std::vector<u64> order;
+    for (size_t g = 0; g < deal; ++g)
+        for (size_t k = g; k < D; k += deal) order.push_back(masks[k]);
+    struct Space {
+        std::vector<u64> basis;  // reduced echelon form, pivot = highest bit of each
+        u64 reduce(u64 v) const {
+            for (u64 b : basis)
+                if ((v >> (63 - __builtin_clzll(b))) & 1) v ^= b;
+            return v;
+        }
+        void insert(u64 v) {  // v reduced and not 0
+            const int p = 63 - __builtin_clzll(v);
+            for (u64& b : basis)
+                if ((b >> p) & 1) b ^= v;
+            basis.push_back(v);
+        }
+    };
+    std::vector<Space> spaces(1);
+    // group of each mask (sorted); a mask in an earlier group's span joins it (searched
+    // while there are few)
+    std::vector<u32> group_of(D, 0);
+    auto index_of = [&](u64 m) { return (size_t)(std::lower_bound(masks.begin(), masks.end(), m) - masks.begin()); };
+    for (u64 m : order) {
+        size_t g = spaces.size() - 1;
+        bool found = false;
+        for (size_t k = D <= 256 ? 0 : g; k <= g && !found; ++k)
+            if (spaces[k].reduce(m) == 0) {
+                group_of[index_of(m)] = (u32)k;
+                found = true;
+            }
+        if (found) continue;
+        if (spaces[g].basis.size() == (size_t)kObsRank || (int)spaces[g].basis.size() == n) {
+            spaces.emplace_back();
+            ++g;
+        }
+        spaces[g].insert(spaces[g].reduce(m));
+        group_of[index_of(m)] = (u32)g;
+    }
+    // fill every basis up to the full rank with single high bits
+    for (Space& sp : spaces)
+        for (int q = n - 1; q >= 0 && sp.basis.size() < (size_t)kObsRank; --q)
+            if (sp.reduce(1ULL << q)) sp.insert(sp.reduce(1ULL << q));
+    std::vector<std::vector<u32>> members(spaces.size());
+    for (u32 k = 0; k < nterms; ++k) members[bf[k] ? group_of[index_of(bf[k])] : 0].push_back(k);
+    for (size_t g = 0; g < spaces.size(); ++g) {
+        std::vector<u64>& b = spaces[g].basis;
+        std::sort(b.begin(), b.end());  // ascending pivots
+        ObsGroup gr{};
+        for (size_t k = 0; k < b.size(); ++k) {
+            gr.basis[k] = b[k];
+            gr.piv[k] = (unsigned char)(63 - __builtin_clzll(b[k]));
+        }
+        gr.term0 = (u32)pl.terms.size();
+        gr.nterm = (u32)members[g].size();
+        for (u32 k : members[g]) {
+            ObsTerm t{};
+            t.bf = bf[k];
+            t.pf = pf[k];
+            for (size_t i = 0; i < b.size(); ++i) t.e |= (u32)((bf[k] >> gr.piv[i]) & 1u) << i;
+            for (u32 m = 0; m < (u32)kObsMembers; ++m) {
+                u64 off = 0;
+                for (size_t i = 0; i < b.size(); ++i)
+                    if ((m >> i) & 1) off ^= b[i];
+                t.pattern |= (u32)(__builtin_popcountll(off & pf[k]) & 1) << m;
+            }
+            // a pair gives 2 Re(z i^rot), z = psi_x conj(psi_y) and x's parity; a Z string |psi_x|^2
+            double f = 1.0;
+            if (bf[k]) {
+                const u32 r = rot[k] & 3u;
+                f = (r == 1 || r == 2) ? -2.0 : 2.0;
+                if (r & 1u) t.e |= 16u;
+            }
+            t.cre = f * coef[k].re;
+            t.cim = f * coef[k].im;
+            pl.terms.push_back(t);
+        }
+        pl.groups.push_back(gr);
+    }
+    return pl;
+}
+
+unsigned obs_blocks(u64 dim) {
+    return dim <= kObsOneBlock ? 1u : (unsigned)std::min<u64>(kObsMaxBlocks, (dim / kObsMembers + kRBlock - 1) / kRBlock);
+}
+
+// Enqueues the groups [g0, g0 + ng) of a plan; their sum goes to out (device or pinned memory).
+// `tables` holds the terms and groups in device memory when they are too many for the arguments.
+bool launch_observable(const ObsPlan& pl, size_t g0, size_t ng, const void* state, u64 dim, hipStream_t st,
+                       double* partials, const ObsTerm* dterms, const ObsGroup* dgroups, double* out, const char* what) {
+    ObsArgs a{};
+    a.state = (const double2*)state;
+    a.dim = dim;
+    a.partials = partials;
+    a.ngroup = (u32)ng;
+    a.terms = dterms;
+    a.groups = dgroups ? dgroups + g0 : nullptr;
+    const unsigned nb = obs_blocks(dim);
+    const unsigned ny = nb == 1 ? 1u : (unsigned)ng;
+    a.out = nb * ny == 1 ? out : nullptr;
+    if (!dterms) {
+        std::copy(pl.terms.begin(), pl.terms.end(), a.term);
+        std::copy(pl.groups.begin(), pl.groups.end(), a.group);
+        k_observable<true><<<dim3(nb, ny), kRBlock, 0, st>>>(a);
+    } else {
+        k_observable<false><<<dim3(nb, ny), kRBlock, 0, st>>>(a);
+    }
+    if (nb * ny > 1) k_finish<<<1, kFinishThreads, 0, st>>>(partials, nb * ny, out);
+    return hip_ok(hipGetLastError(), what);
+}
+bool obs_inline(const ObsPlan& pl) {
+    return pl.terms.size() <= kObsInlineTerms && pl.groups.size() <= kObsInlineGroups;
 }
 
 bool enqueue_observable(const u64* bf, const u64* pf, const u32* rot, const double* coef, u32 nterms,
                         const void* state, u64 dim, hipStream_t st, double* h_out) {
-    std::vector<Term> zt, xt;
-    std::vector<qm_complex> zc, xc;
-    for (u32 k = 0; k < nterms; ++k) {
-        const unsigned pivot = bf[k] ? 63 - __builtin_clzll(bf[k]) : 0;
-        Term t{bf[k], pf[k], rot[k], pivot};
-        if (bf[k]) {
-            xt.push_back(t);
-            xc.push_back(qm_complex{coef[k], 0.0});
-        } else {
-            zt.push_back(t);
-            zc.push_back(qm_complex{coef[k], 0.0});
-        }
+    for (int i = 0; i < 4; ++i) h_out[i] = 0.0;
+    if (nterms == 0) return true;
+    std::vector<qm_complex> c(nterms);
+    for (u32 k = 0; k < nterms; ++k) c[k] = qm_complex{coef[k], 0.0};
+    const ObsPlan pl = plan_observable(bf, pf, rot, c.data(), nterms, log2_dim(dim));
+    Scratch* sc = scratch_for(st);
+    if (!sc) return false;
+    const char* what = "enqueue_observable";
+    const ObsTerm* dt = nullptr;
+    const ObsGroup* dg = nullptr;
+    if (!obs_inline(pl)) {
+        dt = (const ObsTerm*)upload(sc, pl.terms.data(), pl.terms.size() * sizeof(ObsTerm));
+        dg = (const ObsGroup*)upload(sc, pl.groups.data(), pl.groups.size() * sizeof(ObsGroup));
+        if (!dt || !dg) return false;
     }
-    RArgs r{};
-    r.a = (const double2*)state;
-    r.dim = dim;
-    for (int g = 0; g < 2; ++g) {
-        const std::vector<Term>& tv = g ? xt : zt;
-        const std::vector<qm_complex>& cv = g ? xc : zc;
-        if (tv.empty()) {
-            h_out[2 * g] = 0.0;
-            h_out[2 * g + 1] = 0.0;
-            continue;
-        }
-        double* dout = nullptr;
-        unsigned ny = 0;
-        if (!enqueue_reduce<R_PAULI>(r, g ? dim / 2 : dim, tv.data(), (unsigned)tv.size(), cv.data(), st, &dout, &ny))
-            return false;
-        // copied before the next reduction on this stream can reuse the scratch
-        if (!hip_ok(hipMemcpyAsync(h_out + 2 * g, dout, 2 * sizeof(double), hipMemcpyDeviceToHost, st),
-                    "enqueue_observable"))
-            return false;
+    // the last (usually only) launch's sum goes to the caller's pinned buffer; more than
+    // kObsMaxGroups groups add up in pairs there
+    if (pl.groups.size() > 2 * kObsMaxGroups) {
+        set_error(QM_ERR_UNSUPPORTED, "%s: too many terms in one observable (%u)", what, nterms);
+        return false;
     }
+    for (size_t g = 0; g < pl.groups.size(); g += kObsMaxGroups)
+        if (!launch_observable(pl, g, std::min<size_t>(kObsMaxGroups, pl.groups.size() - g), state, dim, st, sc->partials,
+                               dt, dg, h_out + (g ? 2 : 0), what))
+            return false;
     return true;
 }
 
@@ -323,7 +514,7 @@ double pauli_expectation(const Term& t, void* state, u64 dim, void* stream, unsi
     r.a = (const double2*)state;
     r.dim = dim;
     double res[2] = {0, 0};
-    run_reduce<R_PAULI>(r, t.bf ? dim / 2 : dim, &t, 1, nullptr, stream_of(stream), res);
+    run_reduce<R_PAULI>(r, t.bf ? dim / 2 : dim, &t, stream_of(stream), res);
     return res[0];
 }
 
@@ -341,7 +532,7 @@ qm_complex transition(const Term& t, void* bra, void* ket, u64 dim, void* stream
     r.b = (const double2*)bra;
     r.dim = dim;
     double res[2] = {0, 0};
-    if (run_reduce<R_TRANS>(r, t.bf ? dim / 2 : dim, &t, 1, nullptr, stream_of(stream), res)) {
+    if (run_reduce<R_TRANS>(r, t.bf ? dim / 2 : dim, &t, stream_of(stream), res)) {
         z.re = res[0];
         z.im = res[1];
     }
@@ -384,22 +575,20 @@ __global__ __launch_bounds__(512) void k_scale_r(double2* __restrict__ s, u64 di
 }
 
 // ------------------------------------------------------------------ allocation-free observable
-// qm_observable_expectation_noalloc_host runs the same two launches per term
-// group as qm_observable_expectation_host (k_reduce<R_PAULI>, then k_finish),
-// but its term table, coefficients, per-block partials and group results live
-// in `scratch`, a fixed device array, instead of the library's per-stream
-// allocations.  Every block of k_reduce writes its partial slot and k_finish
-// writes every result slot, so nothing in it has to start at zero.  All calls
-// on one device share that device's copy: calls that overlap on one device
-// (other threads, other streams) race.
+// qm_observable_expectation_noalloc_host runs the same launches as
+// qm_observable_expectation_host (k_observable, then k_finish), but its tables, per-block
+// partials and results live in `scratch`, a fixed device array, instead of the library's
+// per-stream allocations.  Every block writes its partial slot and k_finish writes the result,
+// so nothing in it has to start at zero.  All calls on one device share that device's copy: calls
+// that overlap on one device (other threads, other streams) race.
 constexpr unsigned kNoAllocMaxTerms = 128;
 constexpr size_t kNoAllocTermsOff = 0;
-constexpr size_t kNoAllocCoefsOff = 4096;                                        // >= 128 * sizeof(Term)
-constexpr size_t kNoAllocOutOff = kNoAllocCoefsOff + 2048;                       // 128 * 16 bytes
-constexpr size_t kNoAllocOutDoubles = 2 + 2 * kNoAllocMaxTerms;                  // per group
-constexpr size_t kNoAllocPartialsOff = kNoAllocOutOff + 2 * kNoAllocOutDoubles * 8 + 256 - (2 * kNoAllocOutDoubles * 8) % 256;
-constexpr size_t kNoAllocBytes = kNoAllocPartialsOff + (size_t)kMaxRBlocks * kNoAllocMaxTerms * 2 * sizeof(double);
-static_assert(kNoAllocMaxTerms * sizeof(Term) <= kNoAllocCoefsOff, "term table overlaps the coefficients");
+constexpr size_t kNoAllocGroupsOff = 6144;    // >= 128 * sizeof(ObsTerm)
+constexpr size_t kNoAllocOutOff = 14336;      // >= kNoAllocGroupsOff + 128 * sizeof(ObsGroup)
+constexpr size_t kNoAllocPartialsOff = 14592;
+constexpr size_t kNoAllocBytes = kNoAllocPartialsOff + (size_t)kObsMaxBlocks * kNoAllocMaxTerms * 2 * sizeof(double);
+static_assert(kNoAllocMaxTerms * sizeof(ObsTerm) <= kNoAllocGroupsOff, "term table overlaps the groups");
+static_assert(kNoAllocGroupsOff + kNoAllocMaxTerms * sizeof(ObsGroup) <= kNoAllocOutOff, "groups overlap the result");
 static_assert(kNoAllocPartialsOff % 256 == 0, "partials not 256-byte aligned");
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
@@ -436,7 +625,7 @@ double state_norm_squared_host(void* state, ITYPE dim, void* stream, unsigned de
     r.a = (const double2*)state;
     r.dim = dim;
     double res[2] = {0, 0};
-    run_reduce<R_NORM>(r, dim, nullptr, 0, nullptr, stream_of(stream), res);
+    run_reduce<R_NORM>(r, dim, nullptr, stream_of(stream), res);
     return res[0];
 }
 
@@ -450,7 +639,7 @@ double measurement_distribution_entropy_host(void* state, ITYPE dim, void* strea
     r.a = (const double2*)state;
     r.dim = dim;
     double res[2] = {0, 0};
-    run_reduce<R_ENTROPY>(r, dim, nullptr, 0, nullptr, stream_of(stream), res);
+    run_reduce<R_ENTROPY>(r, dim, nullptr, stream_of(stream), res);
     return res[0];
 }
 
@@ -462,7 +651,7 @@ static double masked_prob(u64 mask, u64 value, void* state, ITYPE dim, void* str
     r.mask = mask;
     r.value = value;
     double res[2] = {0, 0};
-    run_reduce<R_MASKED>(r, dim, nullptr, 0, nullptr, stream_of(stream), res);
+    run_reduce<R_MASKED>(r, dim, nullptr, stream_of(stream), res);
     return res[0];
 }
 
@@ -560,7 +749,7 @@ qm_complex inner_product_host(const void* bra, const void* ket, ITYPE dim, void*
     r.b = (const double2*)bra;
     r.dim = dim;
     double res[2] = {0, 0};
-    if (run_reduce<R_INNER>(r, dim, nullptr, 0, nullptr, stream_of(stream), res)) {
+    if (run_reduce<R_INNER>(r, dim, nullptr, stream_of(stream), res)) {
         z.re = res[0];
         z.im = res[1];
     }
@@ -580,35 +769,34 @@ qm_complex qm_observable_expectation_host(const ITYPE* bfs, const ITYPE* pfs, co
     }
     if (!use_device(dev)) return z;
     const int n = log2_dim(dim);
-    // Split into Z-only terms and flip terms: each group runs as one launch
-    // (blockIdx.y = term) so a group never re-launches per term.
-    std::vector<Term> zt, xt;
-    std::vector<qm_complex> zc, xc;
-    for (UINT k = 0; k < nterms; ++k) {
+    for (UINT k = 0; k < nterms; ++k)
         if (((bfs[k] | pfs[k]) >> n) != 0) {
             set_error(QM_ERR_INVALID_ARGUMENT, "%s: term %u acts beyond %d qubits", what, k, n);
             return z;
         }
-        unsigned pivot = bfs[k] ? 63 - __builtin_clzll(bfs[k]) : 0;
-        const Term t = make_term(bfs[k], pfs[k], rots[k], pivot);
-        if (bfs[k]) { xt.push_back(t); xc.push_back(coefs[k]); }
-        else { zt.push_back(t); zc.push_back(coefs[k]); }
-    }
     hipStream_t st = stream_of(stream);
-    RArgs r{};
-    r.a = (const double2*)state;
-    r.dim = dim;
+    Scratch* sc = scratch_for(st);
+    if (!sc) return z;
     double total_re = 0, total_im = 0;
-    const size_t chunk = 256;
-    for (int g = 0; g < 2; ++g) {
-        const std::vector<Term>& tv = g ? xt : zt;
-        const std::vector<qm_complex>& cv = g ? xc : zc;
-        for (size_t off = 0; off < tv.size(); off += chunk) {
-            const unsigned cnt = (unsigned)std::min(chunk, tv.size() - off);
-            double res[2] = {0, 0};
-            if (!run_reduce<R_PAULI>(r, g ? dim / 2 : dim, tv.data() + off, cnt, cv.data() + off, st, res)) return z;
-            total_re += res[0];
-            total_im += res[1];
+    // as many terms at a time as the upload ring takes; a launch per kObsMaxGroups groups
+    const UINT chunk = 1u << 15;
+    for (UINT off = 0; off < nterms; off += chunk) {
+        const UINT cnt = std::min(chunk, nterms - off);
+        const ObsPlan pl = plan_observable(bfs + off, pfs + off, rots + off, coefs + off, cnt, n);
+        const ObsTerm* dt = nullptr;
+        const ObsGroup* dg = nullptr;
+        if (!obs_inline(pl)) {
+            dt = (const ObsTerm*)upload(sc, pl.terms.data(), pl.terms.size() * sizeof(ObsTerm));
+            dg = (const ObsGroup*)upload(sc, pl.groups.data(), pl.groups.size() * sizeof(ObsGroup));
+            if (!dt || !dg) return z;
+        }
+        for (size_t g = 0; g < pl.groups.size(); g += kObsMaxGroups) {
+            if (!launch_observable(pl, g, std::min<size_t>(kObsMaxGroups, pl.groups.size() - g), state, dim, st,
+                                   sc->partials, dt, dg, sc->host_result, what) ||
+                !hip_ok(hipStreamSynchronize(st), what))
+                return z;
+            total_re += sc->host_result[0];
+            total_im += sc->host_result[1];
         }
     }
     z.re = total_re;
@@ -639,56 +827,30 @@ qm_complex qm_observable_expectation_noalloc_host(const ITYPE* bfs, const ITYPE*
             set_error(QM_ERR_INVALID_ARGUMENT, "%s: term %u acts beyond %d qubits", what, k, n);
             return z;
         }
-    // Z-only terms first, then flip terms, each group in input order (the
-    // grouping of the allocating entry point).
-    Term ht[kNoAllocMaxTerms];
-    qm_complex hc[kNoAllocMaxTerms];
-    unsigned count[2] = {0, 0};
-    for (int g = 0; g < 2; ++g)
-        for (UINT k = 0; k < nterms; ++k) {
-            if ((bfs[k] != 0) != (g == 1)) continue;
-            const unsigned pivot = bfs[k] ? 63 - __builtin_clzll(bfs[k]) : 0;
-            ht[count[0] + count[1]] = make_term(bfs[k], pfs[k], rots[k], pivot);
-            hc[count[0] + count[1]] = coefs[k];
-            ++count[g];
-        }
-    const unsigned first[2] = {0, count[0]};
+    const ObsPlan pl = plan_observable(bfs, pfs, rots, coefs, nterms, n);  // at most a group per term
     if (!use_device(dev)) return z;
     unsigned char* base = noalloc_scratch(dev, what);
     if (!base) return z;
-    Term* dterms = (Term*)(base + kNoAllocTermsOff);
-    double2* dcoefs = (double2*)(base + kNoAllocCoefsOff);
     double* dout = (double*)(base + kNoAllocOutOff);
-    double* partials = (double*)(base + kNoAllocPartialsOff);
     hipStream_t st = stream_of(stream);
-    if (!hip_ok(hipMemcpyAsync(dterms, ht, nterms * sizeof(Term), hipMemcpyHostToDevice, st), what) ||
-        !hip_ok(hipMemcpyAsync(dcoefs, hc, nterms * sizeof(double2), hipMemcpyHostToDevice, st), what))
-        return z;
-    RArgs r{};
-    r.a = (const double2*)state;
-    r.dim = dim;
-    r.partials = partials;
-    for (int g = 0; g < 2; ++g) {
-        if (!count[g]) continue;
-        const unsigned nb = reduce_blocks(g ? dim / 2 : dim);
-        r.terms = dterms + first[g];
-        k_reduce<R_PAULI><<<dim3(nb, count[g]), kRBlock, 0, st>>>(r);
-        k_finish<<<1, kFinishThreads, 0, st>>>(partials, nb, count[g], dcoefs + first[g], dout + g * kNoAllocOutDoubles);
-    }
-    double res[2][2] = {{0, 0}, {0, 0}};
-    for (int g = 0; g < 2; ++g)
-        if (count[g] && !hip_ok(hipMemcpyAsync(res[g], dout + g * kNoAllocOutDoubles, 2 * sizeof(double),
-                                               hipMemcpyDeviceToHost, st), what))
+    ObsTerm* dt = nullptr;
+    ObsGroup* dg = nullptr;
+    if (!obs_inline(pl)) {
+        dt = (ObsTerm*)(base + kNoAllocTermsOff);
+        dg = (ObsGroup*)(base + kNoAllocGroupsOff);
+        if (!hip_ok(hipMemcpyAsync(dt, pl.terms.data(), pl.terms.size() * sizeof(ObsTerm), hipMemcpyHostToDevice, st), what) ||
+            !hip_ok(hipMemcpyAsync(dg, pl.groups.data(), pl.groups.size() * sizeof(ObsGroup), hipMemcpyHostToDevice, st),
+                    what))
             return z;
-    if (!hip_ok(hipGetLastError(), what) || !hip_ok(hipStreamSynchronize(st), what)) return z;
-    double total_re = 0, total_im = 0;
-    for (int g = 0; g < 2; ++g)
-        if (count[g]) {
-            total_re += res[g][0];
-            total_im += res[g][1];
-        }
-    z.re = total_re;
-    z.im = total_im;
+    }
+    double res[2] = {0, 0};
+    if (!launch_observable(pl, 0, pl.groups.size(), state, dim, st, (double*)(base + kNoAllocPartialsOff), dt, dg, dout,
+                           what) ||
+        !hip_ok(hipMemcpyAsync(res, dout, sizeof(res), hipMemcpyDeviceToHost, st), what) ||
+        !hip_ok(hipStreamSynchronize(st), what))
+        return z;
+    z.re = 0.0 + res[0];  // summed as in the allocating entry point
+    z.im = 0.0 + res[1];
     return z;
 }
 
