@@ -682,9 +682,12 @@ class QuantumCircuit {
    protected:
     friend class QuantumCircuitOptimizer;
     friend class NoiseSimulator;
-    void touched() { ++version_; }
+    // the gate list changed / an angle changed
+    void touched() { ++version_, ++structure_; }
+    void angle_touched() { ++version_; }
     unsigned qubit_count_;
     std::vector<QuantumGateBase*> gates_;
+    uint64_t structure_ = 0;  // changes with the gate list, not with angles
 
    private:
     // Fused execution of a whole-circuit update on a state vector: maximal runs of
@@ -784,6 +787,26 @@ class ParametricQuantumCircuit : public QuantumCircuit {
    private:
     QuantumGate_SingleParameter* param(size_t i) const;
     std::vector<size_t> param_pos_;  // gate index of parameter i
+    // backprop through the adjoint engine (qm_adjoint_*): the scheduled circuit and its device
+    // buffers, kept until the gate list changes.  A copy of the circuit starts without one.
+    struct Adjoint {
+        Adjoint() = default;
+        Adjoint(const Adjoint&) {}
+        Adjoint& operator=(const Adjoint&) = delete;
+        ~Adjoint() { release(); }
+        void release();
+        std::mutex mutex;
+        uint64_t structure = ~0ULL;
+        qm_adjoint* plan = nullptr;  // null: the circuit has a gate the engine does not take
+        std::vector<double> fixed;   // angles of rotations that are no parameter, after the parameters
+        void* stream = nullptr;
+        void* io = nullptr;          // angles, then the energy and the gradient
+        void* work = nullptr;        // kept between calls up to kKeepBytes
+        size_t work_bytes = 0;
+        static constexpr size_t kKeepBytes = size_t(64) << 20;
+    } adjoint_;
+    bool plan_adjoint();
+    bool backprop_fused(const GeneralQuantumOperator& obs, std::vector<double>* grad);
 };
 
 // Parameter-shift gradient (src/vqcsim/GradCalculator.cpp:8-53).

@@ -306,15 +306,6 @@ __global__ __launch_bounds__(tile_threads<K>(), K == 4 ? 2 : 4) void k_tile(doub
     }
 }
 
-template <class T>
-bool dev_upload(T** dst, const std::vector<T>& src) {
-    *dst = nullptr;
-    if (src.empty()) return true;
-    if (!hip_ok(hipMalloc((void**)dst, src.size() * sizeof(T)), "qm_batch_compile: hipMalloc")) return false;
-    return hip_ok(hipMemcpy(*dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice),
-                  "qm_batch_compile: hipMemcpy");
-}
-
 // Grows *dst to hold `bytes` (contents not kept); capacity in *cap.
 bool dev_reserve(void** dst, size_t* cap, size_t bytes, const char* what) {
     if (*cap >= bytes && *dst) return true;
@@ -400,17 +391,16 @@ struct qm_circuit {
     std::vector<double2> pool;
     int device = -1;
     int per_cu = 0, cus = 0;
+    char* d_program = nullptr;  // one allocation, filled by one copy: passes, sub-operations, pool
     qm::DPass* d_passes = nullptr;
     qm::DSub* d_subs = nullptr;
     double2* d_pool = nullptr;
     void release() {
         if (device >= 0) {
             (void)hipSetDevice(device);
-            void* ptrs[] = {d_passes, d_subs, d_pool};
-            for (void* p : ptrs)
-                if (p) (void)hipFree(p);
+            if (d_program) (void)hipFree(d_program);
         }
-        d_passes = nullptr; d_subs = nullptr; d_pool = nullptr;
+        d_program = nullptr; d_passes = nullptr; d_subs = nullptr; d_pool = nullptr;
         device = -1;
         per_cu = 0;
     }
@@ -805,12 +795,24 @@ namespace qm {
 bool circuit_prepare(qm_circuit* c, unsigned dev) {
     if (c->device != (int)dev) {
         c->release();
-        bool ok = dev_upload(&c->d_passes, c->passes) && dev_upload(&c->d_subs, c->subs) &&
-                  dev_upload(&c->d_pool, c->pool);
-        if (!ok) {
-            c->release();
+        auto round = [](size_t b) { return (b + 255) & ~size_t(255); };
+        const size_t np = round(c->passes.size() * sizeof(DPass)), ns = round(c->subs.size() * sizeof(DSub));
+        const size_t nm = c->pool.size() * sizeof(double2);
+        std::vector<char> host(np + ns + nm);
+        std::memcpy(host.data(), c->passes.data(), c->passes.size() * sizeof(DPass));
+        std::memcpy(host.data() + np, c->subs.data(), c->subs.size() * sizeof(DSub));
+        std::memcpy(host.data() + np + ns, c->pool.data(), nm);
+        const char* what = "qm_circuit_apply: program";
+        char* d = nullptr;
+        if (!hip_ok(hipMalloc((void**)&d, host.size()), what)) return false;
+        if (!hip_ok(hipMemcpy(d, host.data(), host.size(), hipMemcpyHostToDevice), what)) {
+            (void)hipFree(d);
             return false;
         }
+        c->d_program = d;
+        c->d_passes = (DPass*)d;
+        c->d_subs = (DSub*)(d + np);
+        c->d_pool = (double2*)(d + np + ns);
         c->device = (int)dev;
     }
     return true;
