@@ -271,6 +271,8 @@ QM_EXPORT double dm_measurement_distribution_entropy_host(void* state, ITYPE dim
 QM_EXPORT double dm_M0_prob_host(UINT target_qubit_index, void* state, ITYPE dim, void* stream, unsigned int device_number); /* stat_ops_dm.cpp:49-63 */
 QM_EXPORT double dm_marginal_prob_host(const UINT* sorted_target_qubit_index_list, const UINT* measured_value_list, UINT target_qubit_index_count, void* state, ITYPE dim, void* stream, unsigned int device_number); /* stat_ops_dm.cpp:89-114 */
 QM_EXPORT double dm_expectation_value_multi_qubit_Pauli_operator_partial_list_host(const UINT* target_qubit_index_list, const UINT* Pauli_operator_type_list, UINT target_qubit_index_count, void* state, ITYPE dim, void* stream, unsigned int device_number); /* stat_ops_dm.cpp:164-191 */
+/* sum_k coef_k Tr(P_k rho) in one call, terms as in qm_observable_expectation_host. */
+QM_EXPORT qm_complex qm_dm_observable_expectation_host(const ITYPE* bit_flip_masks, const ITYPE* phase_flip_masks, const UINT* global_phase_90rot_counts, const qm_complex* coefs, UINT term_count, void* state, ITYPE dim, void* stream, unsigned int device_number);
 QM_EXPORT void dm_normalize_host(double squared_norm, void* state, ITYPE dim, void* stream, unsigned int device_number); /* update_ops_dm.cpp:14-31 */
 /* DM sampling over |rho_ii| (src/cppsim/state_dm.hpp:383-408), same contract as qm_sampling_host. */
 QM_EXPORT void dm_sampling_host(const double* uniforms, UINT count, ITYPE* out, void* state, ITYPE dim, void* stream, unsigned int device_number);
@@ -310,6 +312,11 @@ QM_EXPORT void dm_state_partial_trace_from_state_vector_host(const UINT* target,
 #define QM_BATCH_DIAG 1u
 #define QM_BATCH_CZ 2u
 #define QM_BATCH_CNOT 3u
+/* qm_circuit_create only, on a density matrix taken as a state of 2 n qubits (qubit t:
+ * column bit t, row bit t + n): uniform depolarizing on one qubit, qubits = {t, t + n}, or on
+ * two, {t, t + n, u, u + n}.  Entries whose row and column bits of those qubits differ are
+ * multiplied by s; the others by s, plus t times their sum; matrix[0] = {s, t}. */
+#define QM_BATCH_DEPOL 5u
 #define QM_BATCH_MAX_QUBITS 20u
 typedef struct qm_batch_gate {
     UINT kind;

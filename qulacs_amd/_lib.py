@@ -32,6 +32,7 @@ class QmBatchGate(C.Structure):
 
 
 BATCH_DENSE, BATCH_DIAG, BATCH_CZ, BATCH_CNOT = 0, 1, 2, 3
+BATCH_DEPOL = 5  # qm_circuit_create only
 ADJ_ROT = 4
 
 
@@ -137,6 +138,7 @@ _SIGS: dict[str, tuple] = {
     "dm_M0_prob_host": (D, [UINT, VP, ITYPE, VP, UINT]),
     "dm_marginal_prob_host": (D, [PU, PU, UINT, VP, ITYPE, VP, UINT]),
     "dm_expectation_value_multi_qubit_Pauli_operator_partial_list_host": (D, [PU, PU, UINT, VP, ITYPE, VP, UINT]),
+    "qm_dm_observable_expectation_host": (QmComplex, [PI, PI, PU, PC, UINT, VP, ITYPE, VP, UINT]),
     "dm_normalize_host": (None, [D, VP, ITYPE, VP, UINT]),
     "dm_sampling_host": (None, [PD, UINT, PI, VP, ITYPE, VP, UINT]),
     "qm_sampling_cdf_host": (None, [PD, VP, ITYPE, VP, UINT]),

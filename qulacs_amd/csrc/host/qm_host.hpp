@@ -698,11 +698,14 @@ class QuantumCircuit {
         size_t begin = 0, end = 0;  // gates [begin, end)
         qm_circuit* program = nullptr;  // null: run the gates one by one
     };
+    // The same for a density matrix, with programs over its 2 n bits: the runs also take
+    // channels on one or two qubits.
     void release_plan();
     void build_plan();
-    void update_dm_fused(DensityMatrixMI355* d);
-    std::vector<FusedRun> plan_;
-    uint64_t version_ = 0, plan_version_ = ~0ULL;
+    void build_dm_plan();
+    void update_dm_gates(DensityMatrixMI355* d, size_t begin, size_t end);
+    std::vector<FusedRun> plan_, dm_plan_;
+    uint64_t version_ = 0, plan_version_ = ~0ULL, dm_plan_version_ = ~0ULL;
     std::mutex plan_mutex_;  // one fused update at a time per circuit (the plan uploads lazily per device)
 };
 

@@ -741,17 +741,19 @@ qm_circuit* qm_circuit_create(UINT n, const qm_batch_gate* gates, UINT gate_coun
     }
     auto* c = new qm_circuit();
     HCirc hc;
-    if (!convert_gates(n, gates, gate_count, hc, what)) {
+    if (!convert_gates(n, gates, gate_count, hc, what, true)) {
         delete c;
         return nullptr;
     }
+    // blocks that hold the widest gate; depolarizing takes 4 (row and column bits of two qubits)
+    auto needs = [](const HOp& o) { return o.type == 4 ? size_t(4) : o.type == 0 ? o.q.size() : size_t(0); };
     if (!block_qubits)  // the default width widens to the largest dense gate (at most 4 qubits)
         for (const HOp& o : hc.ops)
-            if (o.type == 0 && o.q.size() > K && o.q.size() <= 4) K = (u32)o.q.size();
+            if (needs(o) > K && needs(o) <= 4) K = (u32)needs(o);
     for (const HOp& o : hc.ops)
-        if (o.type == 0 && o.q.size() > K) {
+        if (needs(o) > K) {
             set_error(QM_ERR_INVALID_ARGUMENT, "%s: a %zu-qubit dense gate needs block_qubits >= %zu", what, o.q.size(),
-                      o.q.size());
+                      needs(o));
             delete c;
             return nullptr;
         }

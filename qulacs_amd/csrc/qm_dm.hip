@@ -77,6 +77,57 @@ __global__ __launch_bounds__(256) void k_dm_pauli(const double2* __restrict__ r,
     if (threadIdx.x == 0) partials[blockIdx.x] = acc;
 }
 
+// sum_k c_k Tr(P_k rho): every term is one entry per row.  Threads take (term, row) pairs, so that a
+// small matrix with many terms still fills its waves; one block writes the result itself.
+// Latency bounds it (a call per term waited for each).
+struct DmTerm {
+    u64 bf, pf;
+    u32 rot, pad;
+    double cre, cim;
+};
+constexpr u32 kDmInlineTerms = 64;
+constexpr u32 kDmUploadTerms = 4096;  // per launch
+struct DmTerms {
+    const DmTerm* more;  // more terms than the array holds
+    DmTerm t[kDmInlineTerms];
+};
+template <bool INLINE>
+__global__ __launch_bounds__(256) void k_dm_observable(const double2* __restrict__ r, u64 dim, u32 bits, u32 nterms,
+                                                       DmTerms terms, double* __restrict__ out) {
+    __shared__ double lds[32];
+    double re = 0.0, im = 0.0;
+    const u64 total = dim * nterms, stride = (u64)gridDim.x * blockDim.x;
+    for (u64 e = (u64)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += stride) {
+        const u64 i = e & (dim - 1);
+        const DmTerm tm = INLINE ? terms.t[e >> bits] : terms.more[e >> bits];
+        const double2 v = r[i * dim + (i ^ tm.bf)];
+        double x = (tm.rot & 1u) ? v.y : v.x;  // the sign of i^rot is in the coefficient
+        if (__popcll(i & tm.pf) & 1) x = -x;
+        re = fma(tm.cre, x, re);
+        im = fma(tm.cim, x, im);
+    }
+    re = block_sum(re, lds);
+    im = block_sum(im, lds);
+    if (threadIdx.x == 0) {
+        out[2 * blockIdx.x] = re;
+        out[2 * blockIdx.x + 1] = im;
+    }
+}
+__global__ __launch_bounds__(256) void k_dm_sum_pairs(const double* __restrict__ p, u32 n, double* __restrict__ out) {
+    __shared__ double lds[32];
+    double re = 0.0, im = 0.0;
+    for (u32 k = threadIdx.x; k < n; k += blockDim.x) {
+        re += p[2 * k];
+        im += p[2 * k + 1];
+    }
+    re = block_sum(re, lds);
+    im = block_sum(im, lds);
+    if (threadIdx.x == 0) {
+        out[0] = re;
+        out[1] = im;
+    }
+}
+
 __global__ __launch_bounds__(256) void k_sum_partials(const double* __restrict__ p, unsigned n, double* __restrict__ out) {
     __shared__ double lds[32];
     double acc = 0.0;
@@ -85,11 +136,11 @@ __global__ __launch_bounds__(256) void k_sum_partials(const double* __restrict__
     if (threadIdx.x == 0) out[0] = acc;
 }
 
+// Where the nb blocks of a reduction leave their sums: one block writes the result.
+static double* partials_of(Scratch* sc, unsigned nb) { return nb == 1 ? sc->host_result : sc->partials; }
 static double finish_scalar(Scratch* sc, unsigned nb, hipStream_t st, const char* what) {
-    double* dout = sc->partials + nb;
-    k_sum_partials<<<1, 256, 0, st>>>(sc->partials, nb, dout);
-    if (!hip_ok(hipMemcpyAsync(sc->host_result, dout, sizeof(double), hipMemcpyDeviceToHost, st), what)) return 0.0;
-    if (!hip_ok(hipStreamSynchronize(st), what)) return 0.0;
+    if (nb > 1) k_sum_partials<<<1, 256, 0, st>>>(sc->partials, nb, sc->host_result);  // pinned: no copy command
+    if (!hip_ok(hipGetLastError(), what) || !hip_ok(hipStreamSynchronize(st), what)) return 0.0;
     return sc->host_result[0];
 }
 
@@ -102,9 +153,9 @@ static double dm_diag_sum(bool ent, u64 mask, u64 value, void* state, u64 dim, v
     if (!sc) return 0.0;
     const unsigned nb = grid_for(dim, 256 * 4, 1024);
     if (ent)
-        k_dm_diag<true><<<nb, 256, 0, st>>>((const double2*)state, dim, mask, value, sc->partials);
+        k_dm_diag<true><<<nb, 256, 0, st>>>((const double2*)state, dim, mask, value, partials_of(sc, nb));
     else
-        k_dm_diag<false><<<nb, 256, 0, st>>>((const double2*)state, dim, mask, value, sc->partials);
+        k_dm_diag<false><<<nb, 256, 0, st>>>((const double2*)state, dim, mask, value, partials_of(sc, nb));
     return finish_scalar(sc, nb, st, what);
 }
 
@@ -490,8 +541,54 @@ double dm_expectation_value_multi_qubit_Pauli_operator_partial_list_host(const U
     Scratch* sc = scratch_for(st);
     if (!sc) return 0.0;
     const unsigned nb = grid_for(dim, 256 * 4, 1024);
-    k_dm_pauli<<<nb, 256, 0, st>>>((const double2*)state, dim, bf, pf, rot, sc->partials);
+    k_dm_pauli<<<nb, 256, 0, st>>>((const double2*)state, dim, bf, pf, rot, partials_of(sc, nb));
     return finish_scalar(sc, nb, st, what);
+}
+
+qm_complex qm_dm_observable_expectation_host(const ITYPE* bfs, const ITYPE* pfs, const UINT* rots,
+                                             const qm_complex* coefs, UINT nterms, void* state, ITYPE dim, void* stream,
+                                             unsigned dev) {
+    const char* what = "qm_dm_observable_expectation_host";
+    qm_complex z{0, 0};
+    int n;
+    if (!dm_ok(state, dim, &n, what) || nterms == 0) return z;
+    if (!bfs || !pfs || !rots || !coefs) {
+        set_error(QM_ERR_INVALID_ARGUMENT, "%s: null term arrays", what);
+        return z;
+    }
+    std::vector<DmTerm> ht(nterms);
+    for (UINT k = 0; k < nterms; ++k) {
+        if (((bfs[k] | pfs[k]) >> n) != 0) {
+            set_error(QM_ERR_INVALID_ARGUMENT, "%s: term %u acts beyond %d qubits", what, k, n);
+            return z;
+        }
+        // Re(v i^rot): v.x, -v.y, -v.x, v.y
+        const double f = (rots[k] & 3u) == 1 || (rots[k] & 3u) == 2 ? -1.0 : 1.0;
+        ht[k] = DmTerm{bfs[k], pfs[k], rots[k], 0, f * coefs[k].re, f * coefs[k].im};
+    }
+    if (!use_device(dev)) return z;
+    hipStream_t st = stream_of(stream);
+    Scratch* sc = scratch_for(st);
+    if (!sc) return z;
+    const auto* rho = (const double2*)state;
+    for (UINT first = 0; first < nterms; first += kDmUploadTerms) {  // one launch up to kDmUploadTerms terms
+        const UINT m = std::min(nterms - first, kDmUploadTerms);
+        DmTerms terms{};
+        if (m <= kDmInlineTerms) {
+            std::copy(ht.begin() + first, ht.begin() + first + m, terms.t);
+        } else {
+            terms.more = (const DmTerm*)upload(sc, ht.data() + first, m * sizeof(DmTerm));
+            if (!terms.more) return qm_complex{0, 0};
+        }
+        const unsigned nb = dim * m <= 1024 ? 1u : grid_for(dim * m, 256, 1024);
+        if (m <= kDmInlineTerms) k_dm_observable<true><<<nb, 256, 0, st>>>(rho, dim, n, m, terms, partials_of(sc, nb));
+        else k_dm_observable<false><<<nb, 256, 0, st>>>(rho, dim, n, m, terms, partials_of(sc, nb));
+        if (nb > 1) k_dm_sum_pairs<<<1, 256, 0, st>>>(sc->partials, nb, sc->host_result);
+        if (!hip_ok(hipGetLastError(), what) || !hip_ok(hipStreamSynchronize(st), what)) return qm_complex{0, 0};
+        z.re += sc->host_result[0];
+        z.im += sc->host_result[1];
+    }
+    return z;
 }
 
 void dm_normalize_host(double squared_norm, void* state, ITYPE dim, void* stream, unsigned dev) {

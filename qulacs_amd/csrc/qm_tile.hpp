@@ -41,7 +41,10 @@ constexpr u32 kMinQubits = 4;   // smaller circuits run on 4 qubits (extra qubit
 // ZROT: amplitudes with even parity of the index bits of a mask times c + i s, the others
 // times c - i s; a = mask of local positions outside the block | block-bit mask << 16, x[0]:
 // mask of tile bits, data: c + i s.
-enum : u32 { SUB_LAYER = 0, SUB_D2 = 1, SUB_DK = 2, SUB_DIAG = 3, SUB_ZROT = 4 };
+// DEPOL (density matrices, column bits c and row bits r of m qubits): entries whose row and
+// column bits differ times s; those where they agree times s plus t times their sum; a = block bits
+// c0, r0, c1, r1 in bytes, m: qubits (1 or 2), data: s + i t.
+enum : u32 { SUB_LAYER = 0, SUB_D2 = 1, SUB_DK = 2, SUB_DIAG = 3, SUB_ZROT = 4, SUB_DEPOL = 5 };
 // bits 16 i .. 16 i + 15: the register-block indices j (< 16) with bit i set
 constexpr u64 kBlockPatterns = 0xFF00F0F0CCCCAAAAull;
 constexpr u32 kCzPairsMax = 4;
@@ -88,8 +91,10 @@ struct DTerm {
 };
 
 struct HOp {
-    // 0 dense, 1 diag, 2 cz, 3 exp(i phi Z...Z) on q with m[0] = exp(i phi)
+    // 0 dense, 1 diag, 2 cz, 3 exp(i phi Z...Z) on q with m[0] = exp(i phi),
+    // 4 depol on q = c0, r0 (, c1, r1) with m[0] = s + i t
     u32 type;
+    bool dense() const { return type == 0 || type == 4; }  // mixes amplitudes: needs its qubits in a block
     std::vector<u32> q;
     std::vector<cd> m;
     bool reduced = false;  // single-qubit dense: m = {a, b, 0, 0} for [[1, 0], [b, 1]] [[1, a], [0, 1]]
@@ -107,6 +112,9 @@ struct HCirc {
     u32 ne = 0; // as run (>= kMinQubits)
     std::vector<HOp> ops;
     std::vector<DTerm> terms;
+    // operations join qubit t with t + ne / 2 (a density matrix): windows of such pairs are
+    // candidates too
+    bool paired = false;
 };
 
 
@@ -313,6 +321,57 @@ __device__ __forceinline__ void sub_d2(double2* v, const double2* mp) {
     }
 }
 
+// DEPOL on block bits (C0, R0), and (C1, R1) unless C1 < 0: 2.5 operations per component for two
+// qubits, where the 16 x 16 superoperator takes 64.
+template <int K, int C0, int R0, int C1, int R1>
+__device__ __forceinline__ void depol_block(double2 (&v)[1 << K], const double s, const double t) {
+    auto bit = [](int j, int b) { return (j >> b) & 1; };
+#pragma unroll
+    for (int j = 0; j < (1 << K); ++j) {
+        // j: the member of its set of agreeing entries with all column bits 0
+        if (bit(j, C0) || bit(j, R0)) continue;
+        if (C1 >= 0 && (bit(j, C1 < 0 ? 0 : C1) || bit(j, R1 < 0 ? 0 : R1))) continue;
+        const int d0 = (1 << C0) | (1 << R0), d1 = C1 >= 0 ? (1 << (C1 < 0 ? 0 : C1)) | (1 << (R1 < 0 ? 0 : R1)) : 0;
+        double2 sum = cadd(v[j], v[j | d0]);
+        if (C1 >= 0) sum = cadd(sum, cadd(v[j | d1], v[j | d0 | d1]));
+        const double2 add = cscale(sum, t);
+#pragma unroll
+        for (int i = 0; i < (1 << K); ++i) {
+            // the entries of j's group: all settings of the operation's bits
+            if ((i & ~(d0 | d1)) != (j & ~(d0 | d1))) continue;
+            const bool agree = bit(i, C0) == bit(i, R0) && (C1 < 0 || bit(i, C1 < 0 ? 0 : C1) == bit(i, R1 < 0 ? 0 : R1));
+            v[i] = agree ? make_double2(fma(v[i].x, s, add.x), fma(v[i].y, s, add.y)) : cscale(v[i], s);
+        }
+    }
+}
+#define QM_DEPOL1_CASE(A, B)                 \
+    case (A) * 4 + (B):                      \
+        depol_block<4, A, B, -1, -1>(v, s, t); \
+        break;
+#define QM_DEPOL2_CASE(A, B, C, D)         \
+    case (A) * 4 + (B):                    \
+        depol_block<4, A, B, C, D>(v, s, t); \
+        break;
+__device__ __forceinline__ void apply_depol(double2 (&v)[16], u32 a, u32 m, const double s, const double t) {
+    // the pair (c, r) is symmetric, and with two qubits the second pair is what is left of the block
+    const u32 c = byte_at(a, 0), r = byte_at(a, 1), lo = min(c, r), hi = max(c, r);
+    if (m == 1) {
+        switch (lo * 4 + hi) {
+            QM_DEPOL1_CASE(0, 1) QM_DEPOL1_CASE(0, 2) QM_DEPOL1_CASE(0, 3) QM_DEPOL1_CASE(1, 2) QM_DEPOL1_CASE(1, 3)
+            QM_DEPOL1_CASE(2, 3)
+            default: break;
+        }
+    } else {
+        switch (lo * 4 + hi) {
+            QM_DEPOL2_CASE(0, 1, 2, 3) QM_DEPOL2_CASE(0, 2, 1, 3) QM_DEPOL2_CASE(0, 3, 1, 2) QM_DEPOL2_CASE(1, 2, 0, 3)
+            QM_DEPOL2_CASE(1, 3, 0, 2) QM_DEPOL2_CASE(2, 3, 0, 1)
+            default: break;
+        }
+    }
+}
+#undef QM_DEPOL1_CASE
+#undef QM_DEPOL2_CASE
+
 template <int K>
 __device__ __forceinline__ void sub_dk(double2* v, const double2* mp) {
     constexpr int D = 1 << K;
@@ -515,6 +574,15 @@ __device__ __forceinline__ void pass_groups(double2* st, const DPass& ps, const 
         if (k == ps.nsub) break;
         const u32 kind = sub.type & 15u;
         const double2* mp = pool + sub.data;
+        if constexpr (WIDE && K == 4) {
+            if (kind == SUB_DEPOL) {
+                const double2 f = mp[0];
+#pragma unroll
+                for (int g = 0; g < G; ++g) apply_depol(v[g], sub.a, sub.m, f.x, f.y);
+                ++k;
+                continue;
+            }
+        }
         if (kind == SUB_D2) {
 #pragma unroll
             for (int g = 0; g < G; ++g) apply_d2<K>(v[g], byte_at(sub.a, 0), byte_at(sub.a, 1), mp);
@@ -656,7 +724,7 @@ struct Picker {
     std::vector<Item> items;
     std::vector<u32> rest;  // what is left, in order
 
-    static u32 weight_of(const HOp& o) { return o.type == 0 ? 1u << (o.q.size() - 1) : 0u; }
+    static u32 weight_of(const HOp& o) { return o.type == 0 ? 1u << (o.q.size() - 1) : o.type == 4 ? 1u : 0u; }
     void add(const HOp& o) {
         rest.push_back((u32)items.size());
         items.push_back({o.mask(), weight_of(o), o.grad});
@@ -693,13 +761,28 @@ struct Picker {
     }
     // Picks a window of at most `most` positions out of [0, n) that contains `fixed`, and
     // what it takes; the window is filled up to min(n, most) positions.
-    u64 pick(u32 n, u64 fixed, u32 low, u32 most, size_t max_grads, std::vector<u32>& sel) {
+    // `paired`: also windows of qubits s, s + 1, ... of [0, n / 2) with their partners n / 2 above.
+    u64 pick(u32 n, u64 fixed, u32 low, u32 most, size_t max_grads, std::vector<u32>& sel, bool paired = false) {
         u64 best = fixed;
         u64 work = scan(best, true, most, max_grads, nullptr);
         const u32 f = most - low;
         bool grow = true;
         for (u32 s = low; s + f <= n; ++s) {
             u64 w = fixed | (((1ULL << f) - 1) << s);
+            const u64 c = scan(w, false, most, max_grads, nullptr);
+            if (c > work) {
+                work = c;
+                best = w;
+                grow = false;
+            }
+        }
+        for (u32 s = 0; paired && s < n / 2; ++s) {
+            u64 w = fixed;
+            for (u32 q = s; q < n / 2; ++q) {
+                const u64 m = w | (1ULL << q) | (1ULL << (q + n / 2));
+                if ((u32)__builtin_popcountll(m) > most) break;
+                w = m;
+            }
             const u64 c = scan(w, false, most, max_grads, nullptr);
             if (c > work) {
                 work = c;
@@ -737,12 +820,12 @@ void schedule_passes(Flat& f, const std::vector<HOp>& ops, u32 lq, u32 K, DStage
     size_t dense_left = 0;
     for (const HOp& o : ops) {
         pk.add(o);
-        dense_left += o.type == 0;
+        dense_left += o.dense();
     }
     std::vector<u32> sel;
     while (!pk.rest.empty()) {
         const u64 block = pk.pick(lq, 0, 0, K, ~size_t(0), sel);
-        for (u32 i : sel) dense_left -= ops[i].type == 0;
+        for (u32 i : sel) dense_left -= ops[i].dense();
         if (dense_left == 0) sel = pk.rest;  // the last pass takes every diagonal operation that is left
         pk.take(sel);
         DPass ps{};
@@ -774,11 +857,11 @@ void schedule_passes(Flat& f, const std::vector<HOp>& ops, u32 lq, u32 K, DStage
                     if (q >= kTileQubit || !((block >> q) & 1)) continue;
                     const u32 b = bit_of(q);
                     lv = std::max(lv, dense_at[b] + 1);
-                    if (o.type == 0) lv = std::max(lv, diag_at[b]);
+                    if (o.dense()) lv = std::max(lv, diag_at[b]);
                 }
                 for (u32 q : o.q) {
                     if (q >= kTileQubit || !((block >> q) & 1)) continue;
-                    u32& at = (o.type == 0 ? dense_at : diag_at)[bit_of(q)];
+                    u32& at = (o.dense() ? dense_at : diag_at)[bit_of(q)];
                     at = std::max(at, lv);
                 }
                 if (levels.size() < lv) levels.resize(lv);
@@ -884,9 +967,14 @@ void schedule_passes(Flat& f, const std::vector<HOp>& ops, u32 lq, u32 K, DStage
             flush();
             for (u32 i : level) {
                 const HOp& o = ops[i];
-                if (o.type != 0 || o.q.size() == 1) continue;
+                if (!o.dense() || o.q.size() == 1) continue;
                 DSub sb{};
-                if (o.q.size() == 2) {
+                if (o.type == 4) {
+                    sb.type = SUB_DEPOL;
+                    sb.m = (u32)o.q.size() / 2;
+                    for (size_t k = 0; k < o.q.size(); ++k) sb.a |= bit_of(o.q[k]) << (8 * k);
+                    sb.data = pool_put(f, o.m);
+                } else if (o.q.size() == 2) {
                     sb.type = SUB_D2;
                     sb.a = bit_of(o.q[0]) | (bit_of(o.q[1]) << 8);
                     sb.data = pool_put(f, o.m);
@@ -960,7 +1048,7 @@ u32 schedule_circuit(Flat& f, const HCirc& c, u32 K, u32 lq_cap = kMaxLocal, siz
     u32 count = 0;
     std::vector<u32> sel;
     do {  // a circuit without gates still needs one stage to initialise |0>
-        const u64 win = pk.pick(n, low, kLowFixed, lq, max_grads, sel);
+        const u64 win = pk.pick(n, low, kLowFixed, lq, max_grads, sel, c.paired);
         pk.take(sel);
         DStage sg{};
         u32 local_of[64];
@@ -1018,7 +1106,7 @@ struct Converter {
         const long i = (long)c.ops.size() - 1;
         for (u32 q : c.ops.back().q) {
             last[q] = i;
-            if (c.ops.back().type == 0) last_dense[q] = i;
+            if (c.ops.back().dense()) last_dense[q] = i;
         }
     }
     void phase(u32 q, cd d0, cd d1) {
@@ -1036,9 +1124,9 @@ struct Converter {
             ph = Phase{};
         }
         const long p = last[q[0]];
-        if (q.size() == 1 && p >= 0 && c.ops[p].type == 0 && c.ops[p].q.size() == 1) {
+        if (p >= 0 && c.ops[p].type == 0 && c.ops[p].q == q && last[q.back()] == p && q.size() <= 2) {
             std::vector<cd> prod;
-            mat_mul(m, c.ops[p].m, prod, 2);  // new after old
+            mat_mul(m, c.ops[p].m, prod, (int)d);  // new after old
             c.ops[p].m = prod;
             return;
         }
@@ -1107,13 +1195,24 @@ struct Converter {
         o.m = m;
         push(std::move(o));
     }
+    void depol(const std::vector<u32>& q, cd st) {
+        for (u32 x : q) flush(x);
+        HOp o;
+        o.type = 4;
+        o.q = q;
+        o.m = {st};
+        push(std::move(o));
+    }
     // What is left in pend: into the last dense operation on the qubit (only diagonal ones
     // follow it), else a diagonal operation of its own.
     void finish() {
-        for (u32 q = 0; q < c.ne; ++q) {
+        for (u32 q = 0; q < c.ne; ++q) flush(q);
+    }
+    void flush(u32 q) {
+        {
             Phase& ph = pend[q];
-            if (!ph.any) continue;
-            if (last_dense[q] >= 0) {
+            if (!ph.any) return;
+            if (last_dense[q] >= 0 && c.ops[last_dense[q]].type == 0) {
                 HOp& o = c.ops[last_dense[q]];
                 const u32 d = 1u << o.q.size(), t = (u32)(std::find(o.q.begin(), o.q.end(), q) - o.q.begin());
                 for (u32 r = 0; r < d; ++r)
@@ -1141,10 +1240,16 @@ struct Converter {
 // applied.  A matrix is left whole when |u00| < 1/2, when that factor would exceed 2^200 in
 // all, and when it is not unitary (or a multiple of a unitary).
 void reduce_matrices(std::vector<HOp>& ops, u32 n) {
-    std::vector<long> last_dense(n, -1);
-    for (size_t i = 0; i < ops.size(); ++i)
-        if (ops[i].type == 0)
-            for (u32 q : ops[i].q) last_dense[q] = (long)i;
+    // the next operation that mixes amplitudes on the qubit has a matrix to take the diagonal
+    std::vector<bool> absorbed(ops.size(), false);
+    {
+        std::vector<bool> next(n, false);
+        for (size_t i = ops.size(); i-- > 0;) {
+            if (!ops[i].dense()) continue;
+            absorbed[i] = ops[i].q.size() == 1 && next[ops[i].q[0]];
+            for (u32 q : ops[i].q) next[q] = ops[i].type == 0;
+        }
+    }
     struct Left {
         cd d[2] = {1.0, 1.0};
         bool any = false;
@@ -1156,7 +1261,7 @@ void reduce_matrices(std::vector<HOp>& ops, u32 n) {
         HOp& o = ops[i];
         if (o.type != 0) continue;
         bool shear = false;
-        if (o.q.size() == 1 && (long)i != last_dense[o.q[0]]) {
+        if (absorbed[i]) {
             const double c0 = std::norm(o.m[0]) + std::norm(o.m[2]), c1 = std::norm(o.m[1]) + std::norm(o.m[3]);
             const cd dot = std::conj(o.m[0]) * o.m[1] + std::conj(o.m[2]) * o.m[3];
             shear = c0 > 1e-6 && c0 < 1e6 && std::abs(c1 - c0) < 1e-12 * c0 && std::abs(dot) < 1e-12 * c0 &&
@@ -1186,7 +1291,10 @@ void reduce_matrices(std::vector<HOp>& ops, u32 n) {
     }
 }
 
-bool convert_gates(u32 n, const qm_batch_gate* gates, UINT gate_count, HCirc& c, const char* what) {
+// `density`: QM_BATCH_DEPOL is taken, and dense operations on t and t + n / 2 mark the circuit as
+// paired.
+bool convert_gates(u32 n, const qm_batch_gate* gates, UINT gate_count, HCirc& c, const char* what,
+                   bool density = false) {
     c.n = n;
     c.ne = std::max<u32>(n, kMinQubits);
     Converter cv(c);
@@ -1194,7 +1302,8 @@ bool convert_gates(u32 n, const qm_batch_gate* gates, UINT gate_count, HCirc& c,
         const qm_batch_gate& g = gates[gi];
         const u32 k = g.qubit_count;
         const bool two = g.kind == QM_BATCH_CZ || g.kind == QM_BATCH_CNOT;
-        if (g.kind > QM_BATCH_CNOT || k < 1 || k > 4 || (two && k != 2)) {
+        const bool depol = g.kind == QM_BATCH_DEPOL && density;
+        if ((g.kind > QM_BATCH_CNOT && !depol) || k < 1 || k > 4 || (two && k != 2) || (depol && k != 2 && k != 4)) {
             set_error(QM_ERR_INVALID_ARGUMENT, "%s: gate %u: kind %u with %u qubits is not supported", what, gi, g.kind, k);
             return false;
         }
@@ -1206,7 +1315,7 @@ bool convert_gates(u32 n, const qm_batch_gate* gates, UINT gate_count, HCirc& c,
             }
             mask |= 1ULL << g.qubits[i];
         }
-        if ((g.kind == QM_BATCH_DENSE || g.kind == QM_BATCH_DIAG) && !g.matrix) {
+        if ((g.kind == QM_BATCH_DENSE || g.kind == QM_BATCH_DIAG || depol) && !g.matrix) {
             set_error(QM_ERR_INVALID_ARGUMENT, "%s: gate %u: null matrix", what, gi);
             return false;
         }
@@ -1220,11 +1329,15 @@ bool convert_gates(u32 n, const qm_batch_gate* gates, UINT gate_count, HCirc& c,
             if (g.kind == QM_BATCH_CNOT) cv.dense({q[1]}, {1.0, 1.0, 1.0, -1.0});
             cv.push(std::move(cz));
             if (g.kind == QM_BATCH_CNOT) cv.dense({q[1]}, {0.5, 0.5, 0.5, -0.5});
+        } else if (depol) {
+            cv.depol(q, cd(g.matrix[0].re, g.matrix[0].im));
+            c.paired = true;
         } else if (g.kind == QM_BATCH_DIAG) {
             for (u32 i = 0; i < d; ++i) m.push_back(cd(g.matrix[i].re, g.matrix[i].im));
             cv.diagonal(q, m);
         } else {
             for (u32 i = 0; i < d * d; ++i) m.push_back(cd(g.matrix[i].re, g.matrix[i].im));
+            if (density && k == 2 && q[1] == q[0] + n / 2) c.paired = true;
             cv.dense(q, std::move(m));
         }
     }
