@@ -659,7 +659,7 @@ void qm_adjoint::build(const Builder& b) {
     std::reverse(hc.ops.begin(), hc.ops.end());
     for (HOp& o : hc.ops)
         if (o.type == 0 && o.q.size() == 2) {  // 4 x 4: conjugate transpose
-            const std::vector<cd> m = o.m;
+            const std::vector<cx> m = o.m;
             for (int r = 0; r < 4; ++r)
                 for (int c = 0; c < 4; ++c) o.m[r * 4 + c] = std::conj(m[c * 4 + r]);
         }

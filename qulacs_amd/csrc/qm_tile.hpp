@@ -17,6 +17,13 @@ namespace qm {
 namespace {
 
 using cd = std::complex<double>;
+// Host-side products of gate matrices are formed with 64 mantissa bits, so that a merged or
+// factored matrix carries little more than the rounding of its final entries.
+using cx = std::complex<long double>;
+inline cx mul(const cx& a, const cx& b) {  // without the C library's checks for infinities
+    return cx(a.real() * b.real() - a.imag() * b.imag(), a.real() * b.imag() + a.imag() * b.real());
+}
+inline cx quot(const cx& a, const cx& b) { return mul(a, std::conj(b)) / std::norm(b); }
 
 constexpr u32 kMaxLocal = 13;   // qubits resident in LDS
 constexpr u32 kLowFixed = 3;    // qubits 0..2 are local in every stage: a tile is made of 128-byte runs
@@ -96,7 +103,7 @@ struct HOp {
     u32 type;
     bool dense() const { return type == 0 || type == 4; }  // mixes amplitudes: needs its qubits in a block
     std::vector<u32> q;
-    std::vector<cd> m;
+    std::vector<cx> m;
     bool reduced = false;  // single-qubit dense: m = {a, b, 0, 0} for [[1, 0], [b, 1]] [[1, a], [0, 1]]
     long id = -1;       // the caller's number of a single-qubit dense operation (see Flat::mats)
     bool grad = false;  // listed in Flat::grads
@@ -681,11 +688,11 @@ __device__ __forceinline__ void run_passes(double2* st, u32 lq, const DPass* __r
 }
 
 // ------------------------------------------------------------------ host side
-void mat_mul(const std::vector<cd>& a, const std::vector<cd>& b, std::vector<cd>& out, int d) {
+void mat_mul(const std::vector<cx>& a, const std::vector<cx>& b, std::vector<cx>& out, int d) {
     out.assign((size_t)d * d, 0.0);
     for (int i = 0; i < d; ++i)
         for (int k = 0; k < d; ++k)
-            for (int j = 0; j < d; ++j) out[i * d + j] += a[i * d + k] * b[k * d + j];
+            for (int j = 0; j < d; ++j) out[i * d + j] += mul(a[i * d + k], b[k * d + j]);
 }
 
 // Schedules one circuit; appends to the flat arrays.
@@ -700,9 +707,9 @@ struct Flat {
     std::vector<long> grads;
 };
 
-u32 pool_put(Flat& f, const std::vector<cd>& m) {
+u32 pool_put(Flat& f, const std::vector<cx>& m) {
     const u32 off = (u32)f.pool.size();
-    for (const cd& z : m) f.pool.push_back(make_double2(z.real(), z.imag()));
+    for (const cx& z : m) f.pool.push_back(make_double2((double)z.real(), (double)z.imag()));
     return off;
 }
 
@@ -987,7 +994,7 @@ void schedule_passes(Flat& f, const std::vector<HOp>& ops, u32 lq, u32 K, DStage
                         bits[t] = bit_of(o.q[t]);
                         omask |= 1u << bits[t];
                     }
-                    std::vector<cd> M((size_t)D * D, 0.0);
+                    std::vector<cx> M((size_t)D * D, 0.0);
                     for (u32 col = 0; col < D; ++col) {
                         u32 x = 0;
                         for (u32 t = 0; t < k; ++t) x |= ((col >> bits[t]) & 1u) << t;
@@ -1094,7 +1101,7 @@ struct Converter {
     std::vector<long> last;        // last operation that touches each qubit
     std::vector<long> last_dense;  // last dense one
     struct Phase {
-        cd d[2] = {1.0, 1.0};
+        cx d[2] = {1.0, 1.0};
         bool any = false;
     };
     std::vector<Phase> pend;
@@ -1109,23 +1116,23 @@ struct Converter {
             if (c.ops.back().dense()) last_dense[q] = i;
         }
     }
-    void phase(u32 q, cd d0, cd d1) {
-        pend[q].d[0] *= d0;
-        pend[q].d[1] *= d1;
+    void phase(u32 q, cx d0, cx d1) {
+        pend[q].d[0] = mul(pend[q].d[0], d0);
+        pend[q].d[1] = mul(pend[q].d[1], d1);
         pend[q].any = true;
     }
-    void dense(const std::vector<u32>& q, std::vector<cd> m) {
+    void dense(const std::vector<u32>& q, std::vector<cx> m) {
         const u32 d = 1u << q.size();
         for (u32 t = 0; t < q.size(); ++t) {
             Phase& ph = pend[q[t]];
             if (!ph.any) continue;
             for (u32 r = 0; r < d; ++r)
-                for (u32 col = 0; col < d; ++col) m[r * d + col] *= ph.d[(col >> t) & 1u];
+                for (u32 col = 0; col < d; ++col) m[r * d + col] = mul(m[r * d + col], ph.d[(col >> t) & 1u]);
             ph = Phase{};
         }
         const long p = last[q[0]];
         if (p >= 0 && c.ops[p].type == 0 && c.ops[p].q == q && last[q.back()] == p && q.size() <= 2) {
-            std::vector<cd> prod;
+            std::vector<cx> prod;
             mat_mul(m, c.ops[p].m, prod, (int)d);  // new after old
             c.ops[p].m = prod;
             return;
@@ -1136,7 +1143,7 @@ struct Converter {
         o.m = std::move(m);
         push(std::move(o));
     }
-    void zrot(const std::vector<u32>& q, cd z) {
+    void zrot(const std::vector<u32>& q, cx z) {
         if (q.size() == 1) {
             phase(q[0], z, std::conj(z));
             return;
@@ -1147,7 +1154,7 @@ struct Converter {
         o.m = {z};
         push(std::move(o));
     }
-    void diagonal(const std::vector<u32>& q, const std::vector<cd>& m) {
+    void diagonal(const std::vector<u32>& q, const std::vector<cx>& m) {
         const u32 k = (u32)q.size(), d = 1u << k;
         if (k == 1) {
             phase(q[0], m[0], m[1]);
@@ -1170,22 +1177,22 @@ struct Converter {
         bool unit = true;
         for (u32 i = 0; i < d && unit; ++i) unit = std::abs(std::abs(m[i]) - 1.0) < 1e-14;
         if (unit) {
-            double phi[16];
+            long double phi[16];
             for (u32 i = 0; i < d; ++i) phi[i] = std::arg(m[i]);
             for (u32 h = 1; h < d; h <<= 1)  // phi[s] <- sum_i (-1)^popcount(i & s) arg m_i
                 for (u32 i = 0; i < d; ++i)
                     if (!(i & h)) {
-                        const double a = phi[i], b = phi[i | h];
+                        const long double a = phi[i], b = phi[i | h];
                         phi[i] = a + b;
                         phi[i | h] = a - b;
                     }
             u32 many = 0;
             for (u32 s = 1; s < d; ++s) many += (s & (s - 1)) && std::abs(phi[s]) > 1e-15;
             if (many <= 2) {
-                const cd g = std::polar(1.0, phi[0] / d);
+                const cx g = std::polar(1.0L, phi[0] / d);
                 phase(q[0], g, g);
                 for (u32 s = 1; s < d; ++s)
-                    if (std::abs(phi[s]) > 1e-15) zrot(subset(s), std::polar(1.0, phi[s] / d));
+                    if (std::abs(phi[s]) > 1e-15) zrot(subset(s), std::polar(1.0L, phi[s] / d));
                 return;
             }
         }
@@ -1195,7 +1202,7 @@ struct Converter {
         o.m = m;
         push(std::move(o));
     }
-    void depol(const std::vector<u32>& q, cd st) {
+    void depol(const std::vector<u32>& q, cx st) {
         for (u32 x : q) flush(x);
         HOp o;
         o.type = 4;
@@ -1216,8 +1223,8 @@ struct Converter {
                 HOp& o = c.ops[last_dense[q]];
                 const u32 d = 1u << o.q.size(), t = (u32)(std::find(o.q.begin(), o.q.end(), q) - o.q.begin());
                 for (u32 r = 0; r < d; ++r)
-                    for (u32 col = 0; col < d; ++col) o.m[r * d + col] *= ph.d[(r >> t) & 1u];
-            } else if (ph.d[0] != 1.0 || ph.d[1] != 1.0) {
+                    for (u32 col = 0; col < d; ++col) o.m[r * d + col] = mul(o.m[r * d + col], ph.d[(r >> t) & 1u]);
+            } else if (ph.d[0] != cx(1.0) || ph.d[1] != cx(1.0)) {
                 HOp o;
                 o.type = 1;
                 o.q = {q};
@@ -1251,7 +1258,7 @@ void reduce_matrices(std::vector<HOp>& ops, u32 n) {
         }
     }
     struct Left {
-        cd d[2] = {1.0, 1.0};
+        cx d[2] = {1.0, 1.0};
         bool any = false;
         double bits = 0.0;  // |log2| of the larger factor that waits in d
     };
@@ -1263,7 +1270,7 @@ void reduce_matrices(std::vector<HOp>& ops, u32 n) {
         bool shear = false;
         if (absorbed[i]) {
             const double c0 = std::norm(o.m[0]) + std::norm(o.m[2]), c1 = std::norm(o.m[1]) + std::norm(o.m[3]);
-            const cd dot = std::conj(o.m[0]) * o.m[1] + std::conj(o.m[2]) * o.m[3];
+            const cx dot = mul(std::conj(o.m[0]), o.m[1]) + mul(std::conj(o.m[2]), o.m[3]);
             shear = c0 > 1e-6 && c0 < 1e6 && std::abs(c1 - c0) < 1e-12 * c0 && std::abs(dot) < 1e-12 * c0 &&
                     std::norm(o.m[0]) >= 0.25 * c0;
         }
@@ -1272,12 +1279,12 @@ void reduce_matrices(std::vector<HOp>& ops, u32 n) {
             Left& l = left[o.q[t]];
             if (!l.any) continue;
             for (u32 r = 0; r < d; ++r)
-                for (u32 col = 0; col < d; ++col) o.m[r * d + col] *= l.d[(col >> t) & 1u];
+                for (u32 col = 0; col < d; ++col) o.m[r * d + col] = mul(o.m[r * d + col], l.d[(col >> t) & 1u]);
             total -= l.bits;
             l = Left{};
         }
         if (!shear) continue;
-        const cd p = o.m[0], a = o.m[1] / o.m[0], q = o.m[3] - o.m[2] * a;
+        const cx p = o.m[0], a = quot(o.m[1], o.m[0]), q = o.m[3] - mul(o.m[2], a);
         const double bits = std::max(std::abs(std::log2(std::abs(p))), std::abs(std::log2(std::abs(q))));
         if (!(total + bits < 200.0)) continue;
         Left& l = left[o.q[0]];
@@ -1286,7 +1293,7 @@ void reduce_matrices(std::vector<HOp>& ops, u32 n) {
         l.any = true;
         l.bits = bits;
         total += bits;
-        o.m = {a, o.m[2] / q, 0.0, 0.0};
+        o.m = {a, quot(o.m[2], q), 0.0, 0.0};
         o.reduced = true;
     }
 }
@@ -1321,7 +1328,7 @@ bool convert_gates(u32 n, const qm_batch_gate* gates, UINT gate_count, HCirc& c,
         }
         const std::vector<u32> q(g.qubits, g.qubits + k);
         const u32 d = 1u << k;
-        std::vector<cd> m;
+        std::vector<cx> m;
         if (two) {
             HOp cz;
             cz.type = 2;
@@ -1330,13 +1337,13 @@ bool convert_gates(u32 n, const qm_batch_gate* gates, UINT gate_count, HCirc& c,
             cv.push(std::move(cz));
             if (g.kind == QM_BATCH_CNOT) cv.dense({q[1]}, {0.5, 0.5, 0.5, -0.5});
         } else if (depol) {
-            cv.depol(q, cd(g.matrix[0].re, g.matrix[0].im));
+            cv.depol(q, cx(g.matrix[0].re, g.matrix[0].im));
             c.paired = true;
         } else if (g.kind == QM_BATCH_DIAG) {
-            for (u32 i = 0; i < d; ++i) m.push_back(cd(g.matrix[i].re, g.matrix[i].im));
+            for (u32 i = 0; i < d; ++i) m.push_back(cx(g.matrix[i].re, g.matrix[i].im));
             cv.diagonal(q, m);
         } else {
-            for (u32 i = 0; i < d * d; ++i) m.push_back(cd(g.matrix[i].re, g.matrix[i].im));
+            for (u32 i = 0; i < d * d; ++i) m.push_back(cx(g.matrix[i].re, g.matrix[i].im));
             if (density && k == 2 && q[1] == q[0] + n / 2) c.paired = true;
             cv.dense(q, std::move(m));
         }
