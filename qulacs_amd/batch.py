@@ -19,7 +19,7 @@ import time
 
 import numpy as np
 
-from . import _lib
+from . import _core, _lib
 
 _KIND = {"dense": _lib.BATCH_DENSE, "diag": _lib.BATCH_DIAG, "CZ": _lib.BATCH_CZ, "CNOT": _lib.BATCH_CNOT}
 
@@ -173,9 +173,17 @@ class FusedCircuit:
             pass
 
 
+def _as_matrix(m):
+    return np.ascontiguousarray(np.asarray(m, dtype=np.complex128)).ravel()
+
+
 def _marshal(gates):
+    """The gates as a C array, and what has to stay alive while it is used."""
     arr = (_lib.QmBatchGate * max(1, len(gates)))()
-    keep = []
+    keep = _core._pack_gates(gates if type(gates) is list else list(gates), arr, _KIND, _as_matrix)
+    if keep is not None:
+        return arr, keep
+    keep = []  # gates in other containers, and those that are refused
     for i, (kind, qubits, matrix) in enumerate(gates):
         if len(qubits) > 4 or kind not in _KIND:
             raise _lib.QulacsMI355Error(f"batch gate {i}: {kind} on {len(qubits)} qubits is not supported")
@@ -185,7 +193,7 @@ def _marshal(gates):
         for j, q in enumerate(qubits):
             g.qubits[j] = int(q)
         if matrix is not None:
-            m = np.ascontiguousarray(np.asarray(matrix, dtype=np.complex128)).ravel()
+            m = _as_matrix(matrix)
             keep.append(m)
             g.matrix = C.cast(m.ctypes.data, _lib.PC)
     return arr, keep

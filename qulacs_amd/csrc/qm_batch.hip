@@ -319,19 +319,18 @@ bool dev_reserve(void** dst, size_t* cap, size_t bytes, const char* what) {
     return true;
 }
 
-template <class T>
-bool dev_put(T** dst, size_t* cap, const std::vector<T>& src, const char* what) {
-    if (!dev_reserve((void**)dst, cap, src.size() * sizeof(T), what)) return false;
-    return src.empty() || hip_ok(hipMemcpy(*dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice), what);
-}
-
 }  // namespace
+// A circuit ready to join a batch (batch_add_prepared).
+struct PreparedCircuit {
+    HCirc c;
+};
 }  // namespace qm
 
 struct qm_batch {
     std::vector<qm::HCirc> circs;
     // compiled
     int device = -1;
+    char* d_program = nullptr;  // one allocation, filled by one copy: the arrays of the next seven and d_large
     unsigned K = 0;
     int keep = 0;
     std::vector<qm::DCirc> h_circs;
@@ -353,7 +352,7 @@ struct qm_batch {
     std::vector<Level> levels;
     Level energy_items{0, 0, 0};
     qm::u32 n_large = 0;
-    size_t cap[11] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};  // bytes held by each device buffer above
+    size_t cap[4] = {0, 0, 0, 0};  // bytes held: program, scratch, energies, partials
     bool lds_set = false;               // the kernel's LDS limit has been raised on this device
     unsigned lq_cap = 13;               // qubits held in LDS per tile (qm_batch_set_local_qubits)
     hipGraph_t graph = nullptr;         // captured launch (qm_batch_capture)
@@ -370,11 +369,11 @@ struct qm_batch {
         lds_set = false;
         if (device >= 0) {
             (void)hipSetDevice(device);
-            void* ptrs[] = {d_circs, d_stages, d_passes, d_subs, d_pool, d_terms, d_items, d_large, d_scratch, d_energies, d_partials};
+            void* ptrs[] = {d_program, d_scratch, d_energies, d_partials};
             for (void* p : ptrs)
                 if (p) (void)hipFree(p);
         }
-        d_circs = nullptr; d_stages = nullptr; d_passes = nullptr; d_subs = nullptr; d_pool = nullptr;
+        d_program = nullptr; d_circs = nullptr; d_stages = nullptr; d_passes = nullptr; d_subs = nullptr; d_pool = nullptr;
         d_terms = nullptr; d_items = nullptr; d_large = nullptr; d_scratch = nullptr; d_energies = nullptr;
         d_partials = nullptr;
         for (size_t& c : cap) c = 0;
@@ -447,22 +446,31 @@ void qm_batch_destroy(qm_batch* b) {
 
 int qm_batch_add_circuit(qm_batch* b, UINT n, const qm_batch_gate* gates, UINT gate_count, const ITYPE* bf,
                          const ITYPE* pf, const UINT* rot, const double* coefs, UINT term_count) {
+    if (!batch_ok(b, "qm_batch_add_circuit")) return -1;
+    PreparedCircuit* c = batch_prepare_circuit(n, gates, gate_count, bf, pf, rot, coefs, term_count);
+    return c ? batch_add_prepared(b, c) : -1;
+}
+
+}  // extern "C"
+
+namespace qm {
+PreparedCircuit* batch_prepare_circuit(UINT n, const qm_batch_gate* gates, UINT gate_count, const ITYPE* bf,
+                                       const ITYPE* pf, const UINT* rot, const double* coefs, UINT term_count) {
     const char* what = "qm_batch_add_circuit";
-    if (!batch_ok(b, what)) return -1;
     if (n < 1 || n > QM_BATCH_MAX_QUBITS) {
         set_error(QM_ERR_INVALID_ARGUMENT, "%s: qubit count %u outside 1..%u", what, n, QM_BATCH_MAX_QUBITS);
-        return -1;
+        return nullptr;
     }
     if ((gate_count && !gates) || (term_count && (!bf || !pf || !rot || !coefs))) {
         set_error(QM_ERR_INVALID_ARGUMENT, "%s: null gate or term array", what);
-        return -1;
+        return nullptr;
     }
     HCirc c;
-    if (!convert_gates(n, gates, gate_count, c, what)) return -1;
+    if (!convert_gates(n, gates, gate_count, c, what)) return nullptr;
     for (UINT t = 0; t < term_count; ++t) {
         if ((bf[t] >> n) || (pf[t] >> n)) {
             set_error(QM_ERR_INVALID_ARGUMENT, "%s: term %u acts beyond %u qubits", what, t, n);
-            return -1;
+            return nullptr;
         }
         DTerm tm{};
         tm.bf = bf[t];
@@ -471,9 +479,17 @@ int qm_batch_add_circuit(qm_batch* b, UINT n, const qm_batch_gate* gates, UINT g
         tm.coef = coefs[t];
         c.terms.push_back(tm);
     }
-    b->circs.push_back(std::move(c));
+    return new PreparedCircuit{std::move(c)};
+}
+int batch_add_prepared(qm_batch* b, PreparedCircuit* c) {
+    b->circs.push_back(std::move(c->c));
+    delete c;
     return (int)b->circs.size() - 1;
 }
+void batch_destroy_prepared(PreparedCircuit* c) { delete c; }
+}  // namespace qm
+
+extern "C" {
 
 int qm_batch_compile(qm_batch* b, UINT block_qubits, int keep_states, unsigned dev) {
     const char* what = "qm_batch_compile";
@@ -552,16 +568,34 @@ int qm_batch_compile(qm_batch* b, UINT block_qubits, int keep_states, unsigned d
     if (terms.empty()) terms.push_back(DTerm{});
     if (items.empty()) items.push_back(DItem{});
     b->device = (int)dev;
-    bool ok = dev_put(&b->d_circs, &b->cap[0], dc, what) && dev_put(&b->d_stages, &b->cap[1], f.stages, what) &&
-              dev_put(&b->d_passes, &b->cap[2], f.passes, what) && dev_put(&b->d_subs, &b->cap[3], f.subs, what) &&
-              dev_put(&b->d_pool, &b->cap[4], f.pool, what) && dev_put(&b->d_terms, &b->cap[5], terms, what) &&
-              dev_put(&b->d_items, &b->cap[6], items, what) && dev_put(&b->d_large, &b->cap[10], large, what);
+    // one copy: a copy command costs some 30 us, which eight arrays paid each
+    std::vector<char> host;
+    auto put = [&](const auto& v) {
+        const size_t at = (host.size() + 255) & ~size_t(255), bytes = v.size() * sizeof(v[0]);
+        host.resize(at + bytes);
+        if (bytes) std::memcpy(host.data() + at, v.data(), bytes);
+        return at;
+    };
+    const size_t at_circs = put(dc), at_stages = put(f.stages), at_passes = put(f.passes), at_subs = put(f.subs),
+                 at_pool = put(f.pool), at_terms = put(terms), at_items = put(items), at_large = put(large);
+    bool ok = dev_reserve((void**)&b->d_program, &b->cap[0], host.size(), what) &&
+              hip_ok(hipMemcpy(b->d_program, host.data(), host.size(), hipMemcpyHostToDevice), what);
+    if (ok) {
+        b->d_circs = (DCirc*)(b->d_program + at_circs);
+        b->d_stages = (DStage*)(b->d_program + at_stages);
+        b->d_passes = (DPass*)(b->d_program + at_passes);
+        b->d_subs = (DSub*)(b->d_program + at_subs);
+        b->d_pool = (double2*)(b->d_program + at_pool);
+        b->d_terms = (DTerm*)(b->d_program + at_terms);
+        b->d_items = (DItem*)(b->d_program + at_items);
+        b->d_large = (u32*)(b->d_program + at_large);
+    }
     if (ok && state_off) {
-        ok = dev_reserve((void**)&b->d_scratch, &b->cap[7], state_off * sizeof(double2), what);
+        ok = dev_reserve((void**)&b->d_scratch, &b->cap[1], state_off * sizeof(double2), what);
         if (!ok) set_error(QM_ERR_OUT_OF_MEMORY, "%s: %llu bytes of state memory", what, state_off * 16ULL);
     }
-    if (ok) ok = dev_reserve((void**)&b->d_energies, &b->cap[8], std::max<size_t>(1, dc.size()) * sizeof(double), what);
-    if (ok) ok = dev_reserve((void**)&b->d_partials, &b->cap[9], std::max<size_t>(1, nchunk) * sizeof(double), what);
+    if (ok) ok = dev_reserve((void**)&b->d_energies, &b->cap[2], std::max<size_t>(1, dc.size()) * sizeof(double), what);
+    if (ok) ok = dev_reserve((void**)&b->d_partials, &b->cap[3], std::max<size_t>(1, nchunk) * sizeof(double), what);
     if (!ok) {
         b->release();
         return QM_ERR_HIP;

@@ -240,6 +240,13 @@ bool enqueue_sampling_in(void* buffer, const void* state, u64 dim, const double*
                          hipStream_t st, double margin, unsigned char* h_flags);
 // Uploads a fused circuit's program to `dev` ahead of its first launch.
 bool circuit_prepare(qm_circuit* c, unsigned dev);
+// A circuit converted for a batch apart from it: checked (null and an error as from
+// qm_batch_add_circuit), then added once, which takes it over, or destroyed.
+struct PreparedCircuit;
+PreparedCircuit* batch_prepare_circuit(UINT n, const qm_batch_gate* gates, UINT gate_count, const ITYPE* bf,
+                                       const ITYPE* pf, const UINT* rot, const double* coefs, UINT term_count);
+int batch_add_prepared(qm_batch* b, PreparedCircuit* c);
+void batch_destroy_prepared(PreparedCircuit* c);
 // Many small state vectors (dim <= 2^16 each), one work-group per CDF.
 struct SampleJob {
     const double2* state;

@@ -52,13 +52,12 @@ constexpr u32 kBatchBlockQubits = 3;
 struct Request {
     long long id = 0;
     u32 n = 0;
-    std::vector<qm_batch_gate> gates;
-    std::vector<std::vector<qm_complex>> mats;
     std::vector<u64> bf, pf;
     std::vector<u32> rot;
     std::vector<double> coef;
     std::vector<double> uniforms;
-    qm_circuit* circuit = nullptr;  // large requests
+    PreparedCircuit* prepared = nullptr;  // small requests until they join a batch: converted once, by the submitter
+    qm_circuit* circuit = nullptr;        // large requests
     bool small = false;
     u64 bytes = 0;
     clk::time_point t_submit, t_admit, t_done;
@@ -69,6 +68,7 @@ struct Request {
     int status = 0;  // 0 queued, 1 admitted, 2 done, 3 failed
     std::string error;
     ~Request() {
+        if (prepared) batch_destroy_prepared(prepared);
         if (circuit) qm_circuit_destroy(circuit);
     }
 };
@@ -205,11 +205,8 @@ void qm_server::launch_batch() {
     qm_batch_clear(batch);
     size_t total = 0;
     for (const ReqPtr& r : next_batch) {
-        if (qm_batch_add_circuit(batch, r->n, r->gates.data(), (UINT)r->gates.size(), r->bf.data(), r->pf.data(),
-                                 r->rot.data(), r->coef.data(), (UINT)r->coef.size()) < 0) {
-            err = take_error();
-            break;
-        }
+        batch_add_prepared(batch, r->prepared);
+        r->prepared = nullptr;
         total += r->uniforms.size();
     }
     const size_t nb = next_batch.size();
@@ -415,17 +412,6 @@ long long qm_server_submit(qm_server* s, UINT n, const qm_batch_gate* gates, UIN
                   r->bytes);
         return -1;
     }
-    r->gates.assign(gates, gates + gate_count);
-    r->mats.resize(gate_count);
-    for (UINT i = 0; i < gate_count; ++i) {
-        const qm_batch_gate& g = gates[i];
-        if (g.matrix && g.qubit_count >= 1 && g.qubit_count <= 4) {
-            const size_t d = (size_t)1 << g.qubit_count;
-            const size_t len = g.kind == QM_BATCH_DIAG ? d : d * d;
-            r->mats[i].assign(g.matrix, g.matrix + len);
-            r->gates[i].matrix = r->mats[i].data();
-        }
-    }
     r->bf.assign(bf, bf + term_count);
     r->pf.assign(pf, pf + term_count);
     r->rot.assign(rot, rot + term_count);
@@ -437,13 +423,10 @@ long long qm_server_submit(qm_server* s, UINT n, const qm_batch_gate* gates, UIN
             return -1;
         }
     if (r->small) {
-        // validate on a host-only batch (no device work)
-        qm_batch* probe = qm_batch_create();
-        const int idx = qm_batch_add_circuit(probe, n, r->gates.data(), gate_count, bf, pf, rot, coefs, term_count);
-        qm_batch_destroy(probe);
-        if (idx < 0) return -1;
+        r->prepared = batch_prepare_circuit(n, gates, gate_count, bf, pf, rot, coefs, term_count);
+        if (!r->prepared) return -1;
     } else {
-        r->circuit = qm_circuit_create(n, r->gates.data(), gate_count, 0, 0);
+        r->circuit = qm_circuit_create(n, gates, gate_count, 0, 0);
         // the program goes to the device here, in the submitting thread, so the
         // scheduler thread never waits on an upload
         if (!r->circuit || !use_device(s->device) || !circuit_prepare(r->circuit, s->device)) return -1;
