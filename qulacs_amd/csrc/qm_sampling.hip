@@ -31,7 +31,8 @@ constexpr int kCdfChunk = kCdfThreads * kCdfPer; // 4096 (32 KiB of LDS)
 // A block scan that stops within kSerialTrigger elements of where it started is
 // followed by kSerialRun one-by-one additions (see exact_chunk).
 constexpr int kSerialTrigger = 64;
-constexpr int kSerialRun = 512;
+constexpr int kSerialRun = 256;
+constexpr int kCdfPad = 80;  // zeros behind a chunk in LDS (serial_wave)
 
 __device__ __forceinline__ double prob_sv(const double2* __restrict__ a, u64 i) {
     const double2 v = a[i];
@@ -241,6 +242,135 @@ __device__ __forceinline__ void xchg_bcast(bool owner, double& s, int& first, Xc
     first = slot.first;
 }
 
+// out[j] = fl(...fl(s + P[pos]) + ... + P[j]) for j in [pos, end), by one wave; s becomes the last.
+// The chain of dependent additions is all that can cost time here, so the lanes share one chain:
+// element k of a block of 64 is read by every lane (an LDS broadcast) and added by the lanes from
+// k on, which leaves lane k with the sum through element k.  The block's elements behind `end` must
+// be 0 (end - pos a multiple of 64, or P padded).  An element costs 8.9 cycles, the latency of a dependent
+// addition being 8.4; keeping each sum with two selects instead took 16.5.  With the block's scan of some 3 us
+// in mind, runs of 128 to 512 elements came out alike, 2048 and 4096 slower.
+__device__ __forceinline__ void add_from_lane(double& t, const double (&p)[16], int k0) {
+    u64 all;
+    // the caller's wave is full, so exec is all ones before and after
+    switch (k0) {
+        case 0:
+            asm volatile("s_mov_b64 %[all], exec\n\t"
+                         "s_lshl_b64 exec, -1, 0\n\tv_add_f64 %[t], %[t], %[p0]\n\t"
+                         "s_lshl_b64 exec, -1, 1\n\tv_add_f64 %[t], %[t], %[p1]\n\t"
+                         "s_lshl_b64 exec, -1, 2\n\tv_add_f64 %[t], %[t], %[p2]\n\t"
+                         "s_lshl_b64 exec, -1, 3\n\tv_add_f64 %[t], %[t], %[p3]\n\t"
+                         "s_lshl_b64 exec, -1, 4\n\tv_add_f64 %[t], %[t], %[p4]\n\t"
+                         "s_lshl_b64 exec, -1, 5\n\tv_add_f64 %[t], %[t], %[p5]\n\t"
+                         "s_lshl_b64 exec, -1, 6\n\tv_add_f64 %[t], %[t], %[p6]\n\t"
+                         "s_lshl_b64 exec, -1, 7\n\tv_add_f64 %[t], %[t], %[p7]\n\t"
+                         "s_lshl_b64 exec, -1, 8\n\tv_add_f64 %[t], %[t], %[p8]\n\t"
+                         "s_lshl_b64 exec, -1, 9\n\tv_add_f64 %[t], %[t], %[p9]\n\t"
+                         "s_lshl_b64 exec, -1, 10\n\tv_add_f64 %[t], %[t], %[p10]\n\t"
+                         "s_lshl_b64 exec, -1, 11\n\tv_add_f64 %[t], %[t], %[p11]\n\t"
+                         "s_lshl_b64 exec, -1, 12\n\tv_add_f64 %[t], %[t], %[p12]\n\t"
+                         "s_lshl_b64 exec, -1, 13\n\tv_add_f64 %[t], %[t], %[p13]\n\t"
+                         "s_lshl_b64 exec, -1, 14\n\tv_add_f64 %[t], %[t], %[p14]\n\t"
+                         "s_lshl_b64 exec, -1, 15\n\tv_add_f64 %[t], %[t], %[p15]\n\t"
+                         "s_mov_b64 exec, %[all]"
+                         : [t] "+v"(t), [all] "=&s"(all)
+                         : [p0] "v"(p[0]), [p1] "v"(p[1]), [p2] "v"(p[2]), [p3] "v"(p[3]), [p4] "v"(p[4]), [p5] "v"(p[5]), [p6] "v"(p[6]), [p7] "v"(p[7]), [p8] "v"(p[8]), [p9] "v"(p[9]), [p10] "v"(p[10]), [p11] "v"(p[11]), [p12] "v"(p[12]), [p13] "v"(p[13]), [p14] "v"(p[14]), [p15] "v"(p[15])
+                         : "scc");
+            break;
+        case 16:
+            asm volatile("s_mov_b64 %[all], exec\n\t"
+                         "s_lshl_b64 exec, -1, 16\n\tv_add_f64 %[t], %[t], %[p0]\n\t"
+                         "s_lshl_b64 exec, -1, 17\n\tv_add_f64 %[t], %[t], %[p1]\n\t"
+                         "s_lshl_b64 exec, -1, 18\n\tv_add_f64 %[t], %[t], %[p2]\n\t"
+                         "s_lshl_b64 exec, -1, 19\n\tv_add_f64 %[t], %[t], %[p3]\n\t"
+                         "s_lshl_b64 exec, -1, 20\n\tv_add_f64 %[t], %[t], %[p4]\n\t"
+                         "s_lshl_b64 exec, -1, 21\n\tv_add_f64 %[t], %[t], %[p5]\n\t"
+                         "s_lshl_b64 exec, -1, 22\n\tv_add_f64 %[t], %[t], %[p6]\n\t"
+                         "s_lshl_b64 exec, -1, 23\n\tv_add_f64 %[t], %[t], %[p7]\n\t"
+                         "s_lshl_b64 exec, -1, 24\n\tv_add_f64 %[t], %[t], %[p8]\n\t"
+                         "s_lshl_b64 exec, -1, 25\n\tv_add_f64 %[t], %[t], %[p9]\n\t"
+                         "s_lshl_b64 exec, -1, 26\n\tv_add_f64 %[t], %[t], %[p10]\n\t"
+                         "s_lshl_b64 exec, -1, 27\n\tv_add_f64 %[t], %[t], %[p11]\n\t"
+                         "s_lshl_b64 exec, -1, 28\n\tv_add_f64 %[t], %[t], %[p12]\n\t"
+                         "s_lshl_b64 exec, -1, 29\n\tv_add_f64 %[t], %[t], %[p13]\n\t"
+                         "s_lshl_b64 exec, -1, 30\n\tv_add_f64 %[t], %[t], %[p14]\n\t"
+                         "s_lshl_b64 exec, -1, 31\n\tv_add_f64 %[t], %[t], %[p15]\n\t"
+                         "s_mov_b64 exec, %[all]"
+                         : [t] "+v"(t), [all] "=&s"(all)
+                         : [p0] "v"(p[0]), [p1] "v"(p[1]), [p2] "v"(p[2]), [p3] "v"(p[3]), [p4] "v"(p[4]), [p5] "v"(p[5]), [p6] "v"(p[6]), [p7] "v"(p[7]), [p8] "v"(p[8]), [p9] "v"(p[9]), [p10] "v"(p[10]), [p11] "v"(p[11]), [p12] "v"(p[12]), [p13] "v"(p[13]), [p14] "v"(p[14]), [p15] "v"(p[15])
+                         : "scc");
+            break;
+        case 32:
+            asm volatile("s_mov_b64 %[all], exec\n\t"
+                         "s_lshl_b64 exec, -1, 32\n\tv_add_f64 %[t], %[t], %[p0]\n\t"
+                         "s_lshl_b64 exec, -1, 33\n\tv_add_f64 %[t], %[t], %[p1]\n\t"
+                         "s_lshl_b64 exec, -1, 34\n\tv_add_f64 %[t], %[t], %[p2]\n\t"
+                         "s_lshl_b64 exec, -1, 35\n\tv_add_f64 %[t], %[t], %[p3]\n\t"
+                         "s_lshl_b64 exec, -1, 36\n\tv_add_f64 %[t], %[t], %[p4]\n\t"
+                         "s_lshl_b64 exec, -1, 37\n\tv_add_f64 %[t], %[t], %[p5]\n\t"
+                         "s_lshl_b64 exec, -1, 38\n\tv_add_f64 %[t], %[t], %[p6]\n\t"
+                         "s_lshl_b64 exec, -1, 39\n\tv_add_f64 %[t], %[t], %[p7]\n\t"
+                         "s_lshl_b64 exec, -1, 40\n\tv_add_f64 %[t], %[t], %[p8]\n\t"
+                         "s_lshl_b64 exec, -1, 41\n\tv_add_f64 %[t], %[t], %[p9]\n\t"
+                         "s_lshl_b64 exec, -1, 42\n\tv_add_f64 %[t], %[t], %[p10]\n\t"
+                         "s_lshl_b64 exec, -1, 43\n\tv_add_f64 %[t], %[t], %[p11]\n\t"
+                         "s_lshl_b64 exec, -1, 44\n\tv_add_f64 %[t], %[t], %[p12]\n\t"
+                         "s_lshl_b64 exec, -1, 45\n\tv_add_f64 %[t], %[t], %[p13]\n\t"
+                         "s_lshl_b64 exec, -1, 46\n\tv_add_f64 %[t], %[t], %[p14]\n\t"
+                         "s_lshl_b64 exec, -1, 47\n\tv_add_f64 %[t], %[t], %[p15]\n\t"
+                         "s_mov_b64 exec, %[all]"
+                         : [t] "+v"(t), [all] "=&s"(all)
+                         : [p0] "v"(p[0]), [p1] "v"(p[1]), [p2] "v"(p[2]), [p3] "v"(p[3]), [p4] "v"(p[4]), [p5] "v"(p[5]), [p6] "v"(p[6]), [p7] "v"(p[7]), [p8] "v"(p[8]), [p9] "v"(p[9]), [p10] "v"(p[10]), [p11] "v"(p[11]), [p12] "v"(p[12]), [p13] "v"(p[13]), [p14] "v"(p[14]), [p15] "v"(p[15])
+                         : "scc");
+            break;
+        case 48:
+            asm volatile("s_mov_b64 %[all], exec\n\t"
+                         "s_lshl_b64 exec, -1, 48\n\tv_add_f64 %[t], %[t], %[p0]\n\t"
+                         "s_lshl_b64 exec, -1, 49\n\tv_add_f64 %[t], %[t], %[p1]\n\t"
+                         "s_lshl_b64 exec, -1, 50\n\tv_add_f64 %[t], %[t], %[p2]\n\t"
+                         "s_lshl_b64 exec, -1, 51\n\tv_add_f64 %[t], %[t], %[p3]\n\t"
+                         "s_lshl_b64 exec, -1, 52\n\tv_add_f64 %[t], %[t], %[p4]\n\t"
+                         "s_lshl_b64 exec, -1, 53\n\tv_add_f64 %[t], %[t], %[p5]\n\t"
+                         "s_lshl_b64 exec, -1, 54\n\tv_add_f64 %[t], %[t], %[p6]\n\t"
+                         "s_lshl_b64 exec, -1, 55\n\tv_add_f64 %[t], %[t], %[p7]\n\t"
+                         "s_lshl_b64 exec, -1, 56\n\tv_add_f64 %[t], %[t], %[p8]\n\t"
+                         "s_lshl_b64 exec, -1, 57\n\tv_add_f64 %[t], %[t], %[p9]\n\t"
+                         "s_lshl_b64 exec, -1, 58\n\tv_add_f64 %[t], %[t], %[p10]\n\t"
+                         "s_lshl_b64 exec, -1, 59\n\tv_add_f64 %[t], %[t], %[p11]\n\t"
+                         "s_lshl_b64 exec, -1, 60\n\tv_add_f64 %[t], %[t], %[p12]\n\t"
+                         "s_lshl_b64 exec, -1, 61\n\tv_add_f64 %[t], %[t], %[p13]\n\t"
+                         "s_lshl_b64 exec, -1, 62\n\tv_add_f64 %[t], %[t], %[p14]\n\t"
+                         "s_lshl_b64 exec, -1, 63\n\tv_add_f64 %[t], %[t], %[p15]\n\t"
+                         "s_mov_b64 exec, %[all]"
+                         : [t] "+v"(t), [all] "=&s"(all)
+                         : [p0] "v"(p[0]), [p1] "v"(p[1]), [p2] "v"(p[2]), [p3] "v"(p[3]), [p4] "v"(p[4]), [p5] "v"(p[5]), [p6] "v"(p[6]), [p7] "v"(p[7]), [p8] "v"(p[8]), [p9] "v"(p[9]), [p10] "v"(p[10]), [p11] "v"(p[11]), [p12] "v"(p[12]), [p13] "v"(p[13]), [p14] "v"(p[14]), [p15] "v"(p[15])
+                         : "scc");
+            break;
+    }
+}
+__device__ __forceinline__ void serial_wave(const double* P, int pos, int end, double& s, double* __restrict__ out) {
+    const int lane = threadIdx.x & 63;
+    double p[16], q[16];
+    auto load = [&](double (&x)[16], int j) {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) x[k] = P[j + k];
+    };
+    load(p, pos);
+    double t = s;
+    for (int j = pos; j < end; j += 64) {
+        load(q, j + 16);
+        add_from_lane(t, p, 0);
+        load(p, j + 32);
+        add_from_lane(t, q, 16);
+        load(q, j + 48);
+        add_from_lane(t, p, 32);
+        load(p, min(j + 64, kCdfChunk));
+        add_from_lane(t, q, 48);
+        if (j + lane < end) out[j + lane] = t;
+        t = readlane_f64(t, 63);
+    }
+    s = t;
+}
+
 // Sums chunk [c0, c0 + len) onto the running sum s exactly as the sequential
 // loop does and writes cdf[c0 + 1 .. c0 + len].  Called by every thread of a
 // 1024-thread block with the same s; returns with the same s in every thread.
@@ -250,6 +380,7 @@ __device__ __forceinline__ void exact_chunk(const double2* __restrict__ a, u64 d
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (int j = threadIdx.x; j < len; j += kCdfThreads)
         P[j] = DM ? prob_dm(a, c0 + j, dim) : prob_sv(a, c0 + j);
+    if (threadIdx.x < kCdfPad) P[len + threadIdx.x] = 0.0;
     __syncthreads();
     const u64 LIM = 1ULL << 53;
     const int lo = threadIdx.x * kCdfPer;  // this thread's elements: lo .. lo+kCdfPer-1
@@ -257,46 +388,15 @@ __device__ __forceinline__ void exact_chunk(const double2* __restrict__ a, u64 d
     int serial = 0;  // elements to add one by one before the next block scan
     while (pos < len) {
         if (serial > 0 || !isfinite(s)) {
-            // One thread adds the next elements one at a time, the same IEEE
-            // additions as the sequential loop, and leaves the sums in P for the
-            // block to store.  Used after crossings close together (a small
+            // One wave adds the next elements one at a time, the same IEEE additions as the
+            // sequential loop.  Used after crossings close together (a small
             // running sum doubling every few elements), where it is cheaper than
             // a block scan per crossing, and to finish a chunk after an inf/NaN
             // (only reachable from a non-finite amplitude).
             const int end = isfinite(s) ? min(len, pos + serial) : len;
-            if (threadIdx.x == 0) {
-                double t = s;
-                int j = pos;
-                double v[16];
-                if (j + 16 <= end) {
-#pragma unroll
-                    for (int k = 0; k < 16; ++k) v[k] = P[j + k];
-                }
-                for (; j + 16 <= end; j += 16) {
-                    double w[16];  // the next 16, loaded before this block's sums are stored
-                    if (j + 32 <= end) {
-#pragma unroll
-                        for (int k = 0; k < 16; ++k) w[k] = P[j + 16 + k];
-                    }
-#pragma unroll
-                    for (int k = 0; k < 16; ++k) {
-                        t = t + v[k];
-                        v[k] = t;
-                    }
-#pragma unroll
-                    for (int k = 0; k < 16; ++k) P[j + k] = v[k];
-#pragma unroll
-                    for (int k = 0; k < 16; ++k) v[k] = w[k];
-                }
-                for (; j < end; ++j) {
-                    t = t + P[j];
-                    P[j] = t;
-                }
-                s = t;
-            }
+            if (wid == 0) serial_wave(P, pos, end, s, cdf + c0 + 1);
             int unused = 0;
             xchg_bcast(threadIdx.x == 0, s, unused, X, r);
-            for (int j = pos + threadIdx.x; j < end; j += kCdfThreads) cdf[c0 + j + 1] = P[j];
             pos = end;
             serial = 0;
             continue;
@@ -406,7 +506,7 @@ __device__ __forceinline__ void exact_chunk(const double2* __restrict__ a, u64 d
 template <bool DM>
 __global__ __launch_bounds__(kCdfThreads) void k_cdf_exact(const double2* __restrict__ a, u64 dim,
                                                            double* __restrict__ cdf) {
-    __shared__ double P[kCdfChunk];
+    __shared__ double P[kCdfChunk + kCdfPad];
     __shared__ Xchg X[2];
     int r = 0;
     double s = 0.0;  // exact running sum, identical in every thread
@@ -662,27 +762,31 @@ __global__ __launch_bounds__(kIncrThreads) void k_chunk_incr(const double2* __re
     }
 }
 
+// A window of 1024 chunks is loaded and scanned once; its chunks are then walked in runs, each one
+// exchange across the block.  A run ends at the first chunk that is not fast, and the next one
+// starts behind it with the sum that this chunk left, be it settled from the summaries (a tie, a
+// crossing) or summed element by element.  Latency bounds the walk (one work-group).
+// 17 qubits: 59 -> 46 us, 20: 64 -> 37, where a window was loaded and scanned again after every
+// crossing and one thread added the elements of serial_wave; half of what is left is the first chunk's
+// exact_chunk, whose sum crosses a binade each time the position doubles.
 template <bool DM>
 __global__ __launch_bounds__(kCdfThreads) void k_cdf_walk(const double2* __restrict__ a, u64 dim, u64 M,
                                                           ChunkSums cs, double* __restrict__ cdf) {
-    __shared__ double P[kCdfChunk];
+    __shared__ double P[kCdfChunk + kCdfPad];
     __shared__ Xchg X[2];
     int r = 0;
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t = (int)threadIdx.x;
     const u64 LIM = 1ULL << 53;
-    double s = 0.0;  // exact running sum, identical in every thread
+    double s = 0.0;  // exact running sum in front of chunk c + pos, identical in every thread
     if (threadIdx.x == 0) cdf[0] = 0.0;
-    // summaries of this thread's chunk in the window, loaded one window ahead
-    // (the next window's loads are in flight during an exact chunk)
-    double tT = 0.0, tp = 0.0;
-    int tkind = 0, tE = 0, tJ = 0;
-    u64 tN = 0, tA = 0, tR = 0, tB = 0;
-    auto load = [&](u64 cc) {
-        const u64 ci = cc + threadIdx.x;
-        tT = 0.0;
-        tkind = tE = 0;
-        tN = 0;
-        if (ci < M) {
+    for (u64 c = 0; c < M; c += kCdfThreads) {
+        const u64 ci = c + threadIdx.x;
+        const bool in = ci < M;
+        double tT = 0.0, tp = 0.0;
+        int tkind = 0, tE = 0, tJ = 0;
+        u64 tN = 0, tA = 0, tR = 0, tB = 0;
+        if (in) {
             tT = cs.T[ci];
             tkind = cs.kind[ci];
             tE = cs.E[ci];
@@ -693,56 +797,37 @@ __global__ __launch_bounds__(kCdfThreads) void k_cdf_walk(const double2* __restr
             tB = cs.eB[ci];
             tp = cs.ep[ci];
         }
-    };
-    u64 c = 0;
-    load(c);
-    while (c < M) {
-        const u64 ci = c + threadIdx.x;
-        int es = INT_MIN;
-        double u = 0.0;
-        u64 S = 0;
-        if (s != 0.0 && isfinite(s)) {
-            es = max(ilogb(s), -1022);
-            u = ldexp(1.0, es - 52);
-            S = (u64)(s / u);
-        }
-        bool ok = false;
-        u64 v = 0;  // below 2^53 (a chunk whose sum reaches it is not plain)
-        if (ci < M && isfinite(s)) {
-            if (tT == 0.0) {
-                ok = true;
-            } else if (s != 0.0 && tkind == kChunkPlain && tE == es) {
-                ok = true;
-                v = tN;
-            }
-        }
+        // Increments of the plain chunks in front, each in its own predicted binade: between two
+        // chunks of a run, which all lie in the sum's binade, differences are exact (modulo
+        // 2^64, and below 2^63).
+        const u64 v = in && tT != 0.0 && tkind == kChunkPlain ? tN : 0;  // below 2^53
         const XScan xs = xchg_scan_first<>(v, INT_MAX, X, r);
-        // The window is walked in runs: a run ends at its first chunk that is
-        // not fast; a settled tie chunk there adds its increments (delta) to
-        // every later chunk of the window, and the next run starts after it.
-        u64 delta = 0;
+        u64 base = 0;  // the scan in front of chunk c + pos
         int pos = 0;
-        int stop = kCdfThreads;
-        int settled = 0;  // 0, kStartTie or kStartCross for the chunk at stop
-        u64 Sstop = 0;
-        double s_after = 0.0;
-        double rsj = 0.0;  // this thread's sum through its crossing element (last run)
-        for (;;) {  // wave-uniform and block-uniform
-            const int t = (int)threadIdx.x;
-            const u64 S0 = S + xs.excl + delta;  // exact for the chunks of the current run and its stop
-            // Chunk ci is fast when every chunk of the run up to it is ok and
-            // the sum stays below 2^53 units through it; the sums never
-            // decrease, so the fast chunks are the first of the run.
+        while (pos < kCdfThreads && c + (u64)pos < M) {  // block-uniform
+            const bool sum = s != 0.0 && isfinite(s);
+            int es = INT_MIN;
+            double u = 0.0;
+            u64 S = 0;
+            if (sum) {
+                es = max(ilogb(s), -1022);
+                u = ldexp(1.0, es - 52);
+                S = (u64)(s / u);
+            }
+            const u64 S0 = S + (xs.excl - base);  // exact for the chunks of this run and its stop
+            // A chunk is fast when every chunk of the run up to it is ok and the sum stays below
+            // 2^53 units through it; the sums never decrease, so the fast chunks are the first of
+            // the run.  (What later chunks store here they store again in their own run.)
+            const bool ok = in && isfinite(s) && (tT == 0.0 || (sum && tkind == kChunkPlain && tE == es));
             const bool fast = t >= pos && ok && S0 + v < LIM;
             if (fast) {
-                cs.start[ci] = s == 0.0 ? 0.0 : (double)S0 * u;
+                cs.start[ci] = sum ? (double)S0 * u : 0.0;
                 cs.exact[ci] = kStartPlain;
             }
             // the settlement of this chunk, should it be the run's stop
             int rcode = 0;
-            double rend = 0.0;
-            u64 rdelta = 0;
-            if (t >= pos && !fast && ci < M && s != 0.0 && isfinite(s) && tE == es && tT != 0.0) {
+            double rend = 0.0, rsj = 0.0;
+            if (t >= pos && !fast && in && sum && tE == es && tT != 0.0) {
                 if (tkind == kChunkTie) {
                     // fl(x + (F + 1/2) u) rounds to the even neighbour: tie k
                     // adds F + ((sum in front of it) mod 2)
@@ -751,7 +836,6 @@ __global__ __launch_bounds__(kCdfThreads) void k_cdf_walk(const double2* __restr
                     const u64 endS = S0 + tN + add;
                     if (endS < LIM) {
                         rcode = kStartTie;
-                        rdelta = tN + add;
                         rend = (double)endS * u;
                     }
                 } else if (tkind == kChunkCross && S0 + tA < LIM && S0 + tA + tR >= LIM) {
@@ -767,77 +851,48 @@ __global__ __launch_bounds__(kCdfThreads) void k_cdf_walk(const double2* __restr
                     }
                 }
             }
-            // the run's stop, the sum in front of it and its settlement: from
-            // the first wave holding a chunk of the run that is not fast
-            {
-                const u64 nf = __ballot(t >= pos && !fast);
-                const int fl = nf ? __ffsll((unsigned long long)nf) - 1 : 0;
-                Xchg& slot = X[r & 1];
-                const u64 at = readlane_u64(S0, fl);
-                const int rk = __builtin_amdgcn_readlane(rcode, fl);
-                const double re = readlane_f64(rend, fl);
-                const u64 rd = readlane_u64(rdelta, fl);
-                if (lane == 0) {
-                    slot.mn[wid] = nf ? wid * 64 + fl : INT_MAX;
-                    slot.val[wid] = at;
-                    slot.ok[wid] = rk;
-                    slot.dv[wid] = re;
-                    slot.sum2[wid] = rd;
-                }
-                __syncthreads();
-                ++r;
+            if (rcode == 0) rend = sum ? (double)S0 * u : s;  // not settled: the sum in front of it
+            // the run's stop and what it leaves: from the first wave that holds a chunk of the
+            // run that is not fast
+            const u64 nf = __ballot(t >= pos && !fast);
+            const int fl = nf ? __ffsll((unsigned long long)nf) - 1 : 0;
+            Xchg& slot = X[r & 1];
+            const int rk = __builtin_amdgcn_readlane(rcode, fl);
+            const double re = readlane_f64(rend, fl);
+            const u64 through = readlane_u64(xs.excl + v, fl);
+            if (lane == 0) {
+                slot.mn[wid] = nf ? wid * 64 + fl : INT_MAX;
+                slot.ok[wid] = rk;
+                slot.dv[wid] = re;
+                slot.val[wid] = through;
             }
-            const Xchg& got = X[(r - 1) & 1];
-            const int tm = lane < kCdfWaves ? got.mn[lane] : INT_MAX;
+            __syncthreads();
+            const int tm = lane < kCdfWaves ? slot.mn[lane] : INT_MAX;
+            const int tk = lane < kCdfWaves ? slot.ok[lane] : 0;
+            const double td = lane < kCdfWaves ? slot.dv[lane] : 0.0;
+            const u64 tv = lane < kCdfWaves ? slot.val[lane] : 0;
+            ++r;
             const u64 has = __ballot(tm != INT_MAX);
-            stop = kCdfThreads;
-            Sstop = S + xs.total + delta;
-            settled = 0;
-            if (has) {
-                const int w = __ffsll((unsigned long long)has) - 1;
-                stop = __builtin_amdgcn_readlane(tm, w);
-                Sstop = readlane_u64(lane < kCdfWaves ? got.val[lane] : 0, w);
-                settled = __builtin_amdgcn_readlane(lane < kCdfWaves ? got.ok[lane] : 0, w);
-                s_after = readlane_f64(lane < kCdfWaves ? got.dv[lane] : 0.0, w);
-                const u64 dstop = readlane_u64(lane < kCdfWaves ? got.sum2[lane] : 0, w);
-                if (settled == kStartTie && c + (u64)stop < M) {
-                    if (t == stop) {
-                        cs.start[ci] = (double)Sstop * u;
-                        cs.exact[ci] = kStartTie;
-                    }
-                    delta += dstop;
-                    pos = stop + 1;
-                    if (pos < kCdfThreads) continue;
-                    // the window ends with the settled tie
-                    stop = kCdfThreads;
-                    Sstop = S + xs.total + delta;
-                    settled = 0;
-                }
+            if (!has) {  // fast to the window's end
+                if (sum) s = (double)(S + (xs.total - base)) * u;
+                break;
             }
-            break;
-        }
-        if (s != 0.0 && isfinite(s)) s = (double)Sstop * u;  // the sum in front of chunk c + stop
-        c += (u64)stop;
-        const bool handle = stop < kCdfThreads && c < M;
-        if (handle && settled == kStartCross) {
-            if ((int)threadIdx.x == stop) {
-                cs.start[c] = s;
-                cs.exact[c] = kStartCross;
-                cs.ep[c] = rsj;  // the sum through the crossing element
+            const int w = __ffsll((unsigned long long)has) - 1;
+            const int stop = __builtin_amdgcn_readlane(tm, w);
+            const int settled = __builtin_amdgcn_readlane(tk, w);
+            s = readlane_f64(td, w);
+            base = readlane_u64(tv, w);
+            pos = stop + 1;
+            if (c + (u64)stop >= M) break;
+            if (t == stop) {
+                cs.start[ci] = settled && sum ? (double)S0 * u : s;
+                cs.exact[ci] = settled ? settled : kStartExact;
+                if (settled == kStartCross) cs.ep[ci] = rsj;  // the sum through the crossing element
             }
-            s = s_after;
-        }
-        load(c + (handle ? 1 : 0));
-        if (handle) {
-            if (settled != kStartCross) {
-                if (threadIdx.x == 0) {
-                    cs.start[c] = s;
-                    cs.exact[c] = kStartExact;
-                }
-                const int len = (int)min((u64)kCdfChunk, dim - c * kCdfChunk);
-                exact_chunk<DM>(a, dim, c * kCdfChunk, len, s, cdf, P, X, r);
+            if (!settled) {
+                const u64 c0 = (c + (u64)stop) * kCdfChunk;
+                exact_chunk<DM>(a, dim, c0, (int)min((u64)kCdfChunk, dim - c0), s, cdf, P, X, r);
             }
-            c += 1;
         }
     }
 }
@@ -1100,7 +1155,7 @@ struct DevSampleJob {
 };
 
 __global__ __launch_bounds__(kCdfThreads) void k_cdf_jobs(const DevSampleJob* __restrict__ jobs) {
-    __shared__ double P[kCdfChunk];
+    __shared__ double P[kCdfChunk + kCdfPad];
     __shared__ Xchg X[2];
     int r = 0;
     const DevSampleJob jb = jobs[blockIdx.x];
