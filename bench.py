@@ -437,48 +437,14 @@ def dm_sweep(args, lib_mod, hip):
     loop_ms = (time.perf_counter() - t0) * 1e3
     qa.set_synchronous(True)
     tr_loop = dmst.get_squared_norm()
-    # HBM passes the loop issues, by its grouping rule: three to five
-    # single-qubit channels in a row on distinct qubits are one pass; otherwise a
-    # run of gates/channels on at most two qubits together is one pass (a lone
-    # gate on one or two qubits too); a gate on more qubits is two passes (rows,
-    # then columns)
-    seq = []
-    for g in gates:
-        seq.append(("gate", set(g.targets)))
-        seq += [("chan", {q}) for q in g.targets]
-    passes, cur, k = 0, set(), 0
-    while k < len(seq):
-        run = 0
-        while k + run < len(seq) and run < 5 and seq[k + run][0] == "chan" and \
-                not any(seq[k + run][1] <= seq[k + j][1] for j in range(run)):
-            run += 1
-        if run >= 3:
-            passes += (1 if cur else 0) + 1
-            cur = set()
-            k += run
-            continue
-        part = seq[k][1]
-        k += 1
-        if len(part) > 2:
-            passes += (1 if cur else 0) + 2
-            cur = set()
-            continue
-        if len(cur | part) > 2:
-            passes += 1
-            cur = set()
-        cur |= part
-    passes += 1 if cur else 0
-    moved = passes * 32 * dim * dim
     return {"qubits": n, "gates": len(gates), "channels": ops - len(gates), "ms": round(ms, 2),
             "alg_GBps": round(alg / (ms * 1e-3) / 1e9, 1), "trace_after": tr,
-            "circuit_loop": {"ms": round(loop_ms, 2), "passes": passes,
+            "circuit_loop": {"ms": round(loop_ms, 2),
                              "alg_GBps": round(alg / (loop_ms * 1e-3) / 1e9, 1),
-                             "pass_GBps": round(moved / (loop_ms * 1e-3) / 1e9, 1),
-                             "pass_frac_of_peak": round(moved / (loop_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4),
                              "trace_after": tr_loop,
-                             "method": "QuantumCircuit.update_quantum_state on a DensityMatrix (gates and "
-                                       "depolarizing channels fused into superoperators), one run after a warm-up; "
-                                       "pass_GBps = passes x 32 B x 4^n / time"}}
+                             "method": "QuantumCircuit.update_quantum_state on a DensityMatrix (runs of gates "
+                                       "and channels on at most four qubits as programs of tile stages), one run "
+                                       "after a warm-up"}}
 
 
 FP64_PEAK_TFLOPS = 78.6
@@ -578,7 +544,7 @@ def many_small(args, lib_mod, hip):
 def fused_large(args, lib_mod, hip):
     """The fused stage executor alone on one large state: an n-qubit brickwork circuit
     (default 26 qubits, 40 layers: a Haar 2x2 on every qubit, then a CNOT brick) from |0>,
-    at register-block widths 3 and 4 with the 13-qubit window, timed with HIP events on the
+    at register-block widths 3 and 4 with the default 12-qubit window, timed with HIP events on the
     launch stream (best of three runs after a warm-up).  Reports the stage count, the state
     traffic (2 x 16 B x 2^n per stage) and the FP64 rate of the fused arithmetic (one 2x2
     complex matrix per qubit per layer: 16 flops per amplitude) against the 78.6 TFLOP/s
@@ -594,7 +560,7 @@ def fused_large(args, lib_mod, hip):
     hstream = C.c_void_p.from_address(stream).value  # the hipStream_t behind the handle
     flops = 16.0 * layers * n * dim
     out = {"workload": f"{n}-qubit brickwork, {layers} layers ({n * layers} Haar 1q + CNOT bricks), from |0>, "
-                       "13-qubit window", "qubits": n, "layers": layers, "gates": len(gates)}
+                       "12-qubit window", "qubits": n, "layers": layers, "gates": len(gates)}
     states = {}
     lib_mod.call("qm_set_synchronous", 0)
     for K in (3, 4):

@@ -345,10 +345,9 @@ QM_EXPORT const double* qm_batch_run_async(qm_batch* batch, void* stream, unsign
  * compiled with keep_states. */
 QM_EXPORT int qm_batch_get_state(qm_batch* batch, UINT index, qm_complex* out, void* stream, unsigned int device_number);
 /* Qubits held in LDS per tile (8..13, default 13); takes effect at the next
- * compile.  A smaller window halves LDS per work-group (two work-groups per CU
- * at 12) and tiles larger circuits. */
+ * compile; 13 runs as 12 (64 KiB tiles, two work-groups per CU). */
 QM_EXPORT int qm_batch_set_local_qubits(qm_batch* batch, UINT local_qubits);
-/* Captures one run (queue reset + the launch) on `stream` (a created stream,
+/* Captures one run (its launches) on `stream` (a created stream,
  * not NULL) into a HIP graph; qm_batch_run_graph replays it.  A compile drops
  * the graph.  The graph holds kernel nodes only. */
 QM_EXPORT int qm_batch_capture(qm_batch* batch, void* stream, unsigned int device_number);
@@ -362,17 +361,17 @@ QM_EXPORT void qm_batch_stats(const qm_batch* batch, ITYPE* circuits, ITYPE* sta
 
 /* ------------------------------------------------------------------ fused circuits
  * One circuit applied in place to an existing state with the batch scheduler:
- * gates are grouped into stages whose qubits fit a window of `local_qubits`
- * (8..13; qubits 0..3 always included), one launch per stage, each work-group
+ * gates are grouped into stages whose dense part fits a window of `local_qubits`
+ * (8..13; qubits 0..2 always included), one launch per stage, each work-group
  * holding 2^local_qubits-amplitude tiles in LDS and applying every gate of the
  * stage to a tile before writing it back.  Replaces QuantumCircuit::update_quantum_state's
  * one launch per gate (src/cppsim/circuit.cpp:46-57) for circuits of 4..40
  * qubits made of the batch gate kinds.  create() does host work only. */
 #define QM_CIRCUIT_MAX_QUBITS 40u
 typedef struct qm_circuit qm_circuit;
-/* block_qubits 2..4, local_qubits 8..13; 0 picks by qubit count (3 and 12 up to
- * 19 qubits, else 4 and 13; the width grows to the largest dense gate, at most
- * 4 qubits); NULL on error. */
+/* block_qubits 2..4, local_qubits 8..13; 0 picks (3 and 12; 4 and 13 for 20 to 22
+ * qubits with at most one dense gate per qubit; the width grows to the largest
+ * dense gate, at most 4 qubits); NULL on error. */
 QM_EXPORT qm_circuit* qm_circuit_create(UINT qubit_count, const qm_batch_gate* gates, UINT gate_count, UINT block_qubits, UINT local_qubits);
 QM_EXPORT void qm_circuit_destroy(qm_circuit* circuit);
 /* Applies the circuit to `state` (dim = 2^qubit_count) in stream order. */
@@ -384,9 +383,9 @@ QM_EXPORT void qm_circuit_stats(const qm_circuit* circuit, ITYPE* stages, ITYPE*
  * on 1..2 qubits) and parametric rotations exp(i coef theta[param] P / 2) with
  * P a Pauli string on 1..4 qubits, for `batch` parameter sets at once.
  * Restates ParametricQuantumCircuit::backprop (src/vqcsim/parametric_circuit.cpp:205-335):
- * gates are grouped into passes over blocks of 3 qubits held in registers; on
- * the way back each pass adds its rotations' gradient terms and applies the
- * inverses to both states. */
+ * consecutive single-qubit gates become one operation, run stage by stage on tiles in LDS;
+ * on the way back each operation's inverse is applied to both states, with the sums that
+ * its rotations' gradients need. */
 #define QM_ADJ_ROT 4u
 typedef struct qm_adjoint_gate {
     UINT kind;                 /* QM_BATCH_DENSE/DIAG/CZ/CNOT (fixed) or QM_ADJ_ROT */
@@ -417,8 +416,8 @@ QM_EXPORT int qm_adjoint_run(qm_adjoint* circuit, UINT batch, const double* thet
  * |0...0> (batch gate kinds), a real-coefficient Pauli observable and uniforms;
  * it returns <H> and the sampled indices (as qm_sampling_host).  Requests are
  * admitted while the sum of 16 * 2^n bytes stays within `hbm_budget_bytes`;
- * requests of up to `small_max_qubits` (<= 16) qubits are batched into one
- * launch, larger ones run on up to `large_slots` streams at once.  No reference
+ * requests of up to `small_max_qubits` (<= 16) qubits are batched together,
+ * larger ones run on up to `large_slots` streams at once.  No reference
  * counterpart (the reference runs one circuit per call, src/cppsim/circuit.cpp:46-57). */
 typedef struct qm_server qm_server;
 QM_EXPORT qm_server* qm_server_create(ITYPE hbm_budget_bytes, UINT large_slots, UINT small_max_qubits, unsigned int device_number);

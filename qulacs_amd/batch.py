@@ -1,6 +1,6 @@
 """Batched circuits on one device: many small circuits, each run from |0...0>
-and reduced to the expectation value of its observable, in one kernel launch
-(the qm_batch_* entry points of libqulacs_mi355).
+and reduced to the expectation value of its observable, together: one launch per
+stage number of the largest circuit (the qm_batch_* entry points of libqulacs_mi355).
 
     b = Batch()
     b.add(n, gates, terms)          # gates: (kind, qubits, matrix); terms: (bf, pf, rot, coef)
@@ -40,7 +40,7 @@ def pauli_masks(targets, paulis):
 
 
 class Batch:
-    """A set of circuits compiled into one launch."""
+    """A set of circuits compiled together."""
 
     def __init__(self, device: int = 0):
         self.device = device

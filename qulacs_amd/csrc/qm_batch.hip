@@ -1,5 +1,5 @@
 // Batched executor: many small circuits, each run from |0...0> and reduced to
-// the expectation value of its observable, in one launch.
+// the expectation value of its observable, together.
 //
 // What it replaces: for each circuit, QuantumCircuit::update_quantum_state
 // (src/cppsim/circuit.cpp:46-57, one kernel launch and synchronisation per gate
@@ -35,7 +35,8 @@
 // barriers), not HBM: a stage of a 26-qubit brickwork circuit takes 1.13 ms of which its 2.1 GB
 // need 0.4 ms.  26 qubits, 10 layers: 9.87 ms with 13 stages of 13-qubit windows picked in
 // gate order and one work-group per CU; 6.55 ms with Picker's 5 stages and two work-groups per
-// CU; 5.64 ms with shears for three quarters of the matrices.  QAOA (4 layers, ring and
+// CU; 5.64 ms with shears for three quarters of the matrices (all but the last on a qubit since, see
+// reduce_matrices: another 6 % at 20 layers).  QAOA (4 layers, ring and
 // chords, 26 qubits): 13.7 -> 10.2 -> 6.0 ms, the last from Z rotations in place of
 // diagonals read per amplitude.  512 circuits of 8 to 16 qubits: 1.75 -> 0.69 ms, from one
 // work-group per tile instead of per circuit.

@@ -15,7 +15,7 @@
 //     kStarveSeconds, after which admission waits for it;
 //   * small requests (n <= small_max_qubits) join the next batch; whenever the
 //     batch stream is idle, every admitted small request is compiled into one
-//     batched-executor launch (states in LDS) followed by one launch that builds
+//     batched-executor run (states in LDS) followed by one launch that builds
 //     every state's exact CDF and searches its uniforms;
 //   * large requests take one of `large_slots` streams: stream-ordered
 //     allocation, |0>, the fused stage executor, the observable, sampling, free;
