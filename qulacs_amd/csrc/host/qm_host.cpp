@@ -1986,7 +1986,7 @@ struct DmLowering {
             for (size_t x = 0; x < d * d; ++x) {
                 const bool agree = y / d == y % d && x / d == x % d;
                 const double want = (y == x ? *keep : 0.0) + (agree ? share : 0.0);
-                if (std::abs(S(y, x) - want) > eps) return false;
+                if (!(std::abs(S(y, x) - want) <= eps)) return false;  // NaN too
             }
         return true;
     }

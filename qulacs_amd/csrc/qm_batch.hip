@@ -39,7 +39,7 @@
 // reduce_matrices: another 6 % at 20 layers).  QAOA (4 layers, ring and
 // chords, 26 qubits): 13.7 -> 10.2 -> 6.0 ms, the last from Z rotations in place of
 // diagonals read per amplitude.  512 circuits of 8 to 16 qubits: 1.75 -> 0.69 ms, from one
-// work-group per tile instead of per circuit.
+// work-group per tile instead of per circuit; 0.60 -> 0.43 from energy_sum.
 #include <cstring>
 
 #include "qm_tile.hpp"
@@ -58,31 +58,73 @@ struct DItem {
 };
 // Circuits above this size run in tiles; a tile is 64 KiB, so two work-groups share a CU.
 constexpr u32 kTileLocal = 12;
-// This thread's share of sum_k c_k Re <psi|P_k|psi> over amplitudes [x0, x1), reading the
-// state from LDS (swizzled slots) or from device memory; threads [0, stride) take part.
-template <bool FROM_LDS>
+// This thread's share of sum_k c_k Re <psi|P_k|psi> over the `len` amplitudes from x0 on (a power
+// of two, aligned), which lie in LDS (swizzled slots); partners beyond them are read from the state in
+// device memory.  Threads [0, stride) take part.  Eight amplitudes at a time, the terms in the inner loop:
+// a term's eight partners are loaded together, where one amplitude at a time waited for each.  The
+// energies of 512 circuits of 8 to 16 qubits (transverse-field Ising chains): those of more than 12
+// qubits 224 us with a partner at a time from device memory, 116 with eight (11 TB/s from L2),
+// 88 with the tile in LDS, and diagonal terms as one sum of signed coefficients per amplitude.
 __device__ __forceinline__ double energy_sum(const double2* __restrict__ gs, const double2* st, const DCirc& c,
-                                             const DTerm* __restrict__ terms, u64 x0, u64 x1, u32 stride) {
+                                             const DTerm* __restrict__ terms, u32 x0, u32 len, u32 stride) {
+    constexpr int P = 8;
     double acc = 0.0;
     if (threadIdx.x >= stride) return acc;
-    for (u64 x = x0 + threadIdx.x; x < x1; x += stride) {
-        const double2 px = FROM_LDS ? st[slot_of((u32)x)] : gs[x];
+    auto signed_by = [](double v, u32 bits) {  // (-1)^popcount(bits) v
+        return __hiloint2double(__double2hiint(v) ^ (int)(__popc(bits) << 31), __double2loint(v));
+    };
+    for (u32 first = threadIdx.x; first < len; first += P * stride) {
+        u32 x[P], slot[P];
+        double2 px[P];
+        double diag[P];  // sum of the diagonal terms' signed coefficients
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            const u32 at = first + (u32)i * stride;
+            x[i] = at < len ? at : 0;  // an amplitude of 0 behind the end
+            slot[i] = slot_of(x[i]);
+            px[i] = st[slot[i]];
+            if (at >= len) px[i] = make_double2(0.0, 0.0);
+            x[i] += x0;
+            diag[i] = 0.0;
+        }
         for (u32 k = 0; k < c.nterm; ++k) {
             const DTerm tm = terms[c.term0 + k];
-            const u64 y = x ^ tm.bf;
-            const double2 py = FROM_LDS ? st[slot_of((u32)y)] : gs[y];  // y == x when bf == 0
-            // psi_x * conj(psi_y) * i^rot * (-1)^popcount(x & pf)
-            const double re0 = px.x * py.x + px.y * py.y, im0 = px.y * py.x - px.x * py.y;
-            double re;
-            switch (tm.rot & 3u) {
-                case 0: re = re0; break;
-                case 1: re = -im0; break;
-                case 2: re = -re0; break;
-                default: re = im0; break;
+            const u32 bf = (u32)tm.bf, pf = (u32)tm.pf;
+            // Re(z i^rot): z.x, -z.y, -z.x, z.y with z = psi_x conj(psi_y)
+            const double coef = ((tm.rot + 1u) & 2u) ? -tm.coef : tm.coef;
+            if (bf == 0) {
+                if (tm.rot & 1u) continue;  // the imaginary part of |psi_x|^2
+#pragma unroll
+                for (int i = 0; i < P; ++i) diag[i] += signed_by(coef, x[i] & pf);
+                continue;
             }
-            if (__popcll(x & tm.pf) & 1) re = -re;
-            acc = fma(tm.coef, re, acc);
+            double2 py[P];
+            if (bf < len) {
+                const u32 sb = slot_of(bf);
+#pragma unroll
+                for (int i = 0; i < P; ++i) py[i] = st[slot[i] ^ sb];
+            } else {
+#pragma unroll
+                for (int i = 0; i < P; ++i) py[i] = gs[x[i] ^ bf];
+            }
+            if (tm.rot & 1u) {
+#pragma unroll
+                for (int i = 0; i < P; ++i) py[i] = make_double2(-py[i].y, py[i].x);
+            }
+            if (pf) {
+#pragma unroll
+                for (int i = 0; i < P; ++i) {
+                    py[i].x = signed_by(py[i].x, x[i] & pf);
+                    py[i].y = signed_by(py[i].y, x[i] & pf);
+                }
+            }
+            double sum = 0.0;
+#pragma unroll
+            for (int i = 0; i < P; ++i) sum = fma(px[i].x, py[i].x, fma(px[i].y, py[i].y, sum));
+            acc = fma(coef, sum, acc);
         }
+#pragma unroll
+        for (int i = 0; i < P; ++i) acc = fma(diag[i], fma(px[i].x, px[i].x, px[i].y * px[i].y), acc);
     }
     return acc;
 }
@@ -131,22 +173,25 @@ __global__ __launch_bounds__(tile_threads<K>(), K == 4 ? 2 : 4) void k_batch_lev
         for (u32 i = tid; i < L; i += bd) gs[i] = st[slot_of(i)];
     // a thread count that depends on the circuit alone: its energy does not depend on the batch
     const u32 part = min(tile_threads<K>(), max(64u, L >> K));
-    const double total = block_sum(energy_sum<true>(gs, st, c, terms, 0, L, part), red);
+    const double total = block_sum(energy_sum(gs, st, c, terms, 0, L, part), red);
     if (tid == 0) energies[it.circ] = total;
 }
 
 // Energies of the circuits of several tiles: partial sums over 2^12 amplitudes, then one thread per
 // circuit adds them in order.
-__global__ __launch_bounds__(256) void k_batch_energy(const DCirc* __restrict__ circs, const DTerm* __restrict__ terms,
+constexpr u32 kEnergyThreads = 512;
+__global__ __launch_bounds__(kEnergyThreads) void k_batch_energy(const DCirc* __restrict__ circs, const DTerm* __restrict__ terms,
                                                       const DItem* __restrict__ items, const double2* __restrict__ scratch,
                                                       double* __restrict__ partials) {
+    extern __shared__ double2 st[];
     __shared__ double red[16];
     const DItem it = items[blockIdx.x];
     const DCirc c = circs[it.circ];
-    const u64 x0 = (u64)it.tile << kTileLocal;
-    const u64 x1 = x0 + (1ULL << kTileLocal), dim = 1ULL << c.n;
-    const double total =
-        block_sum(energy_sum<false>(scratch + c.state_off, nullptr, c, terms, x0, x1 < dim ? x1 : dim, 256), red);
+    const u32 x0 = it.tile << kTileLocal, len = 1u << min(c.n, kTileLocal);
+    const double2* gs = scratch + c.state_off;
+    for (u32 i = threadIdx.x; i < len; i += kEnergyThreads) st[slot_of(i)] = gs[x0 + i];
+    __syncthreads();
+    const double total = block_sum(energy_sum(gs, st, c, terms, x0, len, kEnergyThreads), red);
     if (threadIdx.x == 0) partials[c.chunk0 + it.tile] = total;
 }
 __global__ __launch_bounds__(64) void k_batch_finish(const DCirc* __restrict__ circs, const u32* __restrict__ large,
@@ -416,6 +461,9 @@ bool batch_prepare_launch(qm_batch* b, const char* what) {
                      : b->K == 3 ? (const void*)k_batch_level<3>
                                  : (const void*)k_batch_level<4>;
     if (!hip_ok(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(sizeof(double2) << kTileLocal)),
+                what) ||
+        !hip_ok(hipFuncSetAttribute((const void*)k_batch_energy, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)(sizeof(double2) << kTileLocal)),
                 what))
         return false;
     b->lds_set = true;
@@ -643,7 +691,7 @@ const double* qm_batch_run_async(qm_batch* b, void* stream, unsigned dev) {
 #undef QM_BATCH_LEVEL
     }
     if (b->n_large) {
-        k_batch_energy<<<b->energy_items.count, 256, 0, st>>>(b->d_circs, b->d_terms, b->d_items + b->energy_items.first,
+        k_batch_energy<<<b->energy_items.count, kEnergyThreads, sizeof(double2) << kTileLocal, st>>>(b->d_circs, b->d_terms, b->d_items + b->energy_items.first,
                                                              b->d_scratch, b->d_partials);
         k_batch_finish<<<(b->n_large + 63) / 64, 64, 0, st>>>(b->d_circs, b->d_large, b->n_large, b->d_partials,
                                                               b->d_energies);
