@@ -156,7 +156,7 @@ __global__ __launch_bounds__(tile_threads<K>(), K == 4 ? 2 : 4) void k_batch_lev
         build_hi_tab(hi_tab, lq, sg);
         __syncthreads();
     }
-    warm_program(passes[sg.pass0], subs, pool);
+    if (sg.npass) warm_program(passes[sg.pass0], subs, pool);  // a circuit without gates has no pass to read
     if (level == 0) {
         // |0...0>: slot_of(0) == 0 and amplitude 0 lies in tile 0
         for (u32 i = tid; i < L; i += bd) st[i] = make_double2((i == 0 && it.tile == 0) ? 1.0 : 0.0, 0.0);

@@ -55,6 +55,29 @@ def test_empty_and_trivial_circuits(oracle):
     assert e[0] == 0.5 and e[1] == 1.0 and e[2] == 0.0
 
 
+def test_circuit_without_gates_behind_a_full_pass_table(oracle):
+    """The stage of a circuit without gates has no pass.  As the last circuit of a batch its first
+    pass would be the one behind the table; with a multiple of 8 passes (32 bytes each, tables
+    256-byte aligned) those bytes are the first sub-operation, here one with a CZ to a qubit
+    outside the window."""
+    n = 13
+    gates = []
+    for k in range(3):
+        gates += [("CZ", [q, (q + 1) % n], None) for q in range(n)]
+        for q in range(n):
+            a = 0.15 + 0.05 * q + 0.5 * k
+            gates.append(("dense", [q], np.array([[np.cos(a), -np.sin(a)], [np.sin(a), np.cos(a)]])))
+    circuits = [(n, gates, [(0, 1, 0, 1.0), (3, 4, 0, 0.5)]), (5, [], [(0, 16, 0, 0.75)]), (14, [], [(0, 1, 0, 0.25)])]
+    b = Batch()
+    for c in circuits:
+        b.add(*c)
+    b.compile(block_qubits=4, keep_states=True)
+    assert b.stats()["passes"] % 8 == 0 and b.stats()["passes"] > 0
+    e = _check(oracle, b, circuits)
+    assert e[1] == 0.75 and e[2] == 0.25
+    b.close()
+
+
 def test_many_small_circuits_workload_subset(oracle):
     cs = many_small_circuits(48, seed=77, n_range=(8, 16), layer_range=(2, 5))
     b = Batch()
