@@ -1095,7 +1095,8 @@ u32 schedule_circuit(Flat& f, const HCirc& c, u32 K, u32 lq_cap = kMaxLocal, siz
 //     the CZ: both exact, where 1/sqrt(2) twice would change the norm by 1.4e-16 per CNOT.
 //   * A diagonal gate with entries of modulus 1 is a product of exp(i phi Z...Z) over subsets of
 //     its qubits: phases on single qubits wait as above, the others become ZROT when they
-//     are few (a two-qubit gate has one), else the gate stays a DIAG.
+//     are few (a two-qubit gate has one), else the gate stays a DIAG.  Moduli that differ from 1
+//     by more than rounding are kept (see diagonal).
 struct Converter {
     HCirc& c;
     std::vector<long> last;        // last operation that touches each qubit
@@ -1177,22 +1178,38 @@ struct Converter {
         bool unit = true;
         for (u32 i = 0; i < d && unit; ++i) unit = std::abs(std::abs(m[i]) - 1.0) < 1e-14;
         if (unit) {
-            long double phi[16];
-            for (u32 i = 0; i < d; ++i) phi[i] = std::arg(m[i]);
-            for (u32 h = 1; h < d; h <<= 1)  // phi[s] <- sum_i (-1)^popcount(i & s) arg m_i
+            // log m_i = sum_s (-1)^popcount(i & s) (rho[s] + i phi[s]) / d.  What a double's rounding
+            // leaves of the moduli (2^-53) may go; more of it is kept: rho of all and of single
+            // qubits in the phases that wait, of more qubits by leaving the gate a DIAG.
+            long double phi[16], rho[16];
+            for (u32 i = 0; i < d; ++i) {
+                phi[i] = std::arg(m[i]);
+                rho[i] = std::log(std::abs(m[i]));
+            }
+            for (u32 h = 1; h < d; h <<= 1)
                 for (u32 i = 0; i < d; ++i)
-                    if (!(i & h)) {
-                        const long double a = phi[i], b = phi[i | h];
-                        phi[i] = a + b;
-                        phi[i | h] = a - b;
-                    }
+                    if (!(i & h))
+                        for (long double* x : {phi, rho}) {
+                            const long double a = x[i], b = x[i | h];
+                            x[i] = a + b;
+                            x[i | h] = a - b;
+                        }
             u32 many = 0;
-            for (u32 s = 1; s < d; ++s) many += (s & (s - 1)) && std::abs(phi[s]) > 1e-15;
-            if (many <= 2) {
-                const cx g = std::polar(1.0L, phi[0] / d);
+            bool kept = true;
+            for (u32 s = 0; s < d; ++s) {
+                if (std::abs(rho[s]) <= d * 0x1p-53L) rho[s] = 0.0L;
+                if (!(s & (s - 1))) continue;
+                many += std::abs(phi[s]) > 1e-15;
+                kept = kept && rho[s] == 0.0L;
+            }
+            if (many <= 2 && kept) {
+                const cx g = std::polar(std::exp(rho[0] / d), phi[0] / d);
                 phase(q[0], g, g);
-                for (u32 s = 1; s < d; ++s)
-                    if (std::abs(phi[s]) > 1e-15) zrot(subset(s), std::polar(1.0L, phi[s] / d));
+                for (u32 s = 1; s < d; ++s) {
+                    if (std::abs(phi[s]) <= 1e-15 && rho[s] == 0.0L) continue;
+                    if (s & (s - 1)) zrot(subset(s), std::polar(1.0L, phi[s] / d));
+                    else phase(q[__builtin_ctz(s)], std::polar(std::exp(rho[s] / d), phi[s] / d), std::polar(std::exp(-rho[s] / d), -phi[s] / d));
+                }
                 return;
             }
         }

@@ -98,6 +98,35 @@ def test_fused_circuit(n, count, style, block, window):
     assert err <= 4 * (count + 1) * 2.0 ** -53
 
 
+@pytest.mark.parametrize("k", [2, 3])
+@pytest.mark.parametrize("moduli", ["common", "per qubit", "any"])
+def test_diagonal_moduli_near_one(moduli, k):
+    """Diagonal entries a few ten units of the last place off the unit circle are applied as given:
+    20 gates of modulus 1 + 9e-15 are 1.8e-13 away from 20 phases."""
+    rng = np.random.default_rng(5 * k + len(moduli))
+    n = 13
+    gates = [("dense", [t], haar_unitary(rng, 1)) for t in range(0, n, 2)]
+    for i in range(20):
+        q = [int(t) for t in rng.choice(n, k, replace=False)]
+        bits = (np.arange(1 << k)[:, None] >> np.arange(k)) & 1
+        r = {"common": 9e-15 + 0 * bits[:, 0], "per qubit": 4e-15 + 4e-15 * bits[:, 0],
+             "any": rng.uniform(0, 9e-15, 1 << k)}[moduli]
+        # phases of one Z string beside those of single qubits, so that the gate may become a ZROT
+        phase = bits @ rng.uniform(0, 2, k) + (1 - 2 * (bits[:, 0] ^ bits[:, 1])) * rng.uniform(0, 2)
+        gates.append(("diag", q, (1 + r) * np.exp(1j * phase)))
+    psi = _random_state(rng, n)
+    fc = FusedCircuit(n, gates)
+    with DevState.from_host(psi) as s:
+        fc.apply(s.ptr)
+        got = s.download()
+    fc.close()
+    for g in gates:
+        psi = _apply(psi, n, *g)
+    err = np.linalg.norm(got - psi) / np.linalg.norm(psi)
+    print(moduli, k, err, flush=True)
+    assert err <= 4 * (len(gates) + 1) * 2.0 ** -53
+
+
 @pytest.mark.parametrize("style", ["chain", "phases", "all"])
 def test_batch_of_uneven_circuits(style):
     """Sizes on both sides of one tile together; each circuit's energy and state, and the
