@@ -535,6 +535,12 @@ int batch_add_prepared(qm_batch* b, PreparedCircuit* c) {
     delete c;
     return (int)b->circs.size() - 1;
 }
+u32 batch_prepared_width(const PreparedCircuit* c) {
+    size_t most = 0;
+    for (const HOp& o : c->c.ops)
+        if (o.type == 0) most = std::max(most, o.q.size());
+    return (u32)most;
+}
 void batch_destroy_prepared(PreparedCircuit* c) { delete c; }
 }  // namespace qm
 

@@ -246,6 +246,7 @@ struct PreparedCircuit;
 PreparedCircuit* batch_prepare_circuit(UINT n, const qm_batch_gate* gates, UINT gate_count, const ITYPE* bf,
                                        const ITYPE* pf, const UINT* rot, const double* coefs, UINT term_count);
 int batch_add_prepared(qm_batch* b, PreparedCircuit* c);
+u32 batch_prepared_width(const PreparedCircuit* c);  // qubits of its widest dense operation
 void batch_destroy_prepared(PreparedCircuit* c);
 // Many small state vectors (dim <= 2^16 each), one work-group per CDF.
 struct SampleJob {

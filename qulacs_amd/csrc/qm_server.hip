@@ -14,7 +14,8 @@
 //     does not fit lets later, smaller ones pass until it has waited
 //     kStarveSeconds, after which admission waits for it;
 //   * small requests (n <= small_max_qubits) join the next batch; whenever the
-//     batch stream is idle, every admitted small request is compiled into one
+//     batch stream is idle, every admitted small request (with a dense gate on four
+//     qubits, or every one without) is compiled into one
 //     batched-executor run (states in LDS) followed by one launch that builds
 //     every state's exact CDF and searches its uniforms;
 //   * large requests take one of `large_slots` streams: stream-ordered
@@ -57,6 +58,7 @@ struct Request {
     std::vector<double> coef;
     std::vector<double> uniforms;
     PreparedCircuit* prepared = nullptr;  // small requests until they join a batch: converted once, by the submitter
+    u32 block = 0;                        // small requests: block width of the batch that can run it
     qm_circuit* circuit = nullptr;        // large requests
     bool small = false;
     u64 bytes = 0;
@@ -203,6 +205,16 @@ void qm_server::launch_large(Slot& s, const ReqPtr& r) {
 void qm_server::launch_batch() {
     std::string err;
     qm_batch_clear(batch);
+    // A batch has one block width: the requests of the first one's, the others wait for the next
+    // batch (a dense gate on four qubits needs blocks of four; in those every other request would take
+    // another schedule than it does alone).
+    const u32 block = next_batch.front()->block;
+    std::vector<ReqPtr> later;
+    {
+        std::vector<ReqPtr> now;
+        for (const ReqPtr& r : next_batch) (r->block == block ? now : later).push_back(r);
+        next_batch.swap(now);
+    }
     size_t total = 0;
     for (const ReqPtr& r : next_batch) {
         batch_add_prepared(batch, r->prepared);
@@ -210,7 +222,7 @@ void qm_server::launch_batch() {
         total += r->uniforms.size();
     }
     const size_t nb = next_batch.size();
-    bool ok = err.empty() && qm_batch_compile(batch, kBatchBlockQubits, 1, device) == QM_OK &&
+    bool ok = err.empty() && qm_batch_compile(batch, block, 1, device) == QM_OK &&
               benergy.reserve(nb * sizeof(double)) && bsamples.reserve(total * 8 + 8) &&
               buniforms.reserve(total * 8 + 8) && bflags.reserve(total + 8);
     const double* d_energy = nullptr;
@@ -239,7 +251,7 @@ void qm_server::launch_batch() {
     }
     if (!ok && err.empty()) err = take_error();
     running_batch.swap(next_batch);
-    next_batch.clear();
+    next_batch.swap(later);
     {
         std::lock_guard<std::mutex> lk(mu);
         ++n_batches;
@@ -425,6 +437,7 @@ long long qm_server_submit(qm_server* s, UINT n, const qm_batch_gate* gates, UIN
     if (r->small) {
         r->prepared = batch_prepare_circuit(n, gates, gate_count, bf, pf, rot, coefs, term_count);
         if (!r->prepared) return -1;
+        r->block = std::max(kBatchBlockQubits, batch_prepared_width(r->prepared));
     } else {
         r->circuit = qm_circuit_create(n, gates, gate_count, 0, 0);
         // the program goes to the device here, in the submitting thread, so the

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from qulacs_amd.serving import Server
-from qulacs_amd.workloads import serving_requests
+from qulacs_amd.workloads import haar_unitary, serving_requests
 from tests.batch_util import oracle_run
 
 pytestmark = pytest.mark.gpu
@@ -63,6 +63,28 @@ def test_admission_respects_budget_and_threads_submit():
     print("stats", st, flush=True)
     assert len(out) == len(rs) and st["failed"] == 0
     assert st["peak_bytes"] <= budget
+
+
+def test_four_qubit_gates_beside_ordinary_requests(oracle):
+    """A dense gate on four qubits needs another block width than the other small requests: all
+    succeed, and the others' results are those of a server without it."""
+    rs = serving_requests(12, rate=1000.0, seed=21, n_range=(5, 14), depth_range=(2, 5), samples=40)
+    rng = np.random.default_rng(3)
+    for k, n in ((2, 4), (5, 9), (9, 14)):
+        q = [int(t) for t in rng.choice(n, 4, replace=False)]
+        rs[k].n = n
+        rs[k].gates = [("dense", [t], haar_unitary(rng, 1)) for t in range(n)] + [("dense", q, haar_unitary(rng, 4))]
+        rs[k].terms = [(1, 1 << (n - 1), 0, 0.5), (0, 6, 0, 1.5)]
+    with Server(hbm_budget_bytes=1 << 33, large_slots=1, small_max_qubits=16) as srv:
+        got = _run_all(srv, rs)
+        assert srv.stats()["failed"] == 0
+    with Server(hbm_budget_bytes=1 << 33, large_slots=1, small_max_qubits=16) as srv:
+        plain = _run_all(srv, [r for k, r in enumerate(rs) if k not in (2, 5, 9)])
+    assert [g[0] for k, g in enumerate(got) if k not in (2, 5, 9)] == [p[0] for p in plain]
+    for r, (e, smp, _) in zip(rs, got):
+        psi, want = oracle_run(oracle, r.n, r.gates, r.terms)
+        assert abs(e - want) < 1e-10 * max(1.0, sum(abs(t[3]) for t in r.terms)), r.n
+        assert np.array_equal(smp, oracle.sampling(psi, r.uniforms)), r.n
 
 
 def test_invalid_requests_rejected():
