@@ -434,6 +434,11 @@ long long qm_server_submit(qm_server* s, UINT n, const qm_batch_gate* gates, UIN
             set_error(QM_ERR_INVALID_ARGUMENT, "%s: term %u acts beyond %u qubits", what, t, n);
             return -1;
         }
+    for (UINT i = 0; i < gate_count; ++i)  // a request's state is a vector: no QM_BATCH_DEPOL
+        if (gates[i].kind > QM_BATCH_CNOT) {
+            set_error(QM_ERR_INVALID_ARGUMENT, "%s: gate %u: kind %u is not supported", what, i, gates[i].kind);
+            return -1;
+        }
     if (r->small) {
         r->prepared = batch_prepare_circuit(n, gates, gate_count, bf, pf, rot, coefs, term_count);
         if (!r->prepared) return -1;

@@ -4,6 +4,7 @@ identical for the same uniforms), and admission keeps the footprint within the
 budget."""
 from __future__ import annotations
 
+import ctypes as C
 import threading
 
 import numpy as np
@@ -97,3 +98,21 @@ def test_invalid_requests_rejected():
             srv.submit(5, [("dense", [7], np.eye(2))], [], [0.5])
         e, s, _ = srv.wait(srv.submit(5, [], [(0, 1, 0, 2.0)], [0.25, 0.75]))
         assert e == 2.0 and list(s) == [0, 0]
+
+
+@pytest.mark.parametrize("n", [6, 17])
+def test_density_matrix_gates_rejected(n):
+    """QM_BATCH_DEPOL belongs to qm_circuit_create on density matrices: a request, batched (6 qubits)
+    or alone (17), has a state vector."""
+    from qulacs_amd import _lib
+
+    z = (_lib.QmComplex * 1)(_lib.QmComplex(0.9, 0.05))
+    g = (_lib.QmBatchGate * 1)()
+    g[0].kind, g[0].qubit_count, g[0].matrix = _lib.BATCH_DEPOL, 2, z
+    g[0].qubits[0], g[0].qubits[1] = 0, 3
+    none = (C.c_ulonglong * 1)()
+    with Server(hbm_budget_bytes=1 << 30, large_slots=1, small_max_qubits=16) as srv:
+        with pytest.raises(_lib.QulacsMI355Error):
+            _lib.call("qm_server_submit", srv.h, n, g, 1, none, none, (C.c_uint * 1)(), (C.c_double * 1)(), 0,
+                      (C.c_double * 1)(0.5), 1)
+        assert srv.stats()["admitted"] == 0
