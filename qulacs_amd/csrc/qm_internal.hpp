@@ -223,8 +223,7 @@ void monomial_any(const u32* targets, u32 nt, const qm_complex* matrix, void* st
 
 // state <- |basis> (qm_runtime.hip)
 void enqueue_basis(void* state, u64 dim, u64 basis, hipStream_t st);
-// sum_k coef_k <P_k>: two partial totals (re, im) are written to h_out[0..1] and h_out[2..3]
-// (pinned memory); the caller adds the two.
+// sum_k coef_k <P_k> (re, im), at most 2^16 terms, to h_out[0..1] (pinned memory).
 // (qm_reduce.hip)
 bool enqueue_observable(const u64* bf, const u64* pf, const u32* rot, const double* coef, u32 nterms,
                         const void* state, u64 dim, hipStream_t st, double* h_out);

@@ -9,6 +9,7 @@
 // stat_ops_transition_amplitude.cpp:19-128, update_ops_named_state.cpp:21-98.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 
 #include "qm_internal.hpp"
 
@@ -143,10 +144,10 @@ __global__ __launch_bounds__(kRBlock) void k_reduce(RArgs r) {
 
 // Sums `count` (re, im) pairs of partials in a fixed order (thread-strided, then a fixed tree)
 // into out, which may be pinned host memory: a copy command for 16 bytes costs more than the
-// kernel.
+// kernel.  add: onto what an earlier launch of the stream left there.
 constexpr int kFinishThreads = 256;
 __global__ __launch_bounds__(kFinishThreads) void k_finish(const double* __restrict__ partials, unsigned count,
-                                                           double* __restrict__ out) {
+                                                           double* __restrict__ out, bool add = false) {
     __shared__ double lds[32];
     double re = 0.0, im = 0.0;
     for (unsigned k = threadIdx.x; k < count; k += kFinishThreads) {
@@ -156,8 +157,8 @@ __global__ __launch_bounds__(kFinishThreads) void k_finish(const double* __restr
     re = block_sum(re, lds);
     im = block_sum(im, lds);
     if (threadIdx.x == 0) {
-        out[0] = re;
-        out[1] = im;
+        out[0] = add ? out[0] + re : re;
+        out[1] = add ? out[1] + im : im;
     }
 }
 
@@ -195,7 +196,8 @@ bool run_reduce(RArgs r, u64 work, const Term* term, hipStream_t st, double res[
 constexpr int kObsRank = 4;
 constexpr int kObsMembers = 1 << kObsRank;
 constexpr unsigned kObsInlineTerms = 48, kObsInlineGroups = 16;  // passed as kernel arguments
-constexpr unsigned kObsMaxBlocks = 2048, kObsMaxGroups = 256;   // per launch
+constexpr unsigned kObsMaxBlocks = 2048, kObsMaxGroups = 256;   // per launch: the partials hold this many pairs
+constexpr unsigned kObsMaxTerms = 1u << 16;                      // of a call that does not wait: the upload ring takes their tables
 constexpr u64 kObsOneBlock = 1ULL << 13;                         // states up to here: one block does all
 
 struct ObsTerm {
@@ -405,10 +407,12 @@ unsigned obs_blocks(u64 dim) {
     return dim <= kObsOneBlock ? 1u : (unsigned)std::min<u64>(kObsMaxBlocks, (dim / kObsMembers + kRBlock - 1) / kRBlock);
 }
 
-// Enqueues the groups [g0, g0 + ng) of a plan; their sum goes to out (device or pinned memory).
-// `tables` holds the terms and groups in device memory when they are too many for the arguments.
+// Enqueues the groups [g0, g0 + ng) of a plan; their sum goes to out (device or pinned memory),
+// added to what is there if `add`.
+// dterms and dgroups hold the terms and groups in device memory when they are too many for the arguments.
 bool launch_observable(const ObsPlan& pl, size_t g0, size_t ng, const void* state, u64 dim, hipStream_t st,
-                       double* partials, const ObsTerm* dterms, const ObsGroup* dgroups, double* out, const char* what) {
+                       double* partials, const ObsTerm* dterms, const ObsGroup* dgroups, double* out, const char* what,
+                       bool add = false) {
     ObsArgs a{};
     a.state = (const double2*)state;
     a.dim = dim;
@@ -418,7 +422,7 @@ bool launch_observable(const ObsPlan& pl, size_t g0, size_t ng, const void* stat
     a.groups = dgroups ? dgroups + g0 : nullptr;
     const unsigned nb = obs_blocks(dim);
     const unsigned ny = nb == 1 ? 1u : (unsigned)ng;
-    a.out = nb * ny == 1 ? out : nullptr;
+    a.out = nb * ny == 1 && !add ? out : nullptr;
     if (!dterms) {
         std::copy(pl.terms.begin(), pl.terms.end(), a.term);
         std::copy(pl.groups.begin(), pl.groups.end(), a.group);
@@ -426,39 +430,47 @@ bool launch_observable(const ObsPlan& pl, size_t g0, size_t ng, const void* stat
     } else {
         k_observable<false><<<dim3(nb, ny), kRBlock, 0, st>>>(a);
     }
-    if (nb * ny > 1) k_finish<<<1, kFinishThreads, 0, st>>>(partials, nb * ny, out);
+    if (!a.out) k_finish<<<1, kFinishThreads, 0, st>>>(partials, nb * ny, out, add);
     return hip_ok(hipGetLastError(), what);
 }
 bool obs_inline(const ObsPlan& pl) {
     return pl.terms.size() <= kObsInlineTerms && pl.groups.size() <= kObsInlineGroups;
 }
 
+// The tables of a plan that the kernel arguments do not hold, in one copy.
+bool upload_plan(Scratch* sc, const ObsPlan& pl, const ObsTerm** dterms, const ObsGroup** dgroups) {
+    const size_t nt = pl.terms.size() * sizeof(ObsTerm), ng = pl.groups.size() * sizeof(ObsGroup);
+    std::vector<char> host(nt + ng);
+    std::memcpy(host.data(), pl.terms.data(), nt);
+    std::memcpy(host.data() + nt, pl.groups.data(), ng);
+    const char* d = (const char*)upload(sc, host.data(), host.size());
+    if (!d) return false;
+    *dterms = (const ObsTerm*)d;
+    *dgroups = (const ObsGroup*)(d + nt);
+    return true;
+}
+static_assert(kObsMaxTerms * (sizeof(ObsTerm) + sizeof(ObsGroup)) <= kRingBytes, "the ring takes a plan's tables");
+
 bool enqueue_observable(const u64* bf, const u64* pf, const u32* rot, const double* coef, u32 nterms,
                         const void* state, u64 dim, hipStream_t st, double* h_out) {
-    for (int i = 0; i < 4; ++i) h_out[i] = 0.0;
+    const char* what = "enqueue_observable";
+    h_out[0] = h_out[1] = 0.0;
     if (nterms == 0) return true;
+    if (nterms > kObsMaxTerms) {
+        set_error(QM_ERR_UNSUPPORTED, "%s: too many terms in one observable (%u)", what, nterms);
+        return false;
+    }
     std::vector<qm_complex> c(nterms);
     for (u32 k = 0; k < nterms; ++k) c[k] = qm_complex{coef[k], 0.0};
     const ObsPlan pl = plan_observable(bf, pf, rot, c.data(), nterms, log2_dim(dim));
     Scratch* sc = scratch_for(st);
     if (!sc) return false;
-    const char* what = "enqueue_observable";
     const ObsTerm* dt = nullptr;
     const ObsGroup* dg = nullptr;
-    if (!obs_inline(pl)) {
-        dt = (const ObsTerm*)upload(sc, pl.terms.data(), pl.terms.size() * sizeof(ObsTerm));
-        dg = (const ObsGroup*)upload(sc, pl.groups.data(), pl.groups.size() * sizeof(ObsGroup));
-        if (!dt || !dg) return false;
-    }
-    // the last (usually only) launch's sum goes to the caller's pinned buffer; more than
-    // kObsMaxGroups groups add up in pairs there
-    if (pl.groups.size() > 2 * kObsMaxGroups) {
-        set_error(QM_ERR_UNSUPPORTED, "%s: too many terms in one observable (%u)", what, nterms);
-        return false;
-    }
+    if (!obs_inline(pl) && !upload_plan(sc, pl, &dt, &dg)) return false;
     for (size_t g = 0; g < pl.groups.size(); g += kObsMaxGroups)
         if (!launch_observable(pl, g, std::min<size_t>(kObsMaxGroups, pl.groups.size() - g), state, dim, st, sc->partials,
-                               dt, dg, h_out + (g ? 2 : 0), what))
+                               dt, dg, h_out, what, g > 0))
             return false;
     return true;
 }
@@ -785,11 +797,7 @@ qm_complex qm_observable_expectation_host(const ITYPE* bfs, const ITYPE* pfs, co
         const ObsPlan pl = plan_observable(bfs + off, pfs + off, rots + off, coefs + off, cnt, n);
         const ObsTerm* dt = nullptr;
         const ObsGroup* dg = nullptr;
-        if (!obs_inline(pl)) {
-            dt = (const ObsTerm*)upload(sc, pl.terms.data(), pl.terms.size() * sizeof(ObsTerm));
-            dg = (const ObsGroup*)upload(sc, pl.groups.data(), pl.groups.size() * sizeof(ObsGroup));
-            if (!dt || !dg) return z;
-        }
+        if (!obs_inline(pl) && !upload_plan(sc, pl, &dt, &dg)) return z;
         for (size_t g = 0; g < pl.groups.size(); g += kObsMaxGroups) {
             if (!launch_observable(pl, g, std::min<size_t>(kObsMaxGroups, pl.groups.size() - g), state, dim, st,
                                    sc->partials, dt, dg, sc->host_result, what) ||

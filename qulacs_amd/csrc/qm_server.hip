@@ -173,7 +173,7 @@ void qm_server::launch_large(Slot& s, const ReqPtr& r) {
     // One stream-ordered allocation holds the state and the sampling CDF with
     // its tables: r->bytes, the amount admission counted for this request.
     void* mem = nullptr;
-    bool ok = s.energy.reserve(4 * sizeof(double)) && s.samples.reserve((size_t)count * 8 + 8) &&
+    bool ok = s.energy.reserve(2 * sizeof(double)) && s.samples.reserve((size_t)count * 8 + 8) &&
               s.uniforms.reserve((size_t)count * 8 + 8) && s.flags.reserve((size_t)count + 8);
     if (ok) {
         std::memcpy(s.uniforms.p, r->uniforms.data(), (size_t)count * 8);
@@ -304,8 +304,7 @@ void qm_server::run() {
             s.req.reset();
             const bool ok = q == hipSuccess && r->error.empty();
             if (ok) {
-                const double* e = (const double*)s.energy.p;
-                r->energy = e[0] + e[2];
+                r->energy = ((const double*)s.energy.p)[0];
                 r->samples.assign((const u64*)s.samples.p, (const u64*)s.samples.p + r->uniforms.size());
                 r->flags.assign((const unsigned char*)s.flags.p,
                                 (const unsigned char*)s.flags.p + r->uniforms.size());

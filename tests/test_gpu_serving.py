@@ -10,6 +10,7 @@ import threading
 import numpy as np
 import pytest
 
+from qulacs_amd.batch import pauli_masks
 from qulacs_amd.serving import Server
 from qulacs_amd.workloads import haar_unitary, serving_requests
 from tests.batch_util import oracle_run
@@ -86,6 +87,35 @@ def test_four_qubit_gates_beside_ordinary_requests(oracle):
         psi, want = oracle_run(oracle, r.n, r.gates, r.terms)
         assert abs(e - want) < 1e-10 * max(1.0, sum(abs(t[3]) for t in r.terms)), r.n
         assert np.array_equal(smp, oracle.sampling(psi, r.uniforms)), r.n
+
+
+@pytest.mark.parametrize("n,count", [(17, 3000), (18, 5000), (20, 4000)])
+def test_observables_of_thousands_of_terms(n, count):
+    """More flip masks than one launch's groups take.  A product state, whose Pauli strings have
+    products as expectation values.  Tolerance: each string's value is exact to a few roundings per
+    qubit and amplitude sum, |d| <= 2^-53 * 8 n * sum |c_k|."""
+    rng = np.random.default_rng(n)
+    gates, bloch = [], []
+    for t in range(n):
+        u = haar_unitary(rng, 1)
+        gates.append(("dense", [t], u))
+        a, b = u[0, 0], u[1, 0]
+        bloch.append([1.0, 2 * (np.conj(a) * b).real, 2 * (np.conj(a) * b).imag, abs(a) ** 2 - abs(b) ** 2])
+    terms, want, scale = [], 0.0, 0.0
+    for _ in range(count):
+        p = np.where(rng.random(n) < 0.5, rng.integers(0, 4, n), 0)
+        c = float(rng.standard_normal())
+        terms.append((*pauli_masks(range(n), [int(x) for x in p]), c))
+        want += c * np.prod([bloch[t][p[t]] for t in range(n)])
+        scale += abs(c)
+    with Server(hbm_budget_bytes=1 << 30, large_slots=1, small_max_qubits=16) as srv:
+        e, _, _ = srv.wait(srv.submit(n, gates, terms, [0.5]))
+        few, _, _ = srv.wait(srv.submit(n, gates, terms[:1], [0.5]))
+    print(n, e - want, scale, flush=True)
+    assert abs(e - want) <= 2.0 ** -53 * 8 * n * scale
+    k = terms[0]
+    assert abs(few - k[3] * np.prod([bloch[t][(2 if k[1] >> t & 1 else 1) if k[0] >> t & 1 else 3 * (k[1] >> t & 1)]
+                                     for t in range(n)])) <= 2.0 ** -53 * 8 * n * abs(k[3])
 
 
 def test_invalid_requests_rejected():
