@@ -191,14 +191,16 @@ bool run_reduce(RArgs r, u64 work, const Term* term, hipStream_t st, double res[
 // are numbered by the index bits that are no pivots, and member m is base ^ (sum of the
 // basis vectors in m); a term is the pairs (m, m ^ e), e = its mask's pivot bits, with the
 // sign (-1)^popcount(index & pf) = (lane: base & pf) x (uniform: bit m of a 16-bit pattern).
-// Bound: HBM.  25 qubits, 24 random terms: 24 passes, 1.91 ms; with 6 groups 0.51 ms (6.3 TB/s).  One block for all up
-// to 2^13 amplitudes, which needs no second launch.
+// Bound: HBM.  25 qubits, 24 random terms: 24 passes, 1.91 ms; with 6 groups 0.51 ms (6.3 TB/s).
 constexpr int kObsRank = 4;
 constexpr int kObsMembers = 1 << kObsRank;
 constexpr unsigned kObsInlineTerms = 48, kObsInlineGroups = 16;  // passed as kernel arguments
 constexpr unsigned kObsMaxBlocks = 2048, kObsMaxGroups = 256;   // per launch: the partials hold this many pairs
 constexpr unsigned kObsMaxTerms = 1u << 16;                      // of a call that does not wait: the upload ring takes their tables
-constexpr u64 kObsOneBlock = 1ULL << 13;                         // states up to here: one block does all
+constexpr u64 kObsOneBlock = 1ULL << 13;  // states up to here may take one block
+constexpr u64 kObsOneTerms = 8;           // terms, times cosets of a thread, per wave or block of that launch
+constexpr unsigned kObsSpread = 1024;     // work-groups that a launch of many terms is spread over
+constexpr u64 kObsByWave = 64 * kObsMembers;  // states up to here: a group per wave
 
 struct ObsTerm {
     u64 bf, pf;
@@ -253,12 +255,13 @@ __global__ __launch_bounds__(kRBlock) void k_observable(ObsArgs a) {
     __shared__ double lds[32];
     double re = 0.0, im = 0.0;
     // up to 64 cosets: a group per wave instead of the groups one after another
-    const bool by_wave = a.dim <= 64 * kObsMembers;
+    const bool by_wave = a.dim <= kObsByWave;
     const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const u64 stride = by_wave ? 64 : (u64)gridDim.x * blockDim.x;
     const u64 t0 = by_wave ? threadIdx.x & 63 : (u64)blockIdx.x * blockDim.x + threadIdx.x;
     const double2* __restrict__ psi = a.state;
-    for (u32 g = by_wave ? wave : blockIdx.y; g < a.ngroup; g += by_wave ? kRBlock / 64 : gridDim.y) {
+    const u32 side = by_wave ? kRBlock / 64 : 1;  // groups side by side in a block
+    for (u32 g = blockIdx.y * side + (by_wave ? wave : 0); g < a.ngroup; g += gridDim.y * side) {
         const ObsGroup gr = INLINE ? a.group[g] : a.groups[g];
         if (a.dim < (u64)kObsMembers) {  // fewer amplitudes than a coset has
             if (t0 < a.dim) {
@@ -310,7 +313,44 @@ __global__ __launch_bounds__(kRBlock) void k_observable(ObsArgs a) {
 struct ObsPlan {
     std::vector<ObsTerm> terms;  // group after group
     std::vector<ObsGroup> groups;
+    unsigned nb = 1;       // blocks along the state
+    bool by_wave = false;  // small states: see k_observable
+    bool one = false;      // one block does all
+    // blocks along the groups for ng of them
+    unsigned ny(size_t ng) const { return one ? 1u : (unsigned)(by_wave ? (ng + 3) / 4 : ng); }
+    // groups of a launch whose partials fit (2^20 doubles)
+    size_t per_launch() const { return std::min<size_t>(1u << 15, (size_t)kObsMaxBlocks * kObsMaxGroups / nb); }
 };
+// The grid.  One block for a small state and few terms needs no second launch; its waves wait
+// out the latency of one term after another (0.4 us each), so it takes kObsOneTerms of them.  Beyond
+// that, and on larger states with few blocks and groups (all Z strings are one group), groups are
+// split until some kObsSpread blocks share the terms: their pieces read the same state, from L2.
+// 12 random terms at 12 qubits: one block 22.8 us, spread 20.4; 4 terms at 13 qubits 19.0 and 20.0.
+// 1000 terms at 13 qubits: one block 1150 us, spread 130; 1000 Z strings at 16: one group 481, spread 78.
+void shape_observable(ObsPlan& pl, u64 dim) {
+    const u64 cosets = std::max<u64>(1, dim / kObsMembers), terms = pl.terms.size();
+    pl.by_wave = dim <= kObsByWave;
+    pl.nb = pl.by_wave ? 1u : (unsigned)std::min<u64>(kObsMaxBlocks, (cosets + kRBlock - 1) / kRBlock);
+    const u64 side = pl.by_wave ? 4 : 1;
+    pl.one = dim <= kObsOneBlock && terms * pl.nb <= kObsOneTerms * side;
+    u64 piece = terms;
+    if (pl.one) {
+        pl.nb = 1;
+        if (pl.by_wave && pl.groups.size() < side) piece = std::max<u64>(4, (terms + side - 1) / side);
+    } else {
+        piece = std::max<u64>(8, (terms * pl.nb + kObsSpread * side - 1) / (kObsSpread * side));
+    }
+    std::vector<ObsGroup> out;
+    for (const ObsGroup& g : pl.groups)
+        for (u32 t = 0; t < g.nterm; t += (u32)piece) {
+            out.push_back(g);
+            out.back().term0 = g.term0 + t;
+            out.back().nterm = std::min<u32>((u32)piece, g.nterm - t);
+        }
+    // (not where the groups alone are kernel arguments: an upload costs more than it saves)
+    if (terms > kObsInlineTerms || out.size() <= kObsInlineGroups || pl.groups.size() > kObsInlineGroups)
+        pl.groups.swap(out);
+}
 ObsPlan plan_observable(const u64* bf, const u64* pf, const u32* rot, const qm_complex* coef, u32 nterms, int n) {
     ObsPlan pl;
     // the distinct flip masks, by their highest bit, dealt out so that the pivots of a group are
@@ -400,11 +440,8 @@ ObsPlan plan_observable(const u64* bf, const u64* pf, const u32* rot, const qm_c
         }
         pl.groups.push_back(gr);
     }
+    shape_observable(pl, 1ULL << n);
     return pl;
-}
-
-unsigned obs_blocks(u64 dim) {
-    return dim <= kObsOneBlock ? 1u : (unsigned)std::min<u64>(kObsMaxBlocks, (dim / kObsMembers + kRBlock - 1) / kRBlock);
 }
 
 // Enqueues the groups [g0, g0 + ng) of a plan; their sum goes to out (device or pinned memory),
@@ -420,8 +457,7 @@ bool launch_observable(const ObsPlan& pl, size_t g0, size_t ng, const void* stat
     a.ngroup = (u32)ng;
     a.terms = dterms;
     a.groups = dgroups ? dgroups + g0 : nullptr;
-    const unsigned nb = obs_blocks(dim);
-    const unsigned ny = nb == 1 ? 1u : (unsigned)ng;
+    const unsigned nb = pl.nb, ny = pl.ny(ng);
     a.out = nb * ny == 1 && !add ? out : nullptr;
     if (!dterms) {
         std::copy(pl.terms.begin(), pl.terms.end(), a.term);
@@ -468,8 +504,8 @@ bool enqueue_observable(const u64* bf, const u64* pf, const u32* rot, const doub
     const ObsTerm* dt = nullptr;
     const ObsGroup* dg = nullptr;
     if (!obs_inline(pl) && !upload_plan(sc, pl, &dt, &dg)) return false;
-    for (size_t g = 0; g < pl.groups.size(); g += kObsMaxGroups)
-        if (!launch_observable(pl, g, std::min<size_t>(kObsMaxGroups, pl.groups.size() - g), state, dim, st, sc->partials,
+    for (size_t g = 0; g < pl.groups.size(); g += pl.per_launch())
+        if (!launch_observable(pl, g, std::min(pl.per_launch(), pl.groups.size() - g), state, dim, st, sc->partials,
                                dt, dg, h_out, what, g > 0))
             return false;
     return true;
@@ -790,7 +826,7 @@ qm_complex qm_observable_expectation_host(const ITYPE* bfs, const ITYPE* pfs, co
     Scratch* sc = scratch_for(st);
     if (!sc) return z;
     double total_re = 0, total_im = 0;
-    // as many terms at a time as the upload ring takes; a launch per kObsMaxGroups groups
+    // as many terms at a time as the upload ring takes
     const UINT chunk = 1u << 15;
     for (UINT off = 0; off < nterms; off += chunk) {
         const UINT cnt = std::min(chunk, nterms - off);
@@ -798,8 +834,8 @@ qm_complex qm_observable_expectation_host(const ITYPE* bfs, const ITYPE* pfs, co
         const ObsTerm* dt = nullptr;
         const ObsGroup* dg = nullptr;
         if (!obs_inline(pl) && !upload_plan(sc, pl, &dt, &dg)) return z;
-        for (size_t g = 0; g < pl.groups.size(); g += kObsMaxGroups) {
-            if (!launch_observable(pl, g, std::min<size_t>(kObsMaxGroups, pl.groups.size() - g), state, dim, st,
+        for (size_t g = 0; g < pl.groups.size(); g += pl.per_launch()) {
+            if (!launch_observable(pl, g, std::min(pl.per_launch(), pl.groups.size() - g), state, dim, st,
                                    sc->partials, dt, dg, sc->host_result, what) ||
                 !hip_ok(hipStreamSynchronize(st), what))
                 return z;

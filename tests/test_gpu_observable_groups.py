@@ -1,6 +1,7 @@
 """qm_observable_expectation_host over the forms its grouping of terms meets: fewer
 amplitudes than a coset (1..3 qubits), one block, several blocks, masks that depend on each
-other, only Z strings, low pivots, more terms than the kernel arguments hold.
+other, only Z strings, low pivots, more terms than the kernel arguments hold, groups
+split over work-groups.
 
 Tolerance: sums of 2^n products of magnitude |psi|^2, each rounded a few times:
 |d| <= 2^-53 * (16 + 2 log2(2^n)) * sum |c_k| for a normalised state."""
@@ -75,6 +76,16 @@ def test_observable_groups(n, kind, count):
         assert abs(got - _want(terms, psi)) <= tol, (got, _want(terms, psi), tol)
         if count <= 128:
             assert _call("qm_observable_expectation_noalloc_host", terms, s) == got
+
+
+@pytest.mark.parametrize("n,kind,count", [
+    (2, "z", 200), (7, "any", 33), (10, "z", 32), (10, "z", 33), (10, "z", 49), (10, "any", 600), (11, "any", 8),
+    (11, "z", 9), (12, "low", 300), (13, "any", 4), (13, "any", 5), (13, "z", 2000), (16, "z", 500), (20, "z", 100),
+    (21, "z", 40)])
+def test_groups_split_over_work_groups(n, kind, count):
+    """Both sides of the rule for one block, groups split into pieces (all Z strings are one group),
+    pieces among the kernel arguments and behind them.  Tolerance as above."""
+    test_observable_groups(n, kind, count)
 
 
 def test_infinities_and_nan_stay_where_they_were():
