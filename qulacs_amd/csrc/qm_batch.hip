@@ -313,11 +313,16 @@ __global__ __launch_bounds__(stage_threads<K>()) void k_stage(double2* __restric
     }
 }
 
-// One stage of a single-state circuit with a work-group per tile of at most 2^12 amplitudes: two or more groups share a
+// A grid has fewer than 2^32 threads, and 34 qubits in windows of 8 are 2^26 tiles of 64: the
+// tiles of a stage go out in launches of this many.
+constexpr u64 kTilesPerLaunch = 1ULL << 20;
+
+// One stage of a single-state circuit with a work-group per tile (tiles from tile0 on) of at most 2^12 amplitudes: two or more groups share a
 // CU and drift apart, so one's memory phase overlaps another's passes without a prefetch.
 template <int K>
 __global__ __launch_bounds__(tile_threads<K>(), K == 4 ? 2 : 4) void k_tile(double2* __restrict__ state, u32 lq, u32 tl,
-                                                                            DStage sg, const DPass* __restrict__ passes,
+                                                                            u64 tile0, DStage sg,
+                                                                            const DPass* __restrict__ passes,
                                                                             const DSub* __restrict__ subs,
                                                                             const double2* __restrict__ pool) {
     extern __shared__ double2 st[];
@@ -325,7 +330,8 @@ __global__ __launch_bounds__(tile_threads<K>(), K == 4 ? 2 : 4) void k_tile(doub
     constexpr u32 T = tile_threads<K>();
     const u32 L = 1u << lq;
     build_hi_tab(hi_tab, lq, sg);
-    const u64 tb = tile_base(blockIdx.x, tl, sg);
+    const u64 tile = tile0 + blockIdx.x;
+    const u64 tb = tile_base(tile, tl, sg);
     __syncthreads();
     constexpr u32 P = (1u << kTileLocal) / T;
     if (L == P * T) {
@@ -340,7 +346,7 @@ __global__ __launch_bounds__(tile_threads<K>(), K == 4 ? 2 : 4) void k_tile(doub
         for (u32 i = threadIdx.x; i < L; i += blockDim.x) st[slot_of(i)] = state[tile_index(tb, hi_tab, i)];
     }
     __syncthreads();
-    run_passes<K, T, 1>(st, lq, passes, sg.pass0, sg.npass, subs, pool, blockIdx.x);
+    run_passes<K, T, 1>(st, lq, passes, sg.pass0, sg.npass, subs, pool, tile);
     if (L == P * T) {
 #pragma unroll
         for (u32 k = 0; k < P; ++k) {
@@ -929,8 +935,11 @@ bool circuit_enqueue(qm_circuit* c, void* state, u64 dim, hipStream_t st, unsign
         const u32 T = std::max(64u, std::min(c->K == 3 ? tile_threads<3>() : tile_threads<4>(), (1u << c->lq) >> c->K));
         for (const DStage& sg : c->stages) {
             if (sg.npass == 0) continue;
-            if (c->K == 3) k_tile<3><<<(u32)ntiles, T, lds, st>>>((double2*)state, c->lq, tl, sg, c->d_passes, c->d_subs, c->d_pool);
-            else k_tile<4><<<(u32)ntiles, T, lds, st>>>((double2*)state, c->lq, tl, sg, c->d_passes, c->d_subs, c->d_pool);
+            for (u64 t0 = 0; t0 < ntiles; t0 += kTilesPerLaunch) {
+                const u32 nt = (u32)std::min<u64>(kTilesPerLaunch, ntiles - t0);
+                if (c->K == 3) k_tile<3><<<nt, T, lds, st>>>((double2*)state, c->lq, tl, t0, sg, c->d_passes, c->d_subs, c->d_pool);
+                else k_tile<4><<<nt, T, lds, st>>>((double2*)state, c->lq, tl, t0, sg, c->d_passes, c->d_subs, c->d_pool);
+            }
         }
         return hip_ok(hipGetLastError(), what);
     }

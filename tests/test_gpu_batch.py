@@ -191,3 +191,33 @@ def test_fused_circuit_above_32_qubits_round_trip(block):
     finally:
         _lib.call("release_quantum_state_host", st, 0)
         fc.close()
+
+
+def test_fused_circuit_of_more_tiles_than_a_launch():
+    """30 qubits in windows of 8: 2^22 tiles, four launches a stage.  Rotations, then CZ from the
+    highest qubits (bits of the tile number) to qubit 0 between two rotations of it: every qubit's
+    probability has a closed form."""
+    from qulacs_amd import _lib
+    from qulacs_amd.batch import FusedCircuit
+
+    def ry(a):
+        return np.array([[np.cos(a), -np.sin(a)], [np.sin(a), np.cos(a)]])
+
+    n = 30
+    a = 0.3 + 0.03 * np.arange(n)
+    gates = [("dense", [t], ry(a[t])) for t in range(n)]
+    gates += [("CZ", [0, 29], None), ("CZ", [28, 0], None), ("dense", [0], ry(0.4))]
+    fc = FusedCircuit(n, gates, block_qubits=3, local_qubits=8)
+    dim = 1 << n
+    st = _lib.call("allocate_quantum_state_host", dim, 0)
+    try:
+        _lib.call("initialize_quantum_state_host", st, dim, None, 0)
+        fc.apply(st)
+        want = np.cos(a) ** 2
+        odd = want[28] * (1 - want[29]) + want[29] * (1 - want[28])  # an odd number of the two is 1
+        want[0] = (1 - odd) * np.cos(a[0] + 0.4) ** 2 + odd * np.cos(0.4 - a[0]) ** 2
+        for t in range(n):
+            assert abs(_lib.call("M0_prob_host", t, st, dim, None, 0) - want[t]) < 1e-13, t
+    finally:
+        _lib.call("release_quantum_state_host", st, 0)
+        fc.close()
