@@ -344,8 +344,9 @@ QM_EXPORT const double* qm_batch_run_async(qm_batch* batch, void* stream, unsign
 /* Copies circuit i's final state (2^n complex128) to host memory after a run
  * compiled with keep_states. */
 QM_EXPORT int qm_batch_get_state(qm_batch* batch, UINT index, qm_complex* out, void* stream, unsigned int device_number);
-/* Qubits held in LDS per tile (8..13, default 13); takes effect at the next
- * compile; 13 runs as 12 (64 KiB tiles, two work-groups per CU). */
+/* Qubits held in LDS per tile at most (8..13, default 13); takes effect at the next
+ * compile.  13 runs as QM_BATCH_TILE_QUBITS: 64 KiB tiles, two work-groups per CU. */
+#define QM_BATCH_TILE_QUBITS 12u
 QM_EXPORT int qm_batch_set_local_qubits(qm_batch* batch, UINT local_qubits);
 /* Captures one run (its launches) on `stream` (a created stream,
  * not NULL) into a HIP graph; qm_batch_run_graph replays it.  A compile drops

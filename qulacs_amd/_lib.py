@@ -34,6 +34,7 @@ class QmBatchGate(C.Structure):
 BATCH_DENSE, BATCH_DIAG, BATCH_CZ, BATCH_CNOT = 0, 1, 2, 3
 BATCH_DEPOL = 5  # qm_circuit_create only
 ADJ_ROT = 4
+BATCH_TILE_QUBITS = 12  # the widest window a batch runs
 
 
 class QmAdjointGate(C.Structure):

@@ -83,7 +83,7 @@ class Batch:
         _lib.call("qm_batch_set_local_qubits", self.h, int(local_qubits))
         _lib.call("qm_batch_compile", self.h, int(block_qubits), 1 if keep_states else 0, self.device)
         self.block_qubits = block_qubits
-        self.local_qubits = local_qubits
+        self.local_qubits = min(local_qubits, _lib.BATCH_TILE_QUBITS)  # wider windows run as this one
         self.keep_states = keep_states
 
     def run(self, stream=None) -> np.ndarray:
@@ -114,13 +114,17 @@ class Batch:
         _lib.call("qm_batch_stats", self.h, *[C.byref(x) for x in v])
         return dict(zip(("circuits", "stages", "passes", "subops"), (int(x.value) for x in v)))
 
-    def autotune(self, candidates=(2, 3, 4), local_candidates=(12, 13), repeats: int = 2,
+    def autotune(self, candidates=(2, 3, 4), local_candidates=(11, 12), repeats: int = 2,
                  keep_states: bool = False) -> dict:
         """Compile with each (register-block size, LDS window) pair, time `repeats`
-        runs of each and keep the fastest.  Returns {(block, window): best seconds}."""
+        runs of each and keep the fastest.  Returns {(block, window): best seconds}, windows as
+        they run: above BATCH_TILE_QUBITS qubits they run as that one, and once.  (512 circuits
+        of 8 to 16 qubits at widths 2, 3, 4: 0.58 / 0.46 / 0.54 ms with 11 qubits, 0.49 / 0.41 /
+        0.46 with 12; 11 is ahead at width 2 for some tens of circuits.)"""
         times = {}
+        windows = dict.fromkeys(min(lq, _lib.BATCH_TILE_QUBITS) for lq in local_candidates)
         for k in candidates:
-            for lq in local_candidates:
+            for lq in windows:
                 try:
                     self.compile(k, keep_states, lq)
                 except _lib.QulacsMI355Error:

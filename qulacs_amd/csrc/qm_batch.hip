@@ -57,7 +57,7 @@ struct DItem {
     u32 circ, tile;
 };
 // Circuits above this size run in tiles; a tile is 64 KiB, so two work-groups share a CU.
-constexpr u32 kTileLocal = 12;
+constexpr u32 kTileLocal = QM_BATCH_TILE_QUBITS;
 // This thread's share of sum_k c_k Re <psi|P_k|psi> over the `len` amplitudes from x0 on (a power
 // of two, aligned), which lie in LDS (swizzled slots); partners beyond them are read from the state in
 // device memory.  Threads [0, stride) take part.  Eight amplitudes at a time, the terms in the inner loop:
@@ -406,7 +406,7 @@ struct qm_batch {
     qm::u32 n_large = 0;
     size_t cap[4] = {0, 0, 0, 0};  // bytes held: program, scratch, energies, partials
     bool lds_set = false;               // the kernel's LDS limit has been raised on this device
-    unsigned lq_cap = 13;               // qubits held in LDS per tile (qm_batch_set_local_qubits)
+    unsigned lq_cap = 13;               // qubits held in LDS per tile, at most kTileLocal (qm_batch_set_local_qubits)
     hipGraph_t graph = nullptr;         // captured launch (qm_batch_capture)
     hipGraphExec_t graph_exec = nullptr;
     void drop_graph() {

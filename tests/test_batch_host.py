@@ -114,6 +114,20 @@ def test_batch_window_setter_validation():
     b.close()
 
 
+@pytest.mark.parametrize("windows,run", [(None, [11, 12]), ((12, 13), [12]), ((13,), [12]), ((9, 13, 12, 9), [9, 12])])
+def test_autotune_times_each_program_once(monkeypatch, windows, run):
+    """A window above the widest that a batch runs is that one: not compiled and timed beside it,
+    and not reported as a choice."""
+    b = Batch()
+    compiled = []
+    monkeypatch.setattr(b, "compile", lambda k, keep, lq: compiled.append((k, lq)))
+    monkeypatch.setattr(b, "run", lambda: None)
+    times = b.autotune((3, 4), repeats=1, **({} if windows is None else {"local_candidates": windows}))
+    want = [(k, lq) for k in (3, 4) for lq in run]
+    assert list(times) == want and compiled[:-1] == want and compiled[-1] in want
+    b.close()
+
+
 def test_adjoint_pass_plan():
     """The adjoint groups gates into passes over 3-qubit register blocks (host
     planning, no device work): the 20-qubit, 12-layer hardware-efficient ansatz
