@@ -710,12 +710,12 @@ void qm_adjoint::build(const Builder& b) {
                 occ_col[f.occ] = col[o];
                 occ_coef[f.occ] = f.coef;
             }
-    par_first.assign(1, 0);
-    for (u32 p = 0; p < nparams; ++p) {
-        for (const Factor& f : b.occ)
-            if (f.param == p) par_occs.push_back(f.occ);
-        par_first.push_back((u32)par_occs.size());
-    }
+    par_first.assign((size_t)nparams + 1, 0);
+    for (const Factor& f : b.occ) ++par_first[f.param + 1];
+    for (u32 p = 0; p < nparams; ++p) par_first[p + 1] += par_first[p];
+    par_occs.assign(b.occ.size(), 0);
+    std::vector<u32> next(par_first.begin(), par_first.end() - 1);
+    for (const Factor& f : b.occ) par_occs[next[f.param]++] = f.occ;  // occurrences in order
 }
 
 namespace {
