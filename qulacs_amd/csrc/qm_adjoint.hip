@@ -44,6 +44,7 @@ constexpr u32 kBwdLocal = 11;        // backward window: 32 KiB of psi and 32 Ki
 constexpr u32 kFwdThreads = 1u << (kFwdLocal - kAdjK);
 constexpr u32 kBwdThreads = 1u << (kBwdLocal - kAdjK);
 constexpr u32 kStageGrads = 64;      // operations with gradients per backward stage (LDS sums)
+constexpr u32 kChunkCols = 1536;     // columns of partial sums held at a time (at least a stage's, 3 * kStageGrads)
 constexpr u64 kBwdMaxBlocks = 4096;  // work-groups per state of a backward stage (more tiles: several each)
 constexpr u32 kHpsiThreads = 256;
 constexpr u32 kHpsiMaxBlocks = 512;
@@ -245,9 +246,9 @@ __device__ __forceinline__ void bwd_bit(double2 (&v)[1 << kAdjK], double2 (&l)[1
 // inverted.  A thread holds one register block of each state; the tile has at most T blocks
 // (threads beyond them hold zeros, so that the wave sums see every lane).  Work-group x takes
 // tiles x, x + gridDim.x, ... and writes its sums of the stage's operations to
-// partials[set][x][3 * (position in grads) ..].
+// partials[set][x][col0 ..].
 __global__ __launch_bounds__(kBwdThreads, 2) void k_adj_bwd(double2* __restrict__ psi, double2* __restrict__ lam, u32 n,
-                                                            u32 lq, u64 ntiles, DStage sg, u32 grad0, u32 ngrad,
+                                                            u32 lq, u64 ntiles, DStage sg, u32 grad0, u32 ngrad, u32 col0,
                                                             const DPass* __restrict__ passes,
                                                             const DSub* __restrict__ subs,
                                                             const double2* __restrict__ pools, u32 stride,
@@ -358,7 +359,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void k_adj_bwd(double2* __restrict_
         }
         __syncthreads();  // the tile has been read out of LDS
     }
-    double* dst = partials + ((u64)blockIdx.y * gridDim.x + blockIdx.x) * ncols + 3 * (u64)grad0;
+    double* dst = partials + ((u64)blockIdx.y * gridDim.x + blockIdx.x) * ncols + col0;
     for (u32 i = tid; i < 3 * ngrad; i += T) {
         double s = 0.0;
         for (u32 w = 0; w < T / 64; ++w) s += acc[w][i / 3][i % 3];
@@ -400,10 +401,11 @@ __global__ __launch_bounds__(kHpsiThreads) void k_adj_hpsi(const double2* __rest
     if (threadIdx.x == 0) epart[(u64)blockIdx.y * gridDim.x + blockIdx.x] = acc;
 }
 
-// Columns of partials[set][block][ncols] summed over the blocks: 16 columns per
-// work-group, 16 threads per column, each over every 16th block, then in order.
+// Columns of partials[set][block][ncols] summed over the blocks into sums[set][total], from
+// sums + col0 on: 16 columns per work-group, 16 threads per column, each over every 16th block,
+// then in order.
 __global__ __launch_bounds__(256) void k_adj_columns(const double* __restrict__ partials, u32 nblk, u32 ncols,
-                                                     double* __restrict__ sums) {
+                                                     double* __restrict__ sums, u32 total, u32 col0) {
     __shared__ double red[16][17];
     const u32 c = threadIdx.x & 15u, part = threadIdx.x >> 4, col = blockIdx.x * 16 + c;
     const double* src = partials + (u64)blockIdx.y * nblk * ncols;
@@ -415,7 +417,7 @@ __global__ __launch_bounds__(256) void k_adj_columns(const double* __restrict__ 
     if (part == 0 && col < ncols) {
         double r = 0.0;
         for (u32 k = 0; k < 16; ++k) r += red[k][c];
-        sums[(u64)blockIdx.y * ncols + col] = r;
+        sums[(u64)blockIdx.y * total + col0 + col] = r;
     }
 }
 
@@ -581,6 +583,10 @@ struct qm_adjoint {
     u64 ngates = 0, blocks3 = 0;
     Flat fwd, bwd;
     std::vector<u32> stage_grad0;  // backward stage -> position in bwd.grads of its first operation
+    // runs of backward stages whose partial sums share the workspace's columns: the first stage
+    // of each, and the widest one's columns
+    std::vector<u32> chunk0;
+    u32 chunk_cols = 0;
     // host tables, uploaded on first use
     std::vector<Factor> factors;
     std::vector<u32> first, fwd_at, bwd_at, copies, par_first, par_occs, occ_col;
@@ -608,7 +614,7 @@ struct qm_adjoint {
     u64 state_bytes(u64 batch) const { return batch * (16ULL << ne); }
     u64 fpool_bytes(u64 batch) const { return batch * fwd.pool.size() * 16; }
     u64 bpool_bytes(u64 batch) const { return batch * bwd.pool.size() * 16; }
-    u64 part_bytes(u64 batch) const { return (batch * blocks_b() * ncols() * 8 + 15) & ~15ULL; }
+    u64 part_bytes(u64 batch) const { return (batch * blocks_b() * chunk_cols * 8 + 15) & ~15ULL; }
     u64 sums_bytes(u64 batch) const { return (batch * ncols() * 8 + 15) & ~15ULL; }
     u64 gvec_bytes(u64 batch) const { return (batch * nocc() * 24 + 15) & ~15ULL; }
     u64 epart_bytes(u64 batch) const { return (batch * blocks_h() * 8 + 15) & ~15ULL; }
@@ -675,6 +681,16 @@ void qm_adjoint::build(const Builder& b) {
         }
     }
     stage_grad0.push_back(g);
+    // Partial sums are blocks x columns: held for the whole sweep they would grow with the
+    // circuit (40000 parameters at 20 qubits: 240 MiB beside 32 of states), so they are added up
+    // when kChunkCols are full.  A launch of some microseconds per chunk; most circuits have one.
+    chunk0.assign(1, 0);
+    chunk_cols = 0;
+    for (u32 s = 0; s < bwd.stages.size(); ++s) {
+        if (3 * (stage_grad0[s + 1] - stage_grad0[chunk0.back()]) > kChunkCols) chunk0.push_back(s);
+        chunk_cols = std::max(chunk_cols, 3 * (stage_grad0[s + 1] - stage_grad0[chunk0.back()]));
+    }
+    chunk0.push_back((u32)bwd.stages.size());
     factors.clear();
     first.assign(1, 0);
     for (const Op1& o : b.op1) {
@@ -897,14 +913,19 @@ int qm_adjoint_run(qm_adjoint* a, UINT batch, const double* theta, const ITYPE* 
                                                                    epart);
     if (a->ncols()) {
         const dim3 grid(a->blocks_b(), batch);
-        for (size_t s = 0; s < a->bwd.stages.size(); ++s) {
-            if (a->stage_grad0[s] == a->ncols() / 3) break;  // no rotation is left: nothing more to differentiate
-            k_adj_bwd<<<grid, threads(a->lqb, kBwdThreads), 2 * sizeof(double2) << a->lqb, st>>>(
-                psi, lam, a->ne, a->lqb, a->tiles_b(), a->bwd.stages[s], a->stage_grad0[s],
-                a->stage_grad0[s + 1] - a->stage_grad0[s], a->d_bpass, a->d_bsub, bpool, (u32)a->bwd.pool.size(),
-                partials, a->ncols());
+        for (size_t c = 0; c + 1 < a->chunk0.size(); ++c) {
+            const u32 first = a->stage_grad0[a->chunk0[c]], cols = 3 * (a->stage_grad0[a->chunk0[c + 1]] - first);
+            if (cols == 0) continue;  // only stages behind the last rotation
+            for (u32 s = a->chunk0[c]; s < a->chunk0[c + 1]; ++s) {
+                if (a->stage_grad0[s] == a->ncols() / 3) break;  // no rotation is left: nothing more to differentiate
+                k_adj_bwd<<<grid, threads(a->lqb, kBwdThreads), 2 * sizeof(double2) << a->lqb, st>>>(
+                    psi, lam, a->ne, a->lqb, a->tiles_b(), a->bwd.stages[s], a->stage_grad0[s],
+                    a->stage_grad0[s + 1] - a->stage_grad0[s], 3 * (a->stage_grad0[s] - first), a->d_bpass, a->d_bsub,
+                    bpool, (u32)a->bwd.pool.size(), partials, cols);
+            }
+            k_adj_columns<<<dim3((cols + 15) / 16, batch), 256, 0, st>>>(partials, a->blocks_b(), cols, sums, a->ncols(),
+                                                                         3 * first);
         }
-        k_adj_columns<<<dim3((a->ncols() + 15) / 16, batch), 256, 0, st>>>(partials, a->blocks_b(), a->ncols(), sums);
     }
     k_adj_grad<<<dim3(std::max(1u, (a->nparams + 63) / 64), batch), 64, 0, st>>>(
         sums, a->ncols(), gvec, a->nocc(), a->d_par_first, a->d_par_occs, a->d_occ_col, a->d_occ_coef, a->nparams, grad,

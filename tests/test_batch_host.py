@@ -124,6 +124,23 @@ def test_adjoint_create_is_linear_in_parameters():
     assert best < 0.3
 
 
+def test_adjoint_workspace_does_not_hold_every_partial_sum():
+    """40000 parameters at 20 qubits: two states of 16 MiB, the matrices of the operations (64 bytes
+    each, forward and backward), 24 bytes per parameter and three sums per operation, and at most
+    12 MiB of partial sums."""
+    pytest.importorskip("torch")
+    from qulacs_amd import _lib
+    from qulacs_amd.adjoint import AdjointCircuit, hardware_efficient_ansatz
+
+    gates, params = hardware_efficient_ansatz(20, 1000)
+    c = AdjointCircuit(20, gates, params)
+    ops = params // 2
+    fixed = 2 * (16 << 20) + 2 * 64 * ops + 24 * params + 24 * ops
+    assert params == 40000
+    assert fixed <= _lib.call("qm_adjoint_workspace_bytes", c.h, 1) <= fixed + (12 << 20)
+    c.close()
+
+
 def test_batch_window_setter_validation():
     from qulacs_amd import _lib
 

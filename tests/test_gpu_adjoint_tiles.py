@@ -113,6 +113,28 @@ def test_adjoint_matches_gate_by_gate(n, count, sets):
         assert np.abs(g[b] - wg).max() <= tol * count / params, (b, np.abs(g[b] - wg).max(), tol)
 
 
+@pytest.mark.parametrize("n,sets", [(5, 3), (12, 2)])
+def test_more_operations_than_the_partial_sums_hold(n, sets):
+    """Some 700 operations with gradients (512 share the workspace's columns), the last ones behind
+    fixed gates only: gradients as a shorter sweep gives them."""
+    rng = np.random.default_rng(n)
+    gates = [("dense", [q], haar_unitary(rng, 1)) for q in range(n)]
+    params = 40
+    while sum(g[0] == "rot" for g in gates) < 700:
+        gates += [("rot", [int(rng.integers(n))], [int(rng.integers(1, 4))], int(rng.integers(params)), 1.0),
+                  ("CZ", [int(x) for x in rng.choice(n, 2, replace=False)], None)]
+    terms = [(3, 3, 2, 1.0), (0, 1 << (n - 1), 0, -0.5)]
+    theta = rng.uniform(0, 2 * np.pi, (sets, params))
+    circ = AdjointCircuit(n, gates, params)
+    e, g = circ.run(torch.tensor(theta, device="cuda:0"), terms)
+    e, g = e.cpu().numpy(), g.cpu().numpy()
+    tol = 4 * len(gates) * 2.0 ** -53 * 1.5
+    for b in range(sets):
+        we, wg = _reference(n, gates, theta[b], terms)
+        assert abs(e[b] - we) <= tol
+        assert np.abs(g[b] - wg).max() <= tol * 700 / params, np.abs(g[b] - wg).max()
+
+
 def test_non_unitary_fixed_gate_keeps_its_own_operation():
     """A projection between two rotations: its conjugate transpose stands for its
     inverse, as for any fixed gate."""
