@@ -3651,15 +3651,90 @@ std::vector<double> ParametricQuantumCircuit::backprop_inner_product(QuantumStat
 // Device 0's gradient through the adjoint engine: forward, H|psi> and backward in a few launches
 // over LDS tiles, where the walk above takes about eight calls per gate (12 qubits, 72
 // parameters: 663 launches; one step of a variational loop 8.15 against 0.29 ms).
+namespace {
+// A stream and buffers for one call.  A stream brings 16 MiB of scratch with it, so circuits do not
+// keep one each: calls take a workspace from here and give it back.  At most kIdle wait
+// for the next call, with buffers up to kKeepBytes; the last circuit that has a plan to go frees
+// them.
+struct Workspace {
+    void* stream = nullptr;
+    void* io = nullptr;    // angles, then the energy and the gradient
+    void* work = nullptr;
+    size_t io_amps = 0, work_bytes = 0;
+    bool fit(void** p, size_t* have, size_t want, size_t unit) {
+        if (*p && *have >= want) return true;
+        if (*p) release_quantum_state_host(*p, 0);
+        *p = allocate_quantum_state_host((want + unit - 1) / unit, 0);
+        *have = *p ? want : 0;
+        return *p != nullptr;
+    }
+    bool reserve(size_t amps, size_t bytes) {
+        if (!stream) stream = allocate_cuda_stream_host(1, 0);
+        return stream && fit(&io, &io_amps, amps, 1) && fit(&work, &work_bytes, bytes, 16);
+    }
+    void drop_work() {
+        if (work) release_quantum_state_host(work, 0);
+        work = nullptr;
+        work_bytes = 0;
+    }
+    void release() {
+        if (stream) qm_synchronize(stream, 0);
+        drop_work();
+        if (io) release_quantum_state_host(io, 0);
+        if (stream) release_cuda_stream_host(stream, 1, 0);
+        *this = Workspace();
+    }
+};
+class WorkspacePool {
+   public:
+    static WorkspacePool& get() {
+        static WorkspacePool* p = new WorkspacePool;  // outlives every circuit
+        return *p;
+    }
+    void enter() {
+        std::lock_guard<std::mutex> lock(mutex_);
+        ++users_;
+    }
+    void leave() {
+        std::vector<Workspace> gone;
+        {
+            std::lock_guard<std::mutex> lock(mutex_);
+            if (--users_ == 0) gone.swap(idle_);
+        }
+        for (Workspace& w : gone) w.release();
+    }
+    Workspace take() {
+        std::lock_guard<std::mutex> lock(mutex_);
+        if (idle_.empty()) return Workspace();
+        const Workspace w = idle_.back();
+        idle_.pop_back();
+        return w;
+    }
+    void give(Workspace w) {
+        if (w.work_bytes > kKeepBytes) w.drop_work();
+        {
+            std::lock_guard<std::mutex> lock(mutex_);
+            if (users_ > 0 && idle_.size() < kIdle) {
+                idle_.push_back(w);
+                return;
+            }
+        }
+        w.release();
+    }
+
+   private:
+    static constexpr size_t kIdle = 2, kKeepBytes = size_t(64) << 20;
+    std::mutex mutex_;
+    std::vector<Workspace> idle_;
+    size_t users_ = 0;  // circuits with a plan
+};
+}  // namespace
 void ParametricQuantumCircuit::Adjoint::release() {
-    if (stream) qm_synchronize(stream, 0);
-    if (plan) qm_adjoint_destroy(plan);
-    if (io) release_quantum_state_host(io, 0);
-    if (work) release_quantum_state_host(work, 0);
-    if (stream) release_cuda_stream_host(stream, 1, 0);
+    if (plan) {
+        qm_adjoint_destroy(plan);
+        WorkspacePool::get().leave();
+    }
     plan = nullptr;
-    io = work = stream = nullptr;
-    work_bytes = 0;
     fixed.clear();
     structure = ~0ULL;
 }
@@ -3720,7 +3795,8 @@ bool ParametricQuantumCircuit::plan_adjoint() {
     }
     adjoint_.plan =
         qm_adjoint_create(qubit_count_, list.data(), (UINT)list.size(), (UINT)(np + adjoint_.fixed.size()));
-    if (!adjoint_.plan) qm_clear_last_error();
+    if (adjoint_.plan) WorkspacePool::get().enter();
+    else qm_clear_last_error();
     return adjoint_.plan != nullptr;
 }
 bool ParametricQuantumCircuit::backprop_fused(const GeneralQuantumOperator& obs, std::vector<double>* grad) {
@@ -3742,33 +3818,23 @@ bool ParametricQuantumCircuit::backprop_fused(const GeneralQuantumOperator& obs,
     if (!plan_adjoint()) return false;
     Adjoint& a = adjoint_;
     const size_t all = np + a.fixed.size(), pad = (all + 1) & ~size_t(1);  // buffers are counted in 16-byte units
-    if (!a.stream) a.stream = allocate_cuda_stream_host(1, 0);
-    if (!a.io) a.io = allocate_quantum_state_host(pad / 2 + 1 + pad / 2, 0);
-    const size_t need = (size_t)qm_adjoint_workspace_bytes(a.plan, 1);
-    if (!a.work) {
-        a.work = allocate_quantum_state_host((need + 15) / 16, 0);
-        a.work_bytes = need;
-    }
-    if (!a.stream || !a.io || !a.work) {  // no memory: the walk needs less at a time
-        qm_clear_last_error();
-        a.release();
+    Workspace w = WorkspacePool::get().take();
+    if (!w.reserve(pad / 2 + 1 + pad / 2, (size_t)qm_adjoint_workspace_bytes(a.plan, 1))) {
+        qm_clear_last_error();  // no memory: the walk needs less at a time
+        w.release();
         return false;
     }
     std::vector<double> host(pad, 0.0);
     for (size_t i = 0; i < np; ++i) host[i] = param(i)->get_parameter_value();
     std::copy(a.fixed.begin(), a.fixed.end(), host.begin() + np);
-    double* theta = static_cast<double*>(a.io);
+    double* theta = static_cast<double*>(w.io);
     double* energy = theta + pad;
     double* out = energy + 2;
-    copy_quantum_state_from_host_to_device(theta, host.data(), pad / 2, a.stream, 0);
-    qm_adjoint_run(a.plan, 1, theta, bf.data(), pf.data(), rot.data(), coef.data(), (UINT)nt, energy, out, a.work,
-                   a.stream, 0);
-    copy_quantum_state_from_device_to_host(host.data(), out, pad / 2, a.stream, 0);
-    if (a.work_bytes > Adjoint::kKeepBytes) {
-        release_quantum_state_host(a.work, 0);
-        a.work = nullptr;
-        a.work_bytes = 0;
-    }
+    copy_quantum_state_from_host_to_device(theta, host.data(), pad / 2, w.stream, 0);
+    qm_adjoint_run(a.plan, 1, theta, bf.data(), pf.data(), rot.data(), coef.data(), (UINT)nt, energy, out, w.work,
+                   w.stream, 0);
+    copy_quantum_state_from_device_to_host(host.data(), out, pad / 2, w.stream, 0);
+    WorkspacePool::get().give(w);
     check_abi("backprop");
     grad->assign(host.begin(), host.begin() + np);
     return true;

@@ -790,8 +790,8 @@ class ParametricQuantumCircuit : public QuantumCircuit {
    private:
     QuantumGate_SingleParameter* param(size_t i) const;
     std::vector<size_t> param_pos_;  // gate index of parameter i
-    // backprop through the adjoint engine (qm_adjoint_*): the scheduled circuit and its device
-    // buffers, kept until the gate list changes.  A copy of the circuit starts without one.
+    // backprop through the adjoint engine (qm_adjoint_*): the scheduled circuit and its tables, kept
+    // until the gate list changes.  A copy of the circuit starts without one.
     struct Adjoint {
         Adjoint() = default;
         Adjoint(const Adjoint&) {}
@@ -802,11 +802,6 @@ class ParametricQuantumCircuit : public QuantumCircuit {
         uint64_t structure = ~0ULL;
         qm_adjoint* plan = nullptr;  // null: the circuit has a gate the engine does not take
         std::vector<double> fixed;   // angles of rotations that are no parameter, after the parameters
-        void* stream = nullptr;
-        void* io = nullptr;          // angles, then the energy and the gradient
-        void* work = nullptr;        // kept between calls up to kKeepBytes
-        size_t work_bytes = 0;
-        static constexpr size_t kKeepBytes = size_t(64) << 20;
     } adjoint_;
     bool plan_adjoint();
     bool backprop_fused(const GeneralQuantumOperator& obs, std::vector<double>* grad);

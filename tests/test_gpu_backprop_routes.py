@@ -90,3 +90,49 @@ def test_backprop_with_a_complex_operator_keeps_the_walk():
     o.add_operator(1.0 + 0.5j, "X 0")
     o.add_operator(0.25, "Z 1")
     _both(c, o, 2.0)
+
+
+def _rings(n, count):
+    out = []
+    for k in range(count):
+        c = q.ParametricQuantumCircuit(n)
+        for i in range(n):
+            c.add_parametric_RX_gate(i, 0.1 + 0.05 * k + 0.01 * i)
+            c.add_CNOT_gate(i, (i + 1) % n)
+        out.append(c)
+    return out
+
+
+def test_circuits_share_their_workspaces():
+    """40 circuits that have run backprop hold their tables (some KiB), not a stream with 16 MiB of
+    scratch and a workspace each; the last one to go gives the rest back."""
+    torch = pytest.importorskip("torch")
+    torch.cuda.init()
+    obs = q.Observable(8)
+    obs.add_operator(1.0, "Z 0 Z 3")
+    for c in _rings(8, 2):  # the runtime's own first allocations
+        c.backprop(obs)
+    del c
+    free = [torch.cuda.mem_get_info()[0]]
+    circuits = _rings(8, 40)
+    for c in circuits:
+        c.backprop(obs)
+    free.append(torch.cuda.mem_get_info()[0])
+    del circuits, c
+    free.append(torch.cuda.mem_get_info()[0])
+    print([(free[0] - f) >> 20 for f in free], flush=True)
+    # tables: 15 allocations a circuit, which the runtime rounds to at most 64 KiB
+    assert free[0] - free[1] < (32 << 20) + 40 * 15 * (64 << 10)
+    assert free[0] - free[2] < 8 << 20
+
+
+def test_threads_with_circuits_of_their_own():
+    from concurrent.futures import ThreadPoolExecutor
+
+    rng = np.random.default_rng(8)
+    obs, _ = _observable(rng, 9, 5)
+    circuits = _rings(9, 6)
+    want = [c.backprop(obs) for c in circuits]
+    with ThreadPoolExecutor(6) as ex:
+        for _ in range(4):
+            assert list(ex.map(lambda c: c.backprop(obs), circuits)) == want
