@@ -48,14 +48,19 @@ constexpr u32 kChunkCols = 1536;     // columns of partial sums held at a time (
 constexpr u64 kBwdMaxBlocks = 4096;  // work-groups per state of a backward stage (more tiles: several each)
 constexpr u32 kHpsiThreads = 256;
 constexpr u32 kHpsiMaxBlocks = 512;
+// the neighbours of 1/sqrt(2), and what the upper one, which is nearer, has too much
+constexpr double kRootHigh = 0.70710678118654757, kRootLow = 0.70710678118654746;
+constexpr double kRootRest = -4.8336466567264567e-17;
 
 // One factor of a single-qubit operation.
 struct Factor {
-    u32 kind;    // 0: fixed matrix, 1 / 2 / 3: exp(i a P / 2) with P = X / Y / Z
-    u32 fixed;   // kind 0: offset into the fixed-matrix pool
+    // 0: fixed matrix, 1 / 2 / 3: exp(i a P / 2) with P = X / Y / Z, 4: fixed matrix over sqrt(2)
+    u32 kind;
+    u32 fixed;   // kinds 0 and 4: offset into the fixed-matrix pool
     u32 param;   // rotation: parameter index
     u32 occ;     // rotation: occurrence number
     double coef; // rotation: a = coef * theta[param]
+    __host__ __device__ bool rotation() const { return kind >= 1 && kind <= 3; }
 };
 
 struct AdjTerm {
@@ -78,21 +83,57 @@ __device__ __forceinline__ double2 ipow(double2 z, u32 k) {  // z * i^k
     }
 }
 
-// out <- a b, 2 x 2 complex
-__device__ __forceinline__ void mul2(double2 (&out)[4], const double2 (&a)[4], const double2 (&b)[4]) {
-    double2 r[4];
-    r[0] = cmac(cmul(a[0], b[0]), a[1], b[2]);
-    r[1] = cmac(cmul(a[0], b[1]), a[1], b[3]);
-    r[2] = cmac(cmul(a[2], b[0]), a[3], b[2]);
-    r[3] = cmac(cmul(a[2], b[1]), a[3], b[3]);
+// hi + lo: a number of about 106 bits; lo is at most half a unit of hi's last place once
+// `settle` has run.
+struct Wide {
+    double hi, lo;
+};
+__device__ __forceinline__ Wide settle(Wide a) {
+#pragma clang fp contract(off)
+    const double s = a.hi + a.lo;
+    return Wide{s, a.lo - (s - a.hi)};
+}
+// acc + a b (b a plain number); contraction would turn the exact differences into something else
+__device__ __forceinline__ Wide wide_mac(Wide acc, Wide a, double b) {
+#pragma clang fp contract(off)
+    const double p = a.hi * b, e = __builtin_fma(a.hi, b, -p);
+    const double s = acc.hi + p, t = s - acc.hi;
+    const double d = (acc.hi - (s - t)) + (p - t);
+    return Wide{s, acc.lo + (d + __builtin_fma(a.lo, b, e))};
+}
+// u <- u m, 2 x 2 complex
+__device__ __forceinline__ void wide_mul2(Wide (&re)[4], Wide (&im)[4], const double2 (&m)[4]) {
+    Wide r[4], i[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) out[i] = r[i];
+    for (int k = 0; k < 4; ++k) {
+        const int row = k & 2, col = k & 1;
+        Wide x = wide_mac(Wide{0.0, 0.0}, re[row], m[col].x), y = wide_mac(Wide{0.0, 0.0}, re[row], m[col].y);
+        x = wide_mac(x, im[row], -m[col].y);
+        y = wide_mac(y, im[row], m[col].x);
+        x = wide_mac(x, re[row + 1], m[2 + col].x);
+        y = wide_mac(y, re[row + 1], m[2 + col].y);
+        r[k] = settle(wide_mac(x, im[row + 1], -m[2 + col].y));
+        i[k] = settle(wide_mac(y, im[row + 1], m[2 + col].x));
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        re[k] = r[k];
+        im[k] = i[k];
+    }
 }
 
 // The matrices of every single-qubit operation for every parameter set: U into the
 // forward pool, U^dagger into the backward pool, and per rotation occurrence the
 // vector g (see the file comment).  blockIdx.y = set; one thread per operation.
 // `copies` lists the pool entries that do not depend on the set (4 x 4 matrices).
+//
+// Products are formed in pairs of doubles and rounded once: an operation has the error of one
+// gate, whatever it was made of.  The factors 1/sqrt(2) of the Hadamards that come with a CNOT or a
+// Pauli string are left out and put in at the end, where pairs of them are exact; rounded, each
+// would change the norm by up to 9e-17, always the same way, and the sweep back multiplies by the
+// conjugate transposes, which doubles the change instead of undoing it.  6 qubits, 12 layers of RY RZ
+// and a CNOT chain, error of the gradient against 80 bits: gate by gate 1.9e-15, products and
+// Hadamards in double 5.7e-15, so 1.95e-15.
 struct MatsArgs {
     const Factor* factors;
     const u32* first;      // factors [first[o], first[o + 1]) of operation o, in gate order
@@ -101,6 +142,7 @@ struct MatsArgs {
     const u32* bwd_at;
     const u32* copies;     // ncopy_f forward offsets, then ncopy_b backward offsets
     const double2* copy_val;
+    const u32* low;        // operation o is a Hadamard that takes the lower neighbour of 1/sqrt(2)
     u32 nops, ncopy_f, ncopy_b, nparams, nocc;
     u32 fwd_stride, bwd_stride;
 };
@@ -115,27 +157,34 @@ __global__ __launch_bounds__(64) void k_adj_mats(MatsArgs a, const double* __res
         else if (c < a.ncopy_f + a.ncopy_b) pb[a.copies[c]] = a.copy_val[c];
         return;
     }
-    // u = F_m ... F_{j+1} while the factors are walked from the last to the first
-    double2 u[4] = {make_double2(1, 0), make_double2(0, 0), make_double2(0, 0), make_double2(1, 0)};
+    // sqrt(2)^roots u = F_m ... F_{j+1} while the factors are walked from the last to the first
+    Wide ur[4] = {{1.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {1.0, 0.0}}, ui[4] = {};
+    double half = 1.0;  // 2^-roots
+    u32 roots = 0;
     for (u32 j = a.first[o + 1]; j-- > a.first[o];) {
         const Factor f = a.factors[j];
         // m = c I + i s P for a rotation about P = X, Y or Z (px, py, pz); selected without
         // branches
         const double px = f.kind == 1 ? 1.0 : 0.0, py = f.kind == 2 ? 1.0 : 0.0, pz = f.kind == 3 ? 1.0 : 0.0;
         double2 m[4];
-        if (f.kind == 0) {
+        if (!f.rotation()) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) m[i] = a.fixed[f.fixed + i];
+            half *= f.kind == 4 ? 0.5 : 1.0;
+            roots += f.kind == 4 ? 1u : 0u;
         } else {
+            double2 u[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) u[i] = make_double2(ur[i].hi, ui[i].hi);
             // u P u^dagger = [[g_Z, g_X - i g_Y], [g_X + i g_Y, -g_Z]], from its entries (0, 0) and (1, 0)
             const double2 c0 = cconj(u[0]), c1 = cconj(u[1]);
             const double2 z20 = cmul(u[2], c0), z21 = cmul(u[2], c1), z30 = cmul(u[3], c0), z31 = cmul(u[3], c1);
             const double2 z01 = cmul(u[0], c1);
             const double n0 = u[0].x * u[0].x + u[0].y * u[0].y, n1 = u[1].x * u[1].x + u[1].y * u[1].y;
             double* g = gvec + ((u64)set * a.nocc + f.occ) * 3;
-            g[0] = px * (z30.x + z21.x) - py * (z30.y - z21.y) + pz * (z20.x - z31.x);
-            g[1] = px * (z30.y + z21.y) + py * (z30.x - z21.x) + pz * (z20.y - z31.y);
-            g[2] = 2.0 * (px * z01.x + py * z01.y) + pz * (n0 - n1);
+            g[0] = half * (px * (z30.x + z21.x) - py * (z30.y - z21.y) + pz * (z20.x - z31.x));
+            g[1] = half * (px * (z30.y + z21.y) + py * (z30.x - z21.x) + pz * (z20.y - z31.y));
+            g[2] = half * (2.0 * (px * z01.x + py * z01.y) + pz * (n0 - n1));
             const double ang = 0.5 * (f.coef * theta[(u64)set * a.nparams + f.param]);
             const double c = cos(ang), s = sin(ang);
             m[0] = make_double2(c, s * pz);
@@ -143,7 +192,18 @@ __global__ __launch_bounds__(64) void k_adj_mats(MatsArgs a, const double* __res
             m[2] = make_double2(-(s * py), s * px);
             m[3] = make_double2(c, -(s * pz));
         }
-        mul2(u, u, m);
+        wide_mul2(ur, ui, m);
+    }
+    // times 2^-(roots / 2), and 1/sqrt(2) for an odd one
+    const double pairs = ldexp(1.0, -(int)(roots / 2));
+    const bool odd = roots & 1u, low = a.low[o];
+    const double rh = odd ? (low ? kRootLow : kRootHigh) : 1.0, rl = odd && !low ? kRootRest : 0.0;
+    double2 u[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const Wide x = wide_mac(wide_mac(Wide{0.0, 0.0}, ur[i], rl), ur[i], rh);
+        const Wide y = wide_mac(wide_mac(Wide{0.0, 0.0}, ui[i], rl), ui[i], rh);
+        u[i] = make_double2(pairs * (x.hi + x.lo), pairs * (y.hi + y.lo));
     }
     double2* uf = pf + a.fwd_at[o];
     double2* ub = pb + a.bwd_at[o];
@@ -453,6 +513,8 @@ __global__ __launch_bounds__(64) void k_adj_grad(const double* __restrict__ sums
 struct Op1 {
     std::vector<Factor> factors;
     bool grad = false;
+    bool given = false;  // has a rotation or a matrix of the caller's
+    u32 roots = 0;       // factors of kind 4
 };
 
 bool unitary2(const cd* m) {
@@ -492,7 +554,9 @@ struct Builder {
         Factor f{};
         f.fixed = (u32)fixed.size();
         for (int i = 0; i < 4; ++i) fixed.push_back(make_double2(m[i].real(), m[i].imag()));
-        open(q).factors.push_back(f);
+        Op1& o = open(q);
+        o.factors.push_back(f);
+        o.given = true;
         if (closed) last[q] = -1;
     }
     void cz(u32 a, u32 b) {
@@ -510,14 +574,17 @@ struct Builder {
         ops.push_back(std::move(h));
         last[a] = last[b] = -1;
     }
-    // H before and after a CZ: the two constants are the neighbours of 1/sqrt(2), whose
-    // product is closer to 1/2 (by 2e-17 relative) than either one's square (1.4e-16), so
-    // that many CNOTs do not change the norm
-    void h(u32 q, bool second) {
-        const double c = second ? 0.70710678118654746 : 0.70710678118654757;
-        const cd m[4] = {c, c, c, -c};
-        put1(q, m);
+    // A matrix of units (1, -1, i, -i and 0), over sqrt(2) if `root`.
+    void put_units(u32 q, const cd (&m)[4], bool root) {
+        Op1& o = open(q);
+        Factor f{};
+        f.kind = root ? 4 : 0;
+        f.fixed = (u32)fixed.size();
+        for (const cd& z : m) fixed.push_back(make_double2(z.real(), z.imag()));
+        o.factors.push_back(f);
+        o.roots += root;
     }
+    void h(u32 q) { put_units(q, {1.0, 1.0, 1.0, -1.0}, true); }
     void rot1(u32 q, u32 pauli, u32 param, double coef) {
         Op1& o = open(q);
         Factor f{};
@@ -527,7 +594,7 @@ struct Builder {
         f.occ = (u32)occ.size();
         occ.push_back(f);
         o.factors.push_back(f);
-        o.grad = true;
+        o.grad = o.given = true;
         ops[last[q]].grad = true;
     }
     // exp(i a P / 2), P a Pauli string on k >= 2 qubits
@@ -535,24 +602,18 @@ struct Builder {
         u32 t = 0;  // the qubit that is rotated: one with an X if there is one, else a Z
         for (u32 j = 0; j < k; ++j)
             if (pauli[j] == 1 || (pauli[t] == 2 && pauli[j] == 3)) t = j;
-        const double c = 0.70710678118654757, d = 0.70710678118654746;
         // basis changes to Z (other qubits) and X (qubit t) and back
         const cd i1(0, 1);
         auto change = [&](u32 j, bool back) {
-            const double r = back ? d : c;
-            const cd h[4] = {r, r, r, -r};
             if (j == t) {
-                if (pauli[j] == 3) put1(q[j], h);
-                if (pauli[j] == 2) {  // diag(1, -i) Y diag(1, i) = X
-                    const cd s[4] = {1.0, 0.0, 0.0, back ? i1 : -i1};
-                    put1(q[j], s);
-                }
+                if (pauli[j] == 3) h(q[j]);
+                if (pauli[j] == 2) put_units(q[j], {1.0, 0.0, 0.0, back ? i1 : -i1}, false);  // diag(1, -i) Y diag(1, i) = X
             } else if (pauli[j] == 1) {
-                put1(q[j], h);
+                h(q[j]);
             } else if (pauli[j] == 2) {
                 // V = (1/sqrt2) [[1, -i], [1, i]]: V Y V^dagger = Z
-                const cd v[4] = {r, -i1 * r, r, i1 * r}, w[4] = {r, r, i1 * r, -i1 * r};
-                put1(q[j], back ? w : v);
+                if (back) put_units(q[j], {1.0, 1.0, i1, -i1}, true);
+                else put_units(q[j], {1.0, -i1, 1.0, i1}, true);
             }
         };
         for (u32 j = 0; j < k; ++j) change(j, false);
@@ -589,13 +650,13 @@ struct qm_adjoint {
     u32 chunk_cols = 0;
     // host tables, uploaded on first use
     std::vector<Factor> factors;
-    std::vector<u32> first, fwd_at, bwd_at, copies, par_first, par_occs, occ_col;
+    std::vector<u32> first, fwd_at, bwd_at, copies, low, par_first, par_occs, occ_col;
     std::vector<double2> fixed, copy_val;
     std::vector<double> occ_coef;
     u32 ncopy_f = 0, ncopy_b = 0;
     int device = -1;
     Factor* d_factors = nullptr;
-    u32 *d_first = nullptr, *d_fwd_at = nullptr, *d_bwd_at = nullptr, *d_copies = nullptr, *d_par_first = nullptr,
+    u32 *d_first = nullptr, *d_fwd_at = nullptr, *d_bwd_at = nullptr, *d_copies = nullptr, *d_low = nullptr, *d_par_first = nullptr,
         *d_par_occs = nullptr, *d_occ_col = nullptr;
     double2 *d_fixed = nullptr, *d_copy_val = nullptr;
     double* d_occ_coef = nullptr;
@@ -622,12 +683,12 @@ struct qm_adjoint {
     void release() {
         if (device >= 0) {
             (void)hipSetDevice(device);
-            void* ptrs[] = {d_factors, d_first, d_fwd_at, d_bwd_at, d_copies, d_par_first, d_par_occs, d_occ_col,
+            void* ptrs[] = {d_factors, d_first, d_fwd_at, d_bwd_at, d_copies, d_low, d_par_first, d_par_occs, d_occ_col,
                             d_fixed, d_copy_val, d_occ_coef, d_fpass, d_bpass, d_fsub, d_bsub};
             for (void* p : ptrs)
                 if (p) (void)hipFree(p);
         }
-        d_factors = nullptr; d_first = nullptr; d_fwd_at = nullptr; d_bwd_at = nullptr; d_copies = nullptr;
+        d_factors = nullptr; d_first = nullptr; d_fwd_at = nullptr; d_bwd_at = nullptr; d_copies = nullptr; d_low = nullptr;
         d_par_first = nullptr; d_par_occs = nullptr; d_occ_col = nullptr; d_fixed = nullptr; d_copy_val = nullptr;
         d_occ_coef = nullptr; d_fpass = nullptr; d_bpass = nullptr; d_fsub = nullptr; d_bsub = nullptr;
         device = -1;
@@ -638,7 +699,7 @@ struct qm_adjoint {
         device = (int)dev;  // release() frees what the uploads below allocate
         const bool ok = put_dev(&d_factors, factors, what) && put_dev(&d_first, first, what) &&
                         put_dev(&d_fwd_at, fwd_at, what) && put_dev(&d_bwd_at, bwd_at, what) &&
-                        put_dev(&d_copies, copies, what) && put_dev(&d_par_first, par_first, what) &&
+                        put_dev(&d_copies, copies, what) && put_dev(&d_low, low, what) && put_dev(&d_par_first, par_first, what) &&
                         put_dev(&d_par_occs, par_occs, what) && put_dev(&d_occ_col, occ_col, what) &&
                         put_dev(&d_fixed, fixed, what) && put_dev(&d_copy_val, copy_val, what) &&
                         put_dev(&d_occ_coef, occ_coef, what) && put_dev(&d_fpass, fwd.passes, what) &&
@@ -697,6 +758,16 @@ void qm_adjoint::build(const Builder& b) {
         factors.insert(factors.end(), o.factors.begin(), o.factors.end());
         first.push_back((u32)factors.size());
     }
+    // Hadamards on their own have the rounded 1/sqrt(2) as it is: each takes the neighbour that
+    // keeps the product of all of them so far nearest to a unitary.
+    low.assign(b.op1.size(), 0);
+    double scale = 0.0;  // log of that product, relative to a unitary
+    const double up = -kRootRest / kRootHigh, down = up - (kRootHigh - kRootLow) / kRootHigh;
+    for (size_t o = 0; o < b.op1.size(); ++o) {
+        if (b.op1[o].given || !(b.op1[o].roots & 1u)) continue;
+        low[o] = std::abs(scale + down) < std::abs(scale + up);
+        scale += low[o] ? down : up;
+    }
     fixed = b.fixed;
     auto place = [&](const Flat& f, std::vector<u32>& at, u32& ncopy) {
         at.assign(b.op1.size(), 0);
@@ -722,7 +793,7 @@ void qm_adjoint::build(const Builder& b) {
     occ_coef.assign(b.occ.size(), 0.0);
     for (size_t o = 0; o < b.op1.size(); ++o)
         for (const Factor& f : b.op1[o].factors)
-            if (f.kind) {
+            if (f.rotation()) {
                 occ_col[f.occ] = col[o];
                 occ_coef[f.occ] = f.coef;
             }
@@ -786,9 +857,9 @@ qm_adjoint* qm_adjoint_create(UINT n, const qm_adjoint_gate* gates, UINT gate_co
             if (ok && in.kind == QM_BATCH_CZ) {
                 b.cz(in.qubits[0], in.qubits[1]);
             } else if (ok && in.kind == QM_BATCH_CNOT) {
-                b.h(in.qubits[1], false);
+                b.h(in.qubits[1]);
                 b.cz(in.qubits[0], in.qubits[1]);
-                b.h(in.qubits[1], true);
+                b.h(in.qubits[1]);
                 need = mask;
             } else if (ok) {
                 const u32 d = 1u << k;
@@ -895,7 +966,7 @@ int qm_adjoint_run(qm_adjoint* a, UINT batch, const double* theta, const ITYPE* 
         if (!dgroups || !dterms) return QM_ERR_HIP;
     }
     MatsArgs ma{a->d_factors, a->d_first, a->d_fixed, a->d_fwd_at, a->d_bwd_at, a->d_copies, a->d_copy_val,
-                a->nops(), a->ncopy_f, a->ncopy_b, a->nparams, a->nocc(), (u32)a->fwd.pool.size(),
+                a->d_low, a->nops(), a->ncopy_f, a->ncopy_b, a->nparams, a->nocc(), (u32)a->fwd.pool.size(),
                 (u32)a->bwd.pool.size()};
     const u32 nmat = a->nops() + a->ncopy_f + a->ncopy_b;
     if (nmat) k_adj_mats<<<dim3((nmat + 63) / 64, batch), 64, 0, st>>>(ma, theta, fpool, bpool, gvec);
