@@ -814,19 +814,8 @@ void* qm_batch_state_device_ptr(qm_batch* b, UINT index) {
 qm_circuit* qm_circuit_create(UINT n, const qm_batch_gate* gates, UINT gate_count, UINT block_qubits,
                               UINT local_qubits) {
     const char* what = "qm_circuit_create";
-    // Defaults (0): 3-qubit blocks and 12-qubit windows (two work-groups per CU).  Against 4-qubit
-    // blocks and 13-qubit windows (one per CU, prefetched), brickwork of 10 layers: 52 / 67 us
-    // at 12 qubits, 83 / 116 at 16, 166 / 191 at 20, 405 / 398 at 22, 1377 / 1654 at 24,
-    // 5.64 / 6.59 ms at 26; QAOA and random circuits alike.  A 13-qubit window only pays where
-    // it saves a stage of a circuit with next to no arithmetic: one layer at 22 qubits 114 / 108 us
-    // (at 20 qubits 37 / 48, at 24 371 / 509), so 20 to 22 qubits with at most one
-    // matrix per qubit keep it.
-    UINT dense = 0;
-    if (gates)
-        for (UINT i = 0; i < gate_count; ++i) dense += gates[i].kind == QM_BATCH_DENSE;
-    const bool wide = n >= 20 && n <= 22 && dense <= n;
-    u32 K = block_qubits ? block_qubits : (wide ? 4 : 3);
-    const u32 lq = local_qubits ? local_qubits : (wide ? kMaxLocal : kTileLocal);
+    u32 K = block_qubits ? block_qubits : 3;
+    u32 lq = local_qubits ? local_qubits : kTileLocal;
     if (n < kMinQubits || n > QM_CIRCUIT_MAX_QUBITS || K < 2 || K > 4 || lq < 8 || lq > kMaxLocal ||
         (gate_count && !gates)) {
         set_error(QM_ERR_INVALID_ARGUMENT,
@@ -852,11 +841,30 @@ qm_circuit* qm_circuit_create(UINT n, const qm_batch_gate* gates, UINT gate_coun
             delete c;
             return nullptr;
         }
+    Flat f;
+    schedule_circuit(f, hc, K, lq);
+    // Defaults (0): 3-qubit blocks and 12-qubit windows (two work-groups per CU).  Against 4-qubit
+    // blocks and 13-qubit windows (one per CU, prefetched), brickwork of 10 layers: 52 / 67 us
+    // at 12 qubits, 83 / 116 at 16, 166 / 191 at 20, 405 / 398 at 22, 1377 / 1654 at 24,
+    // 5.64 / 6.59 ms at 26; QAOA and random circuits alike.  The wider window pays where it saves a
+    // stage, a pass over the state, of a circuit with little arithmetic, taken as two operations a
+    // qubit (a CNOT counts three).  Ten matrices between qubits 3 and 20: one stage instead of two, 46 / 31
+    // us at 20 qubits, 210 / 169 at 24, 3.54 / 2.33 ms at 28; a layer of matrices and CZs at 22: two
+    // instead of three, 118 / 114.  Without a stage saved it loses (that layer at 20: 46 / 57), and so it does
+    // with more arithmetic (four CNOT ladders at 22 saving none 262 / 316, one at 23, three stages to
+    // two, 230 / 250).  Below 20 qubits a state is some tens of tiles and stages cost the same.
+    if (!block_qubits && !local_qubits && n >= 20 && hc.ops.size() <= 2 * n) {
+        Flat wide;
+        schedule_circuit(wide, hc, 4, kMaxLocal);
+        if (wide.stages.size() < f.stages.size()) {
+            f = std::move(wide);
+            K = 4;
+            lq = kMaxLocal;
+        }
+    }
     c->n = n;
     c->K = K;
     c->lq = std::min(n, lq);
-    Flat f;
-    schedule_circuit(f, hc, K, lq);
     c->stages = f.stages;
     c->passes = f.passes;
     c->subs = f.subs;

@@ -61,9 +61,10 @@ def test_fused_circuit_rejects_bad_arguments():
     fc.close()
 
 
-def test_fused_defaults_by_qubit_count():
-    """Width and window 0 pick 3-qubit blocks and 12-qubit windows up to 19
-    qubits, 4 and 13 above; a 4-qubit dense gate widens the default block."""
+def test_fused_defaults():
+    """Width and window 0 pick 3-qubit blocks and 12-qubit windows, and 4 and 13 from 20 qubits on where
+    that saves a stage of a circuit with at most two operations a qubit; a 4-qubit dense gate
+    widens the default block."""
     from qulacs_amd.batch import FusedCircuit
 
     def stats(n, gates, **kw):
@@ -73,11 +74,24 @@ def test_fused_defaults_by_qubit_count():
         finally:
             fc.close()
 
-    for n, (k, lq) in ((8, (3, 12)), (13, (3, 12)), (16, (3, 12)), (19, (3, 12)), (20, (4, 13)), (22, (4, 13))):
-        gates = [("dense", [q], np.eye(2)) for q in range(n)] + [("CZ", [q, q + 1], None) for q in range(n - 1)]
-        assert stats(n, gates) == stats(n, gates, block_qubits=k, local_qubits=lq), n
-    wide = [("dense", [q], np.eye(2)) for q in range(16)] + [("dense", [1, 5, 9, 14], np.eye(16))]
-    assert stats(16, wide) == stats(16, wide, block_qubits=4, local_qubits=12)
+    def layer(n):  # 2 n - 1 operations
+        return [("dense", [q], np.eye(2)) for q in range(n)] + [("CZ", [q, q + 1], None) for q in range(n - 1)]
+
+    def ladder(n):  # 3 n - 3 operations
+        return [("CNOT", [q, q + 1], None) for q in range(n - 1)]
+
+    spread = [("dense", [q], np.eye(2)) for q in (3, 6, 9, 11, 13, 14, 16, 17, 18, 19)]
+    narrow, wide = dict(block_qubits=3, local_qubits=12), dict(block_qubits=4, local_qubits=13)
+    for n, gates, kw in [(8, layer(8), narrow), (13, layer(13), narrow), (16, layer(16), narrow),
+                         (19, spread[:-1], narrow),  # a stage saved, but below 20 qubits
+                         (20, layer(20), narrow), (21, layer(21), narrow),  # no stage saved
+                         (20, spread, wide), (24, spread, wide), (22, layer(22), wide),
+                         (22, 2 * layer(22), narrow), (23, ladder(23), narrow)]:  # too much arithmetic
+        assert stats(n, gates) == stats(n, gates, **kw), (n, len(gates))
+    for n, gates in [(20, spread), (22, layer(22)), (23, ladder(23))]:
+        assert stats(n, gates, **wide)["stages"] < stats(n, gates, **narrow)["stages"]
+    four = [("dense", [q], np.eye(2)) for q in range(16)] + [("dense", [1, 5, 9, 14], np.eye(16))]
+    assert stats(16, four) == stats(16, four, block_qubits=4, local_qubits=12)
 
 
 def test_server_rejects_bad_configuration():
