@@ -401,10 +401,10 @@ typedef struct qm_adjoint_gate {
 typedef struct qm_adjoint qm_adjoint;
 QM_EXPORT qm_adjoint* qm_adjoint_create(UINT qubit_count, const qm_adjoint_gate* gates, UINT gate_count, UINT param_count);
 QM_EXPORT void qm_adjoint_destroy(qm_adjoint* circuit);
-/* Two measures of the gate list: the number of groups it divides into, in order,
- * when the gates of a group act non-diagonally on at most 3 qubits together (0 for
- * states below 3 qubits and when a gate alone needs more), and its gates. */
+/* Passes over tiles that an evaluation runs (register blocks of 3 qubits), and gates. */
 QM_EXPORT void qm_adjoint_stats(const qm_adjoint* circuit, ITYPE* passes, ITYPE* gates);
+/* The same by direction, and stages (launches): the backward ones end with the first rotation. */
+QM_EXPORT void qm_adjoint_schedule(const qm_adjoint* circuit, ITYPE* forward_stages, ITYPE* forward_passes, ITYPE* backward_stages, ITYPE* backward_passes);
 /* Device memory qm_adjoint_run needs for `batch` parameter sets. */
 QM_EXPORT ITYPE qm_adjoint_workspace_bytes(const qm_adjoint* circuit, UINT batch);
 /* theta: device, batch x param_count (row-major); energy: device, batch;

@@ -167,6 +167,7 @@ _SIGS: dict[str, tuple] = {
     "qm_adjoint_destroy": (None, [VP]),
     "qm_adjoint_workspace_bytes": (ITYPE, [VP, UINT]),
     "qm_adjoint_stats": (None, [VP, PI, PI]),
+    "qm_adjoint_schedule": (None, [VP, PI, PI, PI, PI]),
     "qm_adjoint_run": (C.c_int, [VP, UINT, VP, PI, PI, PU, PD, UINT, VP, VP, VP, VP, UINT]),
     "qm_server_create": (VP, [ITYPE, UINT, UINT, UINT]),
     "qm_server_submit": (C.c_longlong, [VP, UINT, C.POINTER(QmBatchGate), UINT, PI, PI, PU, PD, UINT, PD, UINT]),

@@ -57,11 +57,13 @@ class AdjointCircuit:
             raise _lib.QulacsMI355Error("qm_adjoint_create failed")
 
     def stats(self) -> dict:
-        """Groups of gates over at most three non-diagonal qubits, in order (0: none, see
-        qm_adjoint_stats), and gates."""
+        """Gates, passes, and (stages, passes) of the forward and the backward sweep."""
         p, g = C.c_ulonglong(), C.c_ulonglong()
         _lib.call("qm_adjoint_stats", self.h, C.byref(p), C.byref(g))
-        return {"passes": int(p.value), "gates": int(g.value)}
+        v = [C.c_ulonglong() for _ in range(4)]
+        _lib.call("qm_adjoint_schedule", self.h, *[C.byref(x) for x in v])
+        s = [int(x.value) for x in v]
+        return {"passes": int(p.value), "gates": int(g.value), "forward": (s[0], s[1]), "backward": (s[2], s[3])}
 
     def close(self) -> None:
         if self.h:

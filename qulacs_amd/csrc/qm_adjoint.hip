@@ -27,7 +27,7 @@
 // Bound: FP64 issue and LDS round trips.  20 qubits, 12 layers of RY RZ and a CZ chain, 16
 // parameter sets (256 MiB per state array): 42.3 ms with one kernel per 3-qubit register block
 // straight from memory (160 passes at 3.0-3.6 TB/s), 11.3 ms with tiles in the order of the gate
-// list (21 forward and 24 backward stages), 7.5 ms with Picker's 6 and 8 stages.
+// list (21 forward and 24 backward stages), 7.5 ms with Picker's 7 and 8 stages.
 //
 // Layout: `batch` states of 2^max(n, 4) complex128 each, contiguous (state b at
 // b * dim); theta is batch x params (row-major).  Every reduction is a fixed-order
@@ -641,7 +641,7 @@ using namespace qm;
 
 struct qm_adjoint {
     u32 n = 0, ne = 0, nparams = 0, lqf = 0, lqb = 0;
-    u64 ngates = 0, blocks3 = 0;
+    u64 ngates = 0;
     Flat fwd, bwd;
     std::vector<u32> stage_grad0;  // backward stage -> position in bwd.grads of its first operation
     // runs of backward stages whose partial sums share the workspace's columns: the first stage
@@ -805,24 +805,6 @@ void qm_adjoint::build(const Builder& b) {
     for (const Factor& f : b.occ) par_occs[next[f.param]++] = f.occ;  // occurrences in order
 }
 
-namespace {
-// The number of groups that the gate list divides into, in order, when a group's gates act
-// non-diagonally on at most three qubits; 0 if a gate needs more, or below three qubits.
-u64 count_blocks3(u32 n, const std::vector<u64>& needs) {
-    if (n < 3) return 0;
-    u64 groups = 0, blk = 0;
-    for (u64 m : needs) {
-        if (__builtin_popcountll(m) > 3) return 0;
-        if (groups == 0 || __builtin_popcountll(blk | m) > 3) {
-            ++groups;
-            blk = 0;
-        }
-        blk |= m;
-    }
-    return groups;
-}
-}  // namespace
-
 extern "C" {
 
 qm_adjoint* qm_adjoint_create(UINT n, const qm_adjoint_gate* gates, UINT gate_count, UINT nparams) {
@@ -833,21 +815,17 @@ qm_adjoint* qm_adjoint_create(UINT n, const qm_adjoint_gate* gates, UINT gate_co
     }
     const u32 ne = std::max<u32>(n, kMinQubits);
     Builder b(ne);
-    std::vector<u64> needs;  // qubits that each gate acts on non-diagonally
     for (UINT i = 0; i < gate_count; ++i) {
         const qm_adjoint_gate& in = gates[i];
         const u32 k = in.qubit_count;
-        u64 mask = 0, need = 0;
+        u64 mask = 0;
         bool ok = k >= 1 && k <= 4;
         for (u32 j = 0; ok && j < k; ++j) {
             ok = in.qubits[j] < n && !((mask >> in.qubits[j]) & 1);
             mask |= 1ULL << in.qubits[j];
         }
         if (ok && in.kind == QM_ADJ_ROT) {
-            for (u32 j = 0; ok && j < k; ++j) {
-                ok = in.paulis[j] >= 1 && in.paulis[j] <= 3;
-                if (in.paulis[j] != 3) need |= 1ULL << in.qubits[j];
-            }
+            for (u32 j = 0; ok && j < k; ++j) ok = in.paulis[j] >= 1 && in.paulis[j] <= 3;
             ok = ok && in.param < nparams;
             if (ok && k == 1) b.rot1(in.qubits[0], in.paulis[0], in.param, in.coef);
             else if (ok) b.rotation(k, in.qubits, in.paulis, in.param, in.coef);
@@ -860,7 +838,6 @@ qm_adjoint* qm_adjoint_create(UINT n, const qm_adjoint_gate* gates, UINT gate_co
                 b.h(in.qubits[1]);
                 b.cz(in.qubits[0], in.qubits[1]);
                 b.h(in.qubits[1]);
-                need = mask;
             } else if (ok) {
                 const u32 d = 1u << k;
                 std::vector<cd> m((size_t)d * d, 0.0);
@@ -868,7 +845,6 @@ qm_adjoint* qm_adjoint_create(UINT n, const qm_adjoint_gate* gates, UINT gate_co
                     for (u32 c = 0; c < d; ++c) {
                         if (in.kind == QM_BATCH_DENSE) m[r * d + c] = cd(in.matrix[r * d + c].re, in.matrix[r * d + c].im);
                         else if (r == c) m[r * d + c] = cd(in.matrix[r].re, in.matrix[r].im);
-                        if (r != c && m[r * d + c] != cd(0.0)) need = mask;
                     }
                 if (k == 1) b.put1(in.qubits[0], m.data());
                 else b.put2(in.qubits[0], in.qubits[1], m.data());
@@ -878,14 +854,12 @@ qm_adjoint* qm_adjoint_create(UINT n, const qm_adjoint_gate* gates, UINT gate_co
             set_error(QM_ERR_INVALID_ARGUMENT, "%s: gate %u is not a 1..2-qubit fixed gate or a valid rotation", what, i);
             return nullptr;
         }
-        needs.push_back(need);
     }
     auto* a = new qm_adjoint();
     a->n = n;
     a->ne = ne;
     a->nparams = nparams;
     a->ngates = gate_count;
-    a->blocks3 = count_blocks3(n, needs);
     a->build(b);
     return a;
 }
@@ -897,8 +871,24 @@ void qm_adjoint_destroy(qm_adjoint* a) {
 }
 
 void qm_adjoint_stats(const qm_adjoint* a, ITYPE* passes, ITYPE* gates) {
-    if (passes) *passes = a ? (ITYPE)a->blocks3 : 0;
+    ITYPE fs, fp, bs, bp;
+    qm_adjoint_schedule(a, &fs, &fp, &bs, &bp);
+    if (passes) *passes = fp + bp;
     if (gates) *gates = a ? (ITYPE)a->ngates : 0;
+}
+
+void qm_adjoint_schedule(const qm_adjoint* a, ITYPE* fwd_stages, ITYPE* fwd_passes, ITYPE* bwd_stages,
+                         ITYPE* bwd_passes) {
+    ITYPE fs = 0, fp = 0, bs = 0, bp = 0;
+    if (a) {
+        fs = a->fwd.stages.size();
+        fp = a->fwd.passes.size();
+        for (; bs < a->bwd.stages.size() && a->stage_grad0[bs] < a->ncols() / 3; ++bs) bp += a->bwd.stages[bs].npass;
+    }
+    if (fwd_stages) *fwd_stages = fs;
+    if (fwd_passes) *fwd_passes = fp;
+    if (bwd_stages) *bwd_stages = bs;
+    if (bwd_passes) *bwd_passes = bp;
 }
 
 ITYPE qm_adjoint_workspace_bytes(const qm_adjoint* a, UINT batch) {

@@ -182,19 +182,21 @@ def test_autotune_times_each_program_once(monkeypatch, windows, run):
 
 
 def test_adjoint_pass_plan():
-    """The adjoint groups gates into passes over 3-qubit register blocks (host
-    planning, no device work): the 20-qubit, 12-layer hardware-efficient ansatz
-    (480 rotations + 228 CZ) needs about one pass per three qubits per layer, a
-    rotation with four X/Y qubits keeps one kernel per gate, and so does a state
-    below three qubits."""
+    """Stages (launches) and passes of the adjoint's sweeps, planned on the host: the 20-qubit, 12-layer
+    hardware-efficient ansatz (480 rotations, two merged per qubit and layer, 228 CZ) runs in 7
+    forward and 8 backward stages of some 6 passes; a Pauli string is one rotation between CZ gates,
+    and what stands before the first rotation is not swept backwards."""
     pytest.importorskip("torch")
     from qulacs_amd.adjoint import AdjointCircuit, hardware_efficient_ansatz
 
     gates, P = hardware_efficient_ansatz(20, 12)
     st = AdjointCircuit(20, gates, P).stats()
-    assert st["gates"] == 708 and 80 <= st["passes"] <= 84, st
+    assert st["gates"] == 708 and st["passes"] == st["forward"][1] + st["backward"][1]
+    assert st["forward"][0] <= 7 and st["forward"][1] <= 47, st
+    assert st["backward"][0] <= 8 and st["backward"][1] <= 49, st
     wide = AdjointCircuit(6, [("rot", [0, 1, 2, 3], [1, 2, 1, 1], 0, 1.0)], 1).stats()
-    assert wide["passes"] == 0 and wide["gates"] == 1
+    assert wide == {"passes": 6, "gates": 1, "forward": (1, 3), "backward": (1, 3)}
     zrot = AdjointCircuit(6, [("rot", [0, 1, 2, 3], [3, 3, 3, 3], 0, 1.0), ("CZ", [0, 5], None)], 1).stats()
-    assert zrot["passes"] == 1
-    assert AdjointCircuit(2, [("rot", [0], [2], 0, 1.0)], 1).stats()["passes"] == 0
+    assert zrot["forward"] == zrot["backward"] == (1, 1)
+    fixed = AdjointCircuit(14, [("CNOT", [q, q + 1], None) for q in range(13)], 0).stats()
+    assert fixed["forward"][0] >= 2 and fixed["backward"] == (0, 0)
