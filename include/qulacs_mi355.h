@@ -372,8 +372,8 @@ QM_EXPORT void qm_batch_stats(const qm_batch* batch, ITYPE* circuits, ITYPE* sta
 typedef struct qm_circuit qm_circuit;
 /* block_qubits 2..4, local_qubits 8..13; 0 picks: 3 and 12, the width grown to the
  * largest dense gate (at most 4 qubits); both 0: 4 and 13 from 20 qubits on where that
- * takes fewer stages and the circuit has at most two operations a qubit, CNOTs counted as
- * CZ between Hadamards.  NULL on error. */
+ * takes fewer stages and the circuit has at most two single-qubit operations a qubit, CNOTs
+ * counted as CZ between Hadamards, a matrix on k qubits as 2^(k-1).  NULL on error. */
 QM_EXPORT qm_circuit* qm_circuit_create(UINT qubit_count, const qm_batch_gate* gates, UINT gate_count, UINT block_qubits, UINT local_qubits);
 QM_EXPORT void qm_circuit_destroy(qm_circuit* circuit);
 /* Applies the circuit to `state` (dim = 2^qubit_count) in stream order. */

@@ -850,13 +850,15 @@ qm_circuit* qm_circuit_create(UINT n, const qm_batch_gate* gates, UINT gate_coun
     // blocks and 13-qubit windows (one per CU, prefetched), brickwork of 10 layers: 52 / 67 us
     // at 12 qubits, 83 / 116 at 16, 166 / 191 at 20, 405 / 398 at 22, 1377 / 1654 at 24,
     // 5.64 / 6.59 ms at 26; QAOA and random circuits alike.  The wider window pays where it saves a
-    // stage, a pass over the state, of a circuit with little arithmetic, taken as two operations a
-    // qubit (a CNOT counts three).  Ten matrices between qubits 3 and 20: one stage instead of two, 46 / 31
+    // stage, a pass over the state, of a circuit with little arithmetic, taken as two single-qubit
+    // operations a qubit (a CNOT counts three, a matrix on k qubits 2^(k-1)).  Ten matrices between qubits 3 and 20: one stage instead of two, 46 / 31
     // us at 20 qubits, 210 / 169 at 24, 3.54 / 2.33 ms at 28; a layer of matrices and CZs at 22: two
     // instead of three, 118 / 114.  Without a stage saved it loses (that layer at 20: 46 / 57), and so it does
     // with more arithmetic (four CNOT ladders at 22 saving none 262 / 316, one at 23, three stages to
-    // two, 230 / 250).  Below 20 qubits a state is some tens of tiles and stages cost the same.
-    if (!block_qubits && !local_qubits && n >= 20 && hc.ops.size() <= 2 * n) {
+    // two, 230 / 250; 24 three-qubit unitaries on a 12-qubit density matrix 1.52 / 3.15 ms).  Below 20 qubits a state is some tens of tiles and stages cost the same.
+    u64 work = 0;  // multiply-adds per amplitude, in those of a single-qubit matrix
+    for (const HOp& o : hc.ops) work += o.type == 0 ? 1u << (o.q.size() - 1) : o.type == 4 ? o.q.size() : 1u;
+    if (!block_qubits && !local_qubits && n >= 20 && work <= 2 * n) {
         Flat wide;
         schedule_circuit(wide, hc, 4, kMaxLocal);
         if (wide.stages.size() < f.stages.size()) {

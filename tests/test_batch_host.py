@@ -86,7 +86,8 @@ def test_fused_defaults():
                          (19, spread[:-1], narrow),  # a stage saved, but below 20 qubits
                          (20, layer(20), narrow), (21, layer(21), narrow),  # no stage saved
                          (20, spread, wide), (24, spread, wide), (22, layer(22), wide),
-                         (22, 2 * layer(22), narrow), (23, ladder(23), narrow)]:  # too much arithmetic
+                         (22, 2 * layer(22), narrow), (23, ladder(23), narrow),  # too much arithmetic
+                         (24, [("dense", [q, q + 1, q + 2], np.eye(8)) for q in range(20)], narrow)]:
         assert stats(n, gates) == stats(n, gates, **kw), (n, len(gates))
     for n, gates in [(20, spread), (22, layer(22)), (23, ladder(23))]:
         assert stats(n, gates, **wide)["stages"] < stats(n, gates, **narrow)["stages"]
