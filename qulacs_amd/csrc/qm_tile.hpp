@@ -1176,33 +1176,35 @@ struct Converter {
             }
         }
         bool unit = true;
-        for (u32 i = 0; i < d && unit; ++i) unit = std::abs(std::abs(m[i]) - 1.0) < 1e-14;
+        for (u32 i = 0; i < d && unit; ++i) unit = std::abs(std::norm(m[i]) - 1.0L) < 2e-14L;
         if (unit) {
             // log m_i = sum_s (-1)^popcount(i & s) (rho[s] + i phi[s]) / d.  What a double's rounding
             // leaves of the moduli (2^-53) may go; more of it is kept: rho of all and of single
             // qubits in the phases that wait, of more qubits by leaving the gate a DIAG.
             long double phi[16], rho[16];
-            for (u32 i = 0; i < d; ++i) {
-                phi[i] = std::arg(m[i]);
-                rho[i] = std::log(std::abs(m[i]));
-            }
-            for (u32 h = 1; h < d; h <<= 1)
-                for (u32 i = 0; i < d; ++i)
-                    if (!(i & h))
-                        for (long double* x : {phi, rho}) {
+            auto transform = [&](long double* x) {
+                for (u32 h = 1; h < d; h <<= 1)
+                    for (u32 i = 0; i < d; ++i)
+                        if (!(i & h)) {
                             const long double a = x[i], b = x[i | h];
                             x[i] = a + b;
                             x[i | h] = a - b;
                         }
+            };
+            for (u32 i = 0; i < d; ++i) phi[i] = std::arg(m[i]);
+            transform(phi);
             u32 many = 0;
-            bool kept = true;
-            for (u32 s = 0; s < d; ++s) {
-                if (std::abs(rho[s]) <= d * 0x1p-53L) rho[s] = 0.0L;
-                if (!(s & (s - 1))) continue;
-                many += std::abs(phi[s]) > 1e-15;
-                kept = kept && rho[s] == 0.0L;
+            for (u32 s = 1; s < d; ++s) many += (s & (s - 1)) && std::abs(phi[s]) > 1e-15;
+            bool kept = many <= 2;
+            if (kept) {
+                for (u32 i = 0; i < d; ++i) rho[i] = 0.5L * (std::norm(m[i]) - 1.0L);  // log |m_i| up to 1e-28
+                transform(rho);
+                for (u32 s = 0; s < d; ++s) {
+                    if (std::abs(rho[s]) <= d * 0x1p-53L) rho[s] = 0.0L;
+                    kept = kept && (rho[s] == 0.0L || !(s & (s - 1)));
+                }
             }
-            if (many <= 2 && kept) {
+            if (kept) {
                 const cx g = std::polar(std::exp(rho[0] / d), phi[0] / d);
                 phase(q[0], g, g);
                 for (u32 s = 1; s < d; ++s) {
