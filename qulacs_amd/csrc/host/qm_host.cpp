@@ -72,13 +72,21 @@ ComplexMatrix embed(const ComplexMatrix& m, const std::vector<unsigned>& targets
 }
 
 // S = sum_i w_i K_i (x) conj(K_i); member = row bits * 2^k + column bits.
+// Zeros are skipped unless something is not finite: most Kraus operators are Pauli strings.
 void accumulate_superop(ComplexMatrix& S, const ComplexMatrix& K, double w) {
     const size_t d = K.rows;
+    bool finite = std::isfinite(w);
+    for (const auto& z : K.data) finite = finite && std::isfinite(z.real()) && std::isfinite(z.imag());
     for (size_t oy = 0; oy < d; ++oy)
-        for (size_t ox = 0; ox < d; ++ox)
-            for (size_t iy = 0; iy < d; ++iy)
-                for (size_t ix = 0; ix < d; ++ix)
-                    S(oy * d + ox, iy * d + ix) += w * K(oy, iy) * std::conj(K(ox, ix));
+        for (size_t iy = 0; iy < d; ++iy) {
+            const CPPCTYPE a = w * K(oy, iy);
+            if (finite && a == CPPCTYPE(0.0)) continue;
+            for (size_t ox = 0; ox < d; ++ox)
+                for (size_t ix = 0; ix < d; ++ix) {
+                    const CPPCTYPE b = std::conj(K(ox, ix));
+                    if (!finite || b != CPPCTYPE(0.0)) S(oy * d + ox, iy * d + ix) += a * b;
+                }
+        }
 }
 
 std::vector<unsigned> sorted_union(const std::vector<std::vector<unsigned>>& lists) {
@@ -1898,6 +1906,10 @@ struct DmLowering {
     std::vector<qm_batch_gate> gates;
     std::deque<std::vector<qm_complex>> store;
     std::vector<Pend> pend;
+    // the last superoperator on two qubits, if nothing was put behind it (gates.size() == pair_end)
+    ComplexMatrix pair_S;
+    std::vector<unsigned> pair_q;
+    size_t pair_end = 0;
     explicit DmLowering(unsigned qubits) : n(qubits), pend(qubits) {}
 
     void put(UINT kind, const std::vector<unsigned>& q, std::vector<qm_complex> m) {
@@ -1977,6 +1989,20 @@ struct DmLowering {
         }
         p.S = S * p.S;
     }
+    // A channel on two qubits.  In a row on one pair they are one superoperator: 24 on 2 qubits took
+    // 495 us on their first use as 24 operations, 165 as one.
+    __attribute__((noinline)) void pair_channel(const ComplexMatrix& S, const std::vector<unsigned>& q) {
+        if (!gates.empty() && gates.size() == pair_end && pair_q == q) {
+            pair_S = S * pair_S;
+            gates.pop_back();
+            store.pop_back();
+        } else {
+            pair_S = S;
+            pair_q = q;
+        }
+        put_matrix(pair_S, {q[0], q[1], q[0] + n, q[1] + n}, false);
+        pair_end = gates.size();
+    }
     // Superoperator of uniform depolarizing on q.size() qubits: the factor of the traceless part.
     static bool depolarizing(const ComplexMatrix& S, size_t qubits, double* keep) {
         const size_t d = size_t(1) << qubits;
@@ -2048,7 +2074,7 @@ struct DmLowering {
             return true;
         }
         for (unsigned t : q) flush(t);
-        put_matrix(S, {q[0], q[1], q[0] + n, q[1] + n}, false);
+        pair_channel(S, q);
         return true;
     }
     void finish() {

@@ -29,6 +29,7 @@ pytestmark = pytest.mark.gpu
 def _circuit(rng, n, count, style):
     c = q.QuantumCircuit(n)
     kinds = {"depol": ["u", "h", "rz", "cnot", "cz", "d1", "d2", "d1"],
+             "pairs": ["prob2", "prob2", "prob2", "u", "d2", "ad"],  # runs of channels on one pair
              "noise": ["u", "cnot", "d1", "ad", "deph", "bf", "xz", "rx"],
              "all": ["u", "h", "s", "t", "x", "sy", "rz", "cnot", "cz", "swap", "d1", "d2", "ad", "deph", "bf", "xz", "u2", "diag2",
                      "cu", "toffoli", "p0", "prob2", "rot", "id", "u3", "wide"]}[style]
@@ -95,7 +96,7 @@ def _run(c, n, rho, fused):
         q.set_circuit_fusion(True)
 
 
-@pytest.mark.parametrize("n,count,style", [(1, 12, "all"), (2, 7, "depol"), (2, 40, "depol"), (2, 40, "all"), (3, 60, "all"), (4, 80, "noise"),
+@pytest.mark.parametrize("n,count,style", [(2, 30, "pairs"), (3, 60, "pairs"), (1, 12, "all"), (2, 7, "depol"), (2, 40, "depol"), (2, 40, "all"), (3, 60, "all"), (4, 80, "noise"),
                                            (5, 120, "depol"), (5, 120, "all"), (6, 150, "noise"), (6, 150, "all"), (7, 200, "depol"),
                                            (7, 160, "all"), (8, 120, "depol"), (11, 30, "all")])
 def test_noisy_circuit(n, count, style):
