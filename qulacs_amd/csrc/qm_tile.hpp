@@ -730,11 +730,13 @@ struct Picker {
     };
     std::vector<Item> items;
     std::vector<u32> rest;  // what is left, in order
+    u64 left = 0;           // its dense work
 
     static u32 weight_of(const HOp& o) { return o.type == 0 ? 1u << (o.q.size() - 1) : o.type == 4 ? 1u : 0u; }
     void add(const HOp& o) {
         rest.push_back((u32)items.size());
         items.push_back({o.mask(), weight_of(o), o.grad});
+        left += items.back().weight;
     }
     // Scans with window w (grown up to `most` qubits if `grow`); returns the dense work taken.
     u64 scan(u64& w, bool grow, u32 most, size_t max_grads, std::vector<u32>* sel) const {
@@ -774,7 +776,8 @@ struct Picker {
         u64 work = scan(best, true, most, max_grads, nullptr);
         const u32 f = most - low;
         bool grow = true;
-        for (u32 s = low; s + f <= n; ++s) {
+        // (a window that takes all there is cannot be beaten)
+        for (u32 s = low; s + f <= n && work < left; ++s) {
             u64 w = fixed | (((1ULL << f) - 1) << s);
             const u64 c = scan(w, false, most, max_grads, nullptr);
             if (c > work) {
@@ -783,7 +786,7 @@ struct Picker {
                 grow = false;
             }
         }
-        for (u32 s = 0; paired && s < n / 2; ++s) {
+        for (u32 s = 0; paired && s < n / 2 && work < left; ++s) {
             u64 w = fixed;
             for (u32 q = s; q < n / 2; ++q) {
                 const u64 m = w | (1ULL << q) | (1ULL << (q + n / 2));
@@ -812,8 +815,12 @@ struct Picker {
     void take(const std::vector<u32>& sel) {  // sel is ascending in `rest` order
         size_t k = 0, out = 0;
         for (size_t i = 0; i < rest.size(); ++i) {
-            if (k < sel.size() && rest[i] == sel[k]) ++k;
-            else rest[out++] = rest[i];
+            if (k < sel.size() && rest[i] == sel[k]) {
+                left -= items[rest[i]].weight;
+                ++k;
+            } else {
+                rest[out++] = rest[i];
+            }
         }
         rest.resize(out);
     }
