@@ -525,7 +525,8 @@ def many_small(args, lib_mod, hip):
     out = {
         "circuits": len(cs), "qubits": "U{8..16}", "layers": "U{4..12}", "gates": total_gates,
         "ms_per_step": round(ms, 3), "circuits_per_s": round(len(cs) / (ms * 1e-3), 1),
-        "fp64": {"bound": "fp64-valu", "achieved": round(flops / (ms * 1e-3) / 1e12, 2), "peak": FP64_PEAK_TFLOPS,
+        # nominal: whole matrices; most are applied as shears, with half the flops
+        "fp64": {"bound": "fp64-valu", "work": "nominal", "achieved": round(flops / (ms * 1e-3) / 1e12, 2), "peak": FP64_PEAK_TFLOPS,
                  "unit": "TFLOP/s", "frac": round(flops / (ms * 1e-3) / 1e12 / FP64_PEAK_TFLOPS, 4),
                  "flops_per_step": flops},
         "graph_ms_per_step": round(graph_ms, 3), "graph_matches_eager": graph_same,
@@ -546,9 +547,10 @@ def fused_large(args, lib_mod, hip):
     (default 26 qubits, 40 layers: a Haar 2x2 on every qubit, then a CNOT brick) from |0>,
     at register-block widths 3 and 4 with the default 12-qubit window, timed with HIP events on the
     launch stream (best of three runs after a warm-up).  Reports the stage count, the state
-    traffic (2 x 16 B x 2^n per stage) and the FP64 rate of the fused arithmetic (one 2x2
-    complex matrix per qubit per layer: 16 flops per amplitude) against the 78.6 TFLOP/s
-    vector peak; the two widths must agree (|<psi_3|psi_4>| within 1e-10 of 1)."""
+    traffic (2 x 16 B x 2^n per stage) and the nominal FP64 rate: one whole 2x2 complex matrix per
+    qubit per layer, 16 flops per amplitude, over the time.  The executor applies most matrices as
+    two shears, half of that, so this is a rate of work done for the caller and no share of the
+    78.6 TFLOP/s vector peak; the two widths must agree (|<psi_3|psi_4>| within 1e-10 of 1)."""
     from qulacs_amd.batch import FusedCircuit
     from qulacs_amd.workloads import brickwork_circuit
 
@@ -581,7 +583,7 @@ def fused_large(args, lib_mod, hip):
         stats = fc.stats()
         traffic = stats["stages"] * 2.0 * 16 * dim
         out[f"K{K}"] = {"ms": round(best, 2), **stats, "state_traffic_GBps": round(traffic / best / 1e6, 1),
-                        "fp64_TFLOPs": round(flops / best / 1e9, 2), "fp64_frac_of_peak": round(flops / best / 1e9 / 78.6, 4)}
+                        "nominal_fp64_TFLOPs": round(flops / best / 1e9, 2)}
         states[K] = st
         fc.close()
     lib_mod.call("qm_set_synchronous", 1)

@@ -720,7 +720,8 @@ u32 pool_put(Flat& f, const std::vector<cx>& m) {
 // window block nothing: they commute with what is taken.  Candidates: the window that grows
 // in scan order (any circuit), and every run of adjacent qubits (chains and grids, where the
 // order of the gate list would spread the window over the register and leave each stage a few
-// layers: 26-qubit brickwork, 20 layers: 26 -> 8 stages; 20-qubit ansatz: 25 -> 8).
+// layers: 26-qubit brickwork, 20 layers, 12-qubit windows: 9 stages, 26 in list
+// order with 13; 20-qubit ansatz backward: 24 -> 8).
 // The one with the most dense work wins.
 struct Picker {
     struct Item {

@@ -202,8 +202,8 @@ def many_small_circuits(count: int = 4096, seed: int = 3003, n_range=(8, 16), la
 
 
 def small_circuit_alg_flops(c: SmallCircuit) -> float:
-    """FP64 flops of the fused form: one 2x2 complex matrix per qubit per layer
-    (8 real multiply-adds = 16 flops per amplitude)."""
+    """Nominal FP64 flops: one whole 2x2 complex matrix per qubit per layer (8 real
+    multiply-adds = 16 flops per amplitude)."""
     return 16.0 * c.layers * c.n * (1 << c.n)
 
 
